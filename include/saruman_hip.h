@@ -142,7 +142,7 @@ extern float alignment_time[2];                    /* cuda-functions.cu:61 (ms, 
 
 /* kernel selection for srm_job_run */
 #define SRM_KERNEL_AUTO 0    /* banded where eligible, plain otherwise */
-#define SRM_KERNEL_PLAIN 1   /* one alignment per thread, full int16 matrix */
+#define SRM_KERNEL_PLAIN 1   /* the full matrix of every candidate */
 #define SRM_KERNEL_BANDED 2  /* persistent banded kernel (ineligible candidates -> plain) */
 
 /* srm_cand.bits */

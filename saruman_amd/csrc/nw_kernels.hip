@@ -2,9 +2,11 @@
 // traceback (the work of compute_score/get_alignment, src/cuda-functions.cu:76-536).
 //
 // The kernels here compute the same results:
+//   plain_wave_kernel  one candidate per wave, the full matrix a row and a column
+//                 strip at a time in registers, a 2-bit traceback decision per cell
+//                 in HBM.  Any candidate (raw-byte or 2-bit sequences), small costs.
 //   plain_kernel  one candidate per thread, full (w+1)x(L+1) int16 matrix in HBM,
-//                 value-based traceback on that matrix.  Handles every candidate
-//                 (any match/mismatch, raw-byte or 2-bit sequences).
+//                 value-based traceback on that matrix.  Any costs.
 //   band_kernel   persistent: each wave pulls 64-candidate tiles from a device queue;
 //   trace_kernel  one candidate per lane; the exact k-error band of a DP column
 //                 (d = row - col in [-k, max(2s+k, w-L)]) lives in VGPRs, saturated
@@ -126,6 +128,215 @@ __global__ __launch_bounds__(256) void plain_kernel(PlainArgs a)
         r.end_col = (uint16_t)col;
     }
     a.res[t] = r;
+}
+
+// ---------------------------------------------------------------------------
+// plain kernel, one wave per candidate
+// ---------------------------------------------------------------------------
+// The same matrix and decisions with the wave's lanes side by side on one
+// candidate.  Lane l holds columns l*C+1 .. l*C+C (C = ceil(L / 64), at most 4: a
+// longer read goes in strips of 256 columns, each strip's last column kept for the
+// next one) and is one row behind lane l - 1: at step t it fills row t - l + 1 from
+// its own row before and from the value its left neighbour's last column had one
+// step earlier, which a lane shift hands over together with the row's window
+// character.  A cell's
+// traceback decision needs only the values at hand when the cell is filled, so the
+// matrix itself is never stored: 2 bits per cell, the decision, 16 steps to a word
+// (word (t >> 4, column), every lane storing its words at the same step).  The walk
+// then looks 64 diagonal cells ahead at once, one per lane, and takes the run of
+// diagonal decisions in one go.
+//
+// Bound by the steps' serial chain while a launch holds few candidates, by VALU
+// issue otherwise; one thread per candidate instead waits for a matrix load and a
+// store per cell.  50,000 reads of 36-250 bp, 3% of them with an N (about 1,300
+// candidates here): 24.0 -> 0.158 ms; every candidate of 2,000,000 reads of 50-250
+// bp: 1,893 -> 55.7 ms a step.
+//
+// Costs within +-PLAIN_WAVE_COST only: no value of a matrix of up to 900 x 1000
+// cells then leaves 16 bits or meets the row -1 / column -1 sentinels, so nothing
+// wraps and row 0 and column 0 have closed forms; other costs keep the
+// thread-per-candidate kernel, whose int16 matrix wraps as the reference's does.
+constexpr int PLAIN_WAVE_COST = 15;
+
+template <bool CODES, int C>
+__device__ __forceinline__ void plain_wave(const PlainArgs &a, const srm_cand &cd, uint32_t t_cand,
+                                           uint32_t *__restrict__ W)
+{
+    constexpr int SC = 64 * C;             // columns of a strip
+    const int lane = threadIdx.x & 63;
+    const int L = cd.L, w = cd.w, k = cd.k;
+    const int s = flag_s(cd.flag, k), e = flag_e(cd.flag, k);
+    const int ma = a.ma, mm = a.mm;
+    const SeqRef<CODES> rd{a.read_words, a.read_bytes, (int64_t)cd.read_off};
+    const SeqRef<CODES> wn{a.win_words, a.win_bytes, (int64_t)cd.win_off};
+    // decision word (t >> 4, column) of strip b at (b * SC) * T + (t >> 4) * (its
+    // columns) + column - b * SC, T words of steps; after them, a value per row of
+    // the column between two strips
+    const int T = (w + 78) >> 4;
+    int *__restrict__ edge = (int *)(W + (size_t)T * L);
+    int score = L;
+    for (int b0 = 0; b0 < L; b0 += SC) {
+        const int Ls = imin(L - b0, SC);       // the strip's columns b0 + 1 .. b0 + Ls
+        const int nl = (Ls + C - 1) / C;       // lanes with columns
+        const int c0 = b0 + lane * C;          // columns c0 + 1 .. c0 + C
+        const bool more = b0 + Ls < L;
+        uint32_t *__restrict__ Wb = W + (size_t)T * b0;
+        int v[C], rc[C];
+        uint32_t acc[C];
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            v[j] = c0 + j + 1;                 // row 0
+            rc[j] = c0 + j < L ? rd.at(c0 + j) : 0;
+            acc[j] = 0u;
+        }
+        int before = c0;                       // column c0 in the row above
+        int last = 0, g = 0, gbuf = 0, ebuf = 0;
+        const int steps = w > 0 ? w + nl - 1 : 0;
+        for (int t = 0; t < steps; ++t) {
+            if ((t & 63) == 0) {
+                gbuf = t + lane < w ? wn.at(t + lane) : 0;
+                // the strip's left column: column 0, max(0, row - 2s), or the strip
+                // before's last (row t + lane + 1; this strip's last column is
+                // stored over it 63 steps later)
+                if (b0 == 0) ebuf = imax(t + lane + 1 - 2 * s, 0);
+                else if (t + lane < w) ebuf = edge[t + lane];
+            }
+            // this step's left column value and window character from the left lane;
+            // lane 0 takes the strip's left column and the next character
+            const int gin = __builtin_amdgcn_readlane(gbuf, t & 63);
+            const int ein = __builtin_amdgcn_readlane(ebuf, t & 63);
+            int left = __builtin_amdgcn_update_dpp(ein, last, 0x138, 0xF, 0xF, false);
+            g = __builtin_amdgcn_update_dpp(gin, g, 0x138, 0xF, 0xF, false);
+            const int row = t - lane + 1;
+            const uint32_t sh = 2u * (uint32_t)(t & 15);
+            if (row >= 1 && row <= w) {
+                int diag = before;
+                before = left;
+                const int tlast = row - 1 >= w - 2 * e ? 0 : mm;   // column L's top move
+                const bool start = c0 == 0 && s && row - 1 <= 2 * (s + 1);
+#pragma unroll
+                for (int j = 0; j < C; ++j) {
+                    const int top = v[j];
+                    const bool eq = g == rc[j];
+                    const int lf = left + mm;
+                    const int tp = top + (c0 + j == L - 1 ? tlast : mm);
+                    const int m = imin(imin(diag + (eq ? ma : mm), lf), tp);
+                    // decide(): in column 1 the walk's top move is free on the first rows
+                    const int td = j == 0 && start ? top : tp;
+                    const bool dg = diag + mm == m || (eq && diag + ma == m);
+                    const uint32_t op = dg ? 0u : td == m ? 1u : lf == m ? 2u : 3u;
+                    acc[j] |= op << sh;
+                    diag = top;
+                    v[j] = m;
+                    left = m;
+                }
+                last = v[C - 1];
+                if (row == w) {
+#pragma unroll
+                    for (int j = 0; j < C; ++j)
+                        if (c0 + j == L - 1) score = v[j];
+                }
+                if (more && lane == 63) edge[row - 1] = last;
+            }
+            if ((t & 15) == 15 || t == steps - 1) {
+#pragma unroll
+                for (int j = 0; j < C; ++j) {
+                    if (c0 + j < L) Wb[(size_t)(t >> 4) * Ls + lane * C + j] = acc[j];
+                    acc[j] = 0u;
+                }
+            }
+        }
+        // the words and the edge column are read by other lanes
+        __threadfence_block();
+    }
+    score = __builtin_amdgcn_readlane(score, ((L - 1) % SC) / C);   // the lane of column L
+    int row = w, col = L, n = 0;
+    if (score <= k) {                                                    // :504
+        const bool stop_row0 = (cd.bits & SRM_CAND_STOP_ROW0) != 0;
+        uint32_t *__restrict__ ops = a.ops + cd.ops_off;
+        const int cap = w + k;
+        uint32_t opw = 0;
+        // count equal decisions op, all over the wave alike; lane 0 stores the words
+        auto emit = [&](uint32_t op, int count) {
+            while (count > 0) {
+                const int c = imin(count, 16 - (n & 15));
+                const uint32_t f = c == 16 ? 0x55555555u : (1u << (2 * c)) / 3u;
+                opw |= (op * f) << (2 * (n & 15));
+                n += c;
+                count -= c;
+                if ((n & 15) == 0) {
+                    if (lane == 0) ops[(n >> 4) - 1] = opw;
+                    opw = 0;
+                }
+            }
+        };
+        while (!(stop_row0 && row == 0)) {                               // Q1
+            if (col == 0) {
+                // column 0: a top move or the stop
+                if (row == 0 || n >= cap) break;
+                const int vv = imax(row - 2 * s, 0), tp = imax(row - 1 - 2 * s, 0);
+                if (decide(ma, mm, vv, SRM_COL0, SRM_COL0, tp, 0, row - 1, L, w, s, e, false) != 1)
+                    break;
+                emit(1u, 1);
+                --row;
+                continue;
+            }
+            if (row == 0) {
+                // M[0][c] = c: left moves when a gap costs 1, else the stop
+                const int c = mm == 1 ? imin(col, cap - n) : 0;
+                emit(2u, c);
+                col -= c;
+                if (c == 0 || n >= cap) break;
+                continue;
+            }
+            const int r1 = row - lane, c1 = col - lane;
+            const bool in = r1 >= 1 && c1 >= 1;
+            uint32_t op = 3u;
+            if (in) {
+                const int b0 = (c1 - 1) / SC * SC, x = c1 - 1 - b0;
+                const int t = r1 - 1 + x / C;
+                op = (W[(size_t)T * b0 + (size_t)(t >> 4) * imin(L - b0, SC) + x] >> (2 * (t & 15))) & 3u;
+            }
+            const uint64_t off_run = ~__ballot(in && op == 0u);
+            const int run = off_run ? (int)__builtin_ctzll(off_run) : 64;
+            const int c = imin(run, cap - n);
+            emit(0u, c);
+            row -= c;
+            col -= c;
+            if (n >= cap) break;
+            if (run == 64 || row == 0 || col == 0) continue;
+            const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)op, run);
+            if (o == 3u) break;
+            emit(o, 1);
+            row -= o != 2u;
+            col -= o != 1u;
+        }
+        if ((n & 15) && lane == 0) ops[n >> 4] = opw;
+    }
+    if (lane == 0) {
+        srm_result r;
+        r.score = (int16_t)score;
+        r.n_ops = (uint16_t)n;
+        r.end_row = (uint16_t)row;
+        r.end_col = (uint16_t)col;
+        a.res[t_cand] = r;
+    }
+}
+
+// a block's 4 waves take a candidate each; C is the same over a wave
+template <bool CODES>
+__global__ __launch_bounds__(256) void plain_wave_kernel(PlainArgs a)
+{
+    const int j = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+    if (j >= a.n) return;
+    const uint32_t t = a.idx[j];
+    const srm_cand cd = a.cand[t];
+    uint32_t *W = (uint32_t *)(a.mat + a.mat_off[j]);
+    const int L = __builtin_amdgcn_readfirstlane((int)cd.L);
+    if (L <= 64) plain_wave<CODES, 1>(a, cd, t, W);
+    else if (L <= 128) plain_wave<CODES, 2>(a, cd, t, W);
+    else if (L <= 192) plain_wave<CODES, 3>(a, cd, t, W);
+    else plain_wave<CODES, 4>(a, cd, t, W);
 }
 
 // ---------------------------------------------------------------------------
@@ -574,8 +785,14 @@ __global__ void reset_counters(uint32_t *c, int n)
 hipError_t launch_plain(const PlainArgs &a, bool codes, hipStream_t st)
 {
     if (a.n <= 0) return hipSuccess;
-    dim3 block(256), grid((a.n + 255) / 256);
-    if (codes)
+    const bool wave = a.ma >= -PLAIN_WAVE_COST && a.ma <= PLAIN_WAVE_COST &&
+                      a.mm >= -PLAIN_WAVE_COST && a.mm <= PLAIN_WAVE_COST;
+    dim3 block(256), grid(wave ? ((unsigned)a.n + 3u) / 4u : ((unsigned)a.n + 255u) / 256u);
+    if (wave && codes)
+        hipLaunchKernelGGL(plain_wave_kernel<true>, grid, block, 0, st, a);
+    else if (wave)
+        hipLaunchKernelGGL(plain_wave_kernel<false>, grid, block, 0, st, a);
+    else if (codes)
         hipLaunchKernelGGL(plain_kernel<true>, grid, block, 0, st, a);
     else
         hipLaunchKernelGGL(plain_kernel<false>, grid, block, 0, st, a);

@@ -250,10 +250,19 @@ int upload(srm_ctx *ctx, DevBuf &b, const T *src, size_t count)
 }
 
 // builds chunked matrix offsets for a plain index list
-// the plain kernel's int16 matrix of a candidate, in elements, 128-byte aligned
+// the plain kernels' scratch of a candidate in int16 elements: the whole matrix
+// (costs that keep it) or the decision words of the wave kernel, a word per column
+// for every 16 of its at most w + 63 steps and one per row, whichever is more (the
+// words only for windows of a few rows)
+inline size_t plain_elems_of(const srm_cand &c)
+{
+    return std::max(((size_t)c.w + 1) * ((size_t)c.L + 1), 
+                    2 * (((size_t)c.w + 78) / 16) * (size_t)c.L + 2 * (size_t)c.w);
+}
+// and 128-byte aligned
 inline uint32_t plain_mat_elems(const srm_cand &c)
 {
-    return (uint32_t)((((size_t)c.w + 1) * ((size_t)c.L + 1) + 63) & ~(size_t)63);
+    return (uint32_t)((plain_elems_of(c) + 63) & ~(size_t)63);
 }
 
 // matrix offsets and chunks of the candidates idx (mat: every candidate's matrix
@@ -806,7 +815,7 @@ size_t srm_job_bytes_bound(const srm_ctx *ctx, int match, int mismatch, const sr
         }
         if (!banded || all_plain) {
             any_plain = true;
-            plain_elems = std::max(plain_elems, (size_t)(c.w + 1) * (size_t)(c.L + 1) + 64);
+            plain_elems = std::max(plain_elems, plain_elems_of(c) + 64);
         }
     }
     size_t tiles = 0, scratch = 0;
