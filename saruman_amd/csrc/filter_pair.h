@@ -67,6 +67,10 @@ struct FArgs {
     int8_t *out_flag;
     int32_t *out_perf;
     uint32_t *meta;          // [3 * n_todo]: ent_off, perf_off, n_ent | n_perf << 16
+    // the reads' bytes as 2-bit codes and as a mask of the bytes other than ACGT
+    // (pack16), at the same offsets
+    const uint32_t *read_pk;
+    const uint32_t *read_odd;
 };
 
 SRM_HD inline char dcomp(char c)
@@ -98,6 +102,71 @@ SRM_HD inline char obyte(const char *rd, int L, int dr, int j)
     return dr ? dcomp(rd[L - 1 - j]) : rd[j];
 }
 
+// 16 bytes as 16 codes, the first in the top two bits (q-gram codes are read as
+// numbers with the first base most significant); a byte other than ACGT gives some
+// code and sets its bit (byte i: bit i) in odd
+SRM_HD inline uint32_t pack16(const uint32_t (&w)[4], uint32_t &odd)
+{
+    uint32_t pk = 0;
+    odd = 0;
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t c = (w[i >> 2] >> (8 * (i & 3))) & 0xFFu;
+        const uint32_t x = (c >> 1) & 3u, code = x ^ (x >> 1);   // A 0, C 1, G 2, T 3
+        pk = (pk << 2) | code;
+        odd |= (uint32_t)(((0x54474341u >> (8 * code)) & 0xFFu) != c) << i;
+    }
+    return pk;
+}
+
+// 32 codes from code index o, the first in the top bits (words o >> 4 .. + 2)
+SRM_HD inline uint64_t codes32(const uint32_t *pk, uint64_t o)
+{
+    const uint32_t *p = pk + (o >> 4);
+    const int sh = 2 * (int)(o & 15);
+    const uint64_t x = ((uint64_t)p[0] << 32) | p[1];
+    return sh ? (x << sh) | (p[2] >> (32 - sh)) : x;
+}
+
+// 32 mask bits from index o (words o >> 5, + 1)
+SRM_HD inline uint32_t odd32(const uint32_t *odd, uint64_t o)
+{
+    const uint32_t *p = odd + (o >> 5);
+    return (uint32_t)((((uint64_t)p[1] << 32) | p[0]) >> (o & 31));
+}
+
+// the 32 codes of x in reverse order
+SRM_HD inline uint64_t reverse_codes(uint64_t x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    x = __brevll(x);
+    return ((x >> 1) & 0x5555555555555555ull) | ((x & 0x5555555555555555ull) << 1);
+#else
+    x = __builtin_bswap64(x);
+    x = ((x >> 4) & 0x0F0F0F0F0F0F0F0Full) | ((x & 0x0F0F0F0F0F0F0F0Full) << 4);
+    return ((x >> 2) & 0x3333333333333333ull) | ((x & 0x3333333333333333ull) << 2);
+#endif
+}
+
+// the code of the q-gram (q <= 31) at offset g of the read at byte `at`, L bases, as
+// strand dr sees it; false when it holds another byte
+SRM_HD inline bool gram_code(const uint32_t *pk, const uint32_t *odd, uint64_t at, int L, int dr,
+                             int q, int g, uint64_t &code)
+{
+    const uint64_t o = at + (uint64_t)(dr ? L - g - q : g);
+    const uint64_t x = codes32(pk, o);
+    if (odd32(odd, o) & ((1u << q) - 1u)) return false;
+    code = dr ? reverse_codes(~x) & (((uint64_t)1 << (2 * q)) - 1) : x >> (64 - 2 * q);
+    return true;
+}
+
+// offset of q-gram list x: ascending from the read's start, then, when q does not
+// divide L, descending from its end (saruman.c:42-75)
+SRM_HD inline int gram_offset(int L, int q, int x)
+{
+    const int m = L / q;
+    return x < m ? x * q : L - (x - m + 1) * q;
+}
+
 // FNV-1a, 64 bit
 SRM_HD inline uint64_t fnv_step(uint64_t h, unsigned char c)
 {
@@ -108,6 +177,24 @@ constexpr uint64_t FNV_BASIS = 14695981039346656037ull;
 // list_lo of a q-gram whose positions are not one run of keys (it holds a byte
 // other than ACGT: its positions come from the hash table and a byte compare)
 constexpr uint32_t NO_RANGE = 0xFFFFFFFFu;
+
+// the run of keys of the q-gram `code`: its length, the first one's index in lo
+SRM_HD inline uint32_t lookup_code(const DQ &X, uint64_t code, uint32_t &lo)
+{
+    const uint64_t p = code >> (2 * (X.q - X.pre_bases));
+    lo = X.pre[p];
+    const uint32_t end = X.pre[p + 1];
+    uint32_t hi = end;
+    const uint64_t key = code << X.pos_bits;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (X.keys[mid] < key) lo = mid + 1;
+        else hi = mid;
+    }
+    uint32_t i = lo;
+    while (i < end && (X.keys[i] >> X.pos_bits) == code) ++i;
+    return i - lo;
+}
 
 // positions of the q-gram at read offset g, ascending; writes them to out when
 // FILL, returns their number; lo_out (when given) receives the index of the first
@@ -150,20 +237,12 @@ SRM_HD uint32_t lookup(const DQ &X, const char *genome, const char *rd, int L, i
         }
         return cnt;
     }
-    const uint64_t p = code >> (2 * (q - X.pre_bases));
-    uint32_t lo = X.pre[p], hi = X.pre[p + 1];
-    const uint64_t key = code << X.pos_bits;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (X.keys[mid] < key) lo = mid + 1;
-        else hi = mid;
-    }
+    uint32_t lo;
+    cnt = lookup_code(X, code, lo);
     if (lo_out) *lo_out = lo;
-    const uint64_t mask = ((uint64_t)1 << X.pos_bits) - 1;
-    const uint32_t end = X.pre[p + 1];
-    for (uint32_t i = lo; i < end && (X.keys[i] >> X.pos_bits) == code; ++i) {
-        if (FILL) out[cnt] = (uint32_t)(X.keys[i] & mask);
-        ++cnt;
+    if (FILL) {
+        const uint64_t mask = ((uint64_t)1 << X.pos_bits) - 1;
+        for (uint32_t i = 0; i < cnt; ++i) out[i] = (uint32_t)(X.keys[lo + i] & mask);
     }
     return cnt;
 }
