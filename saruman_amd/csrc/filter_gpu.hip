@@ -12,7 +12,7 @@
 //   3. fill    the same threads write the lists: a copy of the key run the
 //              count found, or the hash-table lookup again for a q-gram
 //              holding a byte other than ACGT;
-//   4. pair    one thread per read runs run_seashore (hash.c:502-834) and
+//   4. pair    a group of lanes per read runs run_seashore (hash.c:502-834) and
 //              add_start_position (hash.c:40-178) over the flat array.  A list
 //              index beyond the list runs on into the following lists and the
 //              following reads' lists up to the end of the read's chunk of
@@ -164,13 +164,70 @@ __device__ __forceinline__ uint32_t wave_incl_sum(uint32_t v)
     return v;
 }
 
+// one lane's stores to its read's slots before the group's later loads of them
 template <bool GLOBAL>
+__device__ __forceinline__ void slots_written()
+{
+    if (GLOBAL) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// add_start by a group's G lanes alike (gl: this lane's place, gb: the group's first
+// lane in the wave): the entries in steps of G, the first one that decides decides
+template <int G, bool GLOBAL>
+__device__ __forceinline__ int group_add(Store &s, int32_t pos, int flag, int k, int gl, int gb)
+{
+    constexpr uint64_t GM = G == 64 ? ~0ull : (1ull << (G & 63)) - 1;
+    for (uint32_t e0 = 0; e0 < s.n; e0 += G) {
+        const uint32_t e = e0 + (uint32_t)gl;
+        const int rule = e < s.n ? entry_rule(s.P(e), s.F(e), pos, flag, k) : 0;
+        const uint64_t m = (__ballot(rule != 0) >> gb) & GM;
+        if (m) {
+            const int first = (int)__builtin_ctzll(m);
+            const int decided = __shfl(rule, gb + first, 64);
+            if (decided == 2 && gl == first) s.F(e) = (int8_t)flag;
+            slots_written<GLOBAL>();
+            return decided;
+        }
+    }
+    if (s.n == s.cap) {
+        s.ovf = true;
+        return 2;
+    }
+    if (gl == 0) {
+        s.P(s.n) = pos;
+        s.F(s.n) = (int8_t)flag;
+    }
+    slots_written<GLOBAL>();
+    ++s.n;
+    return 2;
+}
+
+// run_seashore (hash.c:502-834) by G lanes per read: each lane takes a start
+// position (an element of the first half of the read's lists, which lie one after
+// another in the flat array) and finds what it would insert -- that depends on the
+// lists alone -- and the group then adds the results in the reference's order.
+//
+// Latency-bound: a start position is a chain of a few dependent list loads and the
+// perfect check.  A thread per read walked its positions one after another and
+// compared the read with the genome byte by byte, so a call lasted as long as its
+// longest read's chain; here the positions' chains run side by side and the group
+// compares 16 bases per lane at once, a genome start that several positions share
+// only once.  2M reads of 50-250 bp, one strand: 10.6 -> 2.44 ms, the reads of many
+// entries 3.39 -> 0.11 ms; 1,000 reads: 856 -> 45 us.
+template <int G, bool GLOBAL>
 __global__ void __launch_bounds__(FB) fl_pair(FArgs a)
 {
-    __shared__ int32_t s_pos[GLOBAL ? 1 : ECAP * FB];
-    __shared__ int8_t s_flag[GLOBAL ? 1 : ECAP * FB];
-    __shared__ int32_t s_perf[GLOBAL ? 1 : PCAP * FB];
-    const uint32_t j = blockIdx.x * FB + threadIdx.x;
+    constexpr int NG = FB / G;           // reads per block
+    constexpr uint64_t GM = G == 64 ? ~0ull : (1ull << (G & 63)) - 1;
+    __shared__ int32_t s_pos[GLOBAL ? 1 : ECAP * NG];
+    __shared__ int8_t s_flag[GLOBAL ? 1 : ECAP * NG];
+    __shared__ int32_t s_perf[GLOBAL ? 1 : PCAP * NG];
+    const int gl = threadIdx.x & (G - 1);
+    const int gb = threadIdx.x & 63 & ~(G - 1);
+    const uint32_t slot = threadIdx.x / G;
+    const uint32_t j = blockIdx.x * NG + slot;
     const bool active = j < a.n_todo;
     Store s;
     if (GLOBAL) {
@@ -181,15 +238,84 @@ __global__ void __launch_bounds__(FB) fl_pair(FArgs a)
         s.cap = a.cap;
         s.pcap = a.pcap;
     } else {
-        s.pos = s_pos + threadIdx.x;
-        s.flag = s_flag + threadIdx.x;
-        s.perf = s_perf + threadIdx.x;
-        s.stride = FB;
+        s.pos = s_pos + slot;
+        s.flag = s_flag + slot;
+        s.perf = s_perf + slot;
+        s.stride = NG;
         s.cap = ECAP;
         s.pcap = PCAP;
     }
-    if (active) seashore(a, a.todo ? a.todo[j] : j, s);
-    const uint32_t ne = (active && !s.ovf) ? s.n : 0, np = (active && !s.ovf) ? s.np : 0;
+    if (active) {
+        const uint32_t r = a.todo ? a.todo[j] : j;
+        const DParam P = a.par[a.pid[r]];
+        const uint32_t lb = a.list_base[r];
+        const uint32_t i0 = a.list_start[lb], i1 = a.list_start[lb + P.half];
+        // (an empty list is its terminator: nothing to do when all of them are)
+        if (i1 - i0 != (uint32_t)P.half) {
+            const uint64_t flat_end = chunk_end(a, r), at = a.roff[r];
+            for (uint32_t p0 = i0; p0 < i1 && !s.ovf; p0 += G) {
+                const uint32_t p = p0 + (uint32_t)gl;
+                const uint32_t Pa = p < i1 ? a.flat[p] : 0u;
+                int aa = 0;
+                uint32_t off = 0;
+                bool valid = Pa != 0;
+                if (valid) {
+                    for (int n = P.half; n > 1;) {   // the list holding p
+                        const int h = n >> 1;
+                        if (a.list_start[lb + aa + h] <= p) aa += h;
+                        n -= h;
+                    }
+                    const uint32_t first = a.list_start[lb + aa];
+                    off = p - first;
+                    // a list that starts with offset 0 reads as empty (Q14)
+                    valid = off == 0 || a.flat[first] != 0;
+                }
+                const long gs = (long)Pa - ((long)aa * P.q + 1);
+                valid = valid && gs + 1 > 0;
+                const uint32_t S = (uint32_t)(gs + 1);
+                // perfect check (strncpy + strcmp, hash.c:550-583), each genome start
+                // once, the group's lanes 16 bases each
+                const bool check = valid && (uint64_t)S + (uint64_t)P.L <= a.glen;
+                bool perfect = false;
+                uint64_t todo = (__ballot(check) >> gb) & GM;
+                while (todo) {
+                    const uint32_t S0 = (uint32_t)__shfl((int)S, gb + (int)__builtin_ctzll(todo), 64);
+                    bool ok = true;
+                    for (int x = gl; 16 * x < P.L && ok; x += G) ok = same16(a, at, P.L, a.dr, S0, x);
+                    const bool all = ((__ballot(!ok) >> gb) & GM) == 0;
+                    const bool mine = check && S == S0;
+                    if (mine) perfect = all;
+                    todo &= ~((__ballot(mine) >> gb) & GM);
+                }
+                int32_t hpos = 0;
+                int hflag = 0;
+                const bool found = valid && pair_matches(a, P, lb, flat_end, aa, off, Pa, gs, hpos, hflag);
+                const int what = (perfect ? 1 : 0) | (found ? 2 : 0) | (hflag << 2);
+                uint64_t add = (__ballot((what & 3) != 0) >> gb) & GM;
+                while (add && !s.ovf) {
+                    const int src = gb + (int)__builtin_ctzll(add);
+                    add &= add - 1;
+                    const int w = __shfl(what, src, 64);
+                    if (w & 1) {
+                        const int32_t S0 = __shfl((int)S, src, 64);
+                        if (group_add<G, GLOBAL>(s, -S0, 0, P.k, gl, gb) != 1 && !s.ovf) {
+                            if (s.np == s.pcap) {
+                                s.ovf = true;
+                            } else {
+                                if (gl == 0) s.Q(s.np) = S0;
+                                ++s.np;
+                            }
+                        }
+                    }
+                    if ((w & 2) && !s.ovf)
+                        group_add<G, GLOBAL>(s, __shfl(hpos, src, 64), w >> 2, P.k, gl, gb);
+                }
+            }
+        }
+    }
+    // the group's first lane speaks for its read
+    const bool lead = active && gl == 0;
+    const uint32_t ne = (lead && !s.ovf) ? s.n : 0, np = (lead && !s.ovf) ? s.np : 0;
     // one atomic pair per block reserves the block's output (the two counters are
     // words that every wave would otherwise update); the waves take consecutive
     // parts of it
@@ -216,7 +342,7 @@ __global__ void __launch_bounds__(FB) fl_pair(FArgs a)
         be += s_sum[v][0];
         bp += s_sum[v][1];
     }
-    if (!active) return;
+    if (!lead) return;
     for (uint32_t e = 0; e < ne; ++e) {
         a.out_pos[be + e] = s.P(e);
         a.out_flag[be + e] = s.F(e);
@@ -277,7 +403,7 @@ struct srm_dfilter {
     hipStream_t st = nullptr;
     const srm_index *ix = nullptr;
     size_t glen = 0;
-    GBuf genome, dq;
+    GBuf genome, gen_pk, gen_odd, dq;
     std::vector<GBuf> keys, pre, odd_hash, odd_pos;
     GBuf par, gram, reads, read_pk, read_odd, roff, rlen, pid, list_base, list_cnt, list_lo,
         list_start, flat, cub_tmp;
@@ -288,7 +414,7 @@ struct srm_dfilter {
 
     ~srm_dfilter()
     {
-        for (GBuf *b : {&genome, &dq, &par, &gram, &reads, &read_pk, &read_odd, &roff, &rlen, &pid, &list_base,
+        for (GBuf *b : {&genome, &gen_pk, &gen_odd, &dq, &par, &gram, &reads, &read_pk, &read_odd, &roff, &rlen, &pid, &list_base,
                         &list_cnt, &list_lo, &list_start, &flat, &cub_tmp, &slot_pos, &slot_flag,
                         &slot_perf, &out_pos, &out_flag, &out_perf, &meta, &counters, &todo})
             b->release();
@@ -302,6 +428,20 @@ struct srm_dfilter {
     {
         FL_RC(b.ensure(bytes + 64));   // slack: whole 16-byte words are read
         if (bytes) FL_TRY(hipMemcpyAsync(b.p, src, bytes, hipMemcpyHostToDevice, st));
+        return SRM_OK;
+    }
+
+    // the codes and the mask of other bytes of b's bytes (two code words and one mask
+    // word past the last are read beside them)
+    int pack(const GBuf &b, size_t bytes, GBuf &pk, GBuf &odd)
+    {
+        const size_t n16 = (bytes + 15) / 16;
+        FL_RC(pk.ensure((n16 + 4) * 4));
+        FL_RC(odd.ensure((n16 + 4) * 2 + 4));
+        if (n16 == 0) return SRM_OK;
+        hipLaunchKernelGGL(fl_pack, dim3((unsigned)((n16 + FB - 1) / FB)), dim3(FB), 0, st,
+                           b.as<const uint4>(), pk.as<uint32_t>(), odd.as<uint16_t>(), n16);
+        FL_TRY(hipGetLastError());
         return SRM_OK;
     }
 
@@ -338,9 +478,15 @@ struct srm_dfilter {
         a.meta = meta.as<uint32_t>();
         a.counters = counters.as<uint32_t>();
         FL_TRY(hipMemsetAsync(a.counters, 0, 8, st));
-        const unsigned grid = (n + FB - 1) / FB;
-        if (global) hipLaunchKernelGGL(fl_pair<true>, dim3(grid), dim3(FB), 0, st, a);
-        else hipLaunchKernelGGL(fl_pair<false>, dim3(grid), dim3(FB), 0, st, a);
+        // lanes per read: a wave for the reads of hundreds of entries; 8, about the
+        // start positions of a read that maps once, for many reads; 32 for the few
+        // thousand that leave the chip idle either way, where one step covers a
+        // read's lists (1,000 reads, both strands: 0.373 ms on the device with 32,
+        // 0.414 with 8; 2M reads: 38.1 and 32.2 ms)
+        auto grid = [&](unsigned g) { return dim3((n + FB / g - 1) / (FB / g)); };
+        if (global) hipLaunchKernelGGL((fl_pair<64, true>), grid(64), dim3(FB), 0, st, a);
+        else if (n < 4096) hipLaunchKernelGGL((fl_pair<32, false>), grid(32), dim3(FB), 0, st, a);
+        else hipLaunchKernelGGL((fl_pair<8, false>), grid(8), dim3(FB), 0, st, a);
         FL_TRY(hipGetLastError());
         uint32_t tot[2];
         FL_TRY(hipMemcpyAsync(tot, a.counters, 8, hipMemcpyDeviceToHost, st));
@@ -391,14 +537,7 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     FL_RC(G->upload(G->par, dpar.data(), dpar.size() * sizeof(DParam)));
     FL_RC(G->upload(G->gram, gram.data(), gram.size() * 2));
     FL_RC(G->upload(G->reads, reads, rbytes));
-    // (two codes words and one mask word past the last are read beside them)
-    const size_t n16 = (rbytes + 15) / 16;
-    FL_RC(G->read_pk.ensure((n16 + 4) * 4));
-    FL_RC(G->read_odd.ensure((n16 + 4) * 2 + 4));
-    hipLaunchKernelGGL(fl_pack, dim3((unsigned)((n16 + FB - 1) / FB)), dim3(FB), 0, G->st,
-                       G->reads.as<const uint4>(), G->read_pk.as<uint32_t>(),
-                       G->read_odd.as<uint16_t>(), n16);
-    FL_TRY(hipGetLastError());
+    FL_RC(G->pack(G->reads, rbytes, G->read_pk, G->read_odd));
     FL_RC(G->upload(G->roff, read_off, n_reads * 8));
     FL_RC(G->upload(G->rlen, read_len, n_reads * 2));
     FL_RC(G->upload(G->pid, pid.data(), n_reads * 2));
@@ -415,6 +554,8 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     a.reads = G->reads.as<char>();
     a.read_pk = G->read_pk.as<uint32_t>();
     a.read_odd = G->read_odd.as<uint32_t>();
+    a.gen_pk = G->gen_pk.as<uint32_t>();
+    a.gen_odd = G->gen_odd.as<uint32_t>();
     a.roff = G->roff.as<uint64_t>();
     a.rlen = G->rlen.as<uint16_t>();
     a.pid = G->pid.as<uint16_t>();
@@ -546,6 +687,7 @@ int srm_dfilter_create(srm_ctx *ctx, const srm_index *ix, const char *genome, si
         hipEventCreate(&G->ev[0]) != hipSuccess || hipEventCreate(&G->ev[1]) != hipSuccess)
         return fail(srm::set_error(SRM_EDEVICE, "event creation failed"));
     int rc = G->upload(G->genome, genome, glen);
+    if (!rc) rc = G->pack(G->genome, glen, G->gen_pk, G->gen_odd);
     if (rc) return fail(rc);
     std::vector<DQ> dq(32);
     std::memset(dq.data(), 0, dq.size() * sizeof(DQ));

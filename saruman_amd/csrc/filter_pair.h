@@ -71,6 +71,8 @@ struct FArgs {
     // (pack16), at the same offsets
     const uint32_t *read_pk;
     const uint32_t *read_odd;
+    const uint32_t *gen_pk;      // the genome's, likewise
+    const uint32_t *gen_odd;
 };
 
 SRM_HD inline char dcomp(char c)
@@ -157,6 +159,31 @@ SRM_HD inline bool gram_code(const uint32_t *pk, const uint32_t *odd, uint64_t a
     if (odd32(odd, o) & ((1u << q) - 1u)) return false;
     code = dr ? reverse_codes(~x) & (((uint64_t)1 << (2 * q)) - 1) : x >> (64 - 2 * q);
     return true;
+}
+
+// 16 codes from code index o, the first in the top bits (words o >> 4, + 1)
+SRM_HD inline uint32_t codes16(const uint32_t *pk, uint64_t o)
+{
+    const uint32_t *p = pk + (o >> 4);
+    return (uint32_t)(((((uint64_t)p[0] << 32) | p[1]) << (2 * (o & 15))) >> 32);
+}
+
+// bases 16x .. of the read (at most 16, to its end) as strand dr sees it against the
+// genome's from S + 16x: equal as bytes.  at: the read's first byte in a.reads.
+SRM_HD inline bool same16(const FArgs &a, uint64_t at, int L, int dr, uint64_t S, int x)
+{
+    const int j = 16 * x, m = L - j < 16 ? L - j : 16;
+    const uint64_t o = at + (uint64_t)(dr ? L - j - m : j);
+    const uint32_t some = (uint32_t)((1ull << m) - 1u);
+    if ((odd32(a.read_odd, o) | odd32(a.gen_odd, S + (uint64_t)j)) & some) {
+        for (int t = 0; t < m; ++t)
+            if (a.genome[S + (uint64_t)(j + t)] != obyte(a.reads + at, L, dr, j + t)) return false;
+        return true;
+    }
+    uint32_t c = codes16(a.read_pk, o);
+    if (dr)   // the m codes complemented and in reverse order, the first on top again
+        c = (uint32_t)(reverse_codes(~(uint64_t)c << 32)) << (2 * (16 - m));
+    return ((c ^ codes16(a.gen_pk, S + (uint64_t)j)) >> (2 * (16 - m))) == 0u;
 }
 
 // offset of q-gram list x: ascending from the read's start, then, when q does not
@@ -321,142 +348,151 @@ SRM_HD inline bool scan_run(const uint32_t *flat, uint64_t lo, uint64_t hi, uint
     return false;
 }
 
+// what entry (ep, ef) makes of a start (pos, flag): 1 rejected, 2 its flag is lowered,
+// 0 the next entry decides
+SRM_HD inline int entry_rule(int32_t ep, int ef, int32_t pos, int flag, int k)
+{
+    const int dir = flag > 3 ? 1 : 0, tdir = ef > 3 ? 1 : 0;
+    const int64_t d1 = (int64_t)ep - pos, d2 = (int64_t)ep + pos;
+    if (ef <= flag && ((d1 >= -k && d1 <= k) || (d2 >= -k && d2 <= k))) return 1;
+    if (ep == pos && tdir == dir && ef > flag) return 2;
+    return (ep == pos || ep == -pos) && tdir == dir ? 1 : 0;
+}
+
 // add_start_position, hash.c:40-178: 0 first entry, 1 rejected, 2 added or
 // flag lowered.  |pos - e| <= k is the reference's scan of pos + i, i in [-k, k].
 SRM_HD inline int add_start(Store &s, int32_t pos, int flag, int possible, int exact, int k)
 {
     if (possible != exact) return 1;
-    const int dir = flag > 3 ? 1 : 0;
     if (s.n == 0) {
         s.push(pos, flag);
         return 0;
     }
     for (uint32_t e = 0; e < s.n; ++e) {
-        const int32_t ep = s.P(e);
-        const int ef = s.F(e);
-        const int tdir = ef > 3 ? 1 : 0;
-        const int64_t d1 = (int64_t)ep - pos, d2 = (int64_t)ep + pos;
-        if (ef <= flag && ((d1 >= -k && d1 <= k) || (d2 >= -k && d2 <= k))) return 1;
-        if (ep == pos && tdir == dir && ef > flag) {
-            s.F(e) = (int8_t)flag;
-            return 2;
-        } else if ((ep == pos || ep == -pos) && tdir == dir) {
-            return 1;
-        }
+        const int rule = entry_rule(s.P(e), s.F(e), pos, flag, k);
+        if (rule == 2) s.F(e) = (int8_t)flag;
+        if (rule) return rule;
     }
     s.push(pos, flag);
     return 2;
 }
 
+// the end of the position lists a read's list indexes may run into: its chunk's
+SRM_HD inline uint64_t chunk_end(const FArgs &a, uint32_t r)
+{
+    const uint64_t next_chunk = ((uint64_t)(r / a.cv) + 1) * a.cv;
+    return a.list_start[a.list_base[next_chunk < a.n_reads ? next_chunk : a.n_reads]];
+}
+
+// the pair passes of one start position (hash.c:606-794): list aa's element off,
+// value Pa, genome start gs + 1; lb: the read's first list.  Every match raises
+// `possible` and calls add_start_position, which acts only when possible equals
+// exact_tresh (Q13): the need-th match of the two passes in scan order, need =
+// exact_tresh - 1, is the only one that can insert, and the scan stops there.
+// True when there is one, with what it inserts.
+SRM_HD inline bool pair_matches(const FArgs &a, const DParam &P, uint32_t lb, uint64_t flat_end,
+                                int aa, uint64_t off, uint32_t Pa, long gs, int32_t &hpos, int &hflag)
+{
+    const int q = P.q, half = P.half, k = P.k, L = P.L, dr = a.dr;
+    const bool fqm = (aa == 0);
+    const int need = P.exact - 1;
+    if (need < 1) return false;
+    int hits = 0;
+    // first pass, hash.c:606-692.  For every err the reference scans D(b, off), then
+    // D(b, 1), D(b, 2), ... up to the next 0 (Q12): the element at a's index, then
+    // one ascending run of list b (or of the list after b when b is empty).
+    for (int b = aa + 1; b < half; ++b) {
+        const uint64_t at = (uint64_t)a.list_start[lb + b] + off;
+        const uint32_t P0 = at < flat_end ? a.flat[at] : 0u;
+        if (P0 == 0) continue;                 // the scan never starts
+        const long rstart = (long)b * q + 1;
+        uint64_t lo = (uint64_t)a.list_start[lb + b] + 1, hi = lo;
+        const uint64_t nb = a.list_start[lb + b + 1];
+        if (lo < nb) {
+            hi = nb - 1;                       // list b from index 1
+        } else if ((uint64_t)lb + b + 2 <= a.list_base[a.n_reads]) {
+            hi = (uint64_t)a.list_start[lb + b + 2] - 1;   // the next list
+        }
+        if (!scan_run(a.flat, lo, hi, flat_end, gs + rstart - k, gs + rstart + k, true, P0, need, hits))
+            continue;
+        if (b == half - 1 && fqm) {
+            hflag = 1 + dr;
+            hpos = (int32_t)(gs + 1);
+        } else if (aa == half - 1) {
+            hflag = ((long)Pa + q > L ? 3 : 2) + dr;
+            hpos = (int32_t)(gs - k + 1);
+        } else if (fqm) {
+            hflag = 1 + dr;
+            hpos = (int32_t)(gs + 1);
+        } else {
+            hflag = 3 + dr;
+            hpos = (int32_t)(gs - k + 1);
+        }
+        return true;
+    }
+    // second pass, hash.c:695-794: each err scans list half + j from its start up to
+    // its 0; the targets gs + nin + err run downwards when j < a (the reference's err
+    // is negated there)
+    for (int j = 0; j < half; ++j) {
+        const int lim = half - 1 - j - aa < 0 ? -(half - 1 - j - aa) : half - 1 - j - aa;
+        const long nin = (long)(half - j - 1) * q + 1 + P.rest;
+        const uint64_t lo = a.list_start[lb + half + j];
+        const uint64_t hi = (uint64_t)a.list_start[lb + half + j + 1] - 1;
+        if (!scan_run(a.flat, lo, hi, flat_end, gs + nin - lim, gs + nin + lim, j - aa >= 0, 0u, need,
+                      hits))
+            continue;
+        if (j == 0 && fqm) {
+            hflag = 1 + dr;
+            hpos = (int32_t)(gs + 1);
+        } else if (j == 0) {
+            hflag = (nin + q > L ? 3 : 2) + dr;
+            hpos = (int32_t)(gs - k + 1);
+        } else if (fqm) {
+            hflag = 1 + dr;
+            hpos = (int32_t)(gs + 1);
+        } else {
+            hflag = 3 + dr;
+            hpos = (int32_t)(gs - k + 1);
+        }
+        return true;
+    }
+    return false;
+}
+
+// run_seashore of one read, its start positions one after another (the kernels
+// take several at a time)
 SRM_HD inline void seashore(const FArgs &a, uint32_t r, Store &s)
 {
     const DParam P = a.par[a.pid[r]];
-    const int q = P.q, half = P.half, k = P.k, L = P.L, rest = P.rest, dr = a.dr;
+    const int L = P.L, dr = a.dr;
     const char *rd = a.reads + a.roff[r];
     const uint32_t lb = a.list_base[r];
-    const uint32_t next_chunk = (r / a.cv + 1) * a.cv;
-    const uint32_t hi_read = next_chunk < a.n_reads ? next_chunk : a.n_reads;
-    const uint64_t flat_end = a.list_start[a.list_base[hi_read]];
-    auto D = [&](int x, uint64_t idx) -> uint32_t {
-        const uint64_t p = (uint64_t)a.list_start[lb + x] + idx;
-        return p < flat_end ? a.flat[p] : 0u;
-    };
-    for (int aa = 0; aa < half; ++aa) {
-        const bool fqm = (aa == 0);
-        const long in_read = (long)aa * q + 1;
-        uint64_t off = 0;
-        uint32_t Pa = D(aa, off);
-        while (Pa > 0) {
-            const long gs = (long)Pa - in_read;
-            if (gs + 1 > 0) {
-                // perfect check (strncpy + strcmp, hash.c:550-583)
-                const long S = gs + 1;
-                if ((uint64_t)S + (uint64_t)L <= a.glen) {
-                    bool perfect = true;
-                    const char *g = a.genome + S;
-                    for (int j = 0; j < L && perfect; ++j) perfect = g[j] == obyte(rd, L, dr, j);
-                    if (perfect && add_start(s, (int32_t)(-S), 0, P.exact, P.exact, k) != 1) {
-                        if (s.np == s.pcap) s.ovf = true;
-                        else s.Q(s.np++) = (int32_t)S;
-                    }
-                    if (s.ovf) return;
+    const uint64_t flat_end = chunk_end(a, r);
+    for (int aa = 0; aa < P.half; ++aa) {
+        for (uint64_t off = 0;; ++off) {
+            const uint64_t at = (uint64_t)a.list_start[lb + aa] + off;
+            const uint32_t Pa = at < flat_end ? a.flat[at] : 0u;
+            if (Pa == 0) break;
+            const long gs = (long)Pa - ((long)aa * P.q + 1);
+            if (gs + 1 <= 0) continue;
+            // perfect check (strncpy + strcmp, hash.c:550-583)
+            const long S = gs + 1;
+            if ((uint64_t)S + (uint64_t)L <= a.glen) {
+                bool perfect = true;
+                const char *g = a.genome + S;
+                for (int j = 0; j < L && perfect; ++j) perfect = g[j] == obyte(rd, L, dr, j);
+                if (perfect && add_start(s, (int32_t)(-S), 0, P.exact, P.exact, P.k) != 1) {
+                    if (s.np == s.pcap) s.ovf = true;
+                    else s.Q(s.np++) = (int32_t)S;
                 }
-                // the pair passes, hash.c:606-794.  Every match raises `possible` and
-                // calls add_start_position, which acts only when possible equals
-                // exact_tresh (Q13): the need-th match of the two passes in scan order,
-                // need = exact_tresh - 1, is the only one that can insert; the scan stops
-                // there.
-                const int need = P.exact - 1;
-                int hits = 0;
-                bool found = need < 1;
-                int32_t hpos = 0;
-                int hflag = 0;
-                // first pass, hash.c:606-692.  For every err the reference scans
-                // D(b, off), then D(b, 1), D(b, 2), ... up to the next 0 (Q12): the
-                // element at a's index, then one ascending run of list b (or of the
-                // list after b when b is empty).
-                for (int b = aa + 1; b < half && !found; ++b) {
-                    const uint32_t P0 = D(b, off);
-                    if (P0 == 0) continue;                 // the scan never starts
-                    const long rstart = (long)b * q + 1;
-                    uint64_t lo = (uint64_t)a.list_start[lb + b] + 1, hi = lo;
-                    const uint64_t nb = a.list_start[lb + b + 1];
-                    if (lo < nb) {
-                        hi = nb - 1;                       // list b from index 1
-                    } else if ((uint64_t)lb + b + 2 <= a.list_base[a.n_reads]) {
-                        hi = (uint64_t)a.list_start[lb + b + 2] - 1;   // the next list
-                    }
-                    if (scan_run(a.flat, lo, hi, flat_end, gs + rstart - k, gs + rstart + k, true,
-                                 P0, need, hits)) {
-                        found = true;
-                        if (b == half - 1 && fqm) {
-                            hflag = 1 + dr;
-                            hpos = (int32_t)(gs + 1);
-                        } else if (aa == half - 1) {
-                            hflag = ((long)Pa + q > L ? 3 : 2) + dr;
-                            hpos = (int32_t)(gs - k + 1);
-                        } else if (fqm) {
-                            hflag = 1 + dr;
-                            hpos = (int32_t)(gs + 1);
-                        } else {
-                            hflag = 3 + dr;
-                            hpos = (int32_t)(gs - k + 1);
-                        }
-                    }
-                }
-                // second pass, hash.c:695-794: each err scans list half + j from its
-                // start up to its 0; the targets gs + nin + err run downwards when
-                // j < a (the reference's err is negated there)
-                for (int j = 0; j < half && !found; ++j) {
-                    const int lim = half - 1 - j - aa < 0 ? -(half - 1 - j - aa) : half - 1 - j - aa;
-                    const long nin = (long)(half - j - 1) * q + 1 + rest;
-                    const uint64_t lo = a.list_start[lb + half + j];
-                    const uint64_t hi = (uint64_t)a.list_start[lb + half + j + 1] - 1;
-                    if (scan_run(a.flat, lo, hi, flat_end, gs + nin - lim, gs + nin + lim, j - aa >= 0,
-                                 0u, need, hits)) {
-                        found = true;
-                        if (j == 0 && fqm) {
-                            hflag = 1 + dr;
-                            hpos = (int32_t)(gs + 1);
-                        } else if (j == 0) {
-                            hflag = (nin + q > L ? 3 : 2) + dr;
-                            hpos = (int32_t)(gs - k + 1);
-                        } else if (fqm) {
-                            hflag = 1 + dr;
-                            hpos = (int32_t)(gs + 1);
-                        } else {
-                            hflag = 3 + dr;
-                            hpos = (int32_t)(gs - k + 1);
-                        }
-                    }
-                }
-                if (found && need >= 1) {
-                    add_start(s, hpos, hflag, P.exact, P.exact, k);
-                    if (s.ovf) return;
-                }
+                if (s.ovf) return;
             }
-            ++off;
-            Pa = D(aa, off);
+            int32_t hpos;
+            int hflag;
+            if (pair_matches(a, P, lb, flat_end, aa, off, Pa, gs, hpos, hflag)) {
+                add_start(s, hpos, hflag, P.exact, P.exact, P.k);
+                if (s.ovf) return;
+            }
         }
     }
 }

@@ -1,7 +1,9 @@
 // CPU build of the packed-code helpers of the device filter (filter_pair.h: pack16,
-// codes32, odd32, gram_code, gram_offset), with exactly the words the device arrays
+// codes16, codes32, odd32, gram_code, gram_offset, same16), with exactly the words the device arrays
 // hold, against a byte-by-byte reading of the same bases: every q-gram of reads of
-// 1..300 bases at every alignment, q 1..31, both strands, with other bytes mixed in.
+// 1..300 bases at every alignment, q 1..31, both strands, with other bytes mixed in,
+// and every 16-base step of reads against genome stretches equal to them or one
+// byte off.
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -82,6 +84,34 @@ int main()
                     }
                     ++checks;
                 }
+    }
+    for (int round = 0; round < 20000; ++round) {
+        const unsigned other = round % 3 == 0 ? 0 : 2 + (unsigned)(next() % 60);
+        const int L = 1 + (int)(next() % 90);
+        const size_t at = next() % 40, S = next() % 70;
+        const int dr = round & 1 ? 4 : 0;
+        const std::string reads = random_bases(at + (size_t)L, other);
+        std::string genome = random_bases(S + (size_t)L, other);
+        for (int j = 0; j < L; ++j) genome[S + (size_t)j] = obyte(reads.data() + at, L, dr, j);
+        if (next() % 2) genome[S + next() % (size_t)L] = random_bases(1, 2)[0];
+        const Packed R(reads), G(genome);
+        FArgs a{};
+        a.reads = reads.data();
+        a.genome = genome.data();
+        a.read_pk = R.pk.data();
+        a.read_odd = R.odd.data();
+        a.gen_pk = G.pk.data();
+        a.gen_odd = G.odd.data();
+        for (int x = 0; 16 * x < L; ++x) {
+            bool want = true;
+            for (int j = 16 * x; j < L && j < 16 * x + 16; ++j)
+                want &= genome[S + (size_t)j] == obyte(reads.data() + at, L, dr, j);
+            if (same16(a, at, L, dr, S, x) != want) {
+                printf("MISMATCH same16 L=%d at=%zu S=%zu dr=%d x=%d\n", L, at, S, dr, x);
+                return 1;
+            }
+            ++checks;
+        }
     }
     for (int L = 1; L <= 400; ++L)
         for (int k = 0; k <= 40; ++k) {
