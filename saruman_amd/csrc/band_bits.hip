@@ -221,6 +221,21 @@ __device__ __forceinline__ void bits_column(uint32_t (&VP)[NWD], uint32_t (&VN)[
     }
 }
 
+// value of band cell i of a column: cell 0's and the deltas of cells 1 .. i
+template <int NWD>
+__device__ __forceinline__ int column_cell(int v0, const uint32_t (&vp)[NWD],
+                                           const uint32_t (&vn)[NWD], int i)
+{
+#pragma unroll
+    for (int m = 0; m < NWD; ++m) {
+        const int top = i - 32 * m;   // cells 1 .. i of word m
+        uint32_t msk = top < 0 ? 0u : top >= 31 ? ~0u : (2u << top) - 1u;
+        if (m == 0) msk &= ~1u;
+        v0 += __builtin_popcount(vp[m] & msk) - __builtin_popcount(vn[m] & msk);
+    }
+    return v0;
+}
+
 template <int NW>
 struct BitsWaves {
     static constexpr int value = NW <= 4 ? 8 : 6;
@@ -231,8 +246,7 @@ struct BitsWaves {
 // column loop is short, and tiles taken from one global counter serialise on its
 // atomics; the workgroup dispatcher hands out the tiles (longest first) instead.
 template <int NW, bool CK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BitsWaves<NW>::value)))
-void bits_band_kernel(BandArgs a)
+__device__ __forceinline__ void band_tile(const BandArgs &a, uint32_t tile)
 {
     using S = BitsShape<NW>;
     constexpr int BMAX = S::BMAX, NWD = S::NWD, DW = S::DW, WB = S::WB;
@@ -240,9 +254,6 @@ void bits_band_kernel(BandArgs a)
     const int lane = threadIdx.x & 63;
 
     {
-        const uint32_t tile =
-            __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-        if (tile >= a.ntiles) return;
         uint4 td = a.tiles[tile];
         td.x = __builtin_amdgcn_readfirstlane(td.x);
         td.y = __builtin_amdgcn_readfirstlane(td.y);
@@ -489,25 +500,24 @@ void bits_band_kernel(BandArgs a)
     }
 }
 
-// Traceback of every hit of a unit-cost band class (cuda-functions.cu:504-534),
-// one wave per tile of bits_band_kernel.  The first run (column L's free rows)
-// and column 0 are as in trace_kernel; elsewhere the walk goes block by block.
-// occupancy target of the walk: the checkpoint layout holds a segment's 32 D0
-// columns in registers (a lower target leaves room for them without spilling)
 template <int NW, bool CK>
-struct TraceWaves {
-    static constexpr int value = CK ? (NW <= 4 ? 4 : 3) : (NW <= 4 ? 8 : 7);
-};
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BitsWaves<NW>::value)))
+void bits_band_kernel(BandArgs a)
+{
+    const uint32_t tile =
+        __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    if (tile < a.ntiles) band_tile<NW, CK>(a, tile);
+}
 
+// Traceback of every hit of a unit-cost band class (cuda-functions.cu:504-534),
+// one wave per tile of band_tile.  The first run (column L's free rows)
+// and column 0 are as in trace_kernel; elsewhere the walk goes block by block.
 template <int NW, bool CK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TraceWaves<NW, CK>::value)))
-void bits_trace_kernel(BandArgs a)
+__device__ __forceinline__ void trace_tile(const BandArgs &a, uint32_t tile)
 {
     using S = BitsShape<NW>;
     constexpr int BMAX = S::BMAX, NWD = S::NWD, DW = S::DW, WB = S::WB;
     const int lane = threadIdx.x & 63;
-    const uint32_t tile = (uint32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    if (tile >= a.ntiles) return;
     const uint4 td = a.tiles[tile];
     if ((uint32_t)lane >= td.y) return;
     const uint32_t pos = td.x + lane;   // tile order
@@ -597,21 +607,33 @@ void bits_trace_kernel(BandArgs a)
     // in the tile's rows: a segment's words are in the same few rows for the lanes
     const uint32_t *__restrict__ rrow = scr + (size_t)S::template read_at<CK>((int)td.z) * 64 + lane;
     const uint32_t *__restrict__ wrow = scr + (size_t)S::template win_at<CK>((int)td.z) * 64 + lane;
-    // checkpoint layout: the D0 words of the 32 columns of segment rg, recomputed
-    // from the segment's first column, and the state of its four blocks' first
-    // columns (band cell 0's value, the delta vectors)
-    uint32_t dcol[32][NWD];
-    int bv[4] = {0, 0, 0, 0};
-    uint32_t bp[4][NWD], bn[4][NWD];
-    int rg = -1;
-    auto recompute = [&](int g) {
+    // checkpoint layout: the state of column 32 bg (band cell 0's value, the deltas)
+    // and, of segment rg recomputed from it, the D0 bits of the 8 diagonals from wb
+    // on, bit j of a diagonal's word for column 32 rg + 1 + j
+    int bg = -1, bgv = 0;
+    uint32_t bgp[NWD], bgn[NWD];
+    int rg = -1, wb = 0;
+    uint32_t dw[8];
+    auto boundary = [&](int g) {
         const uint32_t *__restrict__ sb = scr + (size_t)g * S::WS * 64 + lane;
-        int v0 = (int)sb[0];
+        bgv = (int)sb[0];
+#pragma unroll
+        for (int m = 0; m < NWD; ++m) {
+            bgp[m] = sb[(1 + m) * 64];
+            bgn[m] = sb[(1 + NWD + m) * 64];
+        }
+        bg = g;
+    };
+    // the 8 diagonals around i: what the walk compares there are i - 1, i and i + 1,
+    // and a gap of up to 3 keeps to them
+    auto recompute = [&](int g, int i) {
+        if (g != bg) boundary(g);
+        wb = imin(imax(i - 4, 0), BMAX - 8);
         uint32_t VPr[NWD], VNr[NWD];
 #pragma unroll
         for (int m = 0; m < NWD; ++m) {
-            VPr[m] = sb[(1 + m) * 64];
-            VNr[m] = sb[(1 + NWD + m) * 64];
+            VPr[m] = bgp[m];
+            VNr[m] = bgn[m];
         }
         // window code planes of chunks g .. g + NWD and the read codes of the
         // segment, from the rows the forward pass left
@@ -621,34 +643,34 @@ void bits_trace_kernel(BandArgs a)
             planes_of(wrow[(2 * (g + m)) * 64], wrow[(2 * (g + m) + 1) * 64], c0[m], c1[m]);
         const uint32_t rw0 = rrow[(2 * g) * 64], rw1 = rrow[(2 * g + 1) * 64];
 #pragma unroll
-        for (int j = 0; j < 32; ++j) {
-            if ((j & 7) == 0) {
-                bv[j >> 3] = v0;
+        for (int j = 0; j < 8; ++j) dw[j] = 0u;
 #pragma unroll
-                for (int m = 0; m < NWD; ++m) {
-                    bp[j >> 3][m] = VPr[m];
-                    bn[j >> 3][m] = VNr[m];
-                }
-            }
-            uint32_t ne[NWD];
+        for (int j = 0; j < 32; ++j) {
+            uint32_t ne[NWD], d0[NWD];
             bits_ne<NWD>(c0, c1, j < 16 ? rw0 : rw1, j, ne);
-            bits_column<NWD>(VPr, VNr, ne, dcol[j], true);
-            v0 += 1 - (int)(dcol[j][0] & 1u);
+            bits_column<NWD>(VPr, VNr, ne, d0, true);
+            // column j's 8 bits to byte j / 8 of word j % 8: the transpose then gives
+            // the diagonals' words
+            const uint32_t x = NWD == 1 ? d0[0] >> wb
+                                        : (uint32_t)((((uint64_t)d0[NWD - 1] << 32) | d0[0]) >> wb);
+            dw[j & 7] |= (x & 0xFFu) << (8 * (j >> 3));
         }
+        transpose8(dw);
+        rg = g;
     };
-    // D0 bits of diagonal di over the segment's columns (bit j: column 32 rg + 1 + j);
-    // 0 outside the band
+    // the recomputed words hold diagonals i - 1, i and i + 1 (as far as they are in
+    // the band)
+    auto held = [&](int g, int i) {
+        return g == rg && imax(i - 1, 0) >= wb && imin(i + 1, BMAX - 1) < wb + 8;
+    };
+    // D0 bits of diagonal di over the segment's columns; 0 outside the band
     auto gather = [&](int di) -> uint32_t {
         if (di < 0 || di >= BMAX) return 0u;
-        const uint32_t b = (uint32_t)(di & 31);
-        const bool hi = NWD == 2 && di >= 32;
-        // bit b of each column word into bit j: a bit-field extract and a shift-or
-        // per column
-        uint32_t x = 0;
-#pragma unroll
-        for (int j = 0; j < 32; ++j)
-            x = (__builtin_amdgcn_ubfe(hi ? dcol[j][NWD - 1] : dcol[j][0], b, 1u) << j) | x;
-        return x;
+        const int t = di - wb;
+        const uint32_t x0 = t & 1 ? dw[1] : dw[0], x1 = t & 1 ? dw[3] : dw[2],
+                       x2 = t & 1 ? dw[5] : dw[4], x3 = t & 1 ? dw[7] : dw[6];
+        const uint32_t y0 = t & 2 ? x1 : x0, y1 = t & 2 ? x3 : x2;
+        return t & 4 ? y1 : y0;
     };
     // the walk goes by segments of 32 columns (4 blocks) along its diagonal: the D0
     // bits of the diagonal in columns 32g+1 .. 32g+32 and the mismatches of those
@@ -678,17 +700,10 @@ void bits_trace_kernel(BandArgs a)
     // K outside the band (never equal to a value <= k)
     auto cell = [&](int i, uint32_t dbits, int nb) -> int {
         if (i < 0 || i >= BMAX) return K;
-        int base = bvt;
-#pragma unroll
-        for (int m = 0; m < NWD; ++m) {
-            // cells 1 .. i of word m
-            const int top = i - 32 * m;
-            uint32_t msk = top < 0 ? 0u : top >= 31 ? ~0u : (2u << top) - 1u;
-            if (m == 0) msk &= ~1u;
-            base += __builtin_popcount(bvp[m] & msk) - __builtin_popcount(bvn[m] & msk);
-        }
-        return base + nb - __builtin_popcount(dbits & ((1u << nb) - 1u));
+        return column_cell<NWD>(bvt, bvp, bvn, i) + nb - __builtin_popcount(dbits & ((1u << nb) - 1u));
     };
+    int need = -1;   // the segment to recompute before the walk can go on
+    auto walk = [&]() {
     while (!done) {
         if (stop_row0 && row == 0) break;
         if (col == 0 && L >= 2) {
@@ -757,11 +772,19 @@ void bits_trace_kernel(BandArgs a)
             } else if (!(mseg & ((2u << j0) - 1u))) {
                 dseg = ~0u;
             } else if (CK) {
-                if (g != rg) {
-                    recompute(g);
-                    rg = g;
+                if (held(g, i)) {
+                    dseg = gather(i);
+                } else {
+                    // the diagonal's value in the segment's first column: each of its
+                    // cells is its predecessor or, only where the characters differ,
+                    // one more, so a fall of as many as differ is one at each of them
+                    if (g != bg) boundary(g);
+                    if (v - column_cell<NWD>(bgv, bgp, bgn, i) != __builtin_popcount(mseg & ((2u << j0) - 1u))) {
+                        need = g;
+                        return;
+                    }
+                    dseg = ~mseg;
                 }
-                dseg = gather(i);
             } else {
                 // D words of blocks 4g .. 4g+3 (clamped to the read's last block: bits
                 // of columns past the walk's cell are never looked at)
@@ -801,49 +824,62 @@ void bits_trace_kernel(BandArgs a)
             j0 -= rr;
         }
         // one cell that is not on a diagonal run (col >= 1)
+        int Tp = SRM_FOREIGN, Lf;
+        if constexpr (CK) {
+            // the cells beside it from the segment's first column and the D0 bits of
+            // their diagonals up to the walk's column; K outside the band (never equal
+            // to a value <= k)
+            if (!held(g, i)) {
+                need = g;
+                return;
+            }
+            auto side = [&](int di, int nb) -> int {
+                if (di < 0 || di >= BMAX) return K;
+                return column_cell<NWD>(bgv, bgp, bgn, di) + nb -
+                       __builtin_popcount(gather(di) & (nb > 31 ? ~0u : (1u << nb) - 1u));
+            };
+            if (row >= 1) Tp = side(i - 1, j0 + 1);
+            Lf = side(i + 1, j0);
+        } else {
         const int q = (col - 1) >> 3, jb = (col - 1) & 7;
         if (i != si || q != sq) {
-            if (CK) {
-                // block q is block u of the walk's segment, recomputed if it is not
-                // the one held
-                const int gq = q >> 2;
-                if (gq != rg) {
-                    recompute(gq);
-                    rg = gq;
-                }
-                const int u = q - 4 * rg;
-                dm = (gather(i - 1) >> (8 * u)) & 0xFFu;
-                dp = (gather(i + 1) >> (8 * u)) & 0xFFu;
-                bvt = u == 0 ? bv[0] : u == 1 ? bv[1] : u == 2 ? bv[2] : bv[3];
+            const uint32_t *__restrict__ blk = scr + (size_t)q * WB * 64 + lane;
+            dm = dbyte(blk, i - 1);
+            dp = dbyte(blk, i + 1);
+            if (q != sq) {   // the boundary belongs to the block, not the diagonal
+                bvt = (int)blk[DW * 64];
 #pragma unroll
                 for (int m = 0; m < NWD; ++m) {
-                    bvp[m] = u == 0 ? bp[0][m] : u == 1 ? bp[1][m] : u == 2 ? bp[2][m] : bp[3][m];
-                    bvn[m] = u == 0 ? bn[0][m] : u == 1 ? bn[1][m] : u == 2 ? bn[2][m] : bn[3][m];
-                }
-            } else {
-                const uint32_t *__restrict__ blk = scr + (size_t)q * WB * 64 + lane;
-                dm = dbyte(blk, i - 1);
-                dp = dbyte(blk, i + 1);
-                if (q != sq) {   // the boundary belongs to the block, not the diagonal
-                    bvt = (int)blk[DW * 64];
-#pragma unroll
-                    for (int m = 0; m < NWD; ++m) {
-                        bvp[m] = blk[(DW + 1 + m) * 64];
-                        bvn[m] = blk[(DW + 1 + NWD + m) * 64];
-                    }
+                    bvp[m] = blk[(DW + 1 + m) * 64];
+                    bvn[m] = blk[(DW + 1 + NWD + m) * 64];
                 }
             }
             si = i;
             sq = q;
         }
+        if (row >= 1) Tp = cell(i - 1, dm, jb + 1);
+        Lf = cell(i + 1, dp, jb);
+        }
         const int Dg = row >= 1 ? v - 1 + (int)((dseg >> j0) & 1u) : SRM_FOREIGN;
-        const int Tp = row >= 1 ? cell(i - 1, dm, jb + 1) : SRM_FOREIGN;
-        const int Lf = cell(i + 1, dp, jb);
         const bool eq = ((mseg >> j0) & 1u) == 0u;   // decides only with row >= 1
         const int op = decide(0, 1, v, Dg, Lf, Tp, col - 1, imax(row - 1, 0), L, w, s, e, eq);
         if (op == 3 || n >= cap) break;
         v = op == 0 ? Dg : op == 1 ? Tp : Lf;
         emit(op);
+    }
+    };
+    // Bound by instructions: a recomputed segment is 32 columns of the recurrence, for
+    // the whole wave whenever one lane asks.  So a segment that the boundary's value
+    // shows to have no gap on the diagonal asks for none (above), and a lane that needs
+    // one waits until every lane of the wave has come to such a point or to its end:
+    // one pass then serves them all, each lane in its own segment.  Only 8 diagonals of
+    // it are kept (8 words; all 32 columns' words took 32-64 registers).  1.77M
+    // candidates of 50-250 bp, forward pass, walk and the results' copy: 1.21 -> 0.98 ms
+    for (;;) {
+        walk();
+        if (!CK || need < 0) break;
+        recompute(need, row - col - dlo);
+        need = -1;
     }
     if (n & 15) put_word(n >> 4, opw);
     if (a.stage_words)
@@ -852,6 +888,21 @@ void bits_trace_kernel(BandArgs a)
     r.end_row = (uint16_t)row;
     r.end_col = (uint16_t)col;
     a.res[t] = r;
+}
+
+// occupancy target of the walk: the checkpoint layout recomputes segments in registers
+// (5: 2-7 of them spilled; 4: 1.01 instead of 0.97 ms for the step above; 6: 17-24)
+template <int NW, bool CK>
+struct TraceWaves {
+    static constexpr int value = CK ? (NW <= 4 ? 5 : 5) : (NW <= 4 ? 8 : 7);
+};
+
+template <int NW, bool CK>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TraceWaves<NW, CK>::value)))
+void bits_trace_kernel(BandArgs a)
+{
+    const uint32_t tile = (uint32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    if (tile < a.ntiles) trace_tile<NW, CK>(a, tile);
 }
 
 // ---------------------------------------------------------------------------
