@@ -905,6 +905,54 @@ void bits_trace_kernel(BandArgs a)
     if (tile < a.ntiles) trace_tile<NW, CK>(a, tile);
 }
 
+// reads of up to 250 codes stage their codes in LDS (a class's longest read: maxL)
+__host__ __device__ constexpr int bits_code_words(int maxL) { return maxL <= 250 ? ((maxL + 15) >> 4) + 3 : 0; }
+// transcript words per lane the walk stages in LDS for reads of up to maxL codes:
+// a band candidate's transcript holds at most w + k <= L + 63 ops (band cells
+// k + max(2s + k, w - L) + 1 <= 64), one more word for a run's lookahead write;
+// none for longer reads (the LDS would cut the walk's occupancy)
+__host__ __device__ constexpr int bits_stage_words(int maxL) { return maxL <= 320 ? ((maxL + 63) >> 4) + 2 : 0; }
+
+// The forward pass and the walk of every band class in one launch, a block of one
+// wave per tile, the widest class first: a tile's walk reads what its own forward
+// pass left, so nothing waits for other tiles.
+//
+// A tile is a serial chain of its columns (40-90 us for 250), whatever else runs.
+// Two launches per class one after another took the sum of the classes' longest
+// chains and left the chip to the last tiles of each: 14 launches, 480 us, for the
+// 53,000 candidates of 60,000 reads of 50-250 bp.  60,000 such reads through
+// srm_align_static: 985 -> 590 us; a batch of 50,000 with its upload and records 2.35
+// -> 2.07 ms; 1.77M candidates, where the classes ran on four streams: 0.98 -> 0.95 ms
+// with their results' copy.  So it runs at every size.  Occupancy: 5 waves per SIMD
+// with the checkpoint layout (4: 0.96 ms, with few registers spilled at 5 and hundreds
+// at 6), 6 with stored D bits.
+template <bool CK>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CK ? 5 : 6)))
+void bits_all_kernel(BandArgs a, BitsSpans sp)
+{
+    uint32_t c = 0;
+    while (c + 1 < sp.n && blockIdx.x >= sp.block[c + 1]) ++c;
+    const uint32_t tile = sp.tile[c] + (blockIdx.x - sp.block[c]);
+    a.code_words = bits_code_words(sp.max_len[c]);
+    a.stage_words = bits_stage_words(sp.max_len[c]);
+    auto both = [&](auto nw) {
+        band_tile<decltype(nw)::value, CK>(a, tile);
+        // both use the block's LDS, under two names: the walk's accesses stay behind
+        asm volatile("" ::: "memory");
+        trace_tile<decltype(nw)::value, CK>(a, tile);
+    };
+    switch (sp.nw[c]) {
+    case 1: both(std::integral_constant<int, 1>{}); break;
+    case 2: both(std::integral_constant<int, 2>{}); break;
+    case 3: both(std::integral_constant<int, 3>{}); break;
+    case 4: both(std::integral_constant<int, 4>{}); break;
+    case 5: both(std::integral_constant<int, 5>{}); break;
+    case 6: both(std::integral_constant<int, 6>{}); break;
+    case 7: both(std::integral_constant<int, 7>{}); break;
+    default: both(std::integral_constant<int, 8>{}); break;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // host-side launch wrappers
 // ---------------------------------------------------------------------------
@@ -952,7 +1000,7 @@ static hipError_t launch_bits_band_nw(const BandArgs &a, int blocks, size_t lds,
 hipError_t launch_bits_band(const BandArgs &args, int nw, int blocks, int maxL, hipStream_t st)
 {
     BandArgs a = args;
-    a.code_words = maxL <= 250 ? ((maxL + 15) >> 4) + 3 : 0;
+    a.code_words = bits_code_words(maxL);
     const size_t lds = (size_t)a.code_words * 64 * bits_block_waves(a) * 4;
     switch (nw) {
     case 1: return launch_bits_band_nw<1>(a, blocks, lds, st);
@@ -1003,12 +1051,8 @@ static hipError_t launch_bits_trace_nw(const BandArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
-// the walk reads the codes from the tile's rows: no LDS
-// transcript words per lane the walk stages in LDS for reads of up to maxL codes:
-// a band candidate's transcript holds at most w + k <= L + 63 ops (band cells
-// k + max(2s + k, w - L) + 1 <= 64), one more word for a run's lookahead write;
-// none for longer reads (the LDS would cut the walk's occupancy)
-int bits_trace_stage_words(int maxL) { return maxL <= 320 ? ((maxL + 63) >> 4) + 2 : 0; }
+// the walk reads the codes from the tile's rows: no LDS but the transcript's
+int bits_trace_stage_words(int maxL) { return bits_stage_words(maxL); }
 
 hipError_t launch_bits_trace(const BandArgs &args, int nw, int maxL, hipStream_t st)
 {
@@ -1025,6 +1069,21 @@ hipError_t launch_bits_trace(const BandArgs &args, int nw, int maxL, hipStream_t
     case 8: return launch_bits_trace_nw<8>(a, st);
     default: return hipErrorInvalidValue;
     }
+}
+
+// every class in one launch: a.tiles and a.tile_scratch are those of all classes
+hipError_t launch_bits_all(const BandArgs &a, const BitsSpans &sp, hipStream_t st)
+{
+    int words = 0;
+    for (uint32_t c = 0; c < sp.n; ++c) {
+        const int u = bits_code_words(sp.max_len[c]), v = bits_stage_words(sp.max_len[c]);
+        words = words > u ? words : u;
+        words = words > v ? words : v;
+    }
+    const size_t lds = (size_t)words * 64 * 4;
+    if (a.walk_ck) hipLaunchKernelGGL((bits_all_kernel<true>), dim3(sp.blocks), dim3(64), lds, st, a, sp);
+    else hipLaunchKernelGGL((bits_all_kernel<false>), dim3(sp.blocks), dim3(64), lds, st, a, sp);
+    return hipGetLastError();
 }
 
 } // namespace srm

@@ -55,6 +55,24 @@ struct BandArgs {
                                     // LDS (0: written straight to the slot)
 };
 
+// the unit-cost classes in the order one launch takes them: span c is blocks
+// block[c] .. block[c + 1] - 1 (a tile each, from tile[c] on) of band words nw[c] and
+// reads of up to max_len[c] codes
+constexpr int MAX_BAND_CLASSES = 16;   // 8 classes, each split at most once by read length
+struct BitsSpans {
+    uint32_t n = 0, blocks = 0;
+    uint32_t block[MAX_BAND_CLASSES], tile[MAX_BAND_CLASSES];
+    int nw[MAX_BAND_CLASSES], max_len[MAX_BAND_CLASSES];
+    void add(int w, uint32_t tile_begin, uint32_t ntiles, int maxL)
+    {
+        block[n] = blocks;
+        tile[n] = tile_begin;
+        nw[n] = w;
+        max_len[n++] = maxL;
+        blocks += ntiles;
+    }
+};
+
 struct RecArgs {
     int n;
     const srm_cand *cand;
@@ -104,6 +122,7 @@ hipError_t launch_trace(const BandArgs &a, int nw, bool unit, int maxL, hipStrea
 // unit costs (band_bits.hip): the bit-parallel forward pass and its walk
 hipError_t launch_bits_band(const BandArgs &a, int nw, int blocks, int maxL, hipStream_t st);
 hipError_t launch_bits_trace(const BandArgs &a, int nw, int maxL, hipStream_t st);
+hipError_t launch_bits_all(const BandArgs &a, const BitsSpans &sp, hipStream_t st);
 int bits_trace_stage_words(int maxL);   // LDS transcript words per lane for a class's walk
 int bits_band_occupancy(int nw);
 size_t bits_tile_words(int nw, int maxL, bool ck);   // one tile's scratch (words)

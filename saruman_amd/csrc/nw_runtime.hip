@@ -180,6 +180,7 @@ struct srm_job {
     bool all_planned = false;        // the plain-kernel plan of every candidate made
     int ma = 0, mm = 1;
     bool unit = true;
+    bool one_launch = false;         // unit costs: every class in one launch (upload)
     bool resident_genome = false;
     // device buffers
     DevBuf d_cand, d_read_words, d_win_words, d_read_bytes, d_win_bytes;
@@ -360,6 +361,27 @@ srm::RecArgs rec_args(srm_job *j, bool set_up)
     return a;
 }
 
+// the band kernels' arguments over the job's buffers; the tiles are the caller's
+srm::BandArgs band_args(srm_job *j)
+{
+    srm::BandArgs a{};
+    a.ma = j->ma;
+    a.mm = j->mm;
+    a.cand = (const srm_cand *)j->d_cand.p;
+    a.perm = (const uint32_t *)j->d_perm.p;
+    a.cand_tile = (const srm_cand *)j->d_cand_tile.p;
+    a.tile_score = (int32_t *)j->d_tile_score.p;
+    a.read_words = (const uint32_t *)j->d_read_words.p + SRM_CODE_PAD / 16;
+    a.win_words = j->resident_genome ? j->ctx->genome_ptr()
+                                     : (const uint32_t *)j->d_win_words.p + SRM_CODE_PAD / 16;
+    a.scratch = (uint32_t *)j->d_scratch.p;
+    a.res = (srm_result *)j->d_res.p;
+    a.ops = (uint32_t *)j->d_ops.p;
+    a.block_waves = j->block_waves;
+    a.walk_ck = j->walk_ck;
+    return a;
+}
+
 int run_launches(srm_job *j, int kernel, bool timed)
 {
     srm_ctx *ctx = j->ctx;
@@ -368,10 +390,21 @@ int run_launches(srm_job *j, int kernel, bool timed)
     if (timed) HIP_TRY(hipEventRecord(j->ev[0], st));
     if (use_band && !j->classes.empty()) {
         HIP_TRY(srm::launch_reset((uint32_t *)j->d_queue.p, (int)j->classes.size(), st));
-        // with class_streams > 1 the classes run side by side on their own streams
-        // (each with its own scratch), widest band first; otherwise in order on st
-        const int S = std::min<int>(j->class_streams, (int)j->classes.size());
-        std::vector<size_t> order(j->classes.size());
+        if (j->one_launch) {   // widest band, the longest tiles, first
+            srm::BitsSpans sp;
+            for (size_t c = j->classes.size(); c-- > 0;) {
+                const BandClass &bc = j->classes[c];
+                sp.add(bc.nw, bc.tile_begin, bc.ntiles, bc.maxL);
+            }
+            srm::BandArgs a = band_args(j);
+            a.tiles = (const uint4 *)j->d_tiles.p;
+            a.tile_scratch = (const uint64_t *)j->d_tile_scratch.p;
+            HIP_TRY(srm::launch_bits_all(a, sp, st));
+        }
+        // otherwise, with class_streams > 1, the classes run side by side on their own
+        // streams (each with its own scratch), widest band first, or in order on st
+        std::vector<size_t> order(j->one_launch ? 0 : j->classes.size());
+        const int S = std::min<int>(j->class_streams, (int)order.size());
         for (size_t c = 0; c < order.size(); ++c) order[c] = c;
         if (S > 1) {
             std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) {
@@ -384,26 +417,11 @@ int run_launches(srm_job *j, int kernel, bool timed)
             const size_t c = order[o];
             const BandClass &bc = j->classes[c];
             hipStream_t cst = S > 1 ? j->side[o % (size_t)S] : st;
-            srm::BandArgs a;
-            a.ma = j->ma;
-            a.mm = j->mm;
-            a.cand = (const srm_cand *)j->d_cand.p;
-            a.perm = (const uint32_t *)j->d_perm.p;
-            a.cand_tile = (const srm_cand *)j->d_cand_tile.p;
-            a.tile_score = (int32_t *)j->d_tile_score.p;
+            srm::BandArgs a = band_args(j);
             a.tiles = (const uint4 *)j->d_tiles.p + bc.tile_begin;
             a.ntiles = bc.ntiles;
             a.queue = (uint32_t *)j->d_queue.p + c;
-            a.read_words = (const uint32_t *)j->d_read_words.p + SRM_CODE_PAD / 16;
-            a.win_words = j->resident_genome
-                              ? ctx->genome_ptr()
-                              : (const uint32_t *)j->d_win_words.p + SRM_CODE_PAD / 16;
-            a.scratch = (uint32_t *)j->d_scratch.p;
             a.tile_scratch = (const uint64_t *)j->d_tile_scratch.p + bc.tile_begin;
-            a.res = (srm_result *)j->d_res.p;
-            a.ops = (uint32_t *)j->d_ops.p;
-            a.block_waves = j->block_waves;
-            a.walk_ck = j->walk_ck;
             if (timed) HIP_TRY(hipEventRecord(j->cs[c], cst));
             HIP_TRY(srm::launch_band(a, bc.nw, j->unit, bc.blocks, bc.maxL, cst));
             HIP_TRY(srm::launch_trace(a, bc.nw, j->unit, bc.maxL, cst));
@@ -1023,8 +1041,10 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
     // band classes run side by side on 4 streams unless the tuning says otherwise
     // (1 = one after another on the context's stream)
     const int want_streams = ctx->tuning.class_streams == 0 ? 4 : ctx->tuning.class_streams;
+    // -- the unit-cost classes side by side in one launch
     const bool concurrent = want_streams > 1;
-    j->class_streams = concurrent ? std::min(want_streams, 8) : 0;
+    j->one_launch = j->unit && concurrent && nb > 0;
+    j->class_streams = concurrent && !j->unit ? std::min(want_streams, 8) : 0;
     while ((int)j->side.size() < j->class_streams) {   // default priority, like every stream here
         hipStream_t q = nullptr;
         HIP_TRY(hipStreamCreateWithFlags(&q, hipStreamNonBlocking));
@@ -1224,9 +1244,9 @@ int srm_job_run(srm_job *j, int kernel)
     if (kernel != SRM_KERNEL_PLAIN)   // the class events are recorded only with band launches
         for (size_t c = 0; c < j->classes.size(); ++c)
         {
-            float ms = 0.f;
-            HIP_TRY(hipEventElapsedTime(&ms, j->cs[c], j->ce[c]));
-            j->class_ms[j->classes[c].nw] += ms;
+            float ms = j->band_ms;   // one launch: the time in which the class ran beside the others
+            if (!j->one_launch) HIP_TRY(hipEventElapsedTime(&ms, j->cs[c], j->ce[c]));
+            j->class_ms[j->classes[c].nw] = j->one_launch ? ms : j->class_ms[j->classes[c].nw] + ms;
         }
     return SRM_OK;
 }

@@ -201,31 +201,38 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
     SA_TRY(hipMemcpyAsync(base + o_tiles, h_tiles, ntiles * 16, hipMemcpyHostToDevice, st));
     SA_TRY(hipMemcpyAsync(base + o_toff, h_tile_off, ntiles * 8, hipMemcpyHostToDevice, st));
     // the class counters of the persistent (other-cost) kernel start at zero
-    SA_TRY(srm::launch_reset((uint32_t *)(base + o_queue), ncls, st));
+    if (!unit) SA_TRY(srm::launch_reset((uint32_t *)(base + o_queue), ncls, st));
 
+    srm::BandArgs a{};
+    a.ma = match;
+    a.mm = mismatch;
+    a.cand = (const srm_cand *)(base + o_cand);
+    a.perm = (const uint32_t *)(base + o_perm);
+    a.cand_tile = (const srm_cand *)(base + o_cand_tile);
+    a.tile_score = (int32_t *)(base + o_score);
+    a.read_words = d_read_words + SRM_CODE_PAD / 16;
+    a.win_words = d_win_words + SRM_CODE_PAD / 16;
+    a.scratch = (uint32_t *)(base + o_band);
+    a.res = d_res;
+    a.ops = d_ops;
+    if (unit) {   // every class in one launch, the widest band first
+        srm::BitsSpans sp;
+        for (int c = ncls; c-- > 0;) sp.add(cls[c].nw, cls[c].tile_begin, cls[c].ntiles, cls[c].maxL);
+        a.tiles = (const uint4 *)(base + o_tiles);
+        a.tile_scratch = (const uint64_t *)(base + o_toff);
+        SA_TRY(srm::launch_bits_all(a, sp, st));
+    }
     int num_cus = 0;
-    SA_TRY(hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, device));
-    for (int c = 0; c < ncls; ++c) {
+    if (!unit) SA_TRY(hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, device));
+    for (int c = 0; !unit && c < ncls; ++c) {
         const Class &bc = cls[c];
-        srm::BandArgs a{};
-        a.ma = match;
-        a.mm = mismatch;
-        a.cand = (const srm_cand *)(base + o_cand);
-        a.perm = (const uint32_t *)(base + o_perm);
-        a.cand_tile = (const srm_cand *)(base + o_cand_tile);
-        a.tile_score = (int32_t *)(base + o_score);
         a.tiles = (const uint4 *)(base + o_tiles) + bc.tile_begin;
         a.ntiles = bc.ntiles;
         a.queue = (uint32_t *)(base + o_queue) + c;
-        a.read_words = d_read_words + SRM_CODE_PAD / 16;
-        a.win_words = d_win_words + SRM_CODE_PAD / 16;
-        a.scratch = (uint32_t *)(base + o_band);
         a.tile_scratch = (const uint64_t *)(base + o_toff) + bc.tile_begin;
-        a.res = d_res;
-        a.ops = d_ops;
-        int blocks = (int)((bc.ntiles + 3) / 4);   // bits_band_kernel: a wave per tile
-        if (!unit)   // persistent grid: the blocks that stay resident, at most a wave per tile
-            blocks = std::min(blocks, std::max(1, num_cus * srm::band_occupancy(bc.nw, false)));
+        // persistent grid: the blocks that stay resident, at most a wave per tile
+        const int blocks = std::min((int)((bc.ntiles + 3) / 4),
+                                    std::max(1, num_cus * srm::band_occupancy(bc.nw, false)));
         SA_TRY(srm::launch_band(a, bc.nw, unit, blocks, bc.maxL, st));
         SA_TRY(srm::launch_trace(a, bc.nw, unit, bc.maxL, st));
     }
