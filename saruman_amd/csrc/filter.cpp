@@ -494,15 +494,32 @@ int srm_filter_run_chunk(const srm_index *ix, const char *chunk_text, size_t tex
 int srm_filter_sizes(const srm_filter *F, uint64_t *n_cand, uint64_t *n_batches,
                      uint64_t *n_perfect)
 {
-    *n_cand = F->c_read.size();
+    *n_cand = F->dense ? F->dense->n_cand : F->c_read.size();
     *n_batches = F->batch_end.size();
-    *n_perfect = F->p_read.size();
+    *n_perfect = F->dense ? F->dense->n_perf : F->p_read.size();
     return SRM_OK;
 }
 
 int srm_filter_copy(const srm_filter *F, int32_t *c_read, int64_t *c_pos, uint8_t *c_flag,
                     uint16_t *c_w, uint64_t *batch_end, int32_t *p_read, int64_t *p_pos)
 {
+    if (F->dense) {
+        const auto &D = *F->dense;
+        auto put = [](auto *dst, const auto *src, uint64_t n) {
+            if (dst && n) std::memcpy(dst, src, n * sizeof *dst);
+            return dst ? dst + n : dst;
+        };
+        for (const auto &P : D.piece) {
+            c_read = put(c_read, D.c_read + P.at, P.n);
+            c_pos = put(c_pos, D.c_pos + P.at, P.n);
+            c_flag = put(c_flag, D.c_flag + P.at, P.n);
+            c_w = put(c_w, D.c_w + P.at, P.n);
+        }
+        put(p_read, D.p_read, D.n_perf);
+        put(p_pos, D.p_pos, D.n_perf);
+        put(batch_end, F->batch_end.data(), F->batch_end.size());
+        return SRM_OK;
+    }
     const size_t n = F->c_read.size();
     if (c_read) std::memcpy(c_read, F->c_read.data(), n * 4);
     if (c_pos) std::memcpy(c_pos, F->c_pos.data(), n * 8);

@@ -21,27 +21,35 @@
 //              hits per read); a read that needs more is marked and run again
 //              with slots in HBM (1024, then 65534 entries);
 //   5. compact every wave reserves space for its reads' entries with one atomic
-//              and writes them contiguously; the host downloads 12 bytes per
-//              read plus the entries.
-// The sequential batch pass (Q10 leak, flush boundaries) then runs on the host
-// over the downloaded entries (filter_internal.h).
+//              and writes them contiguously;
+//   6. batch   the sequential batch pass (Q10 leak, flush boundaries) in parallel:
+//              counts per read, their sum, candidates and perfect hits in read
+//              order in one block that the host copies; the host settles the few
+//              reads whose outcome depends on others (filter_batch.h).
+// blockIdx.y is the strand: a call of both runs each kernel once.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
+#include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
 
+#include "filter_batch.h"
 #include "filter_internal.h"
 #include "filter_pair.h"
 #include "nw_device.h"
 
 using namespace srm_filter_impl;
 using namespace srm_pair;
+using namespace srm_batch;
 
 namespace {
 
@@ -61,6 +69,52 @@ __global__ void __launch_bounds__(FB) fl_pack(const uint4 *__restrict__ src, uin
     uint32_t o;
     pk[i] = pack16(w, o);
     odd[i] = (uint16_t)o;
+}
+
+constexpr uint32_t MAX_FLUSH = 256;      // flushes the device lists
+constexpr uint32_t MAX_UNSAFE = 1 << 16; // reads it lists for the host's walk
+constexpr uint32_t MAX_WALK = 1 << 16;   // words of their entries
+
+// one strand's counters and flushes
+struct Header {
+    uint32_t counters[3];    // entries, perfect hits, reads that outgrew their slots
+    uint32_t n_unsafe, walk_words;
+    uint32_t n_flush;        // MAX_FLUSH + 1: more
+    uint32_t flat;           // list entries (terminators included)
+    uint32_t blob_ok;        // the output fitted
+    Counts total;
+    Flush flush[MAX_FLUSH];
+};
+
+struct Strand {
+    FArgs f;
+    Header *hdr;
+    uint64_t flat_cap;       // entries that flat holds
+    Counts *cnt, *start;     // [n_reads + 1] per read; summed over the reads before
+    uint32_t *by_rank;       // the reads with entries
+    uint32_t *unsafe;        // read | leaky << 31
+    uint32_t *walk;
+};
+
+// one call's strands, in the order the kernels' blockIdx.y takes them
+struct Call {
+    Strand s[2];
+    int n;
+    uint64_t n_lists;        // per strand
+    int kmax;
+    const uint8_t *blocked;
+    unsigned char *blob;     // the strands' candidates and perfect hits, arrays packed
+    uint64_t blob_cap;
+};
+
+// a strand's arguments; false when its lists do not fit (the host makes room and
+// runs the call again)
+__device__ __forceinline__ bool strand_of(const Call &c, FArgs &a)
+{
+    const Strand &s = c.s[blockIdx.y];
+    a = s.f;
+    a.list_org = a.list_start[0];
+    return (uint64_t)list_at(a, c.n_lists) <= s.flat_cap;
 }
 
 // One thread per q-gram list; a block takes the lists of `per` consecutive reads,
@@ -109,9 +163,14 @@ struct BlockReads {
     }
 };
 
-__global__ void __launch_bounds__(FB) fl_count(FArgs a, uint32_t per)
+__global__ void __launch_bounds__(FB) fl_count(Call c_, uint32_t per)
 {
     __shared__ BlockReads s;
+    const FArgs &a = c_.s[blockIdx.y].f;
+    if (blockIdx.x == 0) {   // what later kernels of the call add to
+        if (threadIdx.x < 6) ((uint32_t *)c_.s[blockIdx.y].hdr)[threadIdx.x] = 0;
+        if (threadIdx.x == 0) a.list_cnt[c_.n_lists] = 0;
+    }
     const uint32_t nr = s.load(a, per);
     for (uint32_t i = s.base[0] + threadIdx.x; i < s.base[nr]; i += FB) {
         const uint32_t t = s.read_of(i, nr);
@@ -130,13 +189,15 @@ __global__ void __launch_bounds__(FB) fl_count(FArgs a, uint32_t per)
 
 // the lists themselves, blocks and threads as in fl_count: the positions are the
 // keys it found, or, for a q-gram holding another byte, the hash table's
-__global__ void __launch_bounds__(FB) fl_fill(FArgs a, uint32_t per)
+__global__ void __launch_bounds__(FB) fl_fill(Call c_, uint32_t per)
 {
     __shared__ BlockReads s;
+    FArgs a;
+    if (!strand_of(c_, a)) return;
     const uint32_t nr = s.load(a, per);
     for (uint32_t i = s.base[0] + threadIdx.x; i < s.base[nr]; i += FB) {
         const uint32_t c = a.list_cnt[i] - 1;
-        uint32_t *dst = a.flat + a.list_start[i];
+        uint32_t *dst = a.flat + list_at(a, i);
         if (c) {
             const uint32_t lo = a.list_lo[i], t = s.read_of(i, nr);
             const int q = s.q[t];
@@ -217,8 +278,10 @@ __device__ __forceinline__ int group_add(Store &s, int32_t pos, int flag, int k,
 // only once.  2M reads of 50-250 bp, one strand: 10.6 -> 2.44 ms, the reads of many
 // entries 3.39 -> 0.11 ms; 1,000 reads: 856 -> 45 us.
 template <int G, bool GLOBAL>
-__global__ void __launch_bounds__(FB) fl_pair(FArgs a)
+__global__ void __launch_bounds__(FB) fl_pair(Call c_)
 {
+    FArgs a;
+    if (!strand_of(c_, a)) return;
     constexpr int NG = FB / G;           // reads per block
     constexpr uint64_t GM = G == 64 ? ~0ull : (1ull << (G & 63)) - 1;
     __shared__ int32_t s_pos[GLOBAL ? 1 : ECAP * NG];
@@ -249,7 +312,7 @@ __global__ void __launch_bounds__(FB) fl_pair(FArgs a)
         const uint32_t r = a.todo ? a.todo[j] : j;
         const DParam P = a.par[a.pid[r]];
         const uint32_t lb = a.list_base[r];
-        const uint32_t i0 = a.list_start[lb], i1 = a.list_start[lb + P.half];
+        const uint32_t i0 = list_at(a, lb), i1 = list_at(a, lb + P.half);
         // (an empty list is its terminator: nothing to do when all of them are)
         if (i1 - i0 != (uint32_t)P.half) {
             const uint64_t flat_end = chunk_end(a, r), at = a.roff[r];
@@ -262,10 +325,10 @@ __global__ void __launch_bounds__(FB) fl_pair(FArgs a)
                 if (valid) {
                     for (int n = P.half; n > 1;) {   // the list holding p
                         const int h = n >> 1;
-                        if (a.list_start[lb + aa + h] <= p) aa += h;
+                        if (list_at(a, lb + aa + h) <= p) aa += h;
                         n -= h;
                     }
-                    const uint32_t first = a.list_start[lb + aa];
+                    const uint32_t first = list_at(a, lb + aa);
                     off = p - first;
                     // a list that starts with offset 0 reads as empty (Q14)
                     valid = off == 0 || a.flat[first] != 0;
@@ -348,9 +411,209 @@ __global__ void __launch_bounds__(FB) fl_pair(FArgs a)
         a.out_flag[be + e] = s.F(e);
     }
     for (uint32_t e = 0; e < np; ++e) a.out_perf[bp + e] = s.Q(e);
-    a.meta[3 * (size_t)j + 0] = be;
-    a.meta[3 * (size_t)j + 1] = bp;
-    a.meta[3 * (size_t)j + 2] = s.ovf ? OVERFLOW_MARK : (ne | (np << 16));
+    const uint32_t r = a.todo ? a.todo[j] : j;
+    a.meta[3 * (size_t)r + 0] = be;
+    a.meta[3 * (size_t)r + 1] = bp;
+    a.meta[3 * (size_t)r + 2] = s.ovf ? OVERFLOW_MARK : (ne | (np << 16));
+    if (s.ovf) a.over[atomicAdd(&a.counters[2], 1u)] = r;
+}
+
+// ---- the batch pass (filter_batch.h), a thread per read: counts, and after their
+// sum the candidates and perfect hits at their places in read order.  HBM-bound
+// (12 bytes of meta per read, 5 per entry, 15 out per candidate); the host's pass
+// over the same data and its download took 80 of the 96 ms of a call of 2M reads.
+// With both strands in each launch and two waits in a call (one, while the output fits
+// the first copy) instead of eight, the whole call: 2M reads 96.2 -> 20.8 ms, 100,000 of
+// 36 bp 3.14 -> 0.74 ms, 1,000 0.47 -> 0.22 ms
+__global__ void __launch_bounds__(FB) fl_batch_count(Call c)
+{
+    FArgs a;
+    if (!strand_of(c, a)) return;
+    const Strand &s = c.s[blockIdx.y];
+    const uint32_t r = blockIdx.x * FB + threadIdx.x;
+    if (r > a.n_reads) return;
+    Counts n;
+    if (r < a.n_reads) {
+        const uint32_t m0 = a.meta[3 * (size_t)r], m2 = a.meta[3 * (size_t)r + 2];
+        const DParam P = a.par[a.pid[r]];
+        bool unsafe, leaky;
+        n = count_entries(a.out_pos + m0, a.out_flag + m0, entries_of(m2), P.L, P.k, c.kmax, a.glen,
+                          c.blocked, unsafe, leaky);
+        n.perf = perfects_of(m2);
+        if (unsafe) {
+            const uint32_t u = atomicAdd(&s.hdr->n_unsafe, 1u);
+            if (u < MAX_UNSAFE) s.unsafe[u] = r | (leaky ? 1u << 31 : 0u);
+        }
+    }
+    s.cnt[r] = n;
+}
+
+// the sum over a strand's reads before r
+__device__ __forceinline__ Counts counts_before(const Strand &s, uint32_t r)
+{
+    const Counts x = s.start[r], o = s.start[0];
+    Counts n;
+    n.cand = x.cand - o.cand;
+    n.perf = x.perf - o.perf;
+    n.queued = x.queued - o.queued;
+    n.with = x.with - o.with;
+    return n;
+}
+
+// the byte offsets of the strands' arrays in the blob, widest elements first
+struct BlobAt {
+    uint64_t c_pos[2], p_pos[2], c_read[2], p_read[2], c_w[2], c_flag[2], bytes;
+};
+
+__host__ __device__ inline BlobAt blob_at(const Counts &t0, const Counts &t1)
+{
+    const uint64_t c[2] = {t0.cand, t1.cand}, p[2] = {t0.perf, t1.perf};
+    BlobAt b;
+    uint64_t at = 0;
+    for (int s = 0; s < 2; ++s) {
+        b.c_pos[s] = at;
+        b.p_pos[s] = b.c_pos[s] + 8 * c[s];
+        at = b.p_pos[s] + 8 * p[s];
+    }
+    for (int s = 0; s < 2; ++s) {
+        b.c_read[s] = at;
+        b.p_read[s] = b.c_read[s] + 4 * c[s];
+        at = b.p_read[s] + 4 * p[s];
+    }
+    for (int s = 0; s < 2; ++s) {
+        b.c_w[s] = at;
+        at += 2 * c[s];
+    }
+    for (int s = 0; s < 2; ++s) {
+        b.c_flag[s] = at;
+        at += c[s];
+    }
+    b.bytes = at;
+    return b;
+}
+
+__global__ void __launch_bounds__(FB) fl_batch_write(Call c)
+{
+    FArgs a;
+    if (!strand_of(c, a)) return;
+    const int y = blockIdx.y;
+    const Strand &s = c.s[y];
+    const uint32_t r = blockIdx.x * FB + threadIdx.x;
+    const BlobAt b = blob_at(counts_before(c.s[0], a.n_reads),
+                             c.n > 1 ? counts_before(c.s[1], a.n_reads) : Counts());
+    const bool fits = b.bytes <= c.blob_cap;
+    if (r == 0) s.hdr->blob_ok = fits;
+    if (r >= a.n_reads) return;
+    const uint32_t m0 = a.meta[3 * (size_t)r], m1 = a.meta[3 * (size_t)r + 1], m2 = a.meta[3 * (size_t)r + 2];
+    const uint32_t ne = entries_of(m2), np = perfects_of(m2);
+    const Counts at = counts_before(s, r);
+    if (ne) s.by_rank[at.with] = r;
+    if (!fits) return;
+    const DParam P = a.par[a.pid[r]];
+    int64_t *c_pos = (int64_t *)(c.blob + (y ? b.c_pos[1] : b.c_pos[0])), *p_pos = (int64_t *)(c.blob + (y ? b.p_pos[1] : b.p_pos[0]));
+    int32_t *c_read = (int32_t *)(c.blob + (y ? b.c_read[1] : b.c_read[0])), *p_read = (int32_t *)(c.blob + (y ? b.p_read[1] : b.p_read[0]));
+    uint16_t *c_w = (uint16_t *)(c.blob + (y ? b.c_w[1] : b.c_w[0]));
+    uint8_t *c_flag = c.blob + (y ? b.c_flag[1] : b.c_flag[0]);
+    uint32_t o = at.cand;
+    for (uint32_t e = 0; e < ne; ++e) {
+        const int32_t pos = a.out_pos[m0 + e];
+        const int flag = a.out_flag[m0 + e];
+        const int64_t w = own_window(P.L, flag, P.k);
+        if (pos <= 0 || outside(c.blocked, a.glen, pos, w)) continue;
+        c_pos[o] = pos;
+        c_read[o] = (int32_t)r;
+        c_w[o] = (uint16_t)w;
+        c_flag[o] = (uint8_t)flag;
+        ++o;
+    }
+    for (uint32_t e = 0; e < np; ++e) {
+        p_pos[at.perf + e] = a.out_perf[m1 + e];
+        p_read[at.perf + e] = (int32_t)r;
+    }
+}
+
+// where fl_batch_end does not run: the lists' total
+__global__ void fl_totals(Call c)
+{
+    FArgs a;
+    (void)strand_of(c, a);
+    if (threadIdx.x == 0) c.s[blockIdx.y].hdr->flat = list_at(a, c.n_lists);
+}
+
+// one block per strand: the flushes (a flush ends with the first read that takes the
+// queue past chunk_value; found by a wave's 64-way search of the queued sums), and
+// the entries of the reads the host walks
+__global__ void __launch_bounds__(FB) fl_batch_end(Call c)
+{
+    FArgs a;
+    if (!strand_of(c, a)) {
+        if (threadIdx.x == 0) c.s[blockIdx.y].hdr->flat = list_at(a, c.n_lists);
+        return;
+    }
+    const Strand &s = c.s[blockIdx.y];
+    const uint32_t n = a.n_reads;
+    const Counts total = counts_before(s, n);
+    if (threadIdx.x < 64) {
+        const uint32_t lane = threadIdx.x;
+        uint32_t lo = 0, nf = 0;
+        for (;;) {
+            const uint32_t q0 = counts_before(s, lo).queued;
+            uint32_t x = lo, y = n;          // the read is in [x, y], n: none
+            while (x < y) {
+                const uint32_t step = (y - x + 63) / 64;
+                const uint64_t e = (uint64_t)x + (uint64_t)(lane + 1) * step;
+                const uint32_t r = (uint32_t)(e < y ? e : y) - 1;
+                const uint64_t m = __ballot(counts_before(s, r + 1).queued - q0 > a.cv);
+                if (m == 0) {
+                    x = y;
+                    break;
+                }
+                const uint32_t f = (uint32_t)__builtin_ctzll(m);
+                y = (uint32_t)__shfl((int)r, (int)f, 64);
+                x += f * step;
+            }
+            const bool last = x >= n;
+            if (last && total.queued == q0) break;
+            if (nf == MAX_FLUSH) {
+                nf = MAX_FLUSH + 1;
+                break;
+            }
+            lo = last ? n : x + 1;
+            if (lane == 0) s.hdr->flush[nf] = {lo, counts_before(s, lo).cand};
+            ++nf;
+            if (last) break;
+        }
+        if (lane == 0) {
+            s.hdr->n_flush = nf;
+            s.hdr->flat = list_at(a, c.n_lists);
+            s.hdr->total = total;
+        }
+    }
+    auto put = [&](uint32_t r) {
+        const uint32_t m0 = a.meta[3 * (size_t)r], ne = entries_of(a.meta[3 * (size_t)r + 2]);
+        const Counts at = counts_before(s, r);
+        if (4 + 2 * ne > MAX_WALK / 4) {   // (kept out of the sum, which must not wrap)
+            atomicMax(&s.hdr->walk_words, MAX_WALK + 1);
+            return;
+        }
+        const uint32_t w = atomicAdd(&s.hdr->walk_words, 4 + 2 * ne);
+        if (w + 4 + 2 * ne > MAX_WALK) return;
+        s.walk[w] = r;
+        s.walk[w + 1] = at.with;
+        s.walk[w + 2] = at.cand;
+        s.walk[w + 3] = ne;
+        for (uint32_t e = 0; e < ne; ++e) {
+            s.walk[w + 4 + e] = (uint32_t)a.out_pos[m0 + e];
+            s.walk[w + 4 + ne + e] = (uint32_t)(int32_t)a.out_flag[m0 + e];
+        }
+    };
+    const uint32_t nu = s.hdr->n_unsafe < MAX_UNSAFE ? s.hdr->n_unsafe : MAX_UNSAFE;
+    for (uint32_t u = threadIdx.x; u < nu; u += FB) {
+        const uint32_t r = s.unsafe[u] & 0x7FFFFFFFu;
+        put(r);
+        const uint32_t next = counts_before(s, r).with + 1;
+        if ((s.unsafe[u] >> 31) && next < total.with) put(s.by_rank[next]);
+    }
 }
 
 struct GBuf {
@@ -395,6 +658,80 @@ struct GBuf {
         if (rc_ != SRM_OK) return rc_;   \
     } while (0)
 
+// page-locked blocks for results: at most MAX_BLOCKS exist at a time (a caller that
+// holds more results gets ordinary memory), two of them kept for the next calls.
+// The results hold the pool too, so it outlives the filter for as long as they do.
+class BlockPool : public std::enable_shared_from_this<BlockPool> {
+public:
+    ~BlockPool()
+    {
+        for (auto &b : kept_) (void)hipHostFree(b.p);
+    }
+    // `bytes` of memory, given back when the last owner lets go; null: none to be had
+    std::shared_ptr<void> take(size_t bytes)
+    {
+        Block b;
+        bool make = false;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            for (size_t i = 0; i < kept_.size() && !b.p; ++i)
+                if (kept_[i].bytes >= bytes) {
+                    b = kept_[i];
+                    kept_.erase(kept_.begin() + (std::ptrdiff_t)i);
+                }
+            if (!b.p && !kept_.empty()) {   // too small: make room for this size
+                (void)hipHostFree(kept_.back().p);
+                kept_.pop_back();
+                --made_;
+            }
+            if (!b.p && made_ < MAX_BLOCKS) {
+                make = true;
+                ++made_;
+            }
+        }
+        if (make) {
+            b.bytes = bytes + bytes / 4 + 4096;
+            if (hipHostMalloc(&b.p, b.bytes, hipHostMallocDefault) != hipSuccess) {
+                b.p = nullptr;
+                std::lock_guard<std::mutex> lk(mu_);
+                --made_;
+            }
+        }
+        if (!b.p) {
+            void *p = std::malloc(bytes);
+            return p ? std::shared_ptr<void>(p, std::free) : std::shared_ptr<void>();
+        }
+        auto self = shared_from_this();
+        return std::shared_ptr<void>(b.p, [self, b](void *) { self->give(b); });
+    }
+
+private:
+    static constexpr size_t MAX_BLOCKS = 4, KEEP = 2;
+    struct Block {
+        void *p = nullptr;
+        size_t bytes = 0;
+    };
+    void give(Block b)
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        if (kept_.size() < KEEP) {
+            kept_.push_back(b);
+            return;
+        }
+        (void)hipHostFree(b.p);
+        --made_;
+    }
+    std::mutex mu_;
+    std::vector<Block> kept_;
+    size_t made_ = 0;
+};
+
+// inputs up to this size are put together in page-locked memory and sent in one copy
+// (a copy of a few KB takes 10-30 us of calls, whatever its size)
+constexpr size_t STAGE_IN = (size_t)1 << 20;
+// and this much of the output comes back with the headers, in one copy
+constexpr size_t STAGE_OUT = (size_t)128 << 10;
+
 }  // namespace
 
 struct srm_dfilter {
@@ -405,21 +742,30 @@ struct srm_dfilter {
     size_t glen = 0;
     GBuf genome, gen_pk, gen_odd, dq;
     std::vector<GBuf> keys, pre, odd_hash, odd_pos;
-    GBuf par, gram, reads, read_pk, read_odd, roff, rlen, pid, list_base, list_cnt, list_lo,
-        list_start, flat, cub_tmp;
-    GBuf slot_pos, slot_flag, slot_perf, out_pos, out_flag, out_perf, meta, counters, todo;
+    GBuf in, read_pk, read_odd, blocked, list_cnt, list_lo, list_start, cub_tmp, cnt, start, by_rank,
+        unsafe, walk, out;
+    GBuf flat[2], out_pos[2], out_flag[2], out_perf[2], meta[2], over[2][2];
+    GBuf slot_pos, slot_flag, slot_perf;
+    void *stage_in = nullptr, *stage_out = nullptr;   // page-locked
+    std::shared_ptr<BlockPool> pool = std::make_shared<BlockPool>();
     hipEvent_t ev[2] = {nullptr, nullptr};
     float last_ms = 0.f;
     size_t last_lists = 0, last_flat = 0, last_overflow = 0;
 
     ~srm_dfilter()
     {
-        for (GBuf *b : {&genome, &gen_pk, &gen_odd, &dq, &par, &gram, &reads, &read_pk, &read_odd, &roff, &rlen, &pid, &list_base,
-                        &list_cnt, &list_lo, &list_start, &flat, &cub_tmp, &slot_pos, &slot_flag,
-                        &slot_perf, &out_pos, &out_flag, &out_perf, &meta, &counters, &todo})
+        for (GBuf *b : {&genome, &gen_pk, &gen_odd, &dq, &in, &read_pk, &read_odd, &blocked, &list_cnt,
+                        &list_lo, &list_start, &cub_tmp, &cnt, &start, &by_rank, &unsafe, &walk, &out,
+                        &slot_pos, &slot_flag, &slot_perf})
             b->release();
+        for (int s = 0; s < 2; ++s)
+            for (GBuf *b : {&flat[s], &out_pos[s], &out_flag[s], &out_perf[s], &meta[s], &over[s][0],
+                            &over[s][1]})
+                b->release();
         for (auto *v : {&keys, &pre, &odd_hash, &odd_pos})
             for (auto &b : *v) b.release();
+        if (stage_in) (void)hipHostFree(stage_in);
+        if (stage_out) (void)hipHostFree(stage_out);
         for (auto &e : ev)
             if (e) (void)hipEventDestroy(e);
     }
@@ -431,85 +777,364 @@ struct srm_dfilter {
         return SRM_OK;
     }
 
-    // the codes and the mask of other bytes of b's bytes (two code words and one mask
-    // word past the last are read beside them)
-    int pack(const GBuf &b, size_t bytes, GBuf &pk, GBuf &odd)
+    // the codes and the mask of other bytes of n bytes at src (two code words and one
+    // mask word past the last are read beside them)
+    int pack(const void *src, size_t bytes, GBuf &pk, GBuf &odd)
     {
         const size_t n16 = (bytes + 15) / 16;
         FL_RC(pk.ensure((n16 + 4) * 4));
         FL_RC(odd.ensure((n16 + 4) * 2 + 4));
         if (n16 == 0) return SRM_OK;
         hipLaunchKernelGGL(fl_pack, dim3((unsigned)((n16 + FB - 1) / FB)), dim3(FB), 0, st,
-                           b.as<const uint4>(), pk.as<uint32_t>(), odd.as<uint16_t>(), n16);
+                           (const uint4 *)src, pk.as<uint32_t>(), odd.as<uint16_t>(), n16);
         FL_TRY(hipGetLastError());
         return SRM_OK;
     }
 
-    // runs the pairing kernel over n reads (todo == null: all reads of the call)
-    // and downloads meta and the compact output
-    int pair(FArgs a, bool global, const uint32_t *todo_host, uint32_t n, uint32_t cap,
-             uint32_t pcap, std::vector<uint32_t> &meta_h, std::vector<int32_t> &pos_h,
-             std::vector<int8_t> &flag_h, std::vector<int32_t> &perf_h)
+    // b with room for `bytes`, its first `used` bytes kept
+    int grow(GBuf &b, size_t bytes, size_t used)
     {
-        a.n_todo = n;
-        a.todo = nullptr;
-        if (todo_host) {
-            FL_RC(upload(todo, todo_host, (size_t)n * 4));
-            a.todo = todo.as<uint32_t>();
+        if (bytes <= b.cap) return SRM_OK;
+        GBuf n;
+        FL_RC(n.ensure(bytes));
+        hipError_t e = used ? hipMemcpyAsync(n.p, b.p, used, hipMemcpyDeviceToDevice, st) : hipSuccess;
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        if (e != hipSuccess) {
+            n.release();
+            return srm::set_error(SRM_EDEVICE, "copy to a larger buffer failed: %s", hipGetErrorString(e));
         }
-        if (global) {
-            FL_RC(slot_pos.ensure((size_t)n * cap * 4));
-            FL_RC(slot_flag.ensure((size_t)n * cap));
-            FL_RC(slot_perf.ensure((size_t)n * pcap * 4));
-            a.slot_pos = slot_pos.as<int32_t>();
-            a.slot_flag = slot_flag.as<int8_t>();
-            a.slot_perf = slot_perf.as<int32_t>();
-        }
-        a.cap = cap;
-        a.pcap = pcap;
-        FL_RC(out_pos.ensure((size_t)n * cap * 4));
-        FL_RC(out_flag.ensure((size_t)n * cap));
-        FL_RC(out_perf.ensure((size_t)n * pcap * 4));
-        FL_RC(meta.ensure((size_t)n * 12));
-        FL_RC(counters.ensure(8));
-        a.out_pos = out_pos.as<int32_t>();
-        a.out_flag = out_flag.as<int8_t>();
-        a.out_perf = out_perf.as<int32_t>();
-        a.meta = meta.as<uint32_t>();
-        a.counters = counters.as<uint32_t>();
-        FL_TRY(hipMemsetAsync(a.counters, 0, 8, st));
-        // lanes per read: a wave for the reads of hundreds of entries; 8, about the
-        // start positions of a read that maps once, for many reads; 32 for the few
-        // thousand that leave the chip idle either way, where one step covers a
-        // read's lists (1,000 reads, both strands: 0.373 ms on the device with 32,
-        // 0.414 with 8; 2M reads: 38.1 and 32.2 ms)
-        auto grid = [&](unsigned g) { return dim3((n + FB / g - 1) / (FB / g)); };
-        if (global) hipLaunchKernelGGL((fl_pair<64, true>), grid(64), dim3(FB), 0, st, a);
-        else if (n < 4096) hipLaunchKernelGGL((fl_pair<32, false>), grid(32), dim3(FB), 0, st, a);
-        else hipLaunchKernelGGL((fl_pair<8, false>), grid(8), dim3(FB), 0, st, a);
-        FL_TRY(hipGetLastError());
-        uint32_t tot[2];
-        FL_TRY(hipMemcpyAsync(tot, a.counters, 8, hipMemcpyDeviceToHost, st));
-        meta_h.resize((size_t)n * 3);
-        FL_TRY(hipMemcpyAsync(meta_h.data(), a.meta, (size_t)n * 12, hipMemcpyDeviceToHost, st));
-        FL_TRY(hipStreamSynchronize(st));
-        pos_h.resize(tot[0]);
-        flag_h.resize(tot[0]);
-        perf_h.resize(tot[1]);
-        if (tot[0]) {
-            FL_TRY(hipMemcpyAsync(pos_h.data(), a.out_pos, (size_t)tot[0] * 4,
-                                  hipMemcpyDeviceToHost, st));
-            FL_TRY(hipMemcpyAsync(flag_h.data(), a.out_flag, tot[0], hipMemcpyDeviceToHost, st));
-        }
-        if (tot[1])
-            FL_TRY(hipMemcpyAsync(perf_h.data(), a.out_perf, (size_t)tot[1] * 4,
-                                  hipMemcpyDeviceToHost, st));
-        FL_TRY(hipStreamSynchronize(st));
+        b.release();
+        b = n;
+        return SRM_OK;
+    }
+
+    template <class T> int get(std::vector<T> &h, const GBuf &b, size_t n)
+    {
+        h.resize(n);
+        if (n) FL_TRY(hipMemcpyAsync(h.data(), b.p, n * sizeof(T), hipMemcpyDeviceToHost, st));
         return SRM_OK;
     }
 };
 
 namespace {
+
+// lookups, lists and pairing of the call's strands
+int launch_search(srm_dfilter *G, const Call &c)
+{
+    const uint32_t n = c.s[0].f.n_reads;
+    const uint64_t nl = c.n_lists;
+    // reads per block: CREADS while that fills the chip twice over, fewer below
+    const uint32_t per = (uint32_t)std::min<size_t>(CREADS, std::max<size_t>(4, n / 512));
+    const dim3 grid((n + per - 1) / per, (unsigned)c.n);
+    hipLaunchKernelGGL(fl_count, grid, dim3(FB), 0, G->st, c, per);
+    FL_TRY(hipGetLastError());
+    // both strands' lengths in one sum: the second strand's offsets count from its
+    // first (list_org), modulo 2^32
+    size_t tmp = 0;
+    const int items = (int)((nl + 1) * (uint64_t)c.n);
+    FL_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, G->list_cnt.as<uint32_t>(),
+                                            G->list_start.as<uint32_t>(), items, G->st));
+    FL_RC(G->cub_tmp.ensure(tmp));
+    FL_TRY(hipcub::DeviceScan::ExclusiveSum(G->cub_tmp.p, tmp, G->list_cnt.as<uint32_t>(),
+                                            G->list_start.as<uint32_t>(), items, G->st));
+    hipLaunchKernelGGL(fl_fill, grid, dim3(FB), 0, G->st, c, per);
+    FL_TRY(hipGetLastError());
+    // lanes per read: a wave for the reads of hundreds of entries (below); 8, about
+    // the start positions of a read that maps once, for many reads; 32 for the few
+    // thousand that leave the chip idle either way, where one step covers a read's
+    // lists (1,000 reads, both strands: 0.373 ms on the device with 32, 0.414 with 8;
+    // 2M reads: 38.1 and 32.2 ms)
+    auto pgrid = [&](unsigned g) { return dim3((n + FB / g - 1) / (FB / g), (unsigned)c.n); };
+    if (n < 4096) hipLaunchKernelGGL((fl_pair<32, false>), pgrid(32), dim3(FB), 0, G->st, c);
+    else hipLaunchKernelGGL((fl_pair<8, false>), pgrid(8), dim3(FB), 0, G->st, c);
+    FL_TRY(hipGetLastError());
+    return SRM_OK;
+}
+
+int launch_batch(srm_dfilter *G, const Call &c)
+{
+    const uint32_t n = c.s[0].f.n_reads;
+    const dim3 grid(n / FB + 1, (unsigned)c.n);
+    hipLaunchKernelGGL(fl_batch_count, grid, dim3(FB), 0, G->st, c);
+    FL_TRY(hipGetLastError());
+    size_t tmp = 0;
+    const int items = (int)(((uint64_t)n + 1) * (uint64_t)c.n);
+    FL_TRY(hipcub::DeviceScan::ExclusiveScan(nullptr, tmp, G->cnt.as<Counts>(), G->start.as<Counts>(),
+                                             CountsSum(), Counts(), items, G->st));
+    FL_RC(G->cub_tmp.ensure(tmp));
+    FL_TRY(hipcub::DeviceScan::ExclusiveScan(G->cub_tmp.p, tmp, G->cnt.as<Counts>(),
+                                             G->start.as<Counts>(), CountsSum(), Counts(), items,
+                                             G->st));
+    hipLaunchKernelGGL(fl_batch_write, grid, dim3(FB), 0, G->st, c);
+    FL_TRY(hipGetLastError());
+    hipLaunchKernelGGL(fl_batch_end, dim3(1, (unsigned)c.n), dim3(FB), 0, G->st, c);
+    FL_TRY(hipGetLastError());
+    return SRM_OK;
+}
+
+// strand x's reads that outgrew the LDS slots, run again with slots in HBM (1024, then
+// 65534 entries); their entries follow the others'
+int run_overflow(srm_dfilter *G, const Call &call, int x, Header &h)
+{
+    Call c = call;
+    c.s[0] = call.s[x];
+    c.n = 1;
+    FArgs &a = c.s[0].f;
+    int from = 0;
+    uint32_t left = h.counters[2];
+    // (65534: a count word of 0xFFFF | 0xFFFF << 16 would read as the overflow mark)
+    for (uint32_t cap : {1024u, 65534u}) {
+        if (!left) break;
+        const uint32_t per = (uint32_t)std::max<size_t>(1, ((size_t)256 << 20) / ((size_t)cap * 9));
+        FL_RC(G->over[x][1 - from].ensure((size_t)left * 4));
+        FL_TRY(srm::launch_reset(a.counters + 2, 1, G->st));
+        for (uint32_t b = 0; b < left; b += per) {
+            const uint32_t m = std::min(per, left - b);
+            FL_RC(G->slot_pos.ensure((size_t)m * cap * 4));
+            FL_RC(G->slot_flag.ensure((size_t)m * cap));
+            FL_RC(G->slot_perf.ensure((size_t)m * cap * 4));
+            const size_t ne = h.counters[0], np = h.counters[1];
+            FL_RC(G->grow(G->out_pos[x], (ne + (size_t)m * cap) * 4, ne * 4));
+            FL_RC(G->grow(G->out_flag[x], ne + (size_t)m * cap, ne));
+            FL_RC(G->grow(G->out_perf[x], (np + (size_t)m * cap) * 4, np * 4));
+            a.slot_pos = G->slot_pos.as<int32_t>();
+            a.slot_flag = G->slot_flag.as<int8_t>();
+            a.slot_perf = G->slot_perf.as<int32_t>();
+            a.out_pos = G->out_pos[x].as<int32_t>();
+            a.out_flag = G->out_flag[x].as<int8_t>();
+            a.out_perf = G->out_perf[x].as<int32_t>();
+            a.todo = G->over[x][from].as<uint32_t>() + b;
+            a.n_todo = m;
+            a.over = G->over[x][1 - from].as<uint32_t>();
+            a.cap = a.pcap = cap;
+            hipLaunchKernelGGL((fl_pair<64, true>), dim3((m + FB / 64 - 1) / (FB / 64)), dim3(FB), 0,
+                               G->st, c);
+            FL_TRY(hipGetLastError());
+            FL_TRY(hipMemcpyAsync(h.counters, a.counters, 12, hipMemcpyDeviceToHost, G->st));
+            FL_TRY(hipStreamSynchronize(G->st));
+        }
+        left = h.counters[2];
+        from = 1 - from;
+    }
+    if (left) {
+        uint32_t r = 0;
+        FL_TRY(hipMemcpy(&r, G->over[x][from].p, 4, hipMemcpyDeviceToHost));
+        return srm::set_error(SRM_ENOMEM, "read %u holds more than 65534 filter entries", r);
+    }
+    return SRM_OK;
+}
+
+// one or both strands (strands: bit 0 forward, bit 1 reverse) over the reads on the
+// device, at most one of the strands when `nl` lists leave no room for two in one sum
+int run_strands(srm_dfilter *G, Call c, const uint8_t *blocked, const uint16_t *read_len,
+                const uint8_t *read_k, srm_filter **out)
+{
+    const uint64_t nl = c.n_lists;
+    const uint32_t n = c.s[0].f.n_reads;
+    // the batch pass runs on the device unless separators have to come along that
+    // outweigh it (a byte a base; the host's pass takes tens of nanoseconds a read), or
+    // its lists of flushes and walked reads run over (below): then the host's pass over
+    // the downloaded entries
+    bool on_device = !blocked || G->glen / 64 <= n;
+    if (on_device && blocked) {
+        FL_RC(G->upload(G->blocked, blocked, G->glen));
+        c.blocked = G->blocked.as<uint8_t>();
+    }
+    FL_RC(G->list_cnt.ensure((nl + 1) * 4 * (size_t)c.n));
+    FL_RC(G->list_lo.ensure((nl + 1) * 4 * (size_t)c.n));
+    FL_RC(G->list_start.ensure((nl + 1) * 4 * (size_t)c.n));
+    FL_RC(G->cnt.ensure(((size_t)n + 1) * sizeof(Counts) * (size_t)c.n));
+    FL_RC(G->start.ensure(((size_t)n + 1) * sizeof(Counts) * (size_t)c.n));
+    FL_RC(G->by_rank.ensure((size_t)n * 4 * (size_t)c.n));
+    FL_RC(G->unsafe.ensure((size_t)MAX_UNSAFE * 4 * (size_t)c.n));
+    FL_RC(G->walk.ensure((size_t)MAX_WALK * 4 * (size_t)c.n));
+    // candidates and perfect hits of both strands are 1-1.2 a read, 16-20 bytes each
+    const size_t head = sizeof(Header) * (size_t)c.n;
+    FL_RC(G->out.ensure(head + std::max<size_t>(STAGE_OUT, 28 * (size_t)n)));
+    for (int x = 0; x < c.n; ++x) {
+        // about one position a list beside its terminator
+        FL_RC(G->flat[x].ensure((nl * 2 + 1024) * 4));
+        FL_RC(G->out_pos[x].ensure((size_t)n * ECAP * 4));
+        FL_RC(G->out_flag[x].ensure((size_t)n * ECAP));
+        FL_RC(G->out_perf[x].ensure((size_t)n * PCAP * 4));
+        FL_RC(G->meta[x].ensure((size_t)n * 12));
+        FL_RC(G->over[x][0].ensure((size_t)n * 4));
+    }
+    auto bind = [&] {
+        for (int x = 0; x < c.n; ++x) {
+            Strand &s = c.s[x];
+            FArgs &a = s.f;
+            s.hdr = G->out.as<Header>() + x;
+            s.flat_cap = G->flat[x].cap / 4;
+            s.cnt = G->cnt.as<Counts>() + (size_t)x * ((size_t)n + 1);
+            s.start = G->start.as<Counts>() + (size_t)x * ((size_t)n + 1);
+            s.by_rank = G->by_rank.as<uint32_t>() + (size_t)x * n;
+            s.unsafe = G->unsafe.as<uint32_t>() + (size_t)x * MAX_UNSAFE;
+            s.walk = G->walk.as<uint32_t>() + (size_t)x * MAX_WALK;
+            a.list_cnt = G->list_cnt.as<uint32_t>() + (size_t)x * (nl + 1);
+            a.list_lo = G->list_lo.as<uint32_t>() + (size_t)x * (nl + 1);
+            a.list_start = G->list_start.as<uint32_t>() + (size_t)x * (nl + 1);
+            a.flat = G->flat[x].as<uint32_t>();
+            a.counters = s.hdr->counters;
+            a.out_pos = G->out_pos[x].as<int32_t>();
+            a.out_flag = G->out_flag[x].as<int8_t>();
+            a.out_perf = G->out_perf[x].as<int32_t>();
+            a.meta = G->meta[x].as<uint32_t>();
+            a.over = G->over[x][0].as<uint32_t>();
+            a.todo = nullptr;
+            a.n_todo = n;
+            a.cap = ECAP;
+            a.pcap = PCAP;
+        }
+        c.blob = G->out.as<unsigned char>() + head;
+        c.blob_cap = G->out.cap - head;
+    };
+    bind();
+    FL_RC(launch_search(G, c));
+    if (on_device) FL_RC(launch_batch(G, c));
+    // the headers and the first part of the output; what did not fit is made room for
+    // and run again
+    Header h[2];
+    const auto *so = (const unsigned char *)G->stage_out;
+    auto fetch = [&]() -> int {
+        FL_TRY(hipEventRecord(G->ev[1], G->st));
+        FL_TRY(hipMemcpyAsync(G->stage_out, G->out.p, std::min(G->out.cap, head + STAGE_OUT),
+                              hipMemcpyDeviceToHost, G->st));
+        FL_TRY(hipStreamSynchronize(G->st));
+        std::memcpy(h, so, head);
+        return SRM_OK;
+    };
+    if (!on_device) {   // the list total, which fl_batch_end would have left
+        hipLaunchKernelGGL(fl_totals, dim3(1, (unsigned)c.n), dim3(64), 0, G->st, c);
+        FL_TRY(hipGetLastError());
+    }
+    FL_RC(fetch());
+    bool again = false;
+    for (int x = 0; x < c.n; ++x)
+        if ((uint64_t)h[x].flat > c.s[x].flat_cap) {
+            FL_RC(G->flat[x].ensure(((size_t)h[x].flat + h[x].flat / 8) * 4));
+            again = true;
+        }
+    if (again) {
+        bind();
+        FL_RC(launch_search(G, c));
+        if (on_device) FL_RC(launch_batch(G, c));
+        FL_RC(fetch());
+    }
+    again = false;
+    for (int x = 0; x < c.n; ++x) {
+        G->last_flat += h[x].flat;
+        G->last_overflow += h[x].counters[2];
+        if (h[x].counters[2]) {
+            FL_RC(run_overflow(G, c, x, h[x]));
+            again = true;
+        }
+    }
+    // the counters of the reads the batch pass lists start over
+    auto batch_again = [&]() -> int {
+        bind();
+        for (int x = 0; x < c.n; ++x) FL_TRY(srm::launch_reset(&c.s[x].hdr->n_unsafe, 3, G->st));
+        FL_RC(launch_batch(G, c));
+        return fetch();
+    };
+    if (again && on_device) FL_RC(batch_again());
+    if (on_device && !h[0].blob_ok) {
+        const BlobAt b = blob_at(h[0].total, c.n > 1 ? h[1].total : Counts());
+        // (the headers' entry counts stay: the output is made anew behind them)
+        FL_RC(G->grow(G->out, head + b.bytes, head));
+        FL_RC(batch_again());
+    }
+    FL_TRY(hipEventElapsedTime(&G->last_ms, G->ev[0], G->ev[1]));
+    for (int x = 0; x < c.n; ++x)
+        if (h[x].n_flush > MAX_FLUSH || h[x].n_unsafe > MAX_UNSAFE || h[x].walk_words > MAX_WALK)
+            on_device = false;
+    if (!on_device) {
+        std::vector<uint32_t> meta_h[2];
+        std::vector<int32_t> pos_h[2], perf_h[2];
+        std::vector<int8_t> flag_h[2];
+        for (int x = 0; x < c.n; ++x) {
+            FL_RC(G->get(meta_h[x], G->meta[x], (size_t)n * 3));
+            FL_RC(G->get(pos_h[x], G->out_pos[x], h[x].counters[0]));
+            FL_RC(G->get(flag_h[x], G->out_flag[x], h[x].counters[0]));
+            FL_RC(G->get(perf_h[x], G->out_perf[x], h[x].counters[1]));
+        }
+        FL_TRY(hipStreamSynchronize(G->st));
+        auto pass = [&](int x) {
+            out[x] = batch_pass(MetaAcc{meta_h[x], pos_h[x], flag_h[x], perf_h[x]}, n, read_len, read_k,
+                                G->glen, blocked, (int)c.s[0].f.cv);
+        };
+        std::thread other;   // the two strands' passes side by side
+        if (c.n > 1) {
+            try {
+                other = std::thread(pass, 1);
+            } catch (...) {   // no thread to be had: both passes on this one
+                pass(1);
+            }
+        }
+        pass(0);
+        if (other.joinable()) other.join();
+        return SRM_OK;
+    }
+    // the output: from the first copy when it is all there, else into page-locked memory
+    const BlobAt b = blob_at(h[0].total, c.n > 1 ? h[1].total : Counts());
+    std::shared_ptr<void> hold;
+    if (b.bytes <= STAGE_OUT) {
+        void *p = std::malloc(std::max<size_t>(b.bytes, 1));
+        if (p) hold = std::shared_ptr<void>(p, std::free);
+    } else {
+        hold = G->pool->take(b.bytes);
+    }
+    if (!hold) return srm::set_error(SRM_ENOMEM, "no memory for %zu bytes of filter results", (size_t)b.bytes);
+    auto *m = (unsigned char *)hold.get();
+    std::vector<uint32_t> walk_h[2];
+    bool wait = false;
+    if (b.bytes <= STAGE_OUT) {
+        std::memcpy(m, so + head, b.bytes);
+    } else {
+        FL_TRY(hipMemcpyAsync(m, c.blob, b.bytes, hipMemcpyDeviceToHost, G->st));
+        wait = true;
+    }
+    for (int x = 0; x < c.n; ++x)
+        if (h[x].walk_words) {
+            walk_h[x].resize(h[x].walk_words);
+            FL_TRY(hipMemcpyAsync(walk_h[x].data(), c.s[x].walk, (size_t)h[x].walk_words * 4,
+                                  hipMemcpyDeviceToHost, G->st));
+            wait = true;
+        }
+    if (wait) FL_TRY(hipStreamSynchronize(G->st));
+    for (int x = 0; x < c.n; ++x) {
+        std::vector<Walked> walked;
+        for (size_t w = 0; w < walk_h[x].size();) {
+            const uint32_t *v = walk_h[x].data() + w;
+            Walked k;
+            k.read = v[0];
+            k.rank = v[1];
+            k.cand_start = v[2];
+            const uint32_t ne = v[3];
+            for (uint32_t e = 0; e < ne; ++e) {
+                k.pos.push_back((int32_t)v[4 + e]);
+                k.flag.push_back((int8_t)(int32_t)v[4 + ne + e]);
+            }
+            walked.push_back(std::move(k));
+            w += 4 + 2 * (size_t)ne;
+        }
+        auto F = std::make_unique<srm_filter>();
+        F->dense = std::make_unique<Pieces>();
+        Pieces &R = *F->dense;
+        R.hold = hold;
+        R.c_pos = (int64_t *)(m + b.c_pos[x]);
+        R.p_pos = (int64_t *)(m + b.p_pos[x]);
+        R.c_read = (int32_t *)(m + b.c_read[x]);
+        R.p_read = (int32_t *)(m + b.p_read[x]);
+        R.c_w = (uint16_t *)(m + b.c_w[x]);
+        R.c_flag = m + b.c_flag[x];
+        R.n_perf = h[x].total.perf;
+        finish(R, F->batch_end, std::vector<Flush>(h[x].flush, h[x].flush + h[x].n_flush), walked,
+               read_len, read_k, G->glen, blocked);
+        out[x] = F.release();
+    }
+    return SRM_OK;
+}
 
 // one or both strands (strands: bit 0 forward, bit 1 reverse) over one upload of
 // the reads
@@ -529,136 +1154,93 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     const auto &list_base = plan.list_base;
     const uint64_t nl = list_base[n_reads];
     const uint64_t rbytes = plan.read_bytes;
-    G->last_lists = 0;
+    G->last_lists = nl * (strands == 3 ? 2 : 1);
     G->last_flat = 0;
     G->last_overflow = 0;
     FL_TRY(hipSetDevice(G->device));
     FL_TRY(hipEventRecord(G->ev[0], G->st));
-    FL_RC(G->upload(G->par, dpar.data(), dpar.size() * sizeof(DParam)));
-    FL_RC(G->upload(G->gram, gram.data(), gram.size() * 2));
-    FL_RC(G->upload(G->reads, reads, rbytes));
-    FL_RC(G->pack(G->reads, rbytes, G->read_pk, G->read_odd));
-    FL_RC(G->upload(G->roff, read_off, n_reads * 8));
-    FL_RC(G->upload(G->rlen, read_len, n_reads * 2));
-    FL_RC(G->upload(G->pid, pid.data(), n_reads * 2));
-    FL_RC(G->upload(G->list_base, list_base.data(), (n_reads + 1) * 4));
-    FL_RC(G->list_cnt.ensure((nl + 1) * 4));
-    FL_RC(G->list_lo.ensure((nl + 1) * 4));
-    FL_RC(G->list_start.ensure((nl + 1) * 4));
+    // the inputs, one after another in one buffer
+    struct Part {
+        const void *src;
+        size_t bytes, at;
+    };
+    Part part[] = {{dpar.data(), dpar.size() * sizeof(DParam), 0},
+                   {list_base.data(), (n_reads + 1) * 4, 0},
+                   {pid.data(), n_reads * 2, 0},
+                   {read_off, n_reads * 8, 0},
+                   {reads, rbytes, 0}};
+    size_t all = 0;
+    for (Part &p : part) {
+        p.at = all;
+        all = (all + p.bytes + 255) & ~(size_t)255;
+    }
+    FL_RC(G->in.ensure(all + 64));   // slack: whole 16-byte words of the reads are read
+    if (all <= STAGE_IN) {
+        for (const Part &p : part) std::memcpy((char *)G->stage_in + p.at, p.src, p.bytes);
+        FL_TRY(hipMemcpyAsync(G->in.p, G->stage_in, all, hipMemcpyHostToDevice, G->st));
+    } else {
+        for (const Part &p : part)
+            if (p.bytes)
+                FL_TRY(hipMemcpyAsync(G->in.as<char>() + p.at, p.src, p.bytes, hipMemcpyHostToDevice,
+                                      G->st));
+    }
+    const char *in = G->in.as<char>();
+    FL_RC(G->pack(in + part[4].at, rbytes, G->read_pk, G->read_odd));
+    Call c{};
+    c.n_lists = nl;
+    for (const Params &p : plan.params) c.kmax = std::max(c.kmax, p.k);
     FArgs a{};
     a.qix = G->dq.as<DQ>();
-    a.par = G->par.as<DParam>();
-    a.gram = G->gram.as<uint16_t>();
+    a.par = (const DParam *)(in + part[0].at);
     a.genome = G->genome.as<char>();
     a.glen = G->glen;
-    a.reads = G->reads.as<char>();
+    a.reads = in + part[4].at;
     a.read_pk = G->read_pk.as<uint32_t>();
     a.read_odd = G->read_odd.as<uint32_t>();
     a.gen_pk = G->gen_pk.as<uint32_t>();
     a.gen_odd = G->gen_odd.as<uint32_t>();
-    a.roff = G->roff.as<uint64_t>();
-    a.rlen = G->rlen.as<uint16_t>();
-    a.pid = G->pid.as<uint16_t>();
+    a.roff = (const uint64_t *)(in + part[3].at);
+    a.pid = (const uint16_t *)(in + part[2].at);
     a.n_reads = (uint32_t)n_reads;
     a.cv = (uint32_t)chunk_value;
-    a.list_base = G->list_base.as<uint32_t>();
-    a.list_cnt = G->list_cnt.as<uint32_t>();
-    a.list_lo = G->list_lo.as<uint32_t>();
-    a.list_start = G->list_start.as<uint32_t>();
-    // per strand: the device's entries and perfect hits for the batch pass, which
-    // runs on the host once both strands' device work is done (the two strands'
-    // passes side by side)
-    std::vector<uint32_t> meta_s[2];
-    std::vector<int32_t> pos_s[2], perf_s[2];
-    std::vector<int8_t> flag_s[2];
-    for (int dr : {0, 4}) {
-        if (!(strands & (dr ? 2 : 1))) continue;
-        a.dr = dr;
-        G->last_lists += nl;
-        // reads per block: CREADS while that fills the chip twice over, fewer below
-        const uint32_t per = (uint32_t)std::min<size_t>(CREADS, std::max<size_t>(4, n_reads / 512));
-        const unsigned grid = (unsigned)((n_reads + per - 1) / per);
-        FL_TRY(hipMemsetAsync(a.list_cnt + nl, 0, 4, G->st));
-        hipLaunchKernelGGL(fl_count, dim3(grid), dim3(FB), 0, G->st, a, per);
-        FL_TRY(hipGetLastError());
-        size_t tmp = 0;
-        FL_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, a.list_cnt, G->list_start.as<uint32_t>(),
-                                                (int)(nl + 1), G->st));
-        FL_RC(G->cub_tmp.ensure(tmp));
-        FL_TRY(hipcub::DeviceScan::ExclusiveSum(G->cub_tmp.p, tmp, a.list_cnt,
-                                                G->list_start.as<uint32_t>(), (int)(nl + 1), G->st));
-        uint32_t total = 0;
-        FL_TRY(hipMemcpyAsync(&total, G->list_start.as<uint32_t>() + nl, 4, hipMemcpyDeviceToHost,
-                              G->st));
-        FL_TRY(hipStreamSynchronize(G->st));
-        G->last_flat += total;
-        FL_RC(G->flat.ensure((size_t)total * 4 + 4));
-        a.flat = G->flat.as<uint32_t>();
-        hipLaunchKernelGGL(fl_fill, dim3(grid), dim3(FB), 0, G->st, a, per);
-        FL_TRY(hipGetLastError());
-
-        std::vector<uint32_t> &meta = meta_s[dr ? 1 : 0];
-        std::vector<int32_t> &pos = pos_s[dr ? 1 : 0], &perf = perf_s[dr ? 1 : 0];
-        std::vector<int8_t> &flag = flag_s[dr ? 1 : 0];
-        FL_RC(G->pair(a, false, nullptr, (uint32_t)n_reads, ECAP, PCAP, meta, pos, flag, perf));
-        // reads that outgrew the LDS slots run again with slots in HBM
-        std::vector<uint32_t> over;
-        for (size_t r = 0; r < n_reads; ++r)
-            if (meta[3 * r + 2] == OVERFLOW_MARK) over.push_back((uint32_t)r);
-        G->last_overflow += over.size();
-        // (65534: a count word of 0xFFFF | 0xFFFF << 16 would read as the overflow mark)
-        for (uint32_t cap : {1024u, 65534u}) {
-            if (over.empty()) break;
-            const size_t per = std::max<size_t>(1, ((size_t)256 << 20) / ((size_t)cap * 9));
-            std::vector<uint32_t> still;
-            for (size_t b = 0; b < over.size(); b += per) {
-                const uint32_t m = (uint32_t)std::min(per, over.size() - b);
-                std::vector<uint32_t> m2;
-                std::vector<int32_t> p2, q2;
-                std::vector<int8_t> f2;
-                FL_RC(G->pair(a, true, over.data() + b, m, cap, cap, m2, p2, f2, q2));
-                const uint32_t es = (uint32_t)pos.size(), ps = (uint32_t)perf.size();
-                pos.insert(pos.end(), p2.begin(), p2.end());
-                flag.insert(flag.end(), f2.begin(), f2.end());
-                perf.insert(perf.end(), q2.begin(), q2.end());
-                for (uint32_t t = 0; t < m; ++t) {
-                    const uint32_t r = over[b + t];
-                    if (m2[3 * t + 2] == OVERFLOW_MARK) {
-                        still.push_back(r);
-                        continue;
-                    }
-                    meta[3 * r + 0] = es + m2[3 * t + 0];
-                    meta[3 * r + 1] = ps + m2[3 * t + 1];
-                    meta[3 * r + 2] = m2[3 * t + 2];
-                }
-            }
-            over.swap(still);
-        }
-        if (!over.empty())
-            return srm::set_error(SRM_ENOMEM, "read %u holds more than 65534 filter entries",
-                                  over[0]);
-        FL_TRY(hipEventRecord(G->ev[1], G->st));
-        FL_TRY(hipEventSynchronize(G->ev[1]));
-        FL_TRY(hipEventElapsedTime(&G->last_ms, G->ev[0], G->ev[1]));
+    a.list_base = (const uint32_t *)(in + part[1].at);
+    srm_filter **outs[2] = {out_fwd, out_rev};
+    // both strands in each launch, while their lists fit one sum
+    if (strands == 3 && nl < ((uint64_t)1 << 30) - 1) {
+        c.n = 2;
+        c.s[0].f = c.s[1].f = a;
+        c.s[1].f.dr = 4;
+        srm_filter *F[2] = {nullptr, nullptr};
+        const int rc = run_strands(G, c, blocked, read_len, read_k, F);
+        *out_fwd = F[0];
+        *out_rev = F[1];
+        return rc;
     }
-    auto pass = [&](int x) {
-        *(x ? out_rev : out_fwd) =
-            batch_pass(MetaAcc{meta_s[x], pos_s[x], flag_s[x], perf_s[x]}, n_reads, read_len,
-                       read_k, G->glen, blocked, chunk_value);
-    };
-    if ((strands & 3) == 3) {
-        std::thread other;
-        try {
-            other = std::thread(pass, 1);
-        } catch (...) {   // no thread to be had: both passes on this one
-            pass(1);
-        }
-        pass(0);
-        if (other.joinable()) other.join();
-    } else {
-        pass((strands & 1) ? 0 : 1);
+    for (int x = 0; x < 2; ++x) {
+        if (!(strands & (1 << x))) continue;
+        c.n = 1;
+        c.s[0].f = a;
+        c.s[0].f.dr = x ? 4 : 0;
+        FL_RC(run_strands(G, c, blocked, read_len, read_k, outs[x]));
     }
     return SRM_OK;
+}
+
+// run_device, its exceptions as error codes; whatever fails, nothing of the call's is
+// still being copied when it returns
+int run_call(srm_dfilter *G, const uint8_t *blocked, const char *reads, const uint64_t *read_off,
+             const uint16_t *read_len, const uint8_t *read_k, size_t n_reads, int strands,
+             int chunk_value, srm_filter **out_fwd, srm_filter **out_rev)
+{
+    int rc;
+    try {
+        rc = run_device(G, blocked, reads, read_off, read_len, read_k, n_reads, strands, chunk_value,
+                        out_fwd, out_rev);
+    } catch (const std::bad_alloc &) {
+        rc = srm::set_error(SRM_ENOMEM, "no memory on the host for %zu reads", n_reads);
+    }
+    if (rc != SRM_OK) (void)hipStreamSynchronize(G->st);
+    return rc;
 }
 
 }  // namespace
@@ -686,8 +1268,11 @@ int srm_dfilter_create(srm_ctx *ctx, const srm_index *ix, const char *genome, si
     if (hipSetDevice(G->device) != hipSuccess ||
         hipEventCreate(&G->ev[0]) != hipSuccess || hipEventCreate(&G->ev[1]) != hipSuccess)
         return fail(srm::set_error(SRM_EDEVICE, "event creation failed"));
+    if (hipHostMalloc(&G->stage_in, STAGE_IN, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(&G->stage_out, 2 * sizeof(Header) + STAGE_OUT, hipHostMallocDefault) != hipSuccess)
+        return fail(srm::set_error(SRM_ENOMEM, "no page-locked memory for the filter's staging"));
     int rc = G->upload(G->genome, genome, glen);
-    if (!rc) rc = G->pack(G->genome, glen, G->gen_pk, G->gen_odd);
+    if (!rc) rc = G->pack(G->genome.p, glen, G->gen_pk, G->gen_odd);
     if (rc) return fail(rc);
     std::vector<DQ> dq(32);
     std::memset(dq.data(), 0, dq.size() * sizeof(DQ));
@@ -737,8 +1322,8 @@ int srm_dfilter_run(srm_dfilter *G, const uint8_t *blocked, const char *reads,
         return SRM_OK;
     }
     srm_filter *F = nullptr;
-    const int rc = run_device(G, blocked, reads, read_off, read_len, read_k, n_reads,
-                              do_reverse ? 2 : 1, chunk_value, &F, &F);
+    const int rc = run_call(G, blocked, reads, read_off, read_len, read_k, n_reads,
+                            do_reverse ? 2 : 1, chunk_value, &F, &F);
     if (rc != SRM_OK) {
         delete F;
         return rc;
@@ -760,8 +1345,8 @@ int srm_dfilter_run2(srm_dfilter *G, const uint8_t *blocked, const char *reads,
         return SRM_OK;
     }
     srm_filter *Ff = nullptr, *Fr = nullptr;
-    const int rc = run_device(G, blocked, reads, read_off, read_len, read_k, n_reads, 3,
-                              chunk_value, &Ff, &Fr);
+    const int rc = run_call(G, blocked, reads, read_off, read_len, read_k, n_reads, 3, chunk_value,
+                            &Ff, &Fr);
     if (rc != SRM_OK) {
         delete Ff;
         delete Fr;

@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -115,7 +116,35 @@ struct srm_index {
     }
 };
 
+namespace srm_filter_impl {
+
+// the device filter's result (filter_batch.h): the candidates by each entry's own flag
+// and the perfect hits, in memory that `hold` keeps, and the pieces of the former that
+// are left
+struct Pieces {
+    struct Piece {
+        uint64_t at, n;
+    };
+    std::shared_ptr<void> hold;
+    int32_t *c_read = nullptr, *p_read = nullptr;
+    int64_t *c_pos = nullptr, *p_pos = nullptr;
+    uint8_t *c_flag = nullptr;
+    uint16_t *c_w = nullptr;
+    uint64_t n_cand = 0, n_perf = 0;
+    std::vector<Piece> piece;
+    void add(uint64_t at, uint64_t n)
+    {
+        if (n == 0) return;
+        if (!piece.empty() && piece.back().at + piece.back().n == at) piece.back().n += n;
+        else piece.push_back({at, n});
+    }
+};
+
+}  // namespace srm_filter_impl
+
+// the host's arrays, or (dense set) the device filter's pieces and batch_end
 struct srm_filter {
+    std::unique_ptr<srm_filter_impl::Pieces> dense;
     std::vector<int32_t> c_read;
     std::vector<int64_t> c_pos;
     std::vector<uint8_t> c_flag;

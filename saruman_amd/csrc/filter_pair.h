@@ -62,18 +62,25 @@ struct FArgs {
     int8_t *slot_flag;
     int32_t *slot_perf;
     uint32_t cap, pcap;
-    uint32_t *counters;      // [2] compact entries / perfect hits written so far
+    uint32_t *counters;      // [3] compact entries / perfect hits written so far, overflows
     int32_t *out_pos;
     int8_t *out_flag;
     int32_t *out_perf;
-    uint32_t *meta;          // [3 * n_todo]: ent_off, perf_off, n_ent | n_perf << 16
+    uint32_t *meta;          // [3 * n_reads]: ent_off, perf_off, n_ent | n_perf << 16
     // the reads' bytes as 2-bit codes and as a mask of the bytes other than ACGT
     // (pack16), at the same offsets
     const uint32_t *read_pk;
     const uint32_t *read_odd;
     const uint32_t *gen_pk;      // the genome's, likewise
     const uint32_t *gen_odd;
+    // list_start[0]: nonzero where another strand's lists come before in one sum.
+    // Offsets into flat count from it, modulo 2^32
+    uint32_t list_org;
+    uint32_t *over;              // reads that outgrew their slots (counters[2] of them)
 };
+
+// where list i starts in flat
+SRM_HD inline uint32_t list_at(const FArgs &a, uint64_t i) { return a.list_start[i] - a.list_org; }
 
 SRM_HD inline char dcomp(char c)
 {
@@ -381,7 +388,7 @@ SRM_HD inline int add_start(Store &s, int32_t pos, int flag, int possible, int e
 SRM_HD inline uint64_t chunk_end(const FArgs &a, uint32_t r)
 {
     const uint64_t next_chunk = ((uint64_t)(r / a.cv) + 1) * a.cv;
-    return a.list_start[a.list_base[next_chunk < a.n_reads ? next_chunk : a.n_reads]];
+    return list_at(a, a.list_base[next_chunk < a.n_reads ? next_chunk : a.n_reads]);
 }
 
 // the pair passes of one start position (hash.c:606-794): list aa's element off,
@@ -402,16 +409,16 @@ SRM_HD inline bool pair_matches(const FArgs &a, const DParam &P, uint32_t lb, ui
     // D(b, 1), D(b, 2), ... up to the next 0 (Q12): the element at a's index, then
     // one ascending run of list b (or of the list after b when b is empty).
     for (int b = aa + 1; b < half; ++b) {
-        const uint64_t at = (uint64_t)a.list_start[lb + b] + off;
+        const uint64_t at = (uint64_t)list_at(a, lb + b) + off;
         const uint32_t P0 = at < flat_end ? a.flat[at] : 0u;
         if (P0 == 0) continue;                 // the scan never starts
         const long rstart = (long)b * q + 1;
-        uint64_t lo = (uint64_t)a.list_start[lb + b] + 1, hi = lo;
-        const uint64_t nb = a.list_start[lb + b + 1];
+        uint64_t lo = (uint64_t)list_at(a, lb + b) + 1, hi = lo;
+        const uint64_t nb = list_at(a, lb + b + 1);
         if (lo < nb) {
             hi = nb - 1;                       // list b from index 1
         } else if ((uint64_t)lb + b + 2 <= a.list_base[a.n_reads]) {
-            hi = (uint64_t)a.list_start[lb + b + 2] - 1;   // the next list
+            hi = (uint64_t)list_at(a, lb + b + 2) - 1;   // the next list
         }
         if (!scan_run(a.flat, lo, hi, flat_end, gs + rstart - k, gs + rstart + k, true, P0, need, hits))
             continue;
@@ -436,8 +443,8 @@ SRM_HD inline bool pair_matches(const FArgs &a, const DParam &P, uint32_t lb, ui
     for (int j = 0; j < half; ++j) {
         const int lim = half - 1 - j - aa < 0 ? -(half - 1 - j - aa) : half - 1 - j - aa;
         const long nin = (long)(half - j - 1) * q + 1 + P.rest;
-        const uint64_t lo = a.list_start[lb + half + j];
-        const uint64_t hi = (uint64_t)a.list_start[lb + half + j + 1] - 1;
+        const uint64_t lo = list_at(a, lb + half + j);
+        const uint64_t hi = (uint64_t)list_at(a, lb + half + j + 1) - 1;
         if (!scan_run(a.flat, lo, hi, flat_end, gs + nin - lim, gs + nin + lim, j - aa >= 0, 0u, need,
                       hits))
             continue;
@@ -470,7 +477,7 @@ SRM_HD inline void seashore(const FArgs &a, uint32_t r, Store &s)
     const uint64_t flat_end = chunk_end(a, r);
     for (int aa = 0; aa < P.half; ++aa) {
         for (uint64_t off = 0;; ++off) {
-            const uint64_t at = (uint64_t)a.list_start[lb + aa] + off;
+            const uint64_t at = (uint64_t)list_at(a, lb + aa) + off;
             const uint32_t Pa = at < flat_end ? a.flat[at] : 0u;
             if (Pa == 0) break;
             const long gs = (long)Pa - ((long)aa * P.q + 1);
