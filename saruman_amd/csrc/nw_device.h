@@ -96,7 +96,7 @@ struct RecArgs {
 };
 
 // band height for the banded kernels: d = row - col in [-k, max(2s+k, w-L)]
-inline int band_cells(const srm_cand &c)
+__host__ __device__ inline int band_cells(const srm_cand &c)
 {
     const int k = c.k;
     const int s = (c.flag <= 7 && (c.flag & 2)) ? k : 0;

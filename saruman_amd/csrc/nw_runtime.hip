@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "nw_device.h"
+#include "plan.h"
 #include "saruman_hip.h"
 
 // ---------------------------------------------------------------------------
@@ -169,7 +170,8 @@ struct HostPlan {
     std::vector<UploadPart> part;
     std::vector<uint32_t> band_idx, rest_idx, bytes_idx, all_idx, tiles;
     std::vector<uint64_t> kv, kv_tmp, tile_off, off_rest, off_all, off_bytes;
-    std::vector<uint32_t> mat;   // per candidate: its plain-kernel matrix elements
+    size_t band_n = 0;                   // banded candidates
+    std::vector<srm::PlanSums> sums;     // the device plan's (one)
 };
 }  // namespace
 
@@ -266,9 +268,8 @@ inline uint32_t plain_mat_elems(const srm_cand &c)
     return (uint32_t)((plain_elems_of(c) + 63) & ~(size_t)63);
 }
 
-// matrix offsets and chunks of the candidates idx (mat: every candidate's matrix
-// elements)
-void plan_plain(const std::vector<uint32_t> &idx, const uint32_t *mat, size_t budget_elems,
+// matrix offsets and chunks of the candidates idx
+void plan_plain(const std::vector<uint32_t> &idx, const srm_cand *cand, size_t budget_elems,
                 std::vector<uint64_t> &off, std::vector<PlainChunk> &chunks)
 {
     off.resize(idx.size());
@@ -276,7 +277,7 @@ void plan_plain(const std::vector<uint32_t> &idx, const uint32_t *mat, size_t bu
     PlainChunk cur;
     size_t acc = 0;
     for (size_t j = 0; j < idx.size(); ++j) {
-        const size_t m = mat[idx[j]];
+        const size_t m = plain_mat_elems(cand[idx[j]]);
         if (cur.count && acc + m > budget_elems) {
             cur.mat_elems = acc;
             chunks.push_back(cur);
@@ -320,7 +321,14 @@ int plan_all(srm_job *j)
         }
         all_idx.push_back(t);
     }
-    plan_plain(all_idx, hp.mat.data(), j->mat_budget_elems, hp.off_all, j->chunks_all);
+    // (the descriptors as the upload left them on the device: the caller's are its own)
+    std::vector<srm_cand> cand((size_t)j->n);
+    if (j->n) {
+        HIP_TRY(hipMemcpyAsync(cand.data(), j->d_cand.p, cand.size() * sizeof(srm_cand),
+                               hipMemcpyDeviceToHost, j->ctx->stream));
+        HIP_TRY(hipStreamSynchronize(j->ctx->stream));
+    }
+    plan_plain(all_idx, cand.data(), j->mat_budget_elems, hp.off_all, j->chunks_all);
     int rc;
     if ((rc = upload(j->ctx, j->d_idx_all, all_idx.data(), all_idx.size()))) return rc;
     if ((rc = upload(j->ctx, j->d_off_all, hp.off_all.data(), hp.off_all.size()))) return rc;
@@ -564,6 +572,281 @@ void radix_sort_kv(std::vector<uint64_t> &kv, std::vector<uint64_t> &tmp, int lo
         });
         kv.swap(tmp);
     }
+}
+
+// why candidate t was refused
+int refused(const srm_cand &c, int t, int why)
+{
+    switch (why) {
+    case srm::E_RANGE:
+        return fail(SRM_EINVAL, "candidate %d: L=%d w=%d outside 1..%d / 0..%d", t, c.L, c.w,
+                    SRM_MAX_L, SRM_MAX_W);
+    case srm::E_BYTES: return fail(SRM_EINVAL, "candidate %d: byte range out of bounds", t);
+    case srm::E_READ: return fail(SRM_EINVAL, "candidate %d: read codes out of bounds", t);
+    case srm::E_GENOME: return fail(SRM_EINVAL, "candidate %d: genome window out of bounds", t);
+    default: return fail(SRM_EINVAL, "candidate %d: window codes out of bounds", t);
+    }
+}
+
+// a class whose tiles (the last of plan.tiles) are made: their order, the launch's
+// blocks, their scratch
+void add_class(srm_job *j, BandClass &bc, size_t &scratch_words)
+{
+    std::vector<uint32_t> &tiles = j->plan.tiles;
+    std::vector<uint64_t> &tile_off = j->plan.tile_off;
+    bc.ntiles = (uint32_t)(tiles.size() / 4) - bc.tile_begin;
+    {
+        // longest tiles first (each tile keeps one L mod 8): the persistent
+        // waves then end on the short ones, and the class's last wave
+        // finishes soon after the others
+        std::vector<std::array<uint32_t, 4>> tv(bc.ntiles);
+        std::memcpy(tv.data(), tiles.data() + 4 * (size_t)bc.tile_begin,
+                    sizeof(uint32_t) * 4 * bc.ntiles);
+        std::stable_sort(tv.begin(), tv.end(),
+                         [](const std::array<uint32_t, 4> &x,
+                            const std::array<uint32_t, 4> &y) { return x[2] > y[2]; });
+        std::memcpy(tiles.data() + 4 * (size_t)bc.tile_begin, tv.data(),
+                    sizeof(uint32_t) * 4 * bc.ntiles);
+    }
+    if (j->unit) {
+        // bits_band_kernel: one wave per tile, blocks of block_waves waves
+        bc.blocks = (int)((bc.ntiles + j->block_waves - 1) / j->block_waves);
+    } else {
+        // persistent grid: as many 4-wave blocks as stay resident on every
+        // CU (occupancy of this kernel instance), never more waves than tiles
+        int per_cu = srm::band_occupancy(bc.nw, false);
+        const int tuned = j->ctx->tuning.blocks_per_cu[bc.nw];
+        if (tuned > 0) per_cu = std::min(per_cu, tuned);
+        int max_blocks = std::max(1, j->ctx->num_cus * per_cu);
+        bc.blocks = (int)std::min<size_t>((bc.ntiles + 3) / 4, (size_t)max_blocks);
+    }
+    // every tile keeps its band until trace_kernel has walked it
+    for (uint32_t u = 0; u < bc.ntiles; ++u) {
+        tile_off.push_back(scratch_words);
+        const int tmax = (int)tiles[4 * (bc.tile_begin + u) + 2];
+        scratch_words += (j->unit)
+                             ? srm::bits_tile_words(bc.nw, tmax, j->walk_ck != 0)
+                             : tile_scratch_words(bc.nw, tmax);
+    }
+    j->classes.push_back(bc);
+}
+
+// The plan of an upload on the host: candidates validated and classified over
+// contiguous ranges on several threads (the lists keep index order, ranges
+// concatenated in order; the first failing candidate, the lowest index, is the one
+// reported), the banded ones in tile order
+int plan_host(srm_job *j, const srm::PlanIn &in, const srm_cand *cand, int n, size_t &ops_end,
+              size_t &scratch_words)
+{
+    srm_ctx *ctx = j->ctx;
+    HostPlan &hp = j->plan;
+    const unsigned TV = plan_threads((size_t)n);
+    std::vector<UploadPart> &part = hp.part;
+    part.resize(TV);
+    for (UploadPart &P : part) P.reset();
+    par_ranges(TV, (size_t)n, [&](unsigned u, size_t a, size_t b) {
+        UploadPart &P = part[u];
+        for (size_t t = a; t < b; ++t) {
+            const srm_cand &c = cand[t];
+            const int r = srm::classify(in, c);
+            if (r >= srm::E_RANGE) {
+                P.bad = (int)t;
+                P.why = r;
+                return;
+            }
+            P.ops_end = std::max(P.ops_end, (size_t)c.ops_off + srm_ops_words(c.w, c.k));
+            P.rows += 2 * ((size_t)c.w + c.k);
+            if (r == srm::K_BAND) P.maxL = std::max<uint32_t>(P.maxL, c.L);
+            (r == srm::K_BAND ? P.band : r == srm::K_REST ? P.rest : P.bytes).push_back((uint32_t)t);
+        }
+    });
+    std::vector<uint32_t> &band_idx = hp.band_idx, &rest_idx = hp.rest_idx,
+                          &bytes_idx = hp.bytes_idx;
+    band_idx.clear();
+    rest_idx.clear();
+    bytes_idx.clear();
+    for (const UploadPart &P : part) {
+        if (P.bad >= 0) return refused(cand[P.bad], P.bad, P.why);
+        ops_end = std::max(ops_end, P.ops_end);
+        j->rec_rows_bound += P.rows;
+    }
+    if (TV == 1) {
+        band_idx.swap(part[0].band);
+        rest_idx.swap(part[0].rest);
+        bytes_idx.swap(part[0].bytes);
+    } else {
+        for (const UploadPart &P : part) {
+            band_idx.insert(band_idx.end(), P.band.begin(), P.band.end());
+            rest_idx.insert(rest_idx.end(), P.rest.begin(), P.rest.end());
+            bytes_idx.insert(bytes_idx.end(), P.bytes.begin(), P.bytes.end());
+        }
+    }
+    hp.band_n = band_idx.size();
+
+    // ---- banded plan: sort by (class, L mod 8, L desc), 64-candidate tiles that
+    // never mix L mod 8: a tile's lanes then cross the 8-column blocks of their
+    // band scratch at the same traceback steps (a walk moves one column per
+    // diagonal step), so the wave reloads band words together
+    const uint32_t tile_cands = ctx->tuning.tile_cands == 32 ? 32u : 64u;
+    const size_t nb = band_idx.size();
+    const unsigned TB = plan_threads(nb);
+    // sort word of every banded candidate, in index order: its index (bits 0-31),
+    // k (bits 32-35) and from bit 36 the key: class (5 bits), L mod 8 (3 bits),
+    // then maxL - L in lb bits (L descending), the fields of the order above from
+    // the top down
+    uint32_t maxL = 0;
+    for (const UploadPart &P : part) maxL = std::max(maxL, P.maxL);
+    int lb = 1;
+    while ((1u << lb) <= maxL) ++lb;
+    std::vector<uint64_t> &kv = hp.kv;
+    kv.resize(nb);
+    par_ranges(TB, nb, [&](unsigned, size_t a, size_t b) {
+        for (size_t i = a; i < b; ++i) {
+            const srm_cand &c = cand[band_idx[i]];
+            const uint32_t cl = (uint32_t)srm::band_class(in, c);
+            const uint32_t key = (((cl << 3) | ((uint32_t)c.L & 7u)) << lb) | (maxL - c.L);
+            kv[i] = ((uint64_t)key << 36) | ((uint64_t)c.k << 32) | band_idx[i];
+        }
+    });
+    static_assert(SRM_BAND_KMAX < 16, "k of a banded candidate fits 4 bits");
+    radix_sort_kv(kv, hp.kv_tmp, 36, 8 + lb, TB);
+    par_ranges(TB, nb, [&](unsigned, size_t a, size_t b) {
+        for (size_t i = a; i < b; ++i) band_idx[i] = (uint32_t)kv[i];
+    });
+    // by position in tile order
+    auto cls_at = [&](size_t i) { return (int)(kv[i] >> (36 + lb + 3)); };
+    auto lmod_at = [&](size_t i) { return (int)((kv[i] >> (36 + lb)) & 7u); };
+    auto k_at = [&](size_t i) { return (uint32_t)(kv[i] >> 32) & 15u; };
+    auto L_at = [&](size_t i) { return maxL - ((uint32_t)(kv[i] >> 36) & ((1u << lb) - 1u)); };
+    std::vector<uint32_t> &tiles = hp.tiles;   // uint4 per tile
+    tiles.clear();
+    std::vector<uint64_t> &tile_off = hp.tile_off;   // word offset of each tile's band
+    tile_off.clear();
+    {
+        size_t i = 0;
+        while (i < band_idx.size()) {
+            BandClass bc;
+            const int ci = cls_at(i);
+            bc.nw = ci / 2 + 1;
+            bc.tile_begin = (uint32_t)(tiles.size() / 4);
+            bc.maxL = 0;
+            // the sort words are in key order: the class's end and each run's end by
+            // binary search
+            const size_t e = (size_t)(std::partition_point(
+                                          kv.begin() + (std::ptrdiff_t)i, kv.end(),
+                                          [&](const uint64_t &x) {
+                                              return (int)(x >> (36 + lb + 3)) == ci;
+                                          }) -
+                                      kv.begin());
+            for (size_t g = i; g < e;) {
+                // one run of equal L mod 8, L descending: a tile's first read is its
+                // longest (its k maximum is filled in below, over all tiles at once)
+                const int lm = lmod_at(g);
+                const size_t ge = (size_t)(std::partition_point(
+                                               kv.begin() + (std::ptrdiff_t)g,
+                                               kv.begin() + (std::ptrdiff_t)e,
+                                               [&](const uint64_t &x) {
+                                                   return (int)((x >> (36 + lb)) & 7u) == lm;
+                                               }) -
+                                           kv.begin());
+                for (size_t s = g; s < ge; s += tile_cands) {
+                    const uint32_t cnt = (uint32_t)std::min<size_t>(tile_cands, ge - s);
+                    const uint32_t lmax = L_at(s);
+                    tiles.push_back((uint32_t)s);
+                    tiles.push_back(cnt);
+                    tiles.push_back(lmax);
+                    tiles.push_back(0u);
+                    bc.maxL = std::max(bc.maxL, (int)lmax);
+                }
+                g = ge;
+            }
+            add_class(j, bc, scratch_words);
+            i = e;
+        }
+    }
+    // every tile's largest k, over the tiles on several host threads
+    {
+        const size_t nt = tiles.size() / 4;
+        par_ranges(plan_threads(nt * tile_cands), nt, [&](unsigned, size_t a, size_t b) {
+            for (size_t t = a; t < b; ++t) {
+                const size_t s0 = tiles[4 * t], c0 = tiles[4 * t + 1];
+                uint32_t kmax = 0;
+                for (size_t u = s0; u < s0 + c0; ++u) kmax = std::max(kmax, k_at(u));
+                tiles[4 * t + 3] = kmax;
+            }
+        });
+    }
+    return SRM_OK;
+}
+
+// The same on the device (plan_gpu.hip), for unit costs: the descriptors go up, are
+// checked, counted and put in tile order there, and the host makes the tiles from the
+// counts.  The host's plan of a million candidates read and wrote them five times on
+// up to 8 threads, before the first copy began: a batch of 1,000,000 reads host to host
+// 11.3 -> 7.6 ms, one of 50,000 2.1 -> 1.67 ms.  The plan's scratch is the results'
+// buffer, so the batch has to have as many as fill it (fewer: the host's plan takes
+// 0.1 ms and less).
+constexpr int PLAN_DEVICE_MIN = 16384;
+static_assert(PLAN_DEVICE_MIN * sizeof(srm_result) >= srm::PLAN_SCRATCH, "the results' buffer holds it");
+
+int plan_device(srm_job *j, const srm::PlanIn &in, const srm_cand *cand, int n, size_t &ops_end,
+                size_t &scratch_words, bool &planned)
+{
+    planned = false;
+    if (!j->unit || n < PLAN_DEVICE_MIN) return SRM_OK;
+    srm_ctx *ctx = j->ctx;
+    HostPlan &hp = j->plan;
+    const size_t N = (size_t)n;
+    int rc;
+    if ((rc = upload(ctx, j->d_cand, cand, N))) return rc;
+    if ((rc = ctx->ensure(j->d_cand_tile, N * sizeof(srm_cand) + 64))) return rc;
+    if ((rc = ctx->ensure(j->d_perm, N * 4 + 64))) return rc;
+    if ((rc = ctx->ensure(j->d_idx_rest, N * 4 + 64))) return rc;
+    if ((rc = ctx->ensure(j->d_idx_bytes, N * 4 + 64))) return rc;
+    if ((rc = ctx->ensure(j->d_res, N * sizeof(srm_result)))) return rc;
+    HIP_TRY(srm::launch_plan(in, (const srm_cand *)j->d_cand.p, (uint32_t)n, j->d_res.p,
+                             (uint32_t *)j->d_perm.p, (srm_cand *)j->d_cand_tile.p,
+                             (uint32_t *)j->d_idx_rest.p, (uint32_t *)j->d_idx_bytes.p, ctx->stream));
+    hp.sums.resize(1);
+    srm::PlanSums &S = hp.sums[0];
+    HIP_TRY(hipMemcpyAsync(&S, j->d_res.p, sizeof S, hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if (S.first_bad != ~0u)
+        return refused(cand[S.first_bad], (int)S.first_bad, srm::classify(in, cand[S.first_bad]));
+    if (S.too_long) return SRM_OK;   // beyond the bins
+    ops_end = (size_t)S.ops_end;
+    j->rec_rows_bound = (size_t)S.rows;
+    hp.band_n = S.n_band;
+    hp.band_idx.clear();
+    // the other paths' lists, in index order
+    hp.rest_idx.resize(S.n_rest);
+    hp.bytes_idx.resize(S.n_bytes);
+    if (S.n_rest)
+        HIP_TRY(hipMemcpyAsync(hp.rest_idx.data(), j->d_idx_rest.p, 4 * (size_t)S.n_rest,
+                               hipMemcpyDeviceToHost, ctx->stream));
+    if (S.n_bytes)
+        HIP_TRY(hipMemcpyAsync(hp.bytes_idx.data(), j->d_idx_bytes.p, 4 * (size_t)S.n_bytes,
+                               hipMemcpyDeviceToHost, ctx->stream));
+    if (S.n_rest || S.n_bytes) HIP_TRY(hipStreamSynchronize(ctx->stream));
+    std::sort(hp.rest_idx.begin(), hp.rest_idx.end());
+    std::sort(hp.bytes_idx.begin(), hp.bytes_idx.end());
+    std::vector<uint32_t> &tiles = hp.tiles;
+    tiles.clear();
+    hp.tile_off.clear();
+    BandClass bc;
+    srm::plan_tiles(S.bin, ctx->tuning.tile_cands == 32 ? 32u : 64u,
+                    [&](int cl) {
+                        bc = BandClass();
+                        bc.nw = cl / 2 + 1;
+                        bc.tile_begin = (uint32_t)(tiles.size() / 4);
+                    },
+                    [&](uint32_t at, uint32_t count, int maxL) {
+                        tiles.insert(tiles.end(), {at, count, (uint32_t)maxL, 0u});
+                        bc.maxL = std::max(bc.maxL, maxL);
+                    },
+                    [&] { add_class(j, bc, scratch_words); });
+    planned = true;
+    return SRM_OK;
 }
 }  // namespace
 
@@ -891,261 +1174,50 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
     j->mm = mismatch;
     j->unit = (match == 0 && mismatch == 1);
     j->resident_genome = (win_words == nullptr);
-    const bool band_ok = match >= 0 && mismatch >= 1;
 
-    // ---- validate and classify, over contiguous ranges of candidates on several
-    // host threads; the lists keep index order (ranges concatenated in order) and
-    // the first failing candidate (lowest index) is the one reported
-    const uint64_t read_codes = (uint64_t)n_read_words * 16;
-    const uint64_t win_codes =
-        j->resident_genome ? (uint64_t)ctx->genome_words * 16 : (uint64_t)n_win_words * 16;
-    const uint64_t pad = SRM_CODE_PAD;
-    enum { K_BAND, K_REST, K_BYTES, E_RANGE, E_BYTES, E_READ, E_GENOME, E_WIN };
-    auto classify = [&](const srm_cand &c) -> int {
-        if (c.L < 1 || c.L > SRM_MAX_L || c.w > SRM_MAX_W) return E_RANGE;
-        if (c.bits & SRM_CAND_BYTES) {
-            if ((uint64_t)c.read_off + c.L > n_read_bytes || (uint64_t)c.win_off + c.w > n_win_bytes)
-                return E_BYTES;
-            return K_BYTES;
-        }
-        // code arrays: pad codes readable before 0 and after the end (the caller's
-        // arrays start with SRM_CODE_PAD pad codes for uploaded arrays, and offsets
-        // count from the first code after them).  Written without subtraction: an
-        // array shorter than the padding must fail, not wrap.
-        if ((uint64_t)c.read_off + c.L + 2 * pad > read_codes) return E_READ;
-        if (j->resident_genome) {
-            // the genome carries SRM_CODE_PAD codes of padding at both ends
-            if ((uint64_t)c.win_off < pad || (uint64_t)c.win_off + c.w + pad > win_codes)
-                return E_GENOME;
-        } else if ((uint64_t)c.win_off + c.w + 2 * pad > win_codes) {
-            return E_WIN;
-        }
-        // banded: exact-band conditions, and w >= L - k (a shorter window can never
-        // hold a hit; the window code stream reads up to L + 93 codes past win_off)
-        if (band_ok && c.k <= SRM_BAND_KMAX && band_cells(c) <= SRM_BAND_MAX &&
-            (int)c.w >= (int)c.L - (int)c.k)
-            return K_BAND;
-        return K_REST;
-    };
-    const unsigned TV = plan_threads((size_t)n);
-    HostPlan &hp = j->plan;
-    std::vector<UploadPart> &part = hp.part;
-    part.resize(TV);
-    for (UploadPart &P : part) P.reset();
-    hp.mat.resize((size_t)n);
-    par_ranges(TV, (size_t)n, [&](unsigned u, size_t a, size_t b) {
-        UploadPart &P = part[u];
-        for (size_t t = a; t < b; ++t) {
-            const srm_cand &c = cand[t];
-            const int r = classify(c);
-            if (r >= E_RANGE) {
-                P.bad = (int)t;
-                P.why = r;
-                return;
-            }
-            hp.mat[t] = plain_mat_elems(c);
-            P.ops_end = std::max(P.ops_end, (size_t)c.ops_off + srm_ops_words(c.w, c.k));
-            P.rows += 2 * ((size_t)c.w + c.k);
-            if (r == K_BAND) P.maxL = std::max<uint32_t>(P.maxL, c.L);
-            (r == K_BAND ? P.band : r == K_REST ? P.rest : P.bytes).push_back((uint32_t)t);
-        }
-    });
-    std::vector<uint32_t> &band_idx = hp.band_idx, &rest_idx = hp.rest_idx,
-                          &bytes_idx = hp.bytes_idx;
-    band_idx.clear();
-    rest_idx.clear();
-    bytes_idx.clear();
-    size_t ops_end = 0;
-    j->rec_rows_bound = 0;
-    for (const UploadPart &P : part) {
-        if (P.bad >= 0) {
-            const srm_cand &c = cand[P.bad];
-            switch (P.why) {
-            case E_RANGE:
-                return fail(SRM_EINVAL, "candidate %d: L=%d w=%d outside 1..%d / 0..%d", P.bad,
-                            c.L, c.w, SRM_MAX_L, SRM_MAX_W);
-            case E_BYTES: return fail(SRM_EINVAL, "candidate %d: byte range out of bounds", P.bad);
-            case E_READ: return fail(SRM_EINVAL, "candidate %d: read codes out of bounds", P.bad);
-            case E_GENOME:
-                return fail(SRM_EINVAL, "candidate %d: genome window out of bounds", P.bad);
-            default: return fail(SRM_EINVAL, "candidate %d: window codes out of bounds", P.bad);
-            }
-        }
-        ops_end = std::max(ops_end, P.ops_end);
-        j->rec_rows_bound += P.rows;
-    }
-    if (TV == 1) {
-        band_idx.swap(part[0].band);
-        rest_idx.swap(part[0].rest);
-        bytes_idx.swap(part[0].bytes);
-    } else {
-        for (const UploadPart &P : part) {
-            band_idx.insert(band_idx.end(), P.band.begin(), P.band.end());
-            rest_idx.insert(rest_idx.end(), P.rest.begin(), P.rest.end());
-            bytes_idx.insert(bytes_idx.end(), P.bytes.begin(), P.bytes.end());
-        }
-    }
-    j->n_band = band_idx.size();
-    j->n_rest = rest_idx.size();
-    j->n_bytes = bytes_idx.size();
-    j->ops_words = ops_end;
-
-    // ---- banded plan: sort by (class, L mod 8, L desc), 64-candidate tiles that
-    // never mix L mod 8: a tile's lanes then cross the 8-column blocks of their
-    // band scratch at the same traceback steps (a walk moves one column per
-    // diagonal step), so the wave reloads band words together
-    // cls = 2 nw + (L >= split_len): a class split by read length (tuning) runs as
-    // two launches, the short reads with a smaller LDS staging size
-    const int merge_below = std::max(1, std::min(8, ctx->tuning.merge_below));
-    const int split_len = ctx->tuning.split_len;
-    const uint32_t tile_cands = ctx->tuning.tile_cands == 32 ? 32u : 64u;
+    srm::PlanIn in{};
+    in.read_codes = (uint64_t)n_read_words * 16;
+    in.win_codes = j->resident_genome ? (uint64_t)ctx->genome_words * 16 : (uint64_t)n_win_words * 16;
+    in.read_bytes = n_read_bytes;
+    in.win_bytes = n_win_bytes;
+    in.resident_genome = j->resident_genome;
+    in.band_ok = match >= 0 && mismatch >= 1;
+    in.merge_below = std::max(1, std::min(8, ctx->tuning.merge_below));
+    in.split_len = ctx->tuning.split_len;
     j->block_waves = ctx->tuning.block_waves ? ctx->tuning.block_waves : 4;
     j->walk_ck = ctx->tuning.walk_layout;
-    const size_t nb = band_idx.size();
-    const unsigned TB = plan_threads(nb);
-    // sort word of every banded candidate, in index order: its index (bits 0-31),
-    // k (bits 32-35) and from bit 36 the key: class (5 bits), L mod 8 (3 bits),
-    // then maxL - L in lb bits (L descending), the fields of the order above from
-    // the top down
-    uint32_t maxL = 0;
-    for (const UploadPart &P : part) maxL = std::max(maxL, P.maxL);
-    int lb = 1;
-    while ((1u << lb) <= maxL) ++lb;
-    std::vector<uint64_t> &kv = hp.kv;
-    kv.resize(nb);
-    par_ranges(TB, nb, [&](unsigned, size_t a, size_t b) {
-        for (size_t i = a; i < b; ++i) {
-            const srm_cand &c = cand[band_idx[i]];
-            const uint32_t cl = 2u * (uint32_t)std::max((band_cells(c) + 7) / 8, merge_below) +
-                                (split_len > 0 && (int)c.L >= split_len ? 1u : 0u);
-            const uint32_t key = (((cl << 3) | ((uint32_t)c.L & 7u)) << lb) | (maxL - c.L);
-            kv[i] = ((uint64_t)key << 36) | ((uint64_t)c.k << 32) | band_idx[i];
-        }
-    });
-    static_assert(SRM_BAND_KMAX < 16, "k of a banded candidate fits 4 bits");
-    radix_sort_kv(kv, hp.kv_tmp, 36, 8 + lb, TB);
-    par_ranges(TB, nb, [&](unsigned, size_t a, size_t b) {
-        for (size_t i = a; i < b; ++i) band_idx[i] = (uint32_t)kv[i];
-    });
-    // by position in tile order
-    auto cls_at = [&](size_t i) { return (int)(kv[i] >> (36 + lb + 3)); };
-    auto lmod_at = [&](size_t i) { return (int)((kv[i] >> (36 + lb)) & 7u); };
-    auto k_at = [&](size_t i) { return (uint32_t)(kv[i] >> 32) & 15u; };
-    auto L_at = [&](size_t i) { return maxL - ((uint32_t)(kv[i] >> 36) & ((1u << lb) - 1u)); };
-    std::vector<uint32_t> &tiles = hp.tiles;   // uint4 per tile
-    tiles.clear();
-    j->classes.clear();
-    size_t scratch_words = 0;
-    std::vector<uint64_t> &tile_off = hp.tile_off;   // word offset of each tile's band
-    tile_off.clear();
-    // band classes run side by side on 4 streams unless the tuning says otherwise
-    // (1 = one after another on the context's stream)
+    // band classes run side by side unless the tuning says otherwise (1 = one after
+    // another on the context's stream): the unit-cost ones in one launch, others on 4
+    // streams or as many as it says
     const int want_streams = ctx->tuning.class_streams == 0 ? 4 : ctx->tuning.class_streams;
-    // -- the unit-cost classes side by side in one launch
     const bool concurrent = want_streams > 1;
-    j->one_launch = j->unit && concurrent && nb > 0;
     j->class_streams = concurrent && !j->unit ? std::min(want_streams, 8) : 0;
     while ((int)j->side.size() < j->class_streams) {   // default priority, like every stream here
         hipStream_t q = nullptr;
         HIP_TRY(hipStreamCreateWithFlags(&q, hipStreamNonBlocking));
         j->side.push_back(q);
     }
-    {
-        size_t i = 0;
-        while (i < band_idx.size()) {
-            BandClass bc;
-            const int ci = cls_at(i);
-            bc.nw = ci / 2;
-            bc.tile_begin = (uint32_t)(tiles.size() / 4);
-            bc.maxL = 0;
-            // the sort words are in key order: the class's end and each run's end by
-            // binary search
-            const size_t e = (size_t)(std::partition_point(
-                                          kv.begin() + (std::ptrdiff_t)i, kv.end(),
-                                          [&](const uint64_t &x) {
-                                              return (int)(x >> (36 + lb + 3)) == ci;
-                                          }) -
-                                      kv.begin());
-            for (size_t g = i; g < e;) {
-                // one run of equal L mod 8, L descending: a tile's first read is its
-                // longest (its k maximum is filled in below, over all tiles at once)
-                const int lm = lmod_at(g);
-                const size_t ge = (size_t)(std::partition_point(
-                                               kv.begin() + (std::ptrdiff_t)g,
-                                               kv.begin() + (std::ptrdiff_t)e,
-                                               [&](const uint64_t &x) {
-                                                   return (int)((x >> (36 + lb)) & 7u) == lm;
-                                               }) -
-                                           kv.begin());
-                for (size_t s = g; s < ge; s += tile_cands) {
-                    const uint32_t cnt = (uint32_t)std::min<size_t>(tile_cands, ge - s);
-                    const uint32_t lmax = L_at(s);
-                    tiles.push_back((uint32_t)s);
-                    tiles.push_back(cnt);
-                    tiles.push_back(lmax);
-                    tiles.push_back(0u);
-                    bc.maxL = std::max(bc.maxL, (int)lmax);
-                }
-                g = ge;
-            }
-            bc.ntiles = (uint32_t)(tiles.size() / 4) - bc.tile_begin;
-            {
-                // longest tiles first (each tile keeps one L mod 8): the persistent
-                // waves then end on the short ones, and the class's last wave
-                // finishes soon after the others
-                std::vector<std::array<uint32_t, 4>> tv(bc.ntiles);
-                std::memcpy(tv.data(), tiles.data() + 4 * (size_t)bc.tile_begin,
-                            sizeof(uint32_t) * 4 * bc.ntiles);
-                std::stable_sort(tv.begin(), tv.end(),
-                                 [](const std::array<uint32_t, 4> &x,
-                                    const std::array<uint32_t, 4> &y) { return x[2] > y[2]; });
-                std::memcpy(tiles.data() + 4 * (size_t)bc.tile_begin, tv.data(),
-                            sizeof(uint32_t) * 4 * bc.ntiles);
-            }
-            if (match == 0 && mismatch == 1) {
-                // bits_band_kernel: one wave per tile, blocks of block_waves waves
-                bc.blocks = (int)((bc.ntiles + j->block_waves - 1) / j->block_waves);
-            } else {
-                // persistent grid: as many 4-wave blocks as stay resident on every
-                // CU (occupancy of this kernel instance), never more waves than tiles
-                int per_cu = srm::band_occupancy(bc.nw, false);
-                const int tuned = ctx->tuning.blocks_per_cu[bc.nw];
-                if (tuned > 0) per_cu = std::min(per_cu, tuned);
-                int max_blocks = std::max(1, ctx->num_cus * per_cu);
-                bc.blocks = (int)std::min<size_t>((bc.ntiles + 3) / 4, (size_t)max_blocks);
-            }
-            // every tile keeps its band until trace_kernel has walked it
-            for (uint32_t u = 0; u < bc.ntiles; ++u) {
-                tile_off.push_back(scratch_words);
-                const int tmax = (int)tiles[4 * (bc.tile_begin + u) + 2];
-                scratch_words += (match == 0 && mismatch == 1)
-                                     ? srm::bits_tile_words(bc.nw, tmax, j->walk_ck != 0)
-                                     : tile_scratch_words(bc.nw, tmax);
-            }
-            j->classes.push_back(bc);
-            i = e;
-        }
-    }
-    // every tile's largest k, over the tiles on several host threads
-    {
-        const size_t nt = tiles.size() / 4;
-        par_ranges(plan_threads(nt * tile_cands), nt, [&](unsigned, size_t a, size_t b) {
-            for (size_t t = a; t < b; ++t) {
-                const size_t s0 = tiles[4 * t], c0 = tiles[4 * t + 1];
-                uint32_t kmax = 0;
-                for (size_t u = s0; u < s0 + c0; ++u) kmax = std::max(kmax, k_at(u));
-                tiles[4 * t + 3] = kmax;
-            }
-        });
-    }
-
-    // ---- device buffers
+    size_t ops_end = 0, scratch_words = 0;
+    j->rec_rows_bound = 0;
+    j->classes.clear();
+    HostPlan &hp = j->plan;
+    bool planned = false;
     int rc;
-    if ((rc = upload(ctx, j->d_cand, cand, (size_t)n))) return rc;
+    if ((rc = plan_device(j, in, cand, n, ops_end, scratch_words, planned))) return rc;
+    if (!planned && (rc = plan_host(j, in, cand, n, ops_end, scratch_words))) return rc;
+    j->n_band = hp.band_n;
+    j->n_rest = hp.rest_idx.size();
+    j->n_bytes = hp.bytes_idx.size();
+    j->ops_words = ops_end;
+    j->one_launch = j->unit && concurrent && j->n_band > 0;
+    // ---- device buffers
+    if (!planned && (rc = upload(ctx, j->d_cand, cand, (size_t)n))) return rc;
     if ((rc = upload(ctx, j->d_read_words, read_words, n_read_words))) return rc;
     if (!j->resident_genome && (rc = upload(ctx, j->d_win_words, win_words, n_win_words))) return rc;
     if ((rc = upload(ctx, j->d_read_bytes, read_bytes, read_bytes ? n_read_bytes : 0))) return rc;
     if ((rc = upload(ctx, j->d_win_bytes, win_bytes, win_bytes ? n_win_bytes : 0))) return rc;
+    if (!planned) {
+    const std::vector<uint32_t> &band_idx = hp.band_idx;
     if ((rc = upload(ctx, j->d_perm, band_idx.data(), band_idx.size()))) return rc;
     // the banded candidates in tile order (a wave reads its tile's descriptors as
     // one contiguous run, without the indirection through perm), gathered on the
@@ -1153,11 +1225,12 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
     if ((rc = ctx->ensure(j->d_cand_tile, band_idx.size() * sizeof(srm_cand) + 64))) return rc;
     HIP_TRY(launch_gather_cand((const srm_cand *)j->d_cand.p, (const uint32_t *)j->d_perm.p,
                                (srm_cand *)j->d_cand_tile.p, band_idx.size(), ctx->stream));
-    if ((rc = ctx->ensure(j->d_tile_score, std::max<size_t>(band_idx.size() * 4, 64)))) return rc;
-    if ((rc = upload(ctx, j->d_tiles, tiles.data(), tiles.size()))) return rc;
-    if ((rc = upload(ctx, j->d_tile_scratch, tile_off.data(), tile_off.size()))) return rc;
-    if ((rc = upload(ctx, j->d_idx_rest, rest_idx.data(), rest_idx.size()))) return rc;
-    if ((rc = upload(ctx, j->d_idx_bytes, bytes_idx.data(), bytes_idx.size()))) return rc;
+    }
+    if ((rc = ctx->ensure(j->d_tile_score, std::max<size_t>(j->n_band * 4, 64)))) return rc;
+    if ((rc = upload(ctx, j->d_tiles, hp.tiles.data(), hp.tiles.size()))) return rc;
+    if ((rc = upload(ctx, j->d_tile_scratch, hp.tile_off.data(), hp.tile_off.size()))) return rc;
+    if ((rc = upload(ctx, j->d_idx_rest, hp.rest_idx.data(), hp.rest_idx.size()))) return rc;
+    if ((rc = upload(ctx, j->d_idx_bytes, hp.bytes_idx.data(), hp.bytes_idx.size()))) return rc;
     if ((rc = ctx->ensure(j->d_queue, 64 * sizeof(uint32_t)))) return rc;
     if ((rc = ctx->ensure(j->d_scratch, std::max<size_t>(scratch_words * 4, 256)))) return rc;
     if ((rc = ctx->ensure(j->d_res, std::max<size_t>((size_t)n * sizeof(srm_result), 64)))) return rc;
@@ -1178,8 +1251,8 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
         budget = std::max<size_t>(std::min<size_t>(free_b / 4, (size_t)32 << 30), SRM_PLAIN_CHUNK);
     }
     j->mat_budget_elems = budget / 2;
-    plan_plain(rest_idx, hp.mat.data(), j->mat_budget_elems, off_rest, j->chunks_rest);
-    plan_plain(bytes_idx, hp.mat.data(), j->mat_budget_elems, off_bytes, j->chunks_bytes);
+    plan_plain(hp.rest_idx, cand, j->mat_budget_elems, off_rest, j->chunks_rest);
+    plan_plain(hp.bytes_idx, cand, j->mat_budget_elems, off_bytes, j->chunks_bytes);
     j->mat_elems_band = max_chunk({&j->chunks_rest, &j->chunks_bytes});
     j->chunks_all.clear();
     j->mat_elems_plain = 0;

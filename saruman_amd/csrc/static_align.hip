@@ -9,8 +9,9 @@
 // band scratch of every tile -- lives in one file-scope device array, `scratch`,
 // of SRM_STATIC_SCRATCH_BYTES.  Each GPU holds its own copy until the process
 // ends; its address is taken once per device with hipGetSymbolAddress and used
-// for every kernel argument and copy.  The host plan (the order by band class, L
-// mod 8 and L, and the tiles) is built in fixed host arrays, so the call
+// for every kernel argument and copy.  The plan (the order by band class, L mod 8 and
+// L, and the tiles) is made on the device, or by small calls in fixed host arrays, so
+// the call
 // allocates nothing on the host either.  Calls are serialised by a mutex: a call
 // returns when its results are in the caller's buffers, and the scratch then
 // holds that call's contents.
@@ -22,6 +23,7 @@
 #include <mutex>
 
 #include "nw_device.h"
+#include "plan.h"
 #include "saruman_hip.h"
 
 namespace {
@@ -43,11 +45,36 @@ uint8_t h_cls[SRM_STATIC_MAX_CAND];
 uint32_t h_tiles[4 * MAX_TILES];
 uint64_t h_tile_off[MAX_TILES];
 size_t h_lcount[MAX_L + 2];
+srm::PlanSums h_sums;
 
 struct Class {
     int nw = 0, maxL = 0;
     uint32_t tile_begin = 0, ntiles = 0;
 };
+
+// From this many candidates on the plan is made on the device (plan_gpu.hip), which
+// costs launches and a wait and then little per candidate.  Whole calls, host's plan and
+// device's, 50-250 bp: 3,317 candidates 140 and 146 us, 4,946 162 and 151, 16,408 246 and
+// 162, 49,055 554 and 203
+constexpr int PLAN_DEVICE_MIN = 4096;
+
+// why candidate t was refused
+int refused(const srm_cand &c, int t, int why)
+{
+    using srm::set_error;
+    switch (why) {
+    case srm::E_RANGE:
+        return set_error(SRM_EINVAL, "candidate %d: L=%d w=%d outside 1..%d / 0..%d", t, c.L, c.w,
+                         SRM_MAX_L, SRM_MAX_W);
+    case srm::E_BYTES: return set_error(SRM_EINVAL, "candidate %d: raw bytes need the plain kernel", t);
+    case srm::E_READ: return set_error(SRM_EINVAL, "candidate %d: read codes out of bounds", t);
+    case srm::E_WIN: return set_error(SRM_EINVAL, "candidate %d: window codes out of bounds", t);
+    case srm::E_OPS: return set_error(SRM_EINVAL, "candidate %d: transcript slot out of bounds", t);
+    default:
+        return set_error(SRM_EINVAL, "candidate %d needs the plain kernel (k=%d, band %d)", t, c.k,
+                         srm::band_cells(c));
+    }
+}
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -72,87 +99,19 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
         return set_error(SRM_EINVAL, "srm_align_static: null argument");
     if (n == 0) return SRM_OK;
 
-    // Everything below up to the size check runs on the host: a batch the call
-    // refuses never reaches the device.
-    // ---- validate: every candidate must fit the exact band and its arrays, as
-    // srm_job_upload checks them (the code arrays carry SRM_CODE_PAD codes of
-    // padding at both ends; offsets count from the first code after it)
-    const uint64_t pad = SRM_CODE_PAD;
-    const uint64_t read_codes = (uint64_t)n_read_words * 16, win_codes = (uint64_t)n_win_words * 16;
-    int maxL = 0;
-    for (int t = 0; t < n; ++t) {
-        const srm_cand &c = cand[t];
-        if (c.L < 1 || c.L > SRM_MAX_L || c.w > SRM_MAX_W)
-            return set_error(SRM_EINVAL, "candidate %d: L=%d w=%d outside 1..%d / 0..%d", t, c.L,
-                             c.w, SRM_MAX_L, SRM_MAX_W);
-        if (c.bits & SRM_CAND_BYTES)
-            return set_error(SRM_EINVAL, "candidate %d: raw bytes need the plain kernel", t);
-        if ((uint64_t)c.read_off + c.L + 2 * pad > read_codes)
-            return set_error(SRM_EINVAL, "candidate %d: read codes out of bounds", t);
-        if ((uint64_t)c.win_off + c.w + 2 * pad > win_codes)
-            return set_error(SRM_EINVAL, "candidate %d: window codes out of bounds", t);
-        if ((uint64_t)c.ops_off + srm_ops_words(c.w, c.k) > n_ops_words)
-            return set_error(SRM_EINVAL, "candidate %d: transcript slot out of bounds", t);
-        if (c.k > SRM_BAND_KMAX || srm::band_cells(c) > SRM_BAND_MAX || (int)c.w < (int)c.L - (int)c.k)
-            return set_error(SRM_EINVAL, "candidate %d needs the plain kernel (k=%d, band %d)", t,
-                             c.k, srm::band_cells(c));
-        h_cls[t] = (uint8_t)((srm::band_cells(c) + 7) / 8);
-        maxL = std::max(maxL, (int)c.L);
-    }
-
-    // ---- order by (class, L mod 8, L descending): a counting pass by L, then a
-    // stable one by (class, L mod 8), as srm_job_upload orders them
-    std::fill(h_lcount, h_lcount + maxL + 2, (size_t)0);
-    for (int t = 0; t < n; ++t) ++h_lcount[(size_t)(maxL - cand[t].L) + 1];
-    for (int x = 1; x <= maxL + 1; ++x) h_lcount[x] += h_lcount[x - 1];
-    for (int t = 0; t < n; ++t) h_tmp[h_lcount[maxL - cand[t].L]++] = (uint32_t)t;
-    size_t bk[9 * 8 + 1] = {};
-    auto key = [&](uint32_t t) { return (size_t)h_cls[t] * 8 + (cand[t].L & 7); };
-    for (int i = 0; i < n; ++i) ++bk[key(h_tmp[i]) + 1];
-    for (size_t x = 1; x < 9 * 8 + 1; ++x) bk[x] += bk[x - 1];
-    for (int i = 0; i < n; ++i) h_perm[bk[key(h_tmp[i])]++] = h_tmp[i];
-
-    // ---- tiles of up to 64 candidates of one class and one L mod 8; the band
-    // scratch of every tile, one after another
     const bool unit = match == 0 && mismatch == 1;
-    Class cls[9];
-    int ncls = 0;
-    size_t ntiles = 0, words = 0;
-    for (int i = 0; i < n;) {
-        Class &bc = cls[ncls++];
-        bc.nw = h_cls[h_perm[i]];
-        bc.tile_begin = (uint32_t)ntiles;
-        int e2 = i;
-        while (e2 < n && h_cls[h_perm[e2]] == bc.nw) ++e2;
-        for (int g = i; g < e2;) {
-            int ge = g;
-            while (ge < e2 && (cand[h_perm[ge]].L & 7) == (cand[h_perm[g]].L & 7)) ++ge;
-            for (int s = g; s < ge; s += 64) {
-                const int cnt = std::min(64, ge - s);
-                uint32_t kmax = 0, lmax = 0;
-                for (int u = s; u < s + cnt; ++u) {
-                    kmax = std::max<uint32_t>(kmax, cand[h_perm[u]].k);
-                    lmax = std::max<uint32_t>(lmax, cand[h_perm[u]].L);
-                }
-                h_tiles[4 * ntiles + 0] = (uint32_t)s;
-                h_tiles[4 * ntiles + 1] = (uint32_t)cnt;
-                h_tiles[4 * ntiles + 2] = lmax;
-                h_tiles[4 * ntiles + 3] = kmax;
-                h_tile_off[ntiles] = words;
-                words += unit ? srm::bits_tile_words(bc.nw, (int)lmax, false)
-                              : srm::tile_scratch_words(bc.nw, (int)lmax);
-                bc.maxL = std::max(bc.maxL, (int)lmax);
-                ++ntiles;
-            }
-            g = ge;
-        }
-        bc.ntiles = (uint32_t)ntiles - bc.tile_begin;
-        i = e2;
-    }
-    for (int p = 0; p < n; ++p) h_cand_tile[p] = cand[h_perm[p]];
+    // every candidate must fit the exact band and its arrays, as srm_job_upload checks
+    // them (the code arrays carry SRM_CODE_PAD codes of padding at both ends; offsets
+    // count from the first code after it)
+    srm::PlanIn in{};
+    in.read_codes = (uint64_t)n_read_words * 16;
+    in.win_codes = (uint64_t)n_win_words * 16;
+    in.ops_words = n_ops_words;
+    in.band_ok = in.only_band = true;
+    in.merge_below = 1;
 
-    // ---- the scratch layout: counters, descriptors in candidate and tile order,
-    // perm, scores, tiles, tile offsets, then the band scratch
+    // the scratch: counters, descriptors in candidate and tile order, perm, scores,
+    // then (below) tiles, tile offsets and the band scratch
     size_t at = 0;
     const size_t o_queue = at;
     at = align256(at + 64 * sizeof(uint32_t));
@@ -164,6 +123,116 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
     at = align256(at + (size_t)n * 4);
     const size_t o_score = at;
     at = align256(at + (size_t)n * 4);
+    unsigned char *base = nullptr;
+    hipStream_t st = (hipStream_t)stream;
+#define SA_TRY(expr)                                                                          \
+    do {                                                                                      \
+        hipError_t e_ = (expr);                                                               \
+        if (e_ != hipSuccess)                                                                 \
+            return set_error(SRM_EDEVICE, "%s failed: %s", #expr, hipGetErrorString(e_));     \
+    } while (0)
+
+    auto on_device = [&]() -> int {
+        SA_TRY(hipSetDevice(device));
+        if (!g_scratch[device]) {   // once per device, with the device current
+            void *p = nullptr;
+            const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+            if (e != hipSuccess || !p)
+                return set_error(SRM_EDEVICE, "hipGetSymbolAddress(scratch): %s", hipGetErrorString(e));
+            g_scratch[device] = (unsigned char *)p;
+        }
+        base = g_scratch[device];
+        return SRM_OK;
+    };
+
+    Class cls[9];
+    int ncls = 0;
+    size_t ntiles = 0, words = 0;
+    auto add_tile = [&](Class &bc, uint32_t first, uint32_t count, uint32_t lmax, uint32_t kmax) {
+        h_tiles[4 * ntiles + 0] = first;
+        h_tiles[4 * ntiles + 1] = count;
+        h_tiles[4 * ntiles + 2] = lmax;
+        h_tiles[4 * ntiles + 3] = kmax;
+        h_tile_off[ntiles] = words;
+        words += unit ? srm::bits_tile_words(bc.nw, (int)lmax, false)
+                      : srm::tile_scratch_words(bc.nw, (int)lmax);
+        bc.maxL = std::max(bc.maxL, (int)lmax);
+        ++bc.ntiles;
+        ++ntiles;
+    };
+    // ---- on the device, for unit costs: checked, counted and put in tile order there;
+    // the tiles follow from the counts
+    bool planned = false;
+    if (unit && n >= PLAN_DEVICE_MIN) {
+        if (const int rc = on_device()) return rc;
+        // (its own scratch lies at the end, where the bands come later)
+        unsigned char *sums = base + SRM_STATIC_SCRATCH_BYTES - align256(srm::PLAN_SCRATCH);
+        SA_TRY(hipMemcpyAsync(base + o_cand, cand, (size_t)n * sizeof(srm_cand), hipMemcpyHostToDevice, st));
+        SA_TRY(srm::launch_plan(in, (const srm_cand *)(base + o_cand), (uint32_t)n, sums,
+                                (uint32_t *)(base + o_perm), (srm_cand *)(base + o_cand_tile), nullptr,
+                                nullptr, st));
+        SA_TRY(hipMemcpyAsync(&h_sums, sums, sizeof h_sums, hipMemcpyDeviceToHost, st));
+        SA_TRY(hipStreamSynchronize(st));
+        if (h_sums.first_bad != ~0u)
+            return refused(cand[h_sums.first_bad], (int)h_sums.first_bad,
+                           srm::classify(in, cand[h_sums.first_bad]));
+        planned = h_sums.too_long == 0;
+        if (planned)
+            srm::plan_tiles(h_sums.bin, 64,
+                            [&](int cl) {
+                                cls[ncls].nw = cl / 2 + 1;
+                                cls[ncls].tile_begin = (uint32_t)ntiles;
+                            },
+                            [&](uint32_t first, uint32_t count, int lmax) {
+                                add_tile(cls[ncls], first, count, (uint32_t)lmax, 0u);
+                            },
+                            [&] { ++ncls; });
+    }
+    // ---- on the host: order by (class, L mod 8, L descending), a counting pass by L,
+    // then a stable one by (class, L mod 8); tiles of up to 64 candidates of one class
+    // and one L mod 8
+    if (!planned) {
+        int maxL = 0;
+        for (int t = 0; t < n; ++t) {
+            const int why = srm::classify(in, cand[t]);
+            if (why != srm::K_BAND) return refused(cand[t], t, why);
+            h_cls[t] = (uint8_t)((srm::band_cells(cand[t]) + 7) / 8);
+            maxL = std::max(maxL, (int)cand[t].L);
+        }
+        std::fill(h_lcount, h_lcount + maxL + 2, (size_t)0);
+        for (int t = 0; t < n; ++t) ++h_lcount[(size_t)(maxL - cand[t].L) + 1];
+        for (int x = 1; x <= maxL + 1; ++x) h_lcount[x] += h_lcount[x - 1];
+        for (int t = 0; t < n; ++t) h_tmp[h_lcount[maxL - cand[t].L]++] = (uint32_t)t;
+        size_t bk[9 * 8 + 1] = {};
+        auto key = [&](uint32_t t) { return (size_t)h_cls[t] * 8 + (cand[t].L & 7); };
+        for (int i = 0; i < n; ++i) ++bk[key(h_tmp[i]) + 1];
+        for (size_t x = 1; x < 9 * 8 + 1; ++x) bk[x] += bk[x - 1];
+        for (int i = 0; i < n; ++i) h_perm[bk[key(h_tmp[i])]++] = h_tmp[i];
+        for (int i = 0; i < n;) {
+            Class &bc = cls[ncls++];
+            bc.nw = h_cls[h_perm[i]];
+            bc.tile_begin = (uint32_t)ntiles;
+            int e2 = i;
+            while (e2 < n && h_cls[h_perm[e2]] == bc.nw) ++e2;
+            for (int g = i; g < e2;) {
+                int ge = g;
+                while (ge < e2 && (cand[h_perm[ge]].L & 7) == (cand[h_perm[g]].L & 7)) ++ge;
+                for (int s = g; s < ge; s += 64) {
+                    const int cnt = std::min(64, ge - s);
+                    uint32_t kmax = 0, lmax = 0;
+                    for (int u = s; u < s + cnt; ++u) {
+                        kmax = std::max<uint32_t>(kmax, cand[h_perm[u]].k);
+                        lmax = std::max<uint32_t>(lmax, cand[h_perm[u]].L);
+                    }
+                    add_tile(bc, (uint32_t)s, (uint32_t)cnt, lmax, kmax);
+                }
+                g = ge;
+            }
+            i = e2;
+        }
+        for (int p = 0; p < n; ++p) h_cand_tile[p] = cand[h_perm[p]];
+    }
+
     const size_t o_tiles = at;
     at = align256(at + ntiles * 16);
     const size_t o_toff = at;
@@ -175,29 +244,13 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
                                      "static scratch holds %zu; split the batch",
                          at, (size_t)SRM_STATIC_SCRATCH_BYTES);
 
-    hipError_t e = hipSetDevice(device);
-    if (e != hipSuccess) return set_error(SRM_EDEVICE, "hipSetDevice(%d): %s", device, hipGetErrorString(e));
-    if (!g_scratch[device]) {   // once per device, with the device current
-        void *p = nullptr;
-        e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p)
-            return set_error(SRM_EDEVICE, "hipGetSymbolAddress(scratch): %s", hipGetErrorString(e));
-        g_scratch[device] = (unsigned char *)p;
+    if (!planned) {
+        if (const int rc = on_device()) return rc;
+        SA_TRY(hipMemcpyAsync(base + o_cand, cand, (size_t)n * sizeof(srm_cand), hipMemcpyHostToDevice, st));
+        SA_TRY(hipMemcpyAsync(base + o_cand_tile, h_cand_tile, (size_t)n * sizeof(srm_cand),
+                              hipMemcpyHostToDevice, st));
+        SA_TRY(hipMemcpyAsync(base + o_perm, h_perm, (size_t)n * 4, hipMemcpyHostToDevice, st));
     }
-    unsigned char *base = g_scratch[device];
-    hipStream_t st = (hipStream_t)stream;
-
-#define SA_TRY(expr)                                                                          \
-    do {                                                                                      \
-        hipError_t e_ = (expr);                                                               \
-        if (e_ != hipSuccess)                                                                 \
-            return set_error(SRM_EDEVICE, "%s failed: %s", #expr, hipGetErrorString(e_));     \
-    } while (0)
-
-    SA_TRY(hipMemcpyAsync(base + o_cand, cand, (size_t)n * sizeof(srm_cand), hipMemcpyHostToDevice, st));
-    SA_TRY(hipMemcpyAsync(base + o_cand_tile, h_cand_tile, (size_t)n * sizeof(srm_cand),
-                          hipMemcpyHostToDevice, st));
-    SA_TRY(hipMemcpyAsync(base + o_perm, h_perm, (size_t)n * 4, hipMemcpyHostToDevice, st));
     SA_TRY(hipMemcpyAsync(base + o_tiles, h_tiles, ntiles * 16, hipMemcpyHostToDevice, st));
     SA_TRY(hipMemcpyAsync(base + o_toff, h_tile_off, ntiles * 8, hipMemcpyHostToDevice, st));
     // the class counters of the persistent (other-cost) kernel start at zero
