@@ -37,7 +37,7 @@ struct BandArgs {
     const uint32_t *perm;           // candidate indices, tile-major
     const srm_cand *cand_tile;      // the candidates in the same order (unit-cost kernels)
     int32_t *tile_score;            // scores in the same order (bits_band_kernel -> walk)
-    const uint4 *tiles;             // x perm start, y count (<= 64), z max L, w max k
+    const uint4 *tiles;             // x perm start, y count (<= 64), z max L, w unused
     uint32_t ntiles;
     uint32_t *queue;                // tile counter (zeroed before the launch)
     const uint32_t *read_words;
@@ -55,7 +55,7 @@ struct BandArgs {
                                     // LDS (0: written straight to the slot)
 };
 
-// the unit-cost classes in the order one launch takes them: span c is blocks
+// the band classes in the order one launch takes them: span c is blocks
 // block[c] .. block[c + 1] - 1 (a tile each, from tile[c] on) of band words nw[c] and
 // reads of up to max_len[c] codes
 constexpr int MAX_BAND_CLASSES = 16;   // 8 classes, each split at most once by read length
@@ -122,6 +122,13 @@ hipError_t launch_trace(const BandArgs &a, int nw, bool unit, int maxL, hipStrea
 // unit costs (band_bits.hip): the bit-parallel forward pass and its walk
 hipError_t launch_bits_band(const BandArgs &a, int nw, int blocks, int maxL, hipStream_t st);
 hipError_t launch_bits_trace(const BandArgs &a, int nw, int maxL, hipStream_t st);
+// one launch for every class: always for unit costs, for others while all tiles run at
+// once (3 waves per SIMD, nw_kernels.hip)
+hipError_t launch_all(const BandArgs &a, const BitsSpans &sp, bool unit, hipStream_t st);
+inline bool all_classes_fit(bool unit, size_t ntiles, int num_cus)
+{
+    return unit || ntiles <= (size_t)num_cus * 12;
+}
 hipError_t launch_bits_all(const BandArgs &a, const BitsSpans &sp, hipStream_t st);
 int bits_trace_stage_words(int maxL);   // LDS transcript words per lane for a class's walk
 int bits_band_occupancy(int nw);

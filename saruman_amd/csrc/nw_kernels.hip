@@ -21,6 +21,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "nw_device.h"
 #include "nw_seq.h"
 
@@ -362,170 +365,177 @@ struct BandWaves {
         NW <= 1 ? 8 : NW <= 2 ? 7 : NW <= 3 ? 6 : NW <= 5 ? 4 : NW <= 7 ? 3 : 2;
 };
 
+// the forward pass of one tile by one wave
 template <int NW>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BandWaves<NW>::value)))
-void band_kernel(BandArgs a)
+__device__ __forceinline__ void nibble_band_tile(const BandArgs &a, uint32_t tile)
 {
     constexpr int BMAX = NW * 8;            // band cells per column held in VGPRs
     constexpr int WW = (BMAX + 15) / 16;    // code words of the sliding window
     const int lane = threadIdx.x & 63;
     const int ma = a.ma, mm = a.mm;
 
+    // x: perm start, y: count, z: max L -- one tile per wave: made
+    // wave-uniform so the column loop and its every-8/16-column steps stay
+    // scalar branches
+    uint4 td = a.tiles[tile];
+    td.x = __builtin_amdgcn_readfirstlane(td.x);
+    td.y = __builtin_amdgcn_readfirstlane(td.y);
+    td.z = __builtin_amdgcn_readfirstlane(td.z);
+    uint32_t *__restrict__ scr = a.scratch + a.tile_scratch[tile];
+    const bool active = (uint32_t)lane < td.y;
+    const uint32_t t = active ? a.perm[td.x + lane] : 0u;
+    srm_cand cd = a.cand[t];
+    const int L = active ? (int)cd.L : 0;
+    const int w = cd.w, k = cd.k;
+    const int s = flag_s(cd.flag, k), e = flag_e(cd.flag, k);
+    const int dlo = -k;
+    const int K = k + 1;
+    const int Lmax = (int)td.z;
+
+    // ---- column 0: M[h][0] = max(0, h - 2s) (unit steps, Q7); rows < 0 -> K
+    int v[BMAX];
+    uint32_t acc[BMAX];
+#pragma unroll
+    for (int i = 0; i < BMAX; ++i) {
+        const int h = dlo + i;
+        const int m0 = h < 0 ? K : imin(imax(h - 2 * s, 0), K);
+        v[i] = m0;
+        acc[i] = (uint32_t)v[i];
+    }
+    // window codes for column 1: W[i] = g[dlo + i]; a 16*WW-code window plus a stream
+    uint32_t gw[WW];
+    const int64_t gbase = (int64_t)cd.win_off + dlo;
+#pragma unroll
+    for (int j = 0; j < WW; ++j) gw[j] = active ? fetch16(a.win_words, gbase + 16 * j) : 0u;
+    uint32_t gnext = 0;   // stream of window codes entering the top of the window
+    uint32_t rbuf = 0;    // stream of read codes
+    const int64_t rbase = (int64_t)cd.read_off;
+
+    // one DP column; last selects the free trailing verticals of column L
+    uint32_t lastmis[WW];   // mismatch fields of column L
+    auto column = [&](int c, bool last) {
+        // window for column c (c >= 2): shift by one code, take the next from the stream
+        if (c >= 2) {
+            if (((c - 2) & 15) == 0) gnext = fetch16(a.win_words, gbase + 16 * WW + (c - 2));
+#pragma unroll
+            for (int j = 0; j < WW - 1; ++j)
+                gw[j] = __builtin_amdgcn_alignbit(gw[j + 1], gw[j], 2);
+            gw[WW - 1] = __builtin_amdgcn_alignbit(gnext, gw[WW - 1], 2);
+            gnext >>= 2;
+        }
+        if (((c - 1) & 15) == 0) rbuf = fetch16(a.read_words, rbase + (c - 1));
+        const uint32_t rc = rbuf & 3u;
+        rbuf >>= 2;
+        const uint32_t r8 = rc * 0x5555u;          // 24-bit multiply (full rate)
+        const uint32_t rrep = r8 | (r8 << 16);     // the read code in all 16 fields
+        uint32_t mis[WW];
+#pragma unroll
+        for (int j = 0; j < WW; ++j) {
+            const uint32_t x = gw[j] ^ rrep;
+            mis[j] = x | (x >> 1);   // bit 2i set <=> window code i != read code
+        }
+        if (last) {
+#pragma unroll
+            for (int j = 0; j < WW; ++j) lastmis[j] = mis[j];
+        }
+        int ifree = BMAX;            // first band cell whose top move is free
+        if (last) ifree = w - 2 * e + 1 - c - dlo;
+        const uint32_t sh = (uint32_t)(c & 7) * 4u;
+        int up = 1 << 20;
+#pragma unroll
+        for (int i = 0; i < BMAX; ++i) {
+            const int bit = (int)((mis[i >> 4] >> (2 * (i & 15))) & 1u);
+            const int lf = (i + 1 < BMAX) ? v[i + 1] : (1 << 20);
+            const int dg = v[i] + (bit ? mm : ma);
+            const int tcost = (last && i >= ifree) ? 0 : mm;
+            int nv = imin(imin(dg, lf + mm), up + tcost);
+            nv = imin(nv, K);
+            v[i] = nv;
+            up = nv;
+        }
+        if (c <= k) {
+            // row 0 keeps its unit-step init M[0][c] = c (Q7) whatever the mismatch cost
+            const int i0 = k - c;
+#pragma unroll
+            for (int i = 0; i < BMAX; ++i) v[i] = (i == i0) ? imin(c, K) : v[i];
+        }
+        // nibble c & 7 of every diagonal's word; a block is stored when complete
+        // and its words start again from 0
+#pragma unroll
+        for (int i = 0; i < BMAX; ++i) acc[i] += (uint32_t)v[i] << sh;
+        if ((c & 7) == 7 || last) {
+            // streaming stores: the band is read back only by the walk, much
+            // later; the code words the next columns fetch stay in L2
+            uint32_t *__restrict__ blk = scr + (size_t)(c >> 3) * BMAX * 64 + lane;
+#pragma unroll
+            for (int i = 0; i < BMAX; ++i) __builtin_nontemporal_store(acc[i], &blk[i * 64]);
+#pragma unroll
+            for (int i = 0; i < BMAX; ++i) acc[i] = 0u;
+        }
+    };
+
+    for (int c0 = 1; c0 < Lmax; ++c0) {
+        // the column is the same on every lane: kept scalar, so the steps taken
+        // every 8 and 16 columns are scalar branches, not masked ones
+        const int c = __builtin_amdgcn_readfirstlane(c0);
+        if (c < L) column(c, false);
+    }
+    // tail of the tile's scratch, for the walk's first (vertical) run: columns
+    // L and L - 1 by diagonal (nibble j of word m is diagonal 8m + j), then the
+    // equal-character bits of column L
+    uint32_t *__restrict__ tail = scr + (size_t)((Lmax + 8) >> 3) * BMAX * 64 + lane;
+    auto store_column = [&](int c, int word0) {
+#pragma unroll
+        for (int m = 0; m < NW; ++m) {
+            uint32_t x = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int i = 8 * m + j;
+                x |= ((uint32_t)v[i] & 15u) << (4 * j);
+            }
+            __builtin_nontemporal_store(x, &tail[(word0 + m) * 64]);
+        }
+    };
+    if (active) {
+        store_column(L - 1, NW);
+        column(L, true);
+        store_column(L, 0);
+        uint32_t eqw[2] = {0u, 0u};
+#pragma unroll
+        for (int i = 0; i < BMAX; ++i)
+            if (!((lastmis[i >> 4] >> (2 * (i & 15))) & 1u)) eqw[i >> 5] |= 1u << (i & 31);
+        tail[(2 * NW) * 64] = eqw[0];
+        tail[(2 * NW + 1) * 64] = eqw[1];
+    }
+
+    // ---- score (cuda-functions.cu:495-497); the walk runs in trace_kernel
+    if (active) {
+        int score = K;
+        const int iend = w - L - dlo;
+        if (iend >= 0 && iend < BMAX) {
+            const uint32_t wd0 = band_word<BMAX>(scr, iend, L >> 3, lane);
+            score = imin((int)((wd0 >> ((L & 7) * 4)) & 15u), K);
+        }
+        srm_result r;
+        r.score = (int16_t)score;
+        r.n_ops = 0;
+        r.end_row = (uint16_t)w;
+        r.end_col = (uint16_t)L;
+        a.res[t] = r;
+    }
+}
+
+template <int NW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BandWaves<NW>::value)))
+void band_kernel(BandArgs a)
+{
+    const int lane = threadIdx.x & 63;
     for (;;) {
         uint32_t tile = 0;
         if (lane == 0) tile = atomicAdd(a.queue, 1u);
         tile = __builtin_amdgcn_readfirstlane(tile);
         if (tile >= a.ntiles) break;
-        // x: perm start, y: count, z: max L, w: max k -- one tile per wave: made
-        // wave-uniform so the column loop and its every-8/16-column steps stay
-        // scalar branches
-        uint4 td = a.tiles[tile];
-        td.x = __builtin_amdgcn_readfirstlane(td.x);
-        td.y = __builtin_amdgcn_readfirstlane(td.y);
-        td.z = __builtin_amdgcn_readfirstlane(td.z);
-        td.w = __builtin_amdgcn_readfirstlane(td.w);
-        uint32_t *__restrict__ scr = a.scratch + a.tile_scratch[tile];
-        const bool active = (uint32_t)lane < td.y;
-        const uint32_t t = active ? a.perm[td.x + lane] : 0u;
-        srm_cand cd = a.cand[t];
-        const int L = active ? (int)cd.L : 0;
-        const int w = cd.w, k = cd.k;
-        const int s = flag_s(cd.flag, k), e = flag_e(cd.flag, k);
-        const int dlo = -k;
-        const int K = k + 1;
-        const int Lmax = (int)td.z;
-
-        // ---- column 0: M[h][0] = max(0, h - 2s) (unit steps, Q7); rows < 0 -> K
-        int v[BMAX];
-        uint32_t acc[BMAX];
-#pragma unroll
-        for (int i = 0; i < BMAX; ++i) {
-            const int h = dlo + i;
-            const int m0 = h < 0 ? K : imin(imax(h - 2 * s, 0), K);
-            v[i] = m0;
-            acc[i] = (uint32_t)v[i];
-        }
-        // window codes for column 1: W[i] = g[dlo + i]; a 16*WW-code window plus a stream
-        uint32_t gw[WW];
-        const int64_t gbase = (int64_t)cd.win_off + dlo;
-#pragma unroll
-        for (int j = 0; j < WW; ++j) gw[j] = active ? fetch16(a.win_words, gbase + 16 * j) : 0u;
-        uint32_t gnext = 0;   // stream of window codes entering the top of the window
-        uint32_t rbuf = 0;    // stream of read codes
-        const int64_t rbase = (int64_t)cd.read_off;
-
-        // one DP column; last selects the free trailing verticals of column L
-        uint32_t lastmis[WW];   // mismatch fields of column L
-        auto column = [&](int c, bool last) {
-            // window for column c (c >= 2): shift by one code, take the next from the stream
-            if (c >= 2) {
-                if (((c - 2) & 15) == 0) gnext = fetch16(a.win_words, gbase + 16 * WW + (c - 2));
-#pragma unroll
-                for (int j = 0; j < WW - 1; ++j)
-                    gw[j] = __builtin_amdgcn_alignbit(gw[j + 1], gw[j], 2);
-                gw[WW - 1] = __builtin_amdgcn_alignbit(gnext, gw[WW - 1], 2);
-                gnext >>= 2;
-            }
-            if (((c - 1) & 15) == 0) rbuf = fetch16(a.read_words, rbase + (c - 1));
-            const uint32_t rc = rbuf & 3u;
-            rbuf >>= 2;
-            const uint32_t r8 = rc * 0x5555u;          // 24-bit multiply (full rate)
-            const uint32_t rrep = r8 | (r8 << 16);     // the read code in all 16 fields
-            uint32_t mis[WW];
-#pragma unroll
-            for (int j = 0; j < WW; ++j) {
-                const uint32_t x = gw[j] ^ rrep;
-                mis[j] = x | (x >> 1);   // bit 2i set <=> window code i != read code
-            }
-            if (last) {
-#pragma unroll
-                for (int j = 0; j < WW; ++j) lastmis[j] = mis[j];
-            }
-            int ifree = BMAX;            // first band cell whose top move is free
-            if (last) ifree = w - 2 * e + 1 - c - dlo;
-            const uint32_t sh = (uint32_t)(c & 7) * 4u;
-            int up = 1 << 20;
-#pragma unroll
-            for (int i = 0; i < BMAX; ++i) {
-                const int bit = (int)((mis[i >> 4] >> (2 * (i & 15))) & 1u);
-                const int lf = (i + 1 < BMAX) ? v[i + 1] : (1 << 20);
-                const int dg = v[i] + (bit ? mm : ma);
-                const int tcost = (last && i >= ifree) ? 0 : mm;
-                int nv = imin(imin(dg, lf + mm), up + tcost);
-                nv = imin(nv, K);
-                v[i] = nv;
-                up = nv;
-            }
-            if (c <= k) {
-                // row 0 keeps its unit-step init M[0][c] = c (Q7) whatever the mismatch cost
-                const int i0 = k - c;
-#pragma unroll
-                for (int i = 0; i < BMAX; ++i) v[i] = (i == i0) ? imin(c, K) : v[i];
-            }
-            // nibble c & 7 of every diagonal's word; a block is stored when complete
-            // and its words start again from 0
-#pragma unroll
-            for (int i = 0; i < BMAX; ++i) acc[i] += (uint32_t)v[i] << sh;
-            if ((c & 7) == 7 || last) {
-                // streaming stores: the band is read back only by the walk, much
-                // later; the code words the next columns fetch stay in L2
-                uint32_t *__restrict__ blk = scr + (size_t)(c >> 3) * BMAX * 64 + lane;
-#pragma unroll
-                for (int i = 0; i < BMAX; ++i) __builtin_nontemporal_store(acc[i], &blk[i * 64]);
-#pragma unroll
-                for (int i = 0; i < BMAX; ++i) acc[i] = 0u;
-            }
-        };
-
-        for (int c0 = 1; c0 < Lmax; ++c0) {
-            // the column is the same on every lane: kept scalar, so the steps taken
-            // every 8 and 16 columns are scalar branches, not masked ones
-            const int c = __builtin_amdgcn_readfirstlane(c0);
-            if (c < L) column(c, false);
-        }
-        // tail of the tile's scratch, for the walk's first (vertical) run: columns
-        // L and L - 1 by diagonal (nibble j of word m is diagonal 8m + j), then the
-        // equal-character bits of column L
-        uint32_t *__restrict__ tail = scr + (size_t)((Lmax + 8) >> 3) * BMAX * 64 + lane;
-        auto store_column = [&](int c, int word0) {
-#pragma unroll
-            for (int m = 0; m < NW; ++m) {
-                uint32_t x = 0;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int i = 8 * m + j;
-                    x |= ((uint32_t)v[i] & 15u) << (4 * j);
-                }
-                __builtin_nontemporal_store(x, &tail[(word0 + m) * 64]);
-            }
-        };
-        if (active) {
-            store_column(L - 1, NW);
-            column(L, true);
-            store_column(L, 0);
-            uint32_t eqw[2] = {0u, 0u};
-#pragma unroll
-            for (int i = 0; i < BMAX; ++i)
-                if (!((lastmis[i >> 4] >> (2 * (i & 15))) & 1u)) eqw[i >> 5] |= 1u << (i & 31);
-            tail[(2 * NW) * 64] = eqw[0];
-            tail[(2 * NW + 1) * 64] = eqw[1];
-        }
-
-        // ---- score (cuda-functions.cu:495-497); the walk runs in trace_kernel
-        if (active) {
-            int score = K;
-            const int iend = w - L - dlo;
-            if (iend >= 0 && iend < BMAX) {
-                const uint32_t wd0 = band_word<BMAX>(scr, iend, L >> 3, lane);
-                score = imin((int)((wd0 >> ((L & 7) * 4)) & 15u), K);
-            }
-            srm_result r;
-            r.score = (int16_t)score;
-            r.n_ops = 0;
-            r.end_row = (uint16_t)w;
-            r.end_col = (uint16_t)L;
-            a.res[t] = r;
-        }
+        nibble_band_tile<NW>(a, tile);
     }
 }
 
@@ -554,13 +564,10 @@ __device__ __forceinline__ uint32_t spread2(uint32_t f)
 // (gaps, the free rows of column L, the start of the read) one cell at a time;
 // column 0 comes from its closed form max(0, h - 2s) (Q7) without loads.
 template <int NW>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8)))
-void trace_kernel(BandArgs a)
+__device__ __forceinline__ void nibble_trace_tile(const BandArgs &a, uint32_t tile)
 {
     constexpr int BMAX = NW * 8;
     const int lane = threadIdx.x & 63;
-    const uint32_t tile = (uint32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    if (tile >= a.ntiles) return;
     const uint4 td = a.tiles[tile];
     if ((uint32_t)lane >= td.y) return;
     const uint32_t t = a.perm[td.x + lane];
@@ -754,6 +761,51 @@ void trace_kernel(BandArgs a)
     a.res[t] = r;
 }
 
+template <int NW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8)))
+void trace_kernel(BandArgs a)
+{
+    const uint32_t tile = (uint32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    if (tile < a.ntiles) nibble_trace_tile<NW>(a, tile);
+}
+
+// words per lane that stage a read of length <= maxL in LDS: codes from one
+// before the read's first to 16 past its last, from word boundaries; reads of more
+// than 600 codes (40 KiB per block of 4 waves) are read from read_words
+__host__ __device__ constexpr int trace_code_words(int maxL)
+{
+    return maxL <= 600 ? ((maxL + 15) >> 4) + 3 : 0;
+}
+
+// The forward pass and the walk of every class in one launch, a block of one wave per
+// tile, as bits_all_kernel does for unit costs.  It holds the widest class's registers
+// (3 waves per SIMD), so it takes the batches whose tiles all run at once that way;
+// larger ones keep a launch per class, each at its own occupancy.  13,200 candidates of
+// 100 bp (two classes, four launches of 44-69 us one after another) through
+// srm_align_static, with the plan on the device: 363 -> 197 us.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
+void nibble_all_kernel(BandArgs a, BitsSpans sp)
+{
+    uint32_t c = 0;
+    while (c + 1 < sp.n && blockIdx.x >= sp.block[c + 1]) ++c;
+    const uint32_t tile = sp.tile[c] + (blockIdx.x - sp.block[c]);
+    a.code_words = trace_code_words(sp.max_len[c]);
+    auto both = [&](auto nw) {
+        nibble_band_tile<decltype(nw)::value>(a, tile);
+        nibble_trace_tile<decltype(nw)::value>(a, tile);
+    };
+    switch (sp.nw[c]) {
+    case 1: both(std::integral_constant<int, 1>{}); break;
+    case 2: both(std::integral_constant<int, 2>{}); break;
+    case 3: both(std::integral_constant<int, 3>{}); break;
+    case 4: both(std::integral_constant<int, 4>{}); break;
+    case 5: both(std::integral_constant<int, 5>{}); break;
+    case 6: both(std::integral_constant<int, 6>{}); break;
+    case 7: both(std::integral_constant<int, 7>{}); break;
+    default: both(std::integral_constant<int, 8>{}); break;
+    }
+}
+
 // streaming copy of n 16-byte words (calibrates the HBM traffic counters)
 __global__ __launch_bounds__(256) void copy_kernel(const uint4 *__restrict__ src,
                                                    uint4 *__restrict__ dst, size_t n)
@@ -856,19 +908,13 @@ static hipError_t launch_trace_nw(const BandArgs &a, size_t lds, hipStream_t st)
     return hipGetLastError();
 }
 
-// words per lane that stage a read of length <= maxL in LDS: codes from one
-// before the read's first to 16 past its last, from word boundaries
-static int trace_code_words(int maxL) { return ((maxL + 15) >> 4) + 3; }
-
 // one wave per tile of the class; unit (match 0, mismatch 1): bits_trace_kernel.
-// trace_kernel stages reads of up to 600 codes in LDS (at most 40 KiB per block
-// of 4 waves); longer ones are read from read_words.
 hipError_t launch_trace(const BandArgs &args, int nw, bool unit, int maxL, hipStream_t st)
 {
     if (args.ntiles == 0) return hipSuccess;
     if (unit) return launch_bits_trace(args, nw, maxL, st);
     BandArgs a = args;
-    a.code_words = maxL <= 600 ? trace_code_words(maxL) : 0;
+    a.code_words = trace_code_words(maxL);
     const size_t lds = (size_t)a.code_words * 256 * 4;
     switch (nw) {
     case 1: return launch_trace_nw<1>(a, lds, st);
@@ -881,6 +927,16 @@ hipError_t launch_trace(const BandArgs &args, int nw, bool unit, int maxL, hipSt
     case 8: return launch_trace_nw<8>(a, lds, st);
     default: return hipErrorInvalidValue;
     }
+}
+
+// every class in one launch: a.tiles and a.tile_scratch are those of all classes
+hipError_t launch_all(const BandArgs &a, const BitsSpans &sp, bool unit, hipStream_t st)
+{
+    if (unit) return launch_bits_all(a, sp, st);
+    int words = 0;
+    for (uint32_t c = 0; c < sp.n; ++c) words = std::max(words, trace_code_words(sp.max_len[c]));
+    hipLaunchKernelGGL(nibble_all_kernel, dim3(sp.blocks), dim3(64), (size_t)words * 64 * 4, st, a, sp);
+    return hipGetLastError();
 }
 
 hipError_t launch_reset(uint32_t *counters, int n, hipStream_t st)

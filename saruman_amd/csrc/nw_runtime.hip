@@ -182,7 +182,7 @@ struct srm_job {
     bool all_planned = false;        // the plain-kernel plan of every candidate made
     int ma = 0, mm = 1;
     bool unit = true;
-    bool one_launch = false;         // unit costs: every class in one launch (upload)
+    bool one_launch = false;         // every class in one launch (set at the upload)
     bool resident_genome = false;
     // device buffers
     DevBuf d_cand, d_read_words, d_win_words, d_read_bytes, d_win_bytes;
@@ -407,7 +407,7 @@ int run_launches(srm_job *j, int kernel, bool timed)
             srm::BandArgs a = band_args(j);
             a.tiles = (const uint4 *)j->d_tiles.p;
             a.tile_scratch = (const uint64_t *)j->d_tile_scratch.p;
-            HIP_TRY(srm::launch_bits_all(a, sp, st));
+            HIP_TRY(srm::launch_all(a, sp, j->unit, st));
         }
         // otherwise, with class_streams > 1, the classes run side by side on their own
         // streams (each with its own scratch), widest band first, or in order on st
@@ -690,8 +690,8 @@ int plan_host(srm_job *j, const srm::PlanIn &in, const srm_cand *cand, int n, si
     const uint32_t tile_cands = ctx->tuning.tile_cands == 32 ? 32u : 64u;
     const size_t nb = band_idx.size();
     const unsigned TB = plan_threads(nb);
-    // sort word of every banded candidate, in index order: its index (bits 0-31),
-    // k (bits 32-35) and from bit 36 the key: class (5 bits), L mod 8 (3 bits),
+    // sort word of every banded candidate, in index order: its index (bits 0-31)
+    // and from bit 36 the key: class (5 bits), L mod 8 (3 bits),
     // then maxL - L in lb bits (L descending), the fields of the order above from
     // the top down
     uint32_t maxL = 0;
@@ -705,10 +705,9 @@ int plan_host(srm_job *j, const srm::PlanIn &in, const srm_cand *cand, int n, si
             const srm_cand &c = cand[band_idx[i]];
             const uint32_t cl = (uint32_t)srm::band_class(in, c);
             const uint32_t key = (((cl << 3) | ((uint32_t)c.L & 7u)) << lb) | (maxL - c.L);
-            kv[i] = ((uint64_t)key << 36) | ((uint64_t)c.k << 32) | band_idx[i];
+            kv[i] = ((uint64_t)key << 36) | band_idx[i];
         }
     });
-    static_assert(SRM_BAND_KMAX < 16, "k of a banded candidate fits 4 bits");
     radix_sort_kv(kv, hp.kv_tmp, 36, 8 + lb, TB);
     par_ranges(TB, nb, [&](unsigned, size_t a, size_t b) {
         for (size_t i = a; i < b; ++i) band_idx[i] = (uint32_t)kv[i];
@@ -716,7 +715,6 @@ int plan_host(srm_job *j, const srm::PlanIn &in, const srm_cand *cand, int n, si
     // by position in tile order
     auto cls_at = [&](size_t i) { return (int)(kv[i] >> (36 + lb + 3)); };
     auto lmod_at = [&](size_t i) { return (int)((kv[i] >> (36 + lb)) & 7u); };
-    auto k_at = [&](size_t i) { return (uint32_t)(kv[i] >> 32) & 15u; };
     auto L_at = [&](size_t i) { return maxL - ((uint32_t)(kv[i] >> 36) & ((1u << lb) - 1u)); };
     std::vector<uint32_t> &tiles = hp.tiles;   // uint4 per tile
     tiles.clear();
@@ -740,7 +738,7 @@ int plan_host(srm_job *j, const srm::PlanIn &in, const srm_cand *cand, int n, si
                                       kv.begin());
             for (size_t g = i; g < e;) {
                 // one run of equal L mod 8, L descending: a tile's first read is its
-                // longest (its k maximum is filled in below, over all tiles at once)
+                // longest
                 const int lm = lmod_at(g);
                 const size_t ge = (size_t)(std::partition_point(
                                                kv.begin() + (std::ptrdiff_t)g,
@@ -764,23 +762,10 @@ int plan_host(srm_job *j, const srm::PlanIn &in, const srm_cand *cand, int n, si
             i = e;
         }
     }
-    // every tile's largest k, over the tiles on several host threads
-    {
-        const size_t nt = tiles.size() / 4;
-        par_ranges(plan_threads(nt * tile_cands), nt, [&](unsigned, size_t a, size_t b) {
-            for (size_t t = a; t < b; ++t) {
-                const size_t s0 = tiles[4 * t], c0 = tiles[4 * t + 1];
-                uint32_t kmax = 0;
-                for (size_t u = s0; u < s0 + c0; ++u) kmax = std::max(kmax, k_at(u));
-                tiles[4 * t + 3] = kmax;
-            }
-        });
-    }
     return SRM_OK;
 }
 
-// The same on the device (plan_gpu.hip), for unit costs: the descriptors go up, are
-// checked, counted and put in tile order there, and the host makes the tiles from the
+// The same on the device (plan_gpu.hip): the descriptors go up, are checked, counted and put in tile order there, and the host makes the tiles from the
 // counts.  The host's plan of a million candidates read and wrote them five times on
 // up to 8 threads, before the first copy began: a batch of 1,000,000 reads host to host
 // 11.3 -> 7.6 ms, one of 50,000 2.1 -> 1.67 ms.  The plan's scratch is the results'
@@ -793,7 +778,7 @@ int plan_device(srm_job *j, const srm::PlanIn &in, const srm_cand *cand, int n, 
                 size_t &scratch_words, bool &planned)
 {
     planned = false;
-    if (!j->unit || n < PLAN_DEVICE_MIN) return SRM_OK;
+    if (n < PLAN_DEVICE_MIN) return SRM_OK;
     srm_ctx *ctx = j->ctx;
     HostPlan &hp = j->plan;
     const size_t N = (size_t)n;
@@ -1187,16 +1172,10 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
     j->block_waves = ctx->tuning.block_waves ? ctx->tuning.block_waves : 4;
     j->walk_ck = ctx->tuning.walk_layout;
     // band classes run side by side unless the tuning says otherwise (1 = one after
-    // another on the context's stream): the unit-cost ones in one launch, others on 4
-    // streams or as many as it says
+    // another on the context's stream): in one launch, or for other costs and many tiles
+    // on 4 streams or as many as it says
     const int want_streams = ctx->tuning.class_streams == 0 ? 4 : ctx->tuning.class_streams;
     const bool concurrent = want_streams > 1;
-    j->class_streams = concurrent && !j->unit ? std::min(want_streams, 8) : 0;
-    while ((int)j->side.size() < j->class_streams) {   // default priority, like every stream here
-        hipStream_t q = nullptr;
-        HIP_TRY(hipStreamCreateWithFlags(&q, hipStreamNonBlocking));
-        j->side.push_back(q);
-    }
     size_t ops_end = 0, scratch_words = 0;
     j->rec_rows_bound = 0;
     j->classes.clear();
@@ -1209,7 +1188,14 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
     j->n_rest = hp.rest_idx.size();
     j->n_bytes = hp.bytes_idx.size();
     j->ops_words = ops_end;
-    j->one_launch = j->unit && concurrent && j->n_band > 0;
+    j->one_launch = concurrent && j->n_band > 0 &&
+                    srm::all_classes_fit(j->unit, hp.tiles.size() / 4, ctx->num_cus);
+    j->class_streams = concurrent && !j->one_launch ? std::min(want_streams, 8) : 0;
+    while ((int)j->side.size() < j->class_streams) {   // default priority, like every stream here
+        hipStream_t q = nullptr;
+        HIP_TRY(hipStreamCreateWithFlags(&q, hipStreamNonBlocking));
+        j->side.push_back(q);
+    }
     // ---- device buffers
     if (!planned && (rc = upload(ctx, j->d_cand, cand, (size_t)n))) return rc;
     if ((rc = upload(ctx, j->d_read_words, read_words, n_read_words))) return rc;

@@ -148,11 +148,11 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
     Class cls[9];
     int ncls = 0;
     size_t ntiles = 0, words = 0;
-    auto add_tile = [&](Class &bc, uint32_t first, uint32_t count, uint32_t lmax, uint32_t kmax) {
+    auto add_tile = [&](Class &bc, uint32_t first, uint32_t count, uint32_t lmax) {
         h_tiles[4 * ntiles + 0] = first;
         h_tiles[4 * ntiles + 1] = count;
         h_tiles[4 * ntiles + 2] = lmax;
-        h_tiles[4 * ntiles + 3] = kmax;
+        h_tiles[4 * ntiles + 3] = 0;
         h_tile_off[ntiles] = words;
         words += unit ? srm::bits_tile_words(bc.nw, (int)lmax, false)
                       : srm::tile_scratch_words(bc.nw, (int)lmax);
@@ -160,10 +160,10 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
         ++bc.ntiles;
         ++ntiles;
     };
-    // ---- on the device, for unit costs: checked, counted and put in tile order there;
-    // the tiles follow from the counts
+    // ---- on the device: checked, counted and put in tile order there; the tiles follow
+    // from the counts
     bool planned = false;
-    if (unit && n >= PLAN_DEVICE_MIN) {
+    if (n >= PLAN_DEVICE_MIN) {
         if (const int rc = on_device()) return rc;
         // (its own scratch lies at the end, where the bands come later)
         unsigned char *sums = base + SRM_STATIC_SCRATCH_BYTES - align256(srm::PLAN_SCRATCH);
@@ -184,7 +184,7 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
                                 cls[ncls].tile_begin = (uint32_t)ntiles;
                             },
                             [&](uint32_t first, uint32_t count, int lmax) {
-                                add_tile(cls[ncls], first, count, (uint32_t)lmax, 0u);
+                                add_tile(cls[ncls], first, count, (uint32_t)lmax);
                             },
                             [&] { ++ncls; });
     }
@@ -219,12 +219,9 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
                 while (ge < e2 && (cand[h_perm[ge]].L & 7) == (cand[h_perm[g]].L & 7)) ++ge;
                 for (int s = g; s < ge; s += 64) {
                     const int cnt = std::min(64, ge - s);
-                    uint32_t kmax = 0, lmax = 0;
-                    for (int u = s; u < s + cnt; ++u) {
-                        kmax = std::max<uint32_t>(kmax, cand[h_perm[u]].k);
-                        lmax = std::max<uint32_t>(lmax, cand[h_perm[u]].L);
-                    }
-                    add_tile(bc, (uint32_t)s, (uint32_t)cnt, lmax, kmax);
+                    uint32_t lmax = 0;
+                    for (int u = s; u < s + cnt; ++u) lmax = std::max<uint32_t>(lmax, cand[h_perm[u]].L);
+                    add_tile(bc, (uint32_t)s, (uint32_t)cnt, lmax);
                 }
                 g = ge;
             }
@@ -253,9 +250,6 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
     }
     SA_TRY(hipMemcpyAsync(base + o_tiles, h_tiles, ntiles * 16, hipMemcpyHostToDevice, st));
     SA_TRY(hipMemcpyAsync(base + o_toff, h_tile_off, ntiles * 8, hipMemcpyHostToDevice, st));
-    // the class counters of the persistent (other-cost) kernel start at zero
-    if (!unit) SA_TRY(srm::launch_reset((uint32_t *)(base + o_queue), ncls, st));
-
     srm::BandArgs a{};
     a.ma = match;
     a.mm = mismatch;
@@ -268,26 +262,29 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
     a.scratch = (uint32_t *)(base + o_band);
     a.res = d_res;
     a.ops = d_ops;
-    if (unit) {   // every class in one launch, the widest band first
+    int num_cus = 0;
+    if (!unit) SA_TRY(hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, device));
+    if (srm::all_classes_fit(unit, ntiles, num_cus)) {   // one launch, the widest band first
         srm::BitsSpans sp;
         for (int c = ncls; c-- > 0;) sp.add(cls[c].nw, cls[c].tile_begin, cls[c].ntiles, cls[c].maxL);
         a.tiles = (const uint4 *)(base + o_tiles);
         a.tile_scratch = (const uint64_t *)(base + o_toff);
-        SA_TRY(srm::launch_bits_all(a, sp, st));
-    }
-    int num_cus = 0;
-    if (!unit) SA_TRY(hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, device));
-    for (int c = 0; !unit && c < ncls; ++c) {
-        const Class &bc = cls[c];
-        a.tiles = (const uint4 *)(base + o_tiles) + bc.tile_begin;
-        a.ntiles = bc.ntiles;
-        a.queue = (uint32_t *)(base + o_queue) + c;
-        a.tile_scratch = (const uint64_t *)(base + o_toff) + bc.tile_begin;
-        // persistent grid: the blocks that stay resident, at most a wave per tile
-        const int blocks = std::min((int)((bc.ntiles + 3) / 4),
-                                    std::max(1, num_cus * srm::band_occupancy(bc.nw, false)));
-        SA_TRY(srm::launch_band(a, bc.nw, unit, blocks, bc.maxL, st));
-        SA_TRY(srm::launch_trace(a, bc.nw, unit, bc.maxL, st));
+        SA_TRY(srm::launch_all(a, sp, unit, st));
+    } else {
+        // the class counters of the persistent kernel start at zero
+        SA_TRY(srm::launch_reset((uint32_t *)(base + o_queue), ncls, st));
+        for (int c = 0; c < ncls; ++c) {
+            const Class &bc = cls[c];
+            a.tiles = (const uint4 *)(base + o_tiles) + bc.tile_begin;
+            a.ntiles = bc.ntiles;
+            a.queue = (uint32_t *)(base + o_queue) + c;
+            a.tile_scratch = (const uint64_t *)(base + o_toff) + bc.tile_begin;
+            // persistent grid: the blocks that stay resident, at most a wave per tile
+            const int blocks = std::min((int)((bc.ntiles + 3) / 4),
+                                        std::max(1, num_cus * srm::band_occupancy(bc.nw, false)));
+            SA_TRY(srm::launch_band(a, bc.nw, unit, blocks, bc.maxL, st));
+            SA_TRY(srm::launch_trace(a, bc.nw, unit, bc.maxL, st));
+        }
     }
     // the host arrays and the scratch are reused by the next call
     SA_TRY(hipStreamSynchronize(st));

@@ -32,10 +32,10 @@ def laid_out(seed, n, hi=250, base=1500):
     return cand, lay, int(words.sum())
 
 
-def run(ctx, cand, lay, ops_total, kernel="banded"):
+def run(ctx, cand, lay, ops_total, kernel="banded", costs=(0, 1)):
     job = Job(ctx)
     try:
-        job.upload(0, 1, cand, pack_codes(lay["rcat"]), pack_codes(lay["wcat"]), lay["rcat"],
+        job.upload(*costs, cand, pack_codes(lay["rcat"]), pack_codes(lay["wcat"]), lay["rcat"],
                    lay["wcat"], ops_total=ops_total)
         job.run(kernel)
         return job.download()
@@ -85,6 +85,26 @@ def test_job_plan(ctx, n, hi, raw):
     k1 = cand["k"].astype(np.int64) + 1
     got = run(ctx, cand, lay, int(words.sum()))[0]["score"].astype(np.int64)
     assert (np.minimum(plain, k1) == np.minimum(got, k1)).all()
+
+
+def test_other_costs_beyond_one_launch(ctx):
+    """More tiles than run at once: a launch per class, on streams and one after another."""
+    print("[gpu] device plan, other costs", flush=True)
+    n = 210_000
+    cand, lay, total = laid_out(9, n, 60)
+    want = run(ctx, cand, lay, total, costs=(0, 2))
+    tune.apply(ctx, {"blocks_per_cu": [0] * 9, "class_streams": 1})
+    res, ops = run(ctx, cand, lay, total, costs=(0, 2))
+    tune.apply(ctx, None)
+    assert (res == want[0]).all()
+    parts = []
+    for a in (0, 105_000, 205_000):
+        part = cand[a:a + 5_000].copy()
+        off = int(part["ops_off"][0])
+        part["ops_off"] -= off
+        words = int((part["ops_off"].astype(np.int64) + (part["w"].astype(np.int64) + part["k"] + 15) // 16).max())
+        pres, pops = run(ctx, part, lay, words, costs=(0, 2))
+        same(part, (res[a:a + 5_000], ops[off:off + words]), [(pres, pops, part)])
 
 
 def test_refusals_name_the_first(ctx):
