@@ -56,6 +56,12 @@ namespace {
 constexpr int FB = 256;      // threads per block
 constexpr int ECAP = 16;     // result-hash entries per read kept in LDS
 constexpr int PCAP = 4;      // perfect hits per read kept in LDS
+constexpr int PB = 64;       // threads per block of the pairing pass
+// reads per block of it with G lanes a read: half as many again as it takes at a time,
+// since about half are dropped; one each where a read may take long
+constexpr int pair_reads(int G) { return G == 8 ? PB / G * 3 / 2 : PB / G; }
+constexpr int NSTARTS = 33;  // list starts per read kept in LDS (odd: the groups of a
+constexpr int NVALS = 64;    // wave read from different banks), and list elements
 
 // the reads' (or the genome's) bytes as codes and as a mask of other bytes: 16 bytes
 // a thread; src holds n16 * 16 readable bytes
@@ -71,6 +77,7 @@ __global__ void __launch_bounds__(FB) fl_pack(const uint4 *__restrict__ src, uin
     odd[i] = (uint16_t)o;
 }
 
+constexpr size_t OVER_ROOM = (size_t)1 << 19;   // entries
 constexpr uint32_t MAX_FLUSH = 256;      // flushes the device lists
 constexpr uint32_t MAX_UNSAFE = 1 << 16; // reads it lists for the host's walk
 constexpr uint32_t MAX_WALK = 1 << 16;   // words of their entries
@@ -168,7 +175,10 @@ __global__ void __launch_bounds__(FB) fl_count(Call c_, uint32_t per)
     __shared__ BlockReads s;
     const FArgs &a = c_.s[blockIdx.y].f;
     if (blockIdx.x == 0) {   // what later kernels of the call add to
-        if (threadIdx.x < 6) ((uint32_t *)c_.s[blockIdx.y].hdr)[threadIdx.x] = 0;
+        // (the entries and perfect hits of reads that are run again follow all slots')
+        if (threadIdx.x < 6)
+            ((uint32_t *)c_.s[blockIdx.y].hdr)[threadIdx.x] =
+                threadIdx.x == 0 ? a.n_reads * ECAP : threadIdx.x == 1 ? a.n_reads * PCAP : 0;
         if (threadIdx.x == 0) a.list_cnt[c_.n_lists] = 0;
     }
     const uint32_t nr = s.load(a, per);
@@ -214,17 +224,6 @@ __global__ void __launch_bounds__(FB) fl_fill(Call c_, uint32_t per)
     }
 }
 
-__device__ __forceinline__ uint32_t wave_incl_sum(uint32_t v)
-{
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(v, d, 64);
-        if (lane >= d) v += o;
-    }
-    return v;
-}
-
 // one lane's stores to its read's slots before the group's later loads of them
 template <bool GLOBAL>
 __device__ __forceinline__ void slots_written()
@@ -265,157 +264,198 @@ __device__ __forceinline__ int group_add(Store &s, int32_t pos, int flag, int k,
     return 2;
 }
 
+// a read of the pairing pass: what its loads depend on, found for all of a block's reads
+// at once
+struct PairRead {
+    uint64_t off;            // its first byte
+    uint32_t r, at;          // the read, its place among the launch's
+    uint32_t lb, n;          // its first list, its lists
+    uint32_t i0, i1, end;    // flat indices: its first list, its second half, its end
+    uint32_t flat_end;
+    uint32_t pid;
+};
+
+// the reads of a block (`per` <= PB) that have a position to start from; nothing comes of
+// the others, half of the reads on either strand
+__device__ __forceinline__ uint32_t pair_list(const FArgs &a, PairRead *list, uint32_t per)
+{
+    __shared__ uint32_t s_n;
+    if (PB > 64 && threadIdx.x == 0) s_n = 0;
+    if (PB > 64) __syncthreads();
+    const uint32_t at = blockIdx.x * per + threadIdx.x;
+    PairRead R;
+    bool some = false;
+    if (threadIdx.x < per && at < a.n_todo) {
+        R.at = at;
+        R.r = a.todo ? a.todo[at] : at;
+        R.lb = a.list_base[R.r];
+        R.off = a.roff[R.r];
+        R.pid = a.pid[R.r];
+        R.flat_end = chunk_end(a, R.r);
+        const uint32_t half = (uint32_t)a.par[R.pid].half;
+        R.n = (uint32_t)a.par[R.pid].n;
+        R.i0 = list_at(a, R.lb);
+        R.i1 = list_at(a, R.lb + half);
+        R.end = list_at(a, R.lb + R.n);
+        some = R.i1 - R.i0 != half;   // (an empty list is its terminator)
+        if (!some) {
+            a.meta[3 * (size_t)R.r + 0] = 0;
+            a.meta[3 * (size_t)R.r + 1] = 0;
+            a.meta[3 * (size_t)R.r + 2] = 0;
+        }
+    }
+    const uint64_t m = __ballot(some);
+    const int lane = threadIdx.x & 63;
+    uint32_t n = (uint32_t)__popcll(m), first = 0;
+    if (PB > 64) {
+        if (lane == 0) first = atomicAdd(&s_n, n);
+        first = (uint32_t)__shfl((int)first, 0, 64);
+    }
+    if (some) list[first + (uint32_t)__popcll(m & ((1ull << lane) - 1))] = R;
+    __syncthreads();
+    return PB > 64 ? s_n : n;
+}
+
 // run_seashore (hash.c:502-834) by G lanes per read: each lane takes a start
 // position (an element of the first half of the read's lists, which lie one after
 // another in the flat array) and finds what it would insert -- that depends on the
 // lists alone -- and the group then adds the results in the reference's order.
 //
-// Latency-bound: a start position is a chain of a few dependent list loads and the
-// perfect check.  A thread per read walked its positions one after another and
-// compared the read with the genome byte by byte, so a call lasted as long as its
-// longest read's chain; here the positions' chains run side by side and the group
-// compares 16 bases per lane at once, a genome start that several positions share
-// only once.  2M reads of 50-250 bp, one strand: 10.6 -> 2.44 ms, the reads of many
-// entries 3.39 -> 0.11 ms; 1,000 reads: 856 -> 45 us.
+// Latency-bound: a start position is a chain of dependent list loads and the perfect
+// check.  With the lists in HBM a wave waited 100 times in turn, and where a block's
+// waves had to meet for one reservation of output, all waited for the slowest.  So a
+// read's lists come to LDS in one step, its loads' addresses are found for all of a
+// block's reads at once (without those that nothing comes of), starts that fail at
+// the read's ends are dropped before the group's compare, a start is added once, the
+// slots' entries have places of their own, and a block is one wave.  Both strands: 2M
+// reads of 50-250 bp 4.78 -> 2.82 ms, 100,000 of 36 bp 162 -> 83 us, 1,000 of
+// 36-250 bp 46 -> 22 us (by a thread per read: 21 ms, 1.7 ms for the 1,000).
 template <int G, bool GLOBAL>
-__global__ void __launch_bounds__(FB) fl_pair(Call c_)
+__global__ void __launch_bounds__(PB) fl_pair(Call c_)
 {
     FArgs a;
     if (!strand_of(c_, a)) return;
-    constexpr int NG = FB / G;           // reads per block
+    constexpr int NG = PB / G, LIST = pair_reads(G);   // reads at a time, reads in all
     constexpr uint64_t GM = G == 64 ? ~0ull : (1ull << (G & 63)) - 1;
     __shared__ int32_t s_pos[GLOBAL ? 1 : ECAP * NG];
     __shared__ int8_t s_flag[GLOBAL ? 1 : ECAP * NG];
     __shared__ int32_t s_perf[GLOBAL ? 1 : PCAP * NG];
+    __shared__ uint32_t s_starts[NG][NSTARTS], s_vals[NG][NVALS + 1];
+    __shared__ PairRead s_list[LIST];
     const int gl = threadIdx.x & (G - 1);
     const int gb = threadIdx.x & 63 & ~(G - 1);
     const uint32_t slot = threadIdx.x / G;
-    const uint32_t j = blockIdx.x * NG + slot;
-    const bool active = j < a.n_todo;
-    Store s;
-    if (GLOBAL) {
-        s.pos = a.slot_pos + (size_t)j * a.cap;
-        s.flag = a.slot_flag + (size_t)j * a.cap;
-        s.perf = a.slot_perf + (size_t)j * a.pcap;
-        s.stride = 1;
-        s.cap = a.cap;
-        s.pcap = a.pcap;
-    } else {
-        s.pos = s_pos + slot;
-        s.flag = s_flag + slot;
-        s.perf = s_perf + slot;
-        s.stride = NG;
-        s.cap = ECAP;
-        s.pcap = PCAP;
-    }
-    if (active) {
-        const uint32_t r = a.todo ? a.todo[j] : j;
-        const DParam P = a.par[a.pid[r]];
-        const uint32_t lb = a.list_base[r];
-        const uint32_t i0 = list_at(a, lb), i1 = list_at(a, lb + P.half);
-        // (an empty list is its terminator: nothing to do when all of them are)
-        if (i1 - i0 != (uint32_t)P.half) {
-            const uint64_t flat_end = chunk_end(a, r), at = a.roff[r];
-            for (uint32_t p0 = i0; p0 < i1 && !s.ovf; p0 += G) {
-                const uint32_t p = p0 + (uint32_t)gl;
-                const uint32_t Pa = p < i1 ? a.flat[p] : 0u;
-                int aa = 0;
-                uint32_t off = 0;
-                bool valid = Pa != 0;
-                if (valid) {
-                    for (int n = P.half; n > 1;) {   // the list holding p
-                        const int h = n >> 1;
-                        if (list_at(a, lb + aa + h) <= p) aa += h;
-                        n -= h;
-                    }
-                    const uint32_t first = list_at(a, lb + aa);
-                    off = p - first;
-                    // a list that starts with offset 0 reads as empty (Q14)
-                    valid = off == 0 || a.flat[first] != 0;
+    const uint32_t n_list = pair_list(a, s_list, (uint32_t)LIST);
+    for (uint32_t j = slot; j < n_list; j += NG) {
+        const PairRead R = s_list[j];
+        const uint32_t r = R.r;
+        Store s;
+        if (GLOBAL) {
+            s.pos = a.slot_pos + (size_t)R.at * a.cap;
+            s.flag = a.slot_flag + (size_t)R.at * a.cap;
+            s.perf = a.slot_perf + (size_t)R.at * a.pcap;
+            s.stride = 1;
+            s.cap = a.cap;
+            s.pcap = a.pcap;
+        } else {
+            s.pos = s_pos + slot;
+            s.flag = s_flag + slot;
+            s.perf = s_perf + slot;
+            s.stride = NG;
+            s.cap = ECAP;
+            s.pcap = PCAP;
+        }
+        const DParam P = a.par[R.pid];
+        const uint32_t n_starts = R.n < NSTARTS ? R.n + 1 : NSTARTS;
+        const uint32_t n_vals = R.end - R.i0 < NVALS ? R.end - R.i0 : NVALS;
+        for (uint32_t x = gl; x < n_starts; x += G) s_starts[slot][x] = list_at(a, R.lb + x);
+#pragma unroll 4
+        for (uint32_t x = gl; x < n_vals; x += G) s_vals[slot][x] = a.flat[R.i0 + x];
+        slots_written<false>();
+        const ReadLists ls{a, R.lb, s_starts[slot], n_starts, s_vals[slot], R.i0, n_vals};
+        const uint64_t at = R.off;
+        for (uint32_t p0 = R.i0; p0 < R.i1 && !s.ovf; p0 += G) {
+            const uint32_t p = p0 + (uint32_t)gl;
+            const uint32_t Pa = p < R.i1 ? ls.val(p) : 0u;
+            int aa = 0;
+            uint32_t off = 0;
+            bool valid = Pa != 0;
+            if (valid) {
+                for (int n = P.half; n > 1;) {   // the list holding p
+                    const int h = n >> 1;
+                    if (ls.start(aa + h) <= p) aa += h;
+                    n -= h;
                 }
-                const long gs = (long)Pa - ((long)aa * P.q + 1);
-                valid = valid && gs + 1 > 0;
-                const uint32_t S = (uint32_t)(gs + 1);
-                // perfect check (strncpy + strcmp, hash.c:550-583), each genome start
-                // once, the group's lanes 16 bases each
-                const bool check = valid && (uint64_t)S + (uint64_t)P.L <= a.glen;
-                bool perfect = false;
-                uint64_t todo = (__ballot(check) >> gb) & GM;
-                while (todo) {
-                    const uint32_t S0 = (uint32_t)__shfl((int)S, gb + (int)__builtin_ctzll(todo), 64);
-                    bool ok = true;
-                    for (int x = gl; 16 * x < P.L && ok; x += G) ok = same16(a, at, P.L, a.dr, S0, x);
-                    const bool all = ((__ballot(!ok) >> gb) & GM) == 0;
-                    const bool mine = check && S == S0;
-                    if (mine) perfect = all;
-                    todo &= ~((__ballot(mine) >> gb) & GM);
-                }
-                int32_t hpos = 0;
-                int hflag = 0;
-                const bool found = valid && pair_matches(a, P, lb, flat_end, aa, off, Pa, gs, hpos, hflag);
-                const int what = (perfect ? 1 : 0) | (found ? 2 : 0) | (hflag << 2);
-                uint64_t add = (__ballot((what & 3) != 0) >> gb) & GM;
-                while (add && !s.ovf) {
-                    const int src = gb + (int)__builtin_ctzll(add);
-                    add &= add - 1;
-                    const int w = __shfl(what, src, 64);
-                    if (w & 1) {
-                        const int32_t S0 = __shfl((int)S, src, 64);
-                        if (group_add<G, GLOBAL>(s, -S0, 0, P.k, gl, gb) != 1 && !s.ovf) {
-                            if (s.np == s.pcap) {
-                                s.ovf = true;
-                            } else {
-                                if (gl == 0) s.Q(s.np) = S0;
-                                ++s.np;
-                            }
+                const uint32_t first = ls.start(aa);
+                off = p - first;
+                // a list that starts with offset 0 reads as empty (Q14)
+                valid = off == 0 || ls.val(first) != 0;
+            }
+            const int64_t gs = (int64_t)Pa - ((int64_t)aa * P.q + 1);
+            valid = valid && gs + 1 > 0;
+            const uint32_t S = (uint32_t)(gs + 1);
+            // perfect check (strncpy + strcmp, hash.c:550-583), each genome start once, the
+            // group's lanes 16 bases each.  Most starts of a chance hit fail at the read's
+            // ends, which each lane looks at for its own: the starts of the loop below wait
+            // for memory one after another
+            const bool check = valid && (uint64_t)S + (uint64_t)P.L <= a.glen &&
+                               (same16(a, at, P.L, a.dr, S, 0) &
+                                same16(a, at, P.L, a.dr, S, (P.L - 1) >> 4));
+            bool perfect = false;
+            uint64_t todo = (__ballot(check) >> gb) & GM;
+            while (todo) {
+                const uint32_t S0 = (uint32_t)__shfl((int)S, gb + (int)__builtin_ctzll(todo), 64);
+                bool ok = true;
+                for (int x = gl + 1; 16 * x < P.L && ok; x += G) ok = same16(a, at, P.L, a.dr, S0, x);
+                const bool all = ((__ballot(!ok) >> gb) & GM) == 0;
+                const bool mine = check && S == S0;
+                if (mine) perfect = all;
+                todo &= ~((__ballot(mine) >> gb) & GM);
+            }
+            int32_t hpos = 0;
+            int hflag = 0;
+            const bool found = valid && pair_matches(ls, P, R.flat_end, aa, off, Pa, gs, hpos, hflag);
+            const int what = (perfect ? 1 : 0) | (found ? 2 : 0) | (hflag << 2);
+            uint64_t add = (__ballot((what & 3) != 0) >> gb) & GM;
+            while (add && !s.ovf) {
+                const int src = gb + (int)__builtin_ctzll(add);
+                const int w = __shfl(what, src, 64);
+                const uint32_t S0 = (uint32_t)__shfl((int)S, src, 64);
+                const int32_t hpos0 = __shfl(hpos, src, 64);
+                if (w & 1) {
+                    if (group_add<G, GLOBAL>(s, -(int32_t)S0, 0, P.k, gl, gb) != 1 && !s.ovf) {
+                        if (s.np == s.pcap) {
+                            s.ovf = true;
+                        } else {
+                            if (gl == 0) s.Q(s.np) = (int32_t)S0;
+                            ++s.np;
                         }
                     }
-                    if ((w & 2) && !s.ovf)
-                        group_add<G, GLOBAL>(s, __shfl(hpos, src, 64), w >> 2, P.k, gl, gb);
                 }
+                if ((w & 2) && !s.ovf) group_add<G, GLOBAL>(s, hpos0, w >> 2, P.k, gl, gb);
+                // a start added again is rejected: its entry, or the one that rejected it,
+                // still decides (an entry's flag is only ever lowered)
+                add &= ~((__ballot(what == w && S == S0 && hpos == hpos0) >> gb) & GM);
             }
         }
-    }
-    // the group's first lane speaks for its read
-    const bool lead = active && gl == 0;
-    const uint32_t ne = (lead && !s.ovf) ? s.n : 0, np = (lead && !s.ovf) ? s.np : 0;
-    // one atomic pair per block reserves the block's output (the two counters are
-    // words that every wave would otherwise update); the waves take consecutive
-    // parts of it
-    __shared__ uint32_t s_sum[FB / 64][2], s_base[2];
-    const uint32_t ie = wave_incl_sum(ne), ip = wave_incl_sum(np);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 63) {
-        s_sum[wv][0] = ie;
-        s_sum[wv][1] = ip;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t te = 0, tp = 0;
-        for (int v = 0; v < FB / 64; ++v) {
-            te += s_sum[v][0];
-            tp += s_sum[v][1];
+        // the group's first lane speaks for its read.  The slots' entries go to the read's
+        // own places; those of a read run again follow them all
+        if (gl == 0) {
+            const uint32_t ne = s.ovf ? 0 : s.n, np = s.ovf ? 0 : s.np;
+            const uint32_t be = GLOBAL ? atomicAdd(&a.counters[0], ne) : r * ECAP;
+            const uint32_t bp = GLOBAL ? atomicAdd(&a.counters[1], np) : r * PCAP;
+            for (uint32_t e = 0; e < ne; ++e) {
+                a.out_pos[be + e] = s.P(e);
+                a.out_flag[be + e] = s.F(e);
+            }
+            for (uint32_t e = 0; e < np; ++e) a.out_perf[bp + e] = s.Q(e);
+            a.meta[3 * (size_t)r + 0] = be;
+            a.meta[3 * (size_t)r + 1] = bp;
+            a.meta[3 * (size_t)r + 2] = s.ovf ? OVERFLOW_MARK : (ne | (np << 16));
+            if (s.ovf) a.over[atomicAdd(&a.counters[2], 1u)] = r;
         }
-        s_base[0] = te ? atomicAdd(&a.counters[0], te) : 0u;
-        s_base[1] = tp ? atomicAdd(&a.counters[1], tp) : 0u;
+        slots_written<GLOBAL>();   // before the next read's
     }
-    __syncthreads();
-    uint32_t be = s_base[0] + ie - ne, bp = s_base[1] + ip - np;
-    for (int v = 0; v < wv; ++v) {
-        be += s_sum[v][0];
-        bp += s_sum[v][1];
-    }
-    if (!lead) return;
-    for (uint32_t e = 0; e < ne; ++e) {
-        a.out_pos[be + e] = s.P(e);
-        a.out_flag[be + e] = s.F(e);
-    }
-    for (uint32_t e = 0; e < np; ++e) a.out_perf[bp + e] = s.Q(e);
-    const uint32_t r = a.todo ? a.todo[j] : j;
-    a.meta[3 * (size_t)r + 0] = be;
-    a.meta[3 * (size_t)r + 1] = bp;
-    a.meta[3 * (size_t)r + 2] = s.ovf ? OVERFLOW_MARK : (ne | (np << 16));
-    if (s.ovf) a.over[atomicAdd(&a.counters[2], 1u)] = r;
 }
 
 // ---- the batch pass (filter_batch.h), a thread per read: counts, and after their
@@ -844,9 +884,11 @@ int launch_search(srm_dfilter *G, const Call &c)
     // thousand that leave the chip idle either way, where one step covers a read's
     // lists (1,000 reads, both strands: 0.373 ms on the device with 32, 0.414 with 8;
     // 2M reads: 38.1 and 32.2 ms)
-    auto pgrid = [&](unsigned g) { return dim3((n + FB / g - 1) / (FB / g), (unsigned)c.n); };
-    if (n < 4096) hipLaunchKernelGGL((fl_pair<32, false>), pgrid(32), dim3(FB), 0, G->st, c);
-    else hipLaunchKernelGGL((fl_pair<8, false>), pgrid(8), dim3(FB), 0, G->st, c);
+    auto pgrid = [&](uint32_t reads) { return dim3((n + reads - 1) / reads, (unsigned)c.n); };
+    if (n < 4096)
+        hipLaunchKernelGGL((fl_pair<32, false>), pgrid(pair_reads(32)), dim3(PB), 0, G->st, c);
+    else
+        hipLaunchKernelGGL((fl_pair<8, false>), pgrid(pair_reads(8)), dim3(PB), 0, G->st, c);
     FL_TRY(hipGetLastError());
     return SRM_OK;
 }
@@ -907,8 +949,8 @@ int run_overflow(srm_dfilter *G, const Call &call, int x, Header &h)
             a.n_todo = m;
             a.over = G->over[x][1 - from].as<uint32_t>();
             a.cap = a.pcap = cap;
-            hipLaunchKernelGGL((fl_pair<64, true>), dim3((m + FB / 64 - 1) / (FB / 64)), dim3(FB), 0,
-                               G->st, c);
+            const uint32_t pr = pair_reads(64);
+            hipLaunchKernelGGL((fl_pair<64, true>), dim3((m + pr - 1) / pr), dim3(PB), 0, G->st, c);
             FL_TRY(hipGetLastError());
             FL_TRY(hipMemcpyAsync(h.counters, a.counters, 12, hipMemcpyDeviceToHost, G->st));
             FL_TRY(hipStreamSynchronize(G->st));
@@ -932,10 +974,10 @@ int run_strands(srm_dfilter *G, Call c, const uint8_t *blocked, const uint16_t *
     const uint64_t nl = c.n_lists;
     const uint32_t n = c.s[0].f.n_reads;
     // the batch pass runs on the device unless separators have to come along that
-    // outweigh it (a byte a base; the host's pass takes tens of nanoseconds a read), or
-    // its lists of flushes and walked reads run over (below): then the host's pass over
-    // the downloaded entries
-    bool on_device = !blocked || G->glen / 64 <= n;
+    // outweigh it (a byte a base at 20 GB/s; the host's pass takes tens of nanoseconds a
+    // read and 160 bytes of slots come down for it), or its lists of flushes and walked
+    // reads run over (below): then the host's pass over the downloaded entries
+    bool on_device = !blocked || G->glen / 512 <= n;
     if (on_device && blocked) {
         FL_RC(G->upload(G->blocked, blocked, G->glen));
         c.blocked = G->blocked.as<uint8_t>();
@@ -954,9 +996,10 @@ int run_strands(srm_dfilter *G, Call c, const uint8_t *blocked, const uint16_t *
     for (int x = 0; x < c.n; ++x) {
         // about one position a list beside its terminator
         FL_RC(G->flat[x].ensure((nl * 2 + 1024) * 4));
-        FL_RC(G->out_pos[x].ensure((size_t)n * ECAP * 4));
-        FL_RC(G->out_flag[x].ensure((size_t)n * ECAP));
-        FL_RC(G->out_perf[x].ensure((size_t)n * PCAP * 4));
+        // (behind the slots, room for the first reads that outgrow them)
+        FL_RC(G->out_pos[x].ensure(((size_t)n * ECAP + OVER_ROOM) * 4));
+        FL_RC(G->out_flag[x].ensure((size_t)n * ECAP + OVER_ROOM));
+        FL_RC(G->out_perf[x].ensure(((size_t)n * PCAP + OVER_ROOM) * 4));
         FL_RC(G->meta[x].ensure((size_t)n * 12));
         FL_RC(G->over[x][0].ensure((size_t)n * 4));
     }

@@ -182,15 +182,17 @@ SRM_HD inline bool same16(const FArgs &a, uint64_t at, int L, int dr, uint64_t S
     const int j = 16 * x, m = L - j < 16 ? L - j : 16;
     const uint64_t o = at + (uint64_t)(dr ? L - j - m : j);
     const uint32_t some = (uint32_t)((1ull << m) - 1u);
+    // all words before the first test: one wait for memory
+    uint32_t c = codes16(a.read_pk, o);
+    const uint32_t g = codes16(a.gen_pk, S + (uint64_t)j);
     if ((odd32(a.read_odd, o) | odd32(a.gen_odd, S + (uint64_t)j)) & some) {
         for (int t = 0; t < m; ++t)
             if (a.genome[S + (uint64_t)(j + t)] != obyte(a.reads + at, L, dr, j + t)) return false;
         return true;
     }
-    uint32_t c = codes16(a.read_pk, o);
     if (dr)   // the m codes complemented and in reverse order, the first on top again
         c = (uint32_t)(reverse_codes(~(uint64_t)c << 32)) << (2 * (16 - m));
-    return ((c ^ codes16(a.gen_pk, S + (uint64_t)j)) >> (2 * (16 - m))) == 0u;
+    return ((c ^ g) >> (2 * (16 - m))) == 0u;
 }
 
 // offset of q-gram list x: ascending from the read's start, then, when q does not
@@ -304,15 +306,27 @@ struct Store {
     }
 };
 
-// first index of the ascending run flat[lo, hi) whose value is >= t
-SRM_HD inline uint64_t run_lower(const uint32_t *flat, uint64_t lo, uint64_t hi, long t)
+// A read's lists (lb: its first): list x starts at flat index start(x), and val(i) is
+// the flat array's element i.  A kernel holds the first n_starts starts and the n_vals
+// elements from index v0 in LDS; the rest, and elements of later reads that a scan
+// runs into (Q12), are read from HBM.
+struct ReadLists {
+    const FArgs &a;
+    uint32_t lb;
+    const uint32_t *starts = nullptr;
+    uint32_t n_starts = 0;
+    const uint32_t *vals = nullptr;
+    uint32_t v0 = 0, n_vals = 0;
+    SRM_HD uint32_t start(int x) const { return (uint32_t)x < n_starts ? starts[x] : list_at(a, lb + (uint32_t)x); }
+    SRM_HD uint32_t val(uint32_t i) const { return i - v0 < n_vals ? vals[i - v0] : a.flat[i]; }
+};
+
+// first index of the ascending run of elements [lo, hi) whose value is >= u
+SRM_HD inline uint32_t run_lower(const ReadLists &ls, uint32_t lo, uint32_t hi, uint32_t u)
 {
-    if (t <= 0) return lo;
-    if (t > 0xFFFFFFFFl) return hi;
-    const uint32_t u = (uint32_t)t;
     while (lo < hi) {
-        const uint64_t m = (lo + hi) >> 1;
-        if (flat[m] < u) lo = m + 1;
+        const uint32_t m = lo + ((hi - lo) >> 1);
+        if (ls.val(m) < u) lo = m + 1;
         else hi = m;
     }
     return lo;
@@ -320,23 +334,27 @@ SRM_HD inline uint64_t run_lower(const uint32_t *flat, uint64_t lo, uint64_t hi,
 
 // The pair passes' matches of one list in the reference's scan order.  The scan
 // compares every target tg(err), err = -lim .. lim, with the ascending run
-// flat[lo, min(hi, end)) -- cut at its first 0, as the reference's 0-terminated
+// [lo, min(hi, end)) of elements -- cut at its first 0, as the reference's 0-terminated
 // scans are -- and, in the first pass, first with one more value p0 (p0 == 0:
 // none).  The targets are consecutive (ascending from t_lo when up, descending
 // from t_hi otherwise), so the matches are the run's values in [t_lo, t_hi] found
 // by one search and a walk, p0 merged in before a run value of the same target.
 // Counts them into *hits and returns true when the count reaches need.
-SRM_HD inline bool scan_run(const uint32_t *flat, uint64_t lo, uint64_t hi, uint64_t end,
-                            long t_lo, long t_hi, bool up, uint32_t p0, int need, int &hits)
+SRM_HD inline bool scan_run(const ReadLists &ls, uint32_t lo, uint32_t hi, uint32_t end,
+                            int64_t t_lo, int64_t t_hi, bool up, uint32_t p0, int need, int &hits)
 {
+    if (t_hi < 0) return false;
+    // positions are below 2^31, so the targets that one can equal fit 32 bits
+    const uint32_t u_lo = t_lo > 0 ? (uint32_t)t_lo : 0u, u_hi = (uint32_t)t_hi;
     if (hi > end) hi = end;
-    if (lo >= hi || flat[lo] == 0) hi = lo;    // an empty run
-    bool p0_left = p0 != 0 && (long)p0 >= t_lo && (long)p0 <= t_hi;
+    if (lo >= hi || ls.val(lo) == 0) hi = lo;    // an empty run
+    bool p0_left = p0 != 0 && p0 >= u_lo && p0 <= u_hi;
     if (up) {
-        uint64_t i = run_lower(flat, lo, hi, t_lo);
+        uint32_t i = run_lower(ls, lo, hi, u_lo);
         for (;;) {
-            const bool run_next = i < hi && (long)flat[i] <= t_hi;
-            if (p0_left && (!run_next || (long)p0 <= (long)flat[i])) {
+            const uint32_t v = i < hi ? ls.val(i) : 0xFFFFFFFFu;
+            const bool run_next = v <= u_hi;
+            if (p0_left && (!run_next || p0 <= v)) {
                 p0_left = false;
                 if (++hits == need) return true;
                 continue;
@@ -347,8 +365,8 @@ SRM_HD inline bool scan_run(const uint32_t *flat, uint64_t lo, uint64_t hi, uint
         }
     }
     // descending (second pass only: no p0)
-    uint64_t i = run_lower(flat, lo, hi, t_hi + 1);
-    while (i > lo && (long)flat[i - 1] >= t_lo) {
+    uint32_t i = run_lower(ls, lo, hi, u_hi + 1u);
+    while (i > lo && ls.val(i - 1) >= u_lo) {
         if (++hits == need) return true;
         --i;
     }
@@ -385,7 +403,7 @@ SRM_HD inline int add_start(Store &s, int32_t pos, int flag, int possible, int e
 }
 
 // the end of the position lists a read's list indexes may run into: its chunk's
-SRM_HD inline uint64_t chunk_end(const FArgs &a, uint32_t r)
+SRM_HD inline uint32_t chunk_end(const FArgs &a, uint32_t r)
 {
     const uint64_t next_chunk = ((uint64_t)(r / a.cv) + 1) * a.cv;
     return list_at(a, a.list_base[next_chunk < a.n_reads ? next_chunk : a.n_reads]);
@@ -397,10 +415,10 @@ SRM_HD inline uint64_t chunk_end(const FArgs &a, uint32_t r)
 // exact_tresh (Q13): the need-th match of the two passes in scan order, need =
 // exact_tresh - 1, is the only one that can insert, and the scan stops there.
 // True when there is one, with what it inserts.
-SRM_HD inline bool pair_matches(const FArgs &a, const DParam &P, uint32_t lb, uint64_t flat_end,
-                                int aa, uint64_t off, uint32_t Pa, long gs, int32_t &hpos, int &hflag)
+SRM_HD inline bool pair_matches(const ReadLists &ls, const DParam &P, uint32_t flat_end, int aa,
+                                uint32_t off, uint32_t Pa, int64_t gs, int32_t &hpos, int &hflag)
 {
-    const int q = P.q, half = P.half, k = P.k, L = P.L, dr = a.dr;
+    const int q = P.q, half = P.half, k = P.k, L = P.L, dr = ls.a.dr;
     const bool fqm = (aa == 0);
     const int need = P.exact - 1;
     if (need < 1) return false;
@@ -409,24 +427,21 @@ SRM_HD inline bool pair_matches(const FArgs &a, const DParam &P, uint32_t lb, ui
     // D(b, 1), D(b, 2), ... up to the next 0 (Q12): the element at a's index, then
     // one ascending run of list b (or of the list after b when b is empty).
     for (int b = aa + 1; b < half; ++b) {
-        const uint64_t at = (uint64_t)list_at(a, lb + b) + off;
-        const uint32_t P0 = at < flat_end ? a.flat[at] : 0u;
+        const uint32_t sb = ls.start(b), nb = ls.start(b + 1);
+        const uint64_t at = (uint64_t)sb + off;
+        const uint32_t P0 = at < flat_end ? ls.val((uint32_t)at) : 0u;
         if (P0 == 0) continue;                 // the scan never starts
-        const long rstart = (long)b * q + 1;
-        uint64_t lo = (uint64_t)list_at(a, lb + b) + 1, hi = lo;
-        const uint64_t nb = list_at(a, lb + b + 1);
-        if (lo < nb) {
-            hi = nb - 1;                       // list b from index 1
-        } else if ((uint64_t)lb + b + 2 <= a.list_base[a.n_reads]) {
-            hi = (uint64_t)list_at(a, lb + b + 2) - 1;   // the next list
-        }
-        if (!scan_run(a.flat, lo, hi, flat_end, gs + rstart - k, gs + rstart + k, true, P0, need, hits))
+        const int64_t rstart = (int64_t)b * q + 1;
+        const uint32_t lo = sb + 1;
+        // list b from index 1, or the next list (b + 2 <= half + 1 <= P.n: the read's)
+        const uint32_t hi = (lo < nb ? nb : ls.start(b + 2)) - 1;
+        if (!scan_run(ls, lo, hi, flat_end, gs + rstart - k, gs + rstart + k, true, P0, need, hits))
             continue;
         if (b == half - 1 && fqm) {
             hflag = 1 + dr;
             hpos = (int32_t)(gs + 1);
         } else if (aa == half - 1) {
-            hflag = ((long)Pa + q > L ? 3 : 2) + dr;
+            hflag = ((int64_t)Pa + q > L ? 3 : 2) + dr;
             hpos = (int32_t)(gs - k + 1);
         } else if (fqm) {
             hflag = 1 + dr;
@@ -442,10 +457,9 @@ SRM_HD inline bool pair_matches(const FArgs &a, const DParam &P, uint32_t lb, ui
     // is negated there)
     for (int j = 0; j < half; ++j) {
         const int lim = half - 1 - j - aa < 0 ? -(half - 1 - j - aa) : half - 1 - j - aa;
-        const long nin = (long)(half - j - 1) * q + 1 + P.rest;
-        const uint64_t lo = list_at(a, lb + half + j);
-        const uint64_t hi = (uint64_t)list_at(a, lb + half + j + 1) - 1;
-        if (!scan_run(a.flat, lo, hi, flat_end, gs + nin - lim, gs + nin + lim, j - aa >= 0, 0u, need,
+        const int64_t nin = (int64_t)(half - j - 1) * q + 1 + P.rest;
+        const uint32_t lo = ls.start(half + j), hi = ls.start(half + j + 1) - 1;
+        if (!scan_run(ls, lo, hi, flat_end, gs + nin - lim, gs + nin + lim, j - aa >= 0, 0u, need,
                       hits))
             continue;
         if (j == 0 && fqm) {
@@ -467,18 +481,17 @@ SRM_HD inline bool pair_matches(const FArgs &a, const DParam &P, uint32_t lb, ui
 }
 
 // run_seashore of one read, its start positions one after another (the kernels
-// take several at a time)
-SRM_HD inline void seashore(const FArgs &a, uint32_t r, Store &s)
+// take several at a time); ls: its lists
+SRM_HD inline void seashore(const FArgs &a, uint32_t r, Store &s, const ReadLists &ls)
 {
     const DParam P = a.par[a.pid[r]];
     const int L = P.L, dr = a.dr;
     const char *rd = a.reads + a.roff[r];
-    const uint32_t lb = a.list_base[r];
-    const uint64_t flat_end = chunk_end(a, r);
+    const uint32_t flat_end = chunk_end(a, r);
     for (int aa = 0; aa < P.half; ++aa) {
         for (uint64_t off = 0;; ++off) {
-            const uint64_t at = (uint64_t)list_at(a, lb + aa) + off;
-            const uint32_t Pa = at < flat_end ? a.flat[at] : 0u;
+            const uint64_t at = (uint64_t)ls.start(aa) + off;
+            const uint32_t Pa = at < flat_end ? ls.val((uint32_t)at) : 0u;
             if (Pa == 0) break;
             const long gs = (long)Pa - ((long)aa * P.q + 1);
             if (gs + 1 <= 0) continue;
@@ -496,12 +509,17 @@ SRM_HD inline void seashore(const FArgs &a, uint32_t r, Store &s)
             }
             int32_t hpos;
             int hflag;
-            if (pair_matches(a, P, lb, flat_end, aa, off, Pa, gs, hpos, hflag)) {
+            if (pair_matches(ls, P, flat_end, aa, (uint32_t)off, Pa, gs, hpos, hflag)) {
                 add_start(s, hpos, hflag, P.exact, P.exact, P.k);
                 if (s.ovf) return;
             }
         }
     }
+}
+
+SRM_HD inline void seashore(const FArgs &a, uint32_t r, Store &s)
+{
+    seashore(a, r, s, ReadLists{a, a.list_base[r]});
 }
 
 // the device copies of the per-read parameter sets and their q-gram offsets
