@@ -108,6 +108,7 @@ struct Call {
     Strand s[2];
     int n;
     uint64_t n_lists;        // per strand
+    uint64_t list_stride;    // words from a strand's list arrays to the other's
     int kmax;
     const uint8_t *blocked;
     unsigned char *blob;     // the strands' candidates and perfect hits, arrays packed
@@ -142,10 +143,10 @@ struct BlockReads {
     uint32_t base[CREADS + 1];
     uint64_t off[CREADS];
     int L[CREADS], q[CREADS];
-    __device__ uint32_t load(const FArgs &a, uint32_t per)
+    __device__ uint32_t load(const FArgs &a, uint32_t per, uint32_t lo, uint32_t hi)
     {
-        const uint32_t r0 = blockIdx.x * per;
-        const uint32_t nr = a.n_reads - r0 < per ? a.n_reads - r0 : per;
+        const uint32_t r0 = lo + blockIdx.x * per;
+        const uint32_t nr = hi - r0 < per ? hi - r0 : per;
         for (uint32_t t = threadIdx.x; t <= nr; t += FB) {
             base[t] = a.list_base[r0 + t];
             if (t < nr) {
@@ -170,30 +171,31 @@ struct BlockReads {
     }
 };
 
-__global__ void __launch_bounds__(FB) fl_count(Call c_, uint32_t per)
+// the lists of reads [lo, hi)
+__global__ void __launch_bounds__(FB) fl_count(Call c_, uint32_t per, uint32_t lo, uint32_t hi)
 {
     __shared__ BlockReads s;
     const FArgs &a = c_.s[blockIdx.y].f;
-    if (blockIdx.x == 0) {   // what later kernels of the call add to
+    if (blockIdx.x == 0 && hi == a.n_reads) {   // what later kernels of the call add to
         // (the entries and perfect hits of reads that are run again follow all slots')
         if (threadIdx.x < 6)
             ((uint32_t *)c_.s[blockIdx.y].hdr)[threadIdx.x] =
                 threadIdx.x == 0 ? a.n_reads * ECAP : threadIdx.x == 1 ? a.n_reads * PCAP : 0;
         if (threadIdx.x == 0) a.list_cnt[c_.n_lists] = 0;
     }
-    const uint32_t nr = s.load(a, per);
+    const uint32_t nr = s.load(a, per, lo, hi);
     for (uint32_t i = s.base[0] + threadIdx.x; i < s.base[nr]; i += FB) {
         const uint32_t t = s.read_of(i, nr);
         const int L = s.L[t], q = s.q[t], g = gram_offset(L, q, (int)(i - s.base[t]));
         const DQ X = a.qix[q];
         uint64_t code;
-        uint32_t lo, c;
+        uint32_t first, c;
         if (gram_code(a.read_pk, a.read_odd, s.off[t], L, a.dr, q, g, code))
-            c = lookup_code(X, code, lo);
+            c = lookup_code(X, code, first);
         else
-            c = lookup<false>(X, a.genome, a.reads + s.off[t], L, a.dr, g, nullptr, &lo);
+            c = lookup<false>(X, a.genome, a.reads + s.off[t], L, a.dr, g, nullptr, &first);
         a.list_cnt[i] = c + 1;
-        a.list_lo[i] = lo;
+        a.list_lo[i] = first;
     }
 }
 
@@ -204,7 +206,7 @@ __global__ void __launch_bounds__(FB) fl_fill(Call c_, uint32_t per)
     __shared__ BlockReads s;
     FArgs a;
     if (!strand_of(c_, a)) return;
-    const uint32_t nr = s.load(a, per);
+    const uint32_t nr = s.load(a, per, 0, a.n_reads);
     for (uint32_t i = s.base[0] + threadIdx.x; i < s.base[nr]; i += FB) {
         const uint32_t c = a.list_cnt[i] - 1;
         uint32_t *dst = a.flat + list_at(a, i);
@@ -771,6 +773,9 @@ private:
 constexpr size_t STAGE_IN = (size_t)1 << 20;
 // and this much of the output comes back with the headers, in one copy
 constexpr size_t STAGE_OUT = (size_t)128 << 10;
+// reads of one piece of a large upload, at most, and its plan in page-locked memory
+constexpr size_t PIECE = 131072, PIECE_BYTES = (PIECE + 2) * (8 + 4 + 2);
+constexpr size_t MAX_SETS = 16384;   // parameter sets (length, k) of a call in pieces
 
 }  // namespace
 
@@ -788,7 +793,9 @@ struct srm_dfilter {
     GBuf slot_pos, slot_flag, slot_perf;
     void *stage_in = nullptr, *stage_out = nullptr;   // page-locked
     std::shared_ptr<BlockPool> pool = std::make_shared<BlockPool>();
-    hipEvent_t ev[2] = {nullptr, nullptr};
+    void *stage_plan = nullptr;                       // two pieces' plans, likewise
+    hipStream_t copy_st = nullptr;                    // the pieces' copies
+    hipEvent_t ev[2] = {nullptr, nullptr}, piece_ev[2] = {nullptr, nullptr};
     float last_ms = 0.f;
     size_t last_lists = 0, last_flat = 0, last_overflow = 0;
 
@@ -806,7 +813,11 @@ struct srm_dfilter {
             for (auto &b : *v) b.release();
         if (stage_in) (void)hipHostFree(stage_in);
         if (stage_out) (void)hipHostFree(stage_out);
+        if (stage_plan) (void)hipHostFree(stage_plan);
+        if (copy_st) (void)hipStreamDestroy(copy_st);
         for (auto &e : ev)
+            if (e) (void)hipEventDestroy(e);
+        for (auto &e : piece_ev)
             if (e) (void)hipEventDestroy(e);
     }
 
@@ -817,19 +828,20 @@ struct srm_dfilter {
         return SRM_OK;
     }
 
-    // the codes and the mask of other bytes of n bytes at src (two code words and one
-    // mask word past the last are read beside them)
-    int pack(const void *src, size_t bytes, GBuf &pk, GBuf &odd)
+    // the codes and the mask of other bytes of the bytes [from, to) at src, of which there
+    // will be `bytes` (two code words and one mask word past the last are read beside them)
+    int pack(const void *src, size_t bytes, GBuf &pk, GBuf &odd, size_t from, size_t to)
     {
-        const size_t n16 = (bytes + 15) / 16;
+        const size_t n16 = (bytes + 15) / 16, b = from / 16, e = (to + 15) / 16;
         FL_RC(pk.ensure((n16 + 4) * 4));
         FL_RC(odd.ensure((n16 + 4) * 2 + 4));
-        if (n16 == 0) return SRM_OK;
-        hipLaunchKernelGGL(fl_pack, dim3((unsigned)((n16 + FB - 1) / FB)), dim3(FB), 0, st,
-                           (const uint4 *)src, pk.as<uint32_t>(), odd.as<uint16_t>(), n16);
+        if (e <= b) return SRM_OK;
+        hipLaunchKernelGGL(fl_pack, dim3((unsigned)((e - b + FB - 1) / FB)), dim3(FB), 0, st,
+                           (const uint4 *)src + b, pk.as<uint32_t>() + b, odd.as<uint16_t>() + b, e - b);
         FL_TRY(hipGetLastError());
         return SRM_OK;
     }
+    int pack(const void *src, size_t bytes, GBuf &pk, GBuf &odd) { return pack(src, bytes, pk, odd, 0, bytes); }
 
     // b with room for `bytes`, its first `used` bytes kept
     int grow(GBuf &b, size_t bytes, size_t used)
@@ -858,25 +870,42 @@ struct srm_dfilter {
 
 namespace {
 
-// lookups, lists and pairing of the call's strands
+// reads per block of the lookups and the fill: CREADS while that fills the chip twice
+// over, fewer below
+uint32_t list_reads(size_t n)
+{
+    return (uint32_t)std::min<size_t>(CREADS, std::max<size_t>(4, n / 512));
+}
+
+// the lookups of reads [lo, hi)
+int launch_count(srm_dfilter *G, const Call &c, uint32_t lo, uint32_t hi)
+{
+    const uint32_t per = list_reads(hi - lo);
+    hipLaunchKernelGGL(fl_count, dim3((hi - lo + per - 1) / per, (unsigned)c.n), dim3(FB), 0, G->st, c,
+                       per, lo, hi);
+    FL_TRY(hipGetLastError());
+    return SRM_OK;
+}
+
+// lists and pairing of the call's strands
 int launch_search(srm_dfilter *G, const Call &c)
 {
     const uint32_t n = c.s[0].f.n_reads;
     const uint64_t nl = c.n_lists;
-    // reads per block: CREADS while that fills the chip twice over, fewer below
-    const uint32_t per = (uint32_t)std::min<size_t>(CREADS, std::max<size_t>(4, n / 512));
+    const uint32_t per = list_reads(n);
     const dim3 grid((n + per - 1) / per, (unsigned)c.n);
-    hipLaunchKernelGGL(fl_count, grid, dim3(FB), 0, G->st, c, per);
-    FL_TRY(hipGetLastError());
-    // both strands' lengths in one sum: the second strand's offsets count from its
-    // first (list_org), modulo 2^32
-    size_t tmp = 0;
-    const int items = (int)((nl + 1) * (uint64_t)c.n);
-    FL_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, G->list_cnt.as<uint32_t>(),
-                                            G->list_start.as<uint32_t>(), items, G->st));
-    FL_RC(G->cub_tmp.ensure(tmp));
-    FL_TRY(hipcub::DeviceScan::ExclusiveSum(G->cub_tmp.p, tmp, G->list_cnt.as<uint32_t>(),
-                                            G->list_start.as<uint32_t>(), items, G->st));
+    // both strands' lengths in one sum where they lie together: the second strand's
+    // offsets count from its first (list_org), modulo 2^32
+    const bool one = c.list_stride == nl + 1;
+    const int items = (int)((nl + 1) * (uint64_t)(one ? c.n : 1));
+    for (int x = 0; x < (one ? 1 : c.n); ++x) {
+        size_t tmp = 0;
+        const uint32_t *from = c.s[x].f.list_cnt;
+        uint32_t *to = G->list_start.as<uint32_t>() + (size_t)x * c.list_stride;
+        FL_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, from, to, items, G->st));
+        FL_RC(G->cub_tmp.ensure(tmp));
+        FL_TRY(hipcub::DeviceScan::ExclusiveSum(G->cub_tmp.p, tmp, from, to, items, G->st));
+    }
     hipLaunchKernelGGL(fl_fill, grid, dim3(FB), 0, G->st, c, per);
     FL_TRY(hipGetLastError());
     // lanes per read: a wave for the reads of hundreds of entries (below); 8, about
@@ -966,9 +995,34 @@ int run_overflow(srm_dfilter *G, const Call &call, int x, Header &h)
     return SRM_OK;
 }
 
-// one or both strands (strands: bit 0 forward, bit 1 reverse) over the reads on the
-// device, at most one of the strands when `nl` lists leave no room for two in one sum
-int run_strands(srm_dfilter *G, Call c, const uint8_t *blocked, const uint16_t *read_len,
+// the buffers that the lookups write: lists of c.n strands, list_stride words each, and
+// the headers with the output behind them
+int ensure_lists(srm_dfilter *G, const Call &c)
+{
+    const size_t words = c.list_stride * (size_t)c.n, n = c.s[0].f.n_reads;
+    FL_RC(G->list_cnt.ensure(words * 4));
+    FL_RC(G->list_lo.ensure(words * 4));
+    FL_RC(G->list_start.ensure(words * 4));
+    // candidates and perfect hits of both strands are 1-1.2 a read, 16-20 bytes each
+    FL_RC(G->out.ensure(sizeof(Header) * (size_t)c.n + std::max<size_t>(STAGE_OUT, 28 * n)));
+    return SRM_OK;
+}
+
+void bind_lists(const srm_dfilter *G, Call &c)
+{
+    for (int x = 0; x < c.n; ++x) {
+        FArgs &a = c.s[x].f;
+        c.s[x].hdr = G->out.as<Header>() + x;
+        a.counters = c.s[x].hdr->counters;
+        a.list_cnt = G->list_cnt.as<uint32_t>() + (size_t)x * c.list_stride;
+        a.list_lo = G->list_lo.as<uint32_t>() + (size_t)x * c.list_stride;
+        a.list_start = G->list_start.as<uint32_t>() + (size_t)x * c.list_stride;
+    }
+}
+
+// one or both strands over the reads on the device (both while their lists fit one sum);
+// counted: their lookups are under way (upload_pieces)
+int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, const uint16_t *read_len,
                 const uint8_t *read_k, srm_filter **out)
 {
     const uint64_t nl = c.n_lists;
@@ -982,17 +1036,13 @@ int run_strands(srm_dfilter *G, Call c, const uint8_t *blocked, const uint16_t *
         FL_RC(G->upload(G->blocked, blocked, G->glen));
         c.blocked = G->blocked.as<uint8_t>();
     }
-    FL_RC(G->list_cnt.ensure((nl + 1) * 4 * (size_t)c.n));
-    FL_RC(G->list_lo.ensure((nl + 1) * 4 * (size_t)c.n));
-    FL_RC(G->list_start.ensure((nl + 1) * 4 * (size_t)c.n));
+    if (!counted) FL_RC(ensure_lists(G, c));
     FL_RC(G->cnt.ensure(((size_t)n + 1) * sizeof(Counts) * (size_t)c.n));
     FL_RC(G->start.ensure(((size_t)n + 1) * sizeof(Counts) * (size_t)c.n));
     FL_RC(G->by_rank.ensure((size_t)n * 4 * (size_t)c.n));
     FL_RC(G->unsafe.ensure((size_t)MAX_UNSAFE * 4 * (size_t)c.n));
     FL_RC(G->walk.ensure((size_t)MAX_WALK * 4 * (size_t)c.n));
-    // candidates and perfect hits of both strands are 1-1.2 a read, 16-20 bytes each
     const size_t head = sizeof(Header) * (size_t)c.n;
-    FL_RC(G->out.ensure(head + std::max<size_t>(STAGE_OUT, 28 * (size_t)n)));
     for (int x = 0; x < c.n; ++x) {
         // about one position a list beside its terminator
         FL_RC(G->flat[x].ensure((nl * 2 + 1024) * 4));
@@ -1004,21 +1054,17 @@ int run_strands(srm_dfilter *G, Call c, const uint8_t *blocked, const uint16_t *
         FL_RC(G->over[x][0].ensure((size_t)n * 4));
     }
     auto bind = [&] {
+        bind_lists(G, c);
         for (int x = 0; x < c.n; ++x) {
             Strand &s = c.s[x];
             FArgs &a = s.f;
-            s.hdr = G->out.as<Header>() + x;
             s.flat_cap = G->flat[x].cap / 4;
             s.cnt = G->cnt.as<Counts>() + (size_t)x * ((size_t)n + 1);
             s.start = G->start.as<Counts>() + (size_t)x * ((size_t)n + 1);
             s.by_rank = G->by_rank.as<uint32_t>() + (size_t)x * n;
             s.unsafe = G->unsafe.as<uint32_t>() + (size_t)x * MAX_UNSAFE;
             s.walk = G->walk.as<uint32_t>() + (size_t)x * MAX_WALK;
-            a.list_cnt = G->list_cnt.as<uint32_t>() + (size_t)x * (nl + 1);
-            a.list_lo = G->list_lo.as<uint32_t>() + (size_t)x * (nl + 1);
-            a.list_start = G->list_start.as<uint32_t>() + (size_t)x * (nl + 1);
             a.flat = G->flat[x].as<uint32_t>();
-            a.counters = s.hdr->counters;
             a.out_pos = G->out_pos[x].as<int32_t>();
             a.out_flag = G->out_flag[x].as<int8_t>();
             a.out_perf = G->out_perf[x].as<int32_t>();
@@ -1033,6 +1079,7 @@ int run_strands(srm_dfilter *G, Call c, const uint8_t *blocked, const uint16_t *
         c.blob_cap = G->out.cap - head;
     };
     bind();
+    if (!counted) FL_RC(launch_count(G, c, 0, n));
     FL_RC(launch_search(G, c));
     if (on_device) FL_RC(launch_batch(G, c));
     // the headers and the first part of the output; what did not fit is made room for
@@ -1060,6 +1107,7 @@ int run_strands(srm_dfilter *G, Call c, const uint8_t *blocked, const uint16_t *
         }
     if (again) {
         bind();
+        FL_RC(launch_count(G, c, 0, n));   // (the counters start over)
         FL_RC(launch_search(G, c));
         if (on_device) FL_RC(launch_batch(G, c));
         FL_RC(fetch());
@@ -1179,6 +1227,100 @@ int run_strands(srm_dfilter *G, Call c, const uint8_t *blocked, const uint16_t *
     return SRM_OK;
 }
 
+// The reads and their plan to the device in pieces, the plan and the lookups of one
+// piece made while the next ones are on their way.  c: the strands to look up.  counted
+// stays false where the totals guessed from a sample of the reads do not hold: the call
+// goes on as a small one.
+//
+// Bound by the copy of the reads (57 GB/s from page-locked memory).  With the plan made
+// before it and the lookups after it, 2M reads of 143 bp took 3.5 + 6.6 + 2.9 ms; in
+// pieces 5.9 ms.
+int upload_pieces(srm_dfilter *G, Call &c, const char *reads, const uint64_t *read_off,
+                  const uint16_t *read_len, const uint8_t *read_k, size_t n, bool &counted)
+{
+    Planner plan(G->ix);
+    std::string err;
+    // the totals: the end of the last read, and the lists of every so many reads
+    const size_t bytes = read_off[n - 1] + read_len[n - 1], step = std::max<size_t>(1, n / 512);
+    uint64_t sum = 0, seen = 0;
+    for (size_t i = 0; i < n; i += step, ++seen) {
+        const int32_t id = plan.set_of(read_len[i], read_k[i], err);
+        if (id < 0) return SRM_OK;   // the first bad read's error is the call's
+        sum += plan.lists[(size_t)id];
+    }
+    const uint64_t room = (uint64_t)((double)sum / (double)seen * (double)n * 1.125) + 4096;
+    if (room >= (uint64_t)1 << 30 || plan.params.size() > MAX_SETS) return SRM_OK;
+    size_t at[5] = {MAX_SETS * sizeof(DParam), (n + 1) * 4, n * 2, n * 8, bytes}, all = 0;
+    for (size_t &p : at) {
+        const size_t b = p;
+        p = all;
+        all = (all + b + 255) & ~(size_t)255;
+    }
+    FL_RC(G->in.ensure(all + 64));   // slack: whole 16-byte words of the reads are read
+    char *in = G->in.as<char>();
+    c.list_stride = room;
+    FArgs &a = c.s[0].f;
+    a.par = (const DParam *)(in + at[0]);
+    a.list_base = (const uint32_t *)(in + at[1]);
+    a.pid = (const uint16_t *)(in + at[2]);
+    a.roff = (const uint64_t *)(in + at[3]);
+    a.reads = in + at[4];
+    FL_RC(ensure_lists(G, c));
+    FL_RC(G->pack(a.reads, bytes, G->read_pk, G->read_odd, 0, 0));
+    a.read_pk = G->read_pk.as<uint32_t>();
+    a.read_odd = G->read_odd.as<uint32_t>();
+    if (c.n > 1) {
+        c.s[1].f = a;
+        c.s[1].f.dr = 4;
+    }
+    bind_lists(G, c);
+    size_t sent = 0, sets = 0;
+    std::vector<DParam> dpar;
+    std::vector<uint16_t> gram;
+    // an eighth of the reads, so that little is left to do after the last one's arrival;
+    // a piece below 32,768 costs more calls than it hides
+    const size_t piece = std::min(PIECE, std::max<size_t>(PIECE / 4, (n + 7) / 8));
+    int k = 0;
+    for (size_t lo = 0; lo < n; lo += piece, ++k) {
+        const size_t hi = std::min(n, lo + piece), m = hi - lo;
+        hipEvent_t done = G->piece_ev[k & 1];
+        if (k >= 2) FL_TRY(hipEventSynchronize(done));   // its staging is free again
+        char *st = (char *)G->stage_plan + (size_t)(k & 1) * PIECE_BYTES;
+        auto *off = (uint64_t *)st;
+        auto *base = (uint32_t *)(off + PIECE);
+        auto *pid = (uint16_t *)(base + PIECE + 2);
+        if (int rc = plan.piece(read_off, read_len, read_k, lo, hi, pid, base, err))
+            return srm::set_error(rc, "%s", err.c_str());
+        if (plan.n_lists + 1 > room || plan.read_bytes > bytes || plan.params.size() > MAX_SETS)
+            return SRM_OK;
+        if (plan.params.size() > sets) {
+            dpar.clear();
+            device_params(plan.params, dpar, gram);
+            FL_TRY(hipMemcpyAsync(in + at[0] + sets * sizeof(DParam), dpar.data() + sets,
+                                  (dpar.size() - sets) * sizeof(DParam), hipMemcpyHostToDevice, G->copy_st));
+            FL_TRY(hipStreamSynchronize(G->copy_st));   // (dpar changes with the next sets)
+            sets = plan.params.size();
+        }
+        if (plan.read_bytes > sent)
+            FL_TRY(hipMemcpyAsync(in + at[4] + sent, reads + sent, plan.read_bytes - sent,
+                                  hipMemcpyHostToDevice, G->copy_st));
+        std::memcpy(off, read_off + lo, m * 8);
+        FL_TRY(hipMemcpyAsync(in + at[1] + lo * 4, base, (m + 1) * 4, hipMemcpyHostToDevice, G->copy_st));
+        FL_TRY(hipMemcpyAsync(in + at[2] + lo * 2, pid, m * 2, hipMemcpyHostToDevice, G->copy_st));
+        FL_TRY(hipMemcpyAsync(in + at[3] + lo * 8, off, m * 8, hipMemcpyHostToDevice, G->copy_st));
+        FL_TRY(hipEventRecord(done, G->copy_st));
+        FL_TRY(hipStreamWaitEvent(G->st, done, 0));
+        // (the bytes of a word that two pieces share are packed again with the second)
+        FL_RC(G->pack(a.reads, bytes, G->read_pk, G->read_odd, sent, plan.read_bytes));
+        sent = plan.read_bytes;
+        c.n_lists = plan.n_lists;
+        FL_RC(launch_count(G, c, (uint32_t)lo, (uint32_t)hi));
+    }
+    for (const Params &p : plan.params) c.kmax = std::max(c.kmax, p.k);
+    counted = true;
+    return SRM_OK;
+}
+
 // one or both strands (strands: bit 0 forward, bit 1 reverse) over one upload of
 // the reads
 int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
@@ -1186,6 +1328,41 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
                size_t n_reads, int strands, int chunk_value, srm_filter **out_fwd,
                srm_filter **out_rev)
 {
+    G->last_flat = 0;
+    G->last_overflow = 0;
+    FL_TRY(hipSetDevice(G->device));
+    FL_TRY(hipEventRecord(G->ev[0], G->st));
+    FArgs a{};
+    a.qix = G->dq.as<DQ>();
+    a.genome = G->genome.as<char>();
+    a.glen = G->glen;
+    a.gen_pk = G->gen_pk.as<uint32_t>();
+    a.gen_odd = G->gen_odd.as<uint32_t>();
+    a.n_reads = (uint32_t)n_reads;
+    a.cv = (uint32_t)chunk_value;
+    srm_filter **outs[2] = {out_fwd, out_rev};
+    auto both = [&](Call &c, bool counted) -> int {
+        srm_filter *F[2] = {nullptr, nullptr};
+        const int rc = run_strands(G, c, counted, blocked, read_len, read_k, F);
+        *outs[strands == 2 ? 1 : 0] = F[0];
+        if (strands == 3) *out_rev = F[1];
+        return rc;
+    };
+    Call c{};
+    c.n = strands == 3 ? 2 : 1;
+    c.s[0].f = a;
+    c.s[0].f.dr = strands == 2 ? 4 : 0;
+    // in pieces where the reads make two or more
+    if (n_reads > PIECE / 4) {
+        bool counted = false;
+        FL_RC(upload_pieces(G, c, reads, read_off, read_len, read_k, n_reads, counted));
+        if (counted) {
+            G->last_lists = c.n_lists * (uint64_t)c.n;
+            return both(c, true);
+        }
+        FL_TRY(hipStreamSynchronize(G->copy_st));
+        FL_TRY(hipStreamSynchronize(G->st));
+    }
     ReadPlan plan;
     std::string err;
     if (int rc = plan_reads(G->ix, read_off, read_len, read_k, n_reads, plan, err))
@@ -1198,10 +1375,6 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     const uint64_t nl = list_base[n_reads];
     const uint64_t rbytes = plan.read_bytes;
     G->last_lists = nl * (strands == 3 ? 2 : 1);
-    G->last_flat = 0;
-    G->last_overflow = 0;
-    FL_TRY(hipSetDevice(G->device));
-    FL_TRY(hipEventRecord(G->ev[0], G->st));
     // the inputs, one after another in one buffer
     struct Part {
         const void *src;
@@ -1229,42 +1402,30 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     }
     const char *in = G->in.as<char>();
     FL_RC(G->pack(in + part[4].at, rbytes, G->read_pk, G->read_odd));
-    Call c{};
-    c.n_lists = nl;
-    for (const Params &p : plan.params) c.kmax = std::max(c.kmax, p.k);
-    FArgs a{};
-    a.qix = G->dq.as<DQ>();
     a.par = (const DParam *)(in + part[0].at);
-    a.genome = G->genome.as<char>();
-    a.glen = G->glen;
     a.reads = in + part[4].at;
     a.read_pk = G->read_pk.as<uint32_t>();
     a.read_odd = G->read_odd.as<uint32_t>();
-    a.gen_pk = G->gen_pk.as<uint32_t>();
-    a.gen_odd = G->gen_odd.as<uint32_t>();
     a.roff = (const uint64_t *)(in + part[3].at);
     a.pid = (const uint16_t *)(in + part[2].at);
-    a.n_reads = (uint32_t)n_reads;
-    a.cv = (uint32_t)chunk_value;
     a.list_base = (const uint32_t *)(in + part[1].at);
-    srm_filter **outs[2] = {out_fwd, out_rev};
+    c = Call{};
+    c.n_lists = nl;
+    c.list_stride = nl + 1;
+    for (const Params &p : plan.params) c.kmax = std::max(c.kmax, p.k);
     // both strands in each launch, while their lists fit one sum
     if (strands == 3 && nl < ((uint64_t)1 << 30) - 1) {
         c.n = 2;
         c.s[0].f = c.s[1].f = a;
         c.s[1].f.dr = 4;
-        srm_filter *F[2] = {nullptr, nullptr};
-        const int rc = run_strands(G, c, blocked, read_len, read_k, F);
-        *out_fwd = F[0];
-        *out_rev = F[1];
-        return rc;
+        return both(c, false);
     }
     for (int x = 0; x < 2; ++x) {
         if (!(strands & (1 << x))) continue;
         c.n = 1;
         c.s[0].f = a;
         c.s[0].f.dr = x ? 4 : 0;
-        FL_RC(run_strands(G, c, blocked, read_len, read_k, outs[x]));
+        FL_RC(run_strands(G, c, false, blocked, read_len, read_k, outs[x]));
     }
     return SRM_OK;
 }
@@ -1282,7 +1443,10 @@ int run_call(srm_dfilter *G, const uint8_t *blocked, const char *reads, const ui
     } catch (const std::bad_alloc &) {
         rc = srm::set_error(SRM_ENOMEM, "no memory on the host for %zu reads", n_reads);
     }
-    if (rc != SRM_OK) (void)hipStreamSynchronize(G->st);
+    if (rc != SRM_OK) {
+        (void)hipStreamSynchronize(G->copy_st);
+        (void)hipStreamSynchronize(G->st);
+    }
     return rc;
 }
 
@@ -1309,9 +1473,13 @@ int srm_dfilter_create(srm_ctx *ctx, const srm_index *ix, const char *genome, si
         return rc;
     };
     if (hipSetDevice(G->device) != hipSuccess ||
-        hipEventCreate(&G->ev[0]) != hipSuccess || hipEventCreate(&G->ev[1]) != hipSuccess)
+        hipEventCreate(&G->ev[0]) != hipSuccess || hipEventCreate(&G->ev[1]) != hipSuccess ||
+        hipEventCreateWithFlags(&G->piece_ev[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&G->piece_ev[1], hipEventDisableTiming) != hipSuccess ||
+        hipStreamCreateWithFlags(&G->copy_st, hipStreamNonBlocking) != hipSuccess)
         return fail(srm::set_error(SRM_EDEVICE, "event creation failed"));
     if (hipHostMalloc(&G->stage_in, STAGE_IN, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(&G->stage_plan, 2 * PIECE_BYTES, hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc(&G->stage_out, 2 * sizeof(Header) + STAGE_OUT, hipHostMallocDefault) != hipSuccess)
         return fail(srm::set_error(SRM_ENOMEM, "no page-locked memory for the filter's staging"));
     int rc = G->upload(G->genome, genome, glen);
@@ -1414,6 +1582,7 @@ void srm_dfilter_destroy(srm_dfilter *G)
 {
     if (!G) return;
     (void)hipSetDevice(G->device);
+    (void)hipStreamSynchronize(G->copy_st);
     (void)hipStreamSynchronize(G->st);
     delete G;
 }

@@ -276,48 +276,78 @@ struct ReadPlan {
     uint64_t read_bytes = 0;            // extent of the reads buffer used
 };
 
+// a call's plan, made piece by piece
+struct Planner {
+    const srm_index *ix;
+    std::vector<int32_t> slot;   // parameter set of each (length, k), filled on first use
+    std::vector<Params> params;
+    std::vector<uint32_t> lists; // their numbers of lists
+    uint64_t n_lists = 0;        // of the reads so far
+    uint64_t read_bytes = 0;
+
+    explicit Planner(const srm_index *ix_) : ix(ix_) {}
+
+    // the parameter set of (L, k), < 0: an SRM_E* code with a message in err
+    int32_t set_of(int L, int k, std::string &err)
+    {
+        const size_t at = (size_t)L * 256 + (size_t)k;
+        if (at >= slot.size()) slot.resize(((size_t)L + 1) * 256, -1);
+        if (slot[at] >= 0) return slot[at];
+        if (L < 1) {
+            err = "a read has length 0";
+            return SRM_EINVAL;
+        }
+        params.push_back(derive(L, k));
+        if (!ix->get(params.back().q)) {
+            err = "the index lacks q = " + std::to_string(params.back().q);
+            return SRM_EINVAL;
+        }
+        if (params.size() > 65535) {
+            err = "too many (length, k) classes";
+            return SRM_EINVAL;
+        }
+        lists.push_back((uint32_t)params.back().n);
+        return slot[at] = (int32_t)params.size() - 1;
+    }
+
+    // reads [lo, hi): pid[0..] and list_base[0 .. hi - lo] (the last: the total so far).
+    // SRM_OK or an SRM_E* code with a message in err
+    int piece(const uint64_t *read_off, const uint16_t *read_len, const uint8_t *read_k, size_t lo,
+              size_t hi, uint16_t *pid, uint32_t *list_base, std::string &err)
+    {
+        uint64_t nl = n_lists, bytes = read_bytes;
+        for (size_t i = lo; i < hi; ++i) {
+            const int L = read_len[i], k = read_k[i];
+            const size_t at = (size_t)L * 256 + (size_t)k;
+            int32_t id = at < slot.size() ? slot[at] : -1;
+            if (id < 0 && (id = set_of(L, k, err)) < 0) return id;
+            pid[i - lo] = (uint16_t)id;
+            list_base[i - lo] = (uint32_t)nl;
+            nl += lists[(size_t)id];
+            bytes = std::max<uint64_t>(bytes, read_off[i] + (uint64_t)L);
+            if (nl >= ((uint64_t)1 << 31)) {
+                err = "too many q-gram lists in one call";
+                return SRM_EINVAL;
+            }
+        }
+        list_base[hi - lo] = (uint32_t)nl;
+        n_lists = nl;
+        read_bytes = bytes;
+        return SRM_OK;
+    }
+};
+
 // returns SRM_OK or an SRM_E* code with a message in err
 inline int plan_reads(const srm_index *ix, const uint64_t *read_off, const uint16_t *read_len,
                       const uint8_t *read_k, size_t n_reads, ReadPlan &P, std::string &err)
 {
-    // parameter set of each (length, k): a table over the lengths present and k
-    // 0..255, filled on first use
-    int maxlen = 0;
-    for (size_t i = 0; i < n_reads; ++i) maxlen = std::max(maxlen, (int)read_len[i]);
-    std::vector<int32_t> slot(((size_t)maxlen + 1) * 256, -1);
+    Planner plan(ix);
     P.pid.resize(n_reads);
     P.list_base.resize(n_reads + 1);
-    uint64_t nl = 0;
-    for (size_t i = 0; i < n_reads; ++i) {
-        const int L = read_len[i], k = read_k[i];
-        int32_t &id = slot[(size_t)L * 256 + (size_t)k];
-        if (id < 0) {
-            if (L < 1) {
-                err = "a read has length 0";
-                return SRM_EINVAL;
-            }
-            P.params.push_back(derive(L, k));
-            if (!ix->get(P.params.back().q)) {
-                err = "the index lacks q = " + std::to_string(P.params.back().q);
-                return SRM_EINVAL;
-            }
-            if (P.params.size() > 65535) {
-                err = "too many (length, k) classes";
-                return SRM_EINVAL;
-            }
-            id = (int32_t)P.params.size() - 1;
-        }
-        P.pid[i] = (uint16_t)id;
-        P.list_base[i] = (uint32_t)nl;
-        nl += (uint64_t)P.params[(size_t)id].n;
-        P.read_bytes = std::max<uint64_t>(P.read_bytes, read_off[i] + read_len[i]);
-        if (nl >= ((uint64_t)1 << 31)) {
-            err = "too many q-gram lists in one call";
-            return SRM_EINVAL;
-        }
-    }
-    P.list_base[n_reads] = (uint32_t)nl;
-    return SRM_OK;
+    const int rc = plan.piece(read_off, read_len, read_k, 0, n_reads, P.pid.data(), P.list_base.data(), err);
+    P.params = std::move(plan.params);
+    P.read_bytes = plan.read_bytes;
+    return rc;
 }
 
 // Per-read filter results held as meta words (3 per read: entry offset, perfect
