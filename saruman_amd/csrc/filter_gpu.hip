@@ -78,6 +78,55 @@ __global__ void __launch_bounds__(FB) fl_pack(const uint4 *__restrict__ src, uin
 }
 
 constexpr size_t OVER_ROOM = (size_t)1 << 19;   // entries
+// The reads' codes as the alignment kernels take them (16 per word, the first lowest, other
+// bytes 0), `pad` codes of zero before them, every read's reverse complement after them:
+// a thread per word.  The reads lie one after another from byte 0, `total` in all; off: n.
+//
+// HBM-bound and small beside the lookups (7 MB of reads: 12 us); on the host a request's
+// reverse complements and packing took 1 ms of 7 MB, 0.2 ms of 140 KB.
+__global__ void __launch_bounds__(FB) fl_read_words(const uint32_t *__restrict__ pk,
+                                                    const uint16_t *__restrict__ odd,
+                                                    const uint64_t *__restrict__ off, uint32_t n,
+                                                    uint64_t total, uint32_t pad, uint32_t *__restrict__ out,
+                                                    size_t n_words)
+{
+    const size_t w = (size_t)blockIdx.x * FB + threadIdx.x;
+    if (w >= n_words) return;
+    const int64_t p = (int64_t)(16 * w) - (int64_t)pad;   // the word's first code
+    uint32_t v = 0;
+    uint32_t r = 0;      // the read of the reverse complements' code at hand
+    uint64_t lo = 0, hi = 0;
+    for (int j = 0; j < 16; ++j) {
+        const int64_t c = p + j;
+        if (c < 0 || (uint64_t)c >= 2 * total) continue;
+        uint64_t at = (uint64_t)c;
+        const bool rev = at >= total;
+        if (rev) {
+            at -= total;
+            if (at >= hi) {
+                if (hi == 0) {   // the last read that starts at or before it
+                    uint32_t b = 0;
+                    for (uint32_t m = n; m > 1;) {
+                        const uint32_t h = m >> 1;
+                        if (off[b + h] <= at) b += h;
+                        m -= h;
+                    }
+                    r = b;
+                } else {
+                    ++r;         // (no read is empty)
+                }
+                lo = off[r];
+                hi = r + 1 < n ? off[r + 1] : total;
+            }
+            at = lo + hi - 1 - at;
+        }
+        const uint32_t code = (pk[at >> 4] >> (30 - 2 * (int)(at & 15))) & 3u;
+        if ((odd[at >> 4] >> (at & 15)) & 1u) continue;
+        v |= (rev ? 3u - code : code) << (2 * j);
+    }
+    out[w] = v;
+}
+
 constexpr uint32_t MAX_FLUSH = 256;      // flushes the device lists
 constexpr uint32_t MAX_UNSAFE = 1 << 16; // reads it lists for the host's walk
 constexpr uint32_t MAX_WALK = 1 << 16;   // words of their entries
@@ -787,7 +836,7 @@ struct srm_dfilter {
     size_t glen = 0;
     GBuf genome, gen_pk, gen_odd, dq;
     std::vector<GBuf> keys, pre, odd_hash, odd_pos;
-    GBuf in, read_pk, read_odd, blocked, list_cnt, list_lo, list_start, cub_tmp, cnt, start, by_rank,
+    GBuf in, read_pk, read_odd, words, blocked, list_cnt, list_lo, list_start, cub_tmp, cnt, start, by_rank,
         unsafe, walk, out;
     GBuf flat[2], out_pos[2], out_flag[2], out_perf[2], meta[2], over[2][2];
     GBuf slot_pos, slot_flag, slot_perf;
@@ -795,13 +844,13 @@ struct srm_dfilter {
     std::shared_ptr<BlockPool> pool = std::make_shared<BlockPool>();
     void *stage_plan = nullptr;                       // two pieces' plans, likewise
     hipStream_t copy_st = nullptr;                    // the pieces' copies
-    hipEvent_t ev[2] = {nullptr, nullptr}, piece_ev[2] = {nullptr, nullptr};
+    hipEvent_t ev[2] = {nullptr, nullptr}, piece_ev[2] = {nullptr, nullptr}, words_ev = nullptr;
     float last_ms = 0.f;
     size_t last_lists = 0, last_flat = 0, last_overflow = 0;
 
     ~srm_dfilter()
     {
-        for (GBuf *b : {&genome, &gen_pk, &gen_odd, &dq, &in, &read_pk, &read_odd, &blocked, &list_cnt,
+        for (GBuf *b : {&genome, &gen_pk, &gen_odd, &dq, &in, &read_pk, &read_odd, &words, &blocked, &list_cnt,
                         &list_lo, &list_start, &cub_tmp, &cnt, &start, &by_rank, &unsafe, &walk, &out,
                         &slot_pos, &slot_flag, &slot_perf})
             b->release();
@@ -819,6 +868,7 @@ struct srm_dfilter {
             if (e) (void)hipEventDestroy(e);
         for (auto &e : piece_ev)
             if (e) (void)hipEventDestroy(e);
+        if (words_ev) (void)hipEventDestroy(words_ev);
     }
 
     int upload(GBuf &b, const void *src, size_t bytes)
@@ -1321,12 +1371,28 @@ int upload_pieces(srm_dfilter *G, Call &c, const char *reads, const uint64_t *re
     return SRM_OK;
 }
 
+// the codes of the call's reads to words (srm::dfilter_run2_words), copied beside the
+// kernels that follow
+int send_words(srm_dfilter *G, const FArgs &a, uint64_t total, uint32_t *words)
+{
+    const size_t n_words = (2 * total + 2 * SRM_CODE_PAD + 15) / 16 + 1;
+    FL_RC(G->words.ensure(n_words * 4));
+    hipLaunchKernelGGL(fl_read_words, dim3((unsigned)((n_words + FB - 1) / FB)), dim3(FB), 0, G->st,
+                       a.read_pk, (const uint16_t *)a.read_odd, a.roff, a.n_reads, total,
+                       (uint32_t)SRM_CODE_PAD, G->words.as<uint32_t>(), n_words);
+    FL_TRY(hipGetLastError());
+    FL_TRY(hipEventRecord(G->words_ev, G->st));
+    FL_TRY(hipStreamWaitEvent(G->copy_st, G->words_ev, 0));
+    FL_TRY(hipMemcpyAsync(words, G->words.p, n_words * 4, hipMemcpyDeviceToHost, G->copy_st));
+    return SRM_OK;
+}
+
 // one or both strands (strands: bit 0 forward, bit 1 reverse) over one upload of
 // the reads
 int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
                const uint64_t *read_off, const uint16_t *read_len, const uint8_t *read_k,
-               size_t n_reads, int strands, int chunk_value, srm_filter **out_fwd,
-               srm_filter **out_rev)
+               size_t n_reads, int strands, int chunk_value, uint32_t *words,
+               srm_filter **out_fwd, srm_filter **out_rev)
 {
     G->last_flat = 0;
     G->last_overflow = 0;
@@ -1358,6 +1424,7 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
         FL_RC(upload_pieces(G, c, reads, read_off, read_len, read_k, n_reads, counted));
         if (counted) {
             G->last_lists = c.n_lists * (uint64_t)c.n;
+            if (words) FL_RC(send_words(G, c.s[0].f, read_off[n_reads - 1] + read_len[n_reads - 1], words));
             return both(c, true);
         }
         FL_TRY(hipStreamSynchronize(G->copy_st));
@@ -1409,6 +1476,7 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     a.roff = (const uint64_t *)(in + part[3].at);
     a.pid = (const uint16_t *)(in + part[2].at);
     a.list_base = (const uint32_t *)(in + part[1].at);
+    if (words) FL_RC(send_words(G, a, rbytes, words));
     c = Call{};
     c.n_lists = nl;
     c.list_stride = nl + 1;
@@ -1434,12 +1502,14 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
 // still being copied when it returns
 int run_call(srm_dfilter *G, const uint8_t *blocked, const char *reads, const uint64_t *read_off,
              const uint16_t *read_len, const uint8_t *read_k, size_t n_reads, int strands,
-             int chunk_value, srm_filter **out_fwd, srm_filter **out_rev)
+             int chunk_value, uint32_t *words, srm_filter **out_fwd, srm_filter **out_rev)
 {
     int rc;
     try {
         rc = run_device(G, blocked, reads, read_off, read_len, read_k, n_reads, strands, chunk_value,
-                        out_fwd, out_rev);
+                        words, out_fwd, out_rev);
+        if (rc == SRM_OK && words && hipStreamSynchronize(G->copy_st) != hipSuccess)
+            rc = srm::set_error(SRM_EDEVICE, "the copy of the reads' codes failed");
     } catch (const std::bad_alloc &) {
         rc = srm::set_error(SRM_ENOMEM, "no memory on the host for %zu reads", n_reads);
     }
@@ -1451,6 +1521,36 @@ int run_call(srm_dfilter *G, const uint8_t *blocked, const char *reads, const ui
 }
 
 }  // namespace
+
+namespace srm {
+
+int dfilter_run2_words(srm_dfilter *G, const uint8_t *blocked, const char *reads,
+                       const uint64_t *read_off, const uint16_t *read_len, const uint8_t *read_k,
+                       size_t n_reads, int chunk_value, uint32_t *words, srm_filter **out_fwd,
+                       srm_filter **out_rev)
+{
+    *out_fwd = nullptr;
+    *out_rev = nullptr;
+    if (!G || chunk_value < 1) return srm::set_error(SRM_EINVAL, "bad filter arguments");
+    if (n_reads == 0) {
+        *out_fwd = new srm_filter();
+        *out_rev = new srm_filter();
+        return SRM_OK;
+    }
+    srm_filter *Ff = nullptr, *Fr = nullptr;
+    const int rc = run_call(G, blocked, reads, read_off, read_len, read_k, n_reads, 3, chunk_value,
+                            words, &Ff, &Fr);
+    if (rc != SRM_OK) {
+        delete Ff;
+        delete Fr;
+        return rc;
+    }
+    *out_fwd = Ff;
+    *out_rev = Fr;
+    return SRM_OK;
+}
+
+}  // namespace srm
 
 extern "C" {
 
@@ -1476,6 +1576,7 @@ int srm_dfilter_create(srm_ctx *ctx, const srm_index *ix, const char *genome, si
         hipEventCreate(&G->ev[0]) != hipSuccess || hipEventCreate(&G->ev[1]) != hipSuccess ||
         hipEventCreateWithFlags(&G->piece_ev[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&G->piece_ev[1], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&G->words_ev, hipEventDisableTiming) != hipSuccess ||
         hipStreamCreateWithFlags(&G->copy_st, hipStreamNonBlocking) != hipSuccess)
         return fail(srm::set_error(SRM_EDEVICE, "event creation failed"));
     if (hipHostMalloc(&G->stage_in, STAGE_IN, hipHostMallocDefault) != hipSuccess ||
@@ -1534,7 +1635,7 @@ int srm_dfilter_run(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     }
     srm_filter *F = nullptr;
     const int rc = run_call(G, blocked, reads, read_off, read_len, read_k, n_reads,
-                            do_reverse ? 2 : 1, chunk_value, &F, &F);
+                            do_reverse ? 2 : 1, chunk_value, nullptr, &F, &F);
     if (rc != SRM_OK) {
         delete F;
         return rc;
@@ -1547,25 +1648,8 @@ int srm_dfilter_run2(srm_dfilter *G, const uint8_t *blocked, const char *reads,
                      const uint64_t *read_off, const uint16_t *read_len, const uint8_t *read_k,
                      size_t n_reads, int chunk_value, srm_filter **out_fwd, srm_filter **out_rev)
 {
-    *out_fwd = nullptr;
-    *out_rev = nullptr;
-    if (!G || chunk_value < 1) return srm::set_error(SRM_EINVAL, "bad filter arguments");
-    if (n_reads == 0) {
-        *out_fwd = new srm_filter();
-        *out_rev = new srm_filter();
-        return SRM_OK;
-    }
-    srm_filter *Ff = nullptr, *Fr = nullptr;
-    const int rc = run_call(G, blocked, reads, read_off, read_len, read_k, n_reads, 3, chunk_value,
-                            &Ff, &Fr);
-    if (rc != SRM_OK) {
-        delete Ff;
-        delete Fr;
-        return rc;
-    }
-    *out_fwd = Ff;
-    *out_rev = Fr;
-    return SRM_OK;
+    return srm::dfilter_run2_words(G, blocked, reads, read_off, read_len, read_k, n_reads, chunk_value,
+                                   nullptr, out_fwd, out_rev);
 }
 
 int srm_dfilter_stats(const srm_dfilter *G, float *device_ms, uint64_t *n_lists,

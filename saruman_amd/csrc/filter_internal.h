@@ -375,3 +375,17 @@ struct MetaAcc {
 };
 
 }  // namespace srm_filter_impl
+
+struct srm_dfilter;
+
+namespace srm {
+// srm_dfilter_run2 that also leaves the reads' codes in words, as srm_pack_codes gives
+// them: SRM_CODE_PAD codes of zero, the reads, their reverse complements (a byte other
+// than ACGT is its own complement and has code 0), and zeros to the last of
+// (2 * total + 2 * SRM_CODE_PAD + 15) / 16 + 1 words.  The reads are not empty and lie one
+// after another from byte 0.  words may be null.
+int dfilter_run2_words(srm_dfilter *G, const uint8_t *blocked, const char *reads,
+                       const uint64_t *read_off, const uint16_t *read_len, const uint8_t *read_k,
+                       size_t n_reads, int chunk_value, uint32_t *words, srm_filter **out_fwd,
+                       srm_filter **out_rev);
+}  // namespace srm

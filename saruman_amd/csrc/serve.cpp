@@ -29,6 +29,7 @@
 #include <thread>
 #include <vector>
 
+#include "filter_internal.h"
 #include "saruman_hip.h"
 
 namespace {
@@ -99,27 +100,88 @@ void pack_codes_par(const char *seq, size_t n, uint32_t *words, size_t code_off)
     });
 }
 
+// Page-locked host memory for the requests' reads, codes and text: copies to and from the
+// device at full rate and on their own, and pages that are there already (a request of
+// 50,000 reads touches 30 MB).  At most MAX_BYTES of it, kept until the server goes;
+// ordinary memory beyond.
+class HostPool : public std::enable_shared_from_this<HostPool> {
+public:
+    ~HostPool()
+    {
+        for (auto &b : free_) srm_host_free(b.second);
+    }
+    std::shared_ptr<char> take(size_t bytes)
+    {
+        const size_t want = (bytes + bytes / 4 + ROUND) / ROUND * ROUND;
+        size_t cap = 0;
+        char *p = nullptr;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            auto it = free_.lower_bound(bytes);
+            if (it != free_.end() && it->first <= 4 * want) {
+                cap = it->first;
+                p = it->second;
+                free_.erase(it);
+            } else {
+                // room by giving free blocks back, the smallest first
+                while (total_ + want > MAX_BYTES && !free_.empty()) {
+                    total_ -= free_.begin()->first;
+                    srm_host_free(free_.begin()->second);
+                    free_.erase(free_.begin());
+                }
+                if (total_ + want <= MAX_BYTES) {
+                    total_ += want;
+                    cap = want;
+                }
+            }
+        }
+        if (cap && !p && !(p = (char *)srm_host_alloc(cap))) {
+            std::lock_guard<std::mutex> lk(mu_);
+            total_ -= cap;
+        }
+        if (!p) return std::shared_ptr<char>(new char[std::max<size_t>(bytes, 1)], std::default_delete<char[]>());
+        auto self = shared_from_this();
+        return std::shared_ptr<char>(p, [self, cap](char *q) {
+            std::lock_guard<std::mutex> lk(self->mu_);
+            self->free_.emplace(cap, q);
+        });
+    }
+
+private:
+    static constexpr size_t MAX_BYTES = (size_t)512 << 20, ROUND = (size_t)256 << 10;
+    std::mutex mu_;
+    std::multimap<size_t, char *> free_;
+    size_t total_ = 0;
+};
+
 struct Request {
     uint64_t id = 0;
     size_t max_len = 0;   // longest read
-    std::string reads;
+    std::shared_ptr<char> reads;
+    size_t total = 0;     // their bytes
     std::vector<uint64_t> off;
     std::vector<uint16_t> len;
     std::vector<uint8_t> k;
     // after the filter
-    std::string reads_rev;
+    std::string reads_rev;             // where the host packs or formats
     std::vector<srm_cand> cand;
     std::vector<int64_t> pos;
     std::vector<int32_t> rid;
-    std::vector<uint64_t> roff_bytes;
-    std::vector<uint32_t> read_words;
+    std::vector<uint64_t> roff_bytes;  // where the host formats
+    std::shared_ptr<char> read_words;
+    size_t n_words = 0;
     std::vector<int32_t> perf_read[2];
     std::vector<int64_t> perf_pos[2];
     size_t ops_total = 0;
     size_t dev_bytes = 0;
     // results
-    std::string records;              // perfect hits, then (host formatting) aligned hits
-    std::unique_ptr<char[]> rec_text; // aligned hits formatted on the device (after records)
+    struct Text {
+        std::shared_ptr<char> mem;
+        size_t n;
+    };
+    std::vector<Text> perfect;        // perfect hits' records in order
+    std::string records;              // aligned hits formatted on the host (after perfect)
+    std::shared_ptr<char> rec_text;   // aligned hits formatted on the device (likewise)
     size_t rec_len = 0;
     srm_request_stats st{};
     bool done = false;
@@ -142,8 +204,7 @@ struct srm_server {
     srm_dfilter *dfilter = nullptr;   // set when the filter runs on the device
     std::vector<srm_ctx *> ctx;       // one per slot; slot 0 owns the resident genome
     std::vector<srm_job *> job;
-    std::vector<char *> stage;        // per slot: page-locked buffer for the record text
-    std::vector<size_t> stage_cap;
+    std::shared_ptr<HostPool> pool = std::make_shared<HostPool>();
     Clock::time_point t0;
 
     std::mutex mu;
@@ -184,25 +245,110 @@ struct srm_server {
     void run_on_slot(int s, Request &r);
 };
 
+namespace {
+
+// room for a perfect hit's record: three numbers, strand, separators and two rows
+size_t perfect_room(const Request &r, int32_t i) { return 2 * (size_t)r.len[(size_t)i] + 48; }
+
+size_t perfect_bound(const Request &r)
+{
+    size_t bytes = 0;
+    for (const auto &hits : r.perf_read)
+        for (int32_t i : hits) bytes += perfect_room(r, i);
+    return bytes;
+}
+
+// perfect hits: "r<id>\t<start>\t<stop>\t<strand>\t<genome>\t<read>\t0\n", as the
+// reference prints them (%d fields), written directly; the hits of both strands in order,
+// split over threads that each write their own part
+void perfect_records(Request &r, HostPool &pool, const std::string &genome)
+{
+    const size_t n0 = r.perf_read[0].size(), np = n0 + r.perf_read[1].size();
+    const unsigned T = host_threads(perfect_bound(r));
+    r.perfect.assign(T, Request::Text{nullptr, 0});
+    par_ranges(T, np, [&](unsigned u, size_t lo, size_t hi) {
+        size_t room = 0;
+        for (size_t x = lo; x < hi; ++x) {
+            const int sd = x < n0 ? 0 : 1;
+            room += perfect_room(r, r.perf_read[sd][sd ? x - n0 : x]);
+        }
+        const auto mem = pool.take(room);
+        char *o = mem.get();
+        auto put_int = [&](long long v) {
+            char d[24];
+            int q = 0;
+            const bool neg = v < 0;
+            unsigned long long w = neg ? 0ull - (unsigned long long)v : (unsigned long long)v;
+            do {
+                d[q++] = (char)('0' + w % 10);
+                w /= 10;
+            } while (w);
+            if (neg) *o++ = '-';
+            while (q) *o++ = d[--q];
+        };
+        auto put = [&](const char *p, size_t n) {
+            std::memcpy(o, p, n);
+            o += n;
+        };
+        for (size_t x = lo; x < hi; ++x) {
+            const int sd = x < n0 ? 0 : 1;
+            const size_t p = sd ? x - n0 : x;
+            const int32_t i = r.perf_read[sd][p];
+            const int64_t S = r.perf_pos[sd][p];
+            const int L = r.len[(size_t)i];
+            const char *rd = r.reads.get() + r.off[(size_t)i];
+            *o++ = 'r';
+            put_int(i);
+            *o++ = '\t';
+            put_int((int)S);
+            *o++ = '\t';
+            put_int((int)(S + L - 1));
+            put(sd ? "\t<<\t" : "\t>>\t", 4);
+            put(genome.data() + S, strnlen(genome.data() + S, (size_t)L));   // %.*s
+            *o++ = '\t';
+            if (sd) {
+                char *row = o;
+                for (int j = 0; j < L; ++j) *o++ = comp(rd[L - 1 - j]);
+                o = row + strnlen(row, (size_t)L);
+            } else {
+                put(rd, strnlen(rd, (size_t)L));
+            }
+            put("\t0\n", 3);
+        }
+        r.perfect[u] = Request::Text{mem, (size_t)(o - mem.get())};
+    });
+}
+
+}  // namespace
+
 void srm_server::prepare(Request &r)
 {
     const size_t n = r.len.size();
-    const size_t total = r.reads.size();
-    r.reads_rev.resize(total);
-    // reverse complements, reads split over the threads
-    par_ranges(host_threads(total), n, [&](unsigned, size_t lo, size_t hi) {
-        for (size_t i = lo; i < hi; ++i) {
-            const char *src = r.reads.data() + r.off[i];
-            char *dst = &r.reads_rev[r.off[i]];
-            for (int j = 0; j < r.len[i]; ++j) dst[j] = comp(src[r.len[i] - 1 - j]);
-        }
-    });
+    const size_t total = r.total;
+    // read codes (forward reads, then their reverse complements): the device filter leaves
+    // them; else from the reverse complements, which the host's formatting needs too
+    r.n_words = (2 * total + 2 * SRM_CODE_PAD + 15) / 16 + 1;
+    r.read_words = pool->take(r.n_words * 4);
+    auto *words = (uint32_t *)r.read_words.get();
+    const bool device_words = dfilter && n > 0;
+    if (!device_words || !cfg.gpu_records) {
+        r.reads_rev.resize(total);
+        // reads split over the threads
+        par_ranges(host_threads(total), n, [&](unsigned, size_t lo, size_t hi) {
+            for (size_t i = lo; i < hi; ++i) {
+                const char *src = r.reads.get() + r.off[i];
+                char *dst = &r.reads_rev[r.off[i]];
+                for (int j = 0; j < r.len[i]; ++j) dst[j] = comp(src[r.len[i] - 1 - j]);
+            }
+        });
+    }
     // both strands through the reference filter semantics (the device filter runs
     // both over one upload of the reads)
     srm_filter *both[2] = {nullptr, nullptr};
     if (dfilter) {
-        int rc = srm_dfilter_run2(dfilter, nullptr, r.reads.data(), r.off.data(), r.len.data(),
-                                  r.k.data(), n, cfg.chunk_value, &both[0], &both[1]);
+        int rc = srm::dfilter_run2_words(dfilter, nullptr, r.reads.get(), r.off.data(), r.len.data(),
+                                         r.k.data(), n, cfg.chunk_value, device_words ? words : nullptr,
+                                         &both[0], &both[1]);
         if (rc != SRM_OK) {
             set_failed(r.st, rc, srm_last_error());
             return;
@@ -211,7 +357,7 @@ void srm_server::prepare(Request &r)
     for (int s = 0; s < 2; ++s) {
         srm_filter *F = both[s];
         if (!F) {
-            int rc = srm_filter_run(index, genome.data(), genome.size(), nullptr, r.reads.data(),
+            int rc = srm_filter_run(index, genome.data(), genome.size(), nullptr, r.reads.get(),
                                     r.off.data(), r.len.data(), r.k.data(), n, s ? 4 : 0,
                                     cfg.chunk_value, cfg.filter_threads, &F);
             if (rc != SRM_OK) {
@@ -222,20 +368,23 @@ void srm_server::prepare(Request &r)
         }
         uint64_t nc, nb, np;
         srm_filter_sizes(F, &nc, &nb, &np);
-        std::vector<int32_t> cr(nc);
-        std::vector<int64_t> cp(nc);
+        const size_t at = r.cand.size();
         std::vector<uint8_t> cf(nc);
         std::vector<uint16_t> cw(nc);
+        r.cand.resize(at + nc);
+        r.pos.resize(at + nc);
+        r.rid.resize(at + nc);
+        if (!cfg.gpu_records) r.roff_bytes.resize(at + nc);
         r.perf_read[s].resize(np);
         r.perf_pos[s].resize(np);
-        srm_filter_copy(F, cr.data(), cp.data(), cf.data(), cw.data(), nullptr,
+        srm_filter_copy(F, r.rid.data() + at, r.pos.data() + at, cf.data(), cw.data(), nullptr,
                         r.perf_read[s].data(), r.perf_pos[s].data());
         srm_filter_destroy(F);
         for (size_t t = 0; t < nc; ++t) {
-            const int32_t i = cr[t];
-            srm_cand c;
+            const int32_t i = r.rid[at + t];
+            srm_cand &c = r.cand[at + t];
             c.read_off = (uint32_t)(r.off[(size_t)i] + (cf[t] > 3 ? total : 0));
-            c.win_off = (uint32_t)(cp[t] + SRM_CODE_PAD);
+            c.win_off = (uint32_t)(r.pos[at + t] + SRM_CODE_PAD);
             c.ops_off = (uint32_t)r.ops_total;
             c.L = r.len[(size_t)i];
             c.w = cw[t];
@@ -244,23 +393,21 @@ void srm_server::prepare(Request &r)
             c.bits = 0;
             c.pad = 0;
             r.ops_total += srm_ops_words(c.w, c.k);
-            r.cand.push_back(c);
-            r.pos.push_back(cp[t]);
-            r.rid.push_back(i);
-            r.roff_bytes.push_back(r.off[(size_t)i]);
+            if (!cfg.gpu_records) r.roff_bytes[at + t] = r.off[(size_t)i];
         }
     }
-    // read codes: forward reads, then their reverse complements
-    r.read_words.assign((2 * total + 2 * SRM_CODE_PAD + 15) / 16 + 1, 0u);
-    pack_codes_par(r.reads.data(), total, r.read_words.data(), SRM_CODE_PAD);
-    pack_codes_par(r.reads_rev.data(), total, r.read_words.data(), SRM_CODE_PAD + total);
+    if (!device_words) {
+        std::fill(words, words + r.n_words, 0u);
+        pack_codes_par(r.reads.get(), total, words, SRM_CODE_PAD);
+        pack_codes_par(r.reads_rev.data(), total, words, SRM_CODE_PAD + total);
+    }
     size_t maxL = 0;
     for (auto L : r.len) maxL = std::max<size_t>(maxL, L);
     r.max_len = maxL;
     const size_t nc = r.cand.size();
     // device footprint: the library's bound for this job, record stage included
     // when the records are formatted on the device (names "r" + decimal id)
-    r.dev_bytes = srm_job_bytes_bound(nullptr, 0, 1, r.cand.data(), (int)nc, r.read_words.size(), 0,
+    r.dev_bytes = srm_job_bytes_bound(nullptr, 0, 1, r.cand.data(), (int)nc, r.n_words, 0,
                                       0, 0, cfg.kernel, cfg.gpu_records, 2, 1 + 11);
     r.st.n_reads = (long long)n;
     r.st.n_candidates = (long long)nc;
@@ -272,16 +419,34 @@ void srm_server::run_on_slot(int s, Request &r)
     srm_job *j = job[(size_t)s];
     const int n = (int)r.cand.size();
     int rc = SRM_OK;
-    std::vector<srm_result> res((size_t)n);
+    // the perfect hits' records beside the device's work, where they are many
+    std::thread beside;
+    const size_t perfect_bytes = perfect_bound(r);
+    if (n > 0 && perfect_bytes >= ((size_t)1 << 18)) {
+        try {
+            beside = std::thread([&] { perfect_records(r, *pool, genome); });
+        } catch (...) {   // no thread to be had: below, on this one
+        }
+    }
+    struct Join {
+        std::thread &t;
+        ~Join()
+        {
+            if (t.joinable()) t.join();
+        }
+    } join{beside};
+    const bool apart = beside.joinable();
+    const auto res_mem = pool->take(sizeof(srm_result) * (size_t)n);
+    auto *res = (srm_result *)res_mem.get();
     // transcripts come to the host only when the host formats the records
     std::vector<uint32_t> ops(cfg.gpu_records ? 0 : r.ops_total + 1);
     if (n > 0) {
-        rc = srm_job_upload(j, 0, 1, r.cand.data(), n, r.read_words.data(), r.read_words.size(),
+        rc = srm_job_upload(j, 0, 1, r.cand.data(), n, (const uint32_t *)r.read_words.get(), r.n_words,
                             nullptr, 0, nullptr, 0, nullptr, 0);
         if (rc == SRM_OK) rc = srm_job_run(j, cfg.kernel);
         if (rc == SRM_OK) r.st.device_ms = srm_job_last_ms(j);
         if (rc == SRM_OK)   // the transcripts stay on the device when it formats the records
-            rc = srm_job_download(j, res.data(), cfg.gpu_records ? nullptr : ops.data(),
+            rc = srm_job_download(j, res, cfg.gpu_records ? nullptr : ops.data(),
                                   cfg.gpu_records ? 0 : ops.size());
     }
     r.st.t_aligned = now();
@@ -291,99 +456,21 @@ void srm_server::run_on_slot(int s, Request &r)
     }
     // records: perfect hits (hash.c:580) of each strand, then aligned hits in
     // candidate order
+    if (!apart) perfect_records(r, *pool, genome);
     std::string out;
     std::vector<char> mapped(r.len.size(), 0);
-    {
-        // perfect hits: "r<id>\t<start>\t<stop>\t<strand>\t<genome>\t<read>\t0\n", as
-        // the reference prints them (%d fields), written directly; the hits of both
-        // strands in order, split over threads that each write their own part
-        const size_t n0 = r.perf_read[0].size(), np = n0 + r.perf_read[1].size();
-        size_t bytes = 0;
-        for (int sd = 0; sd < 2; ++sd)
-            for (int32_t i : r.perf_read[sd]) bytes += 2 * (size_t)r.len[(size_t)i] + 48;
-        const unsigned T = host_threads(bytes);
-        std::vector<std::string> part(T);
-        par_ranges(T, np, [&](unsigned u, size_t lo, size_t hi) {
-            std::string &o = part[u];
-            size_t b = 0;
-            for (size_t x = lo; x < hi; ++x) {
-                const int sd = x < n0 ? 0 : 1;
-                b += 2 * (size_t)r.len[(size_t)r.perf_read[sd][sd ? x - n0 : x]] + 48;
-            }
-            o.reserve(b);
-            auto put_int = [&](long long v) {
-                char d[24];
-                int q = 0;
-                const bool neg = v < 0;
-                unsigned long long w = neg ? 0ull - (unsigned long long)v : (unsigned long long)v;
-                do {
-                    d[q++] = (char)('0' + w % 10);
-                    w /= 10;
-                } while (w);
-                if (neg) o.push_back('-');
-                while (q) o.push_back(d[--q]);
-            };
-            for (size_t x = lo; x < hi; ++x) {
-                const int sd = x < n0 ? 0 : 1;
-                const size_t p = sd ? x - n0 : x;
-                const int32_t i = r.perf_read[sd][p];
-                const int64_t S = r.perf_pos[sd][p];
-                const int L = r.len[(size_t)i];
-                const char *rd = (sd ? r.reads_rev.data() : r.reads.data()) + r.off[(size_t)i];
-                o.push_back('r');
-                put_int(i);
-                o.push_back('\t');
-                put_int((int)S);
-                o.push_back('\t');
-                put_int((int)(S + L - 1));
-                o.append(sd ? "\t<<\t" : "\t>>\t");
-                o.append(genome.data() + S, strnlen(genome.data() + S, (size_t)L));   // %.*s
-                o.push_back('\t');
-                o.append(rd, strnlen(rd, (size_t)L));
-                o.append("\t0\n");
-            }
-        });
-        size_t tot = 0;
-        for (auto &x : part) tot += x.size();
-        out.reserve(tot);
-        for (auto &x : part) out.append(x);
-        for (int sd = 0; sd < 2; ++sd)
-            for (int32_t i : r.perf_read[sd]) mapped[(size_t)i] = 1;
-    }
+    for (int sd = 0; sd < 2; ++sd)
+        for (int32_t i : r.perf_read[sd]) mapped[(size_t)i] = 1;
     r.st.n_perfect = (long long)(r.perf_read[0].size() + r.perf_read[1].size());
     if (n > 0 && cfg.gpu_records) {
-        // the text's exact size first, then the text into a buffer of that size
-        // (no zero-filled allocation of an estimate)
+        // into a buffer with room for all lines: a name of 12 bytes at most, two rows of
+        // at most the transcript's slot, three numbers, strand and separators
         long long hits = 0;
+        const size_t cap = 32 * r.ops_total + (size_t)n * 64 + 256;
+        r.rec_text = pool->take(cap);
         long long total = srm_job_records(j, r.pos.data(), r.rid.data(), nullptr, 0, 0, "r",
-                                          nullptr, 0, &hits);
-        if (total > 0) {
-            // the text comes back into the slot's page-locked buffer (a fast copy),
-            // then goes to the request's own buffer on several threads
-            const size_t want = (size_t)total;
-            if (stage_cap[(size_t)s] < want) {
-                srm_host_free(stage[(size_t)s]);
-                const size_t cap = want + want / 4 + 4096;
-                stage[(size_t)s] = (char *)srm_host_alloc(cap);
-                stage_cap[(size_t)s] = stage[(size_t)s] ? cap : 0;
-            }
-            char *dst = stage[(size_t)s];
-            std::unique_ptr<char[]> direct;
-            if (!dst) {   // no page-locked memory: straight into the request's buffer
-                direct.reset(new char[want]);
-                dst = direct.get();
-            }
-            total = srm_job_records(j, r.pos.data(), r.rid.data(), nullptr, 0, 0, "r", dst, want,
-                                    &hits);
-            if (total > 0 && direct) {
-                r.rec_text = std::move(direct);
-            } else if (total > 0) {
-                r.rec_text.reset(new char[(size_t)total]);
-                char *to = r.rec_text.get();
-                par_ranges(host_threads((size_t)total), (size_t)total,
-                           [&](unsigned, size_t lo, size_t hi) { std::memcpy(to + lo, dst + lo, hi - lo); });
-            }
-        }
+                                          r.rec_text.get(), cap, &hits);
+        if (total > (long long)cap) total = SRM_EDEVICE;   // (it cannot be)
         if (total < 0) {
             set_failed(r.st, (int)total, srm_last_error());
             return;
@@ -394,8 +481,8 @@ void srm_server::run_on_slot(int s, Request &r)
             if (res[(size_t)t].score <= (int)r.cand[(size_t)t].k) mapped[(size_t)r.rid[(size_t)t]] = 1;
     } else if (n > 0) {
         long long hits = 0;
-        long long need = srm_format_records(n, res.data(), ops.data(), r.cand.data(), genome.data(),
-                                            r.pos.data(), r.reads.data(), r.reads_rev.data(),
+        long long need = srm_format_records(n, res, ops.data(), r.cand.data(), genome.data(),
+                                            r.pos.data(), r.reads.get(), r.reads_rev.data(),
                                             r.roff_bytes.data(), r.rid.data(), "r", nullptr, 0,
                                             &hits, cfg.format_threads);
         if (need < 0) {
@@ -404,8 +491,8 @@ void srm_server::run_on_slot(int s, Request &r)
         }
         size_t base = out.size();
         out.resize(base + (size_t)need);
-        srm_format_records(n, res.data(), ops.data(), r.cand.data(), genome.data(), r.pos.data(),
-                           r.reads.data(), r.reads_rev.data(), r.roff_bytes.data(), r.rid.data(),
+        srm_format_records(n, res, ops.data(), r.cand.data(), genome.data(), r.pos.data(),
+                           r.reads.get(), r.reads_rev.data(), r.roff_bytes.data(), r.rid.data(),
                            "r", &out[base], (size_t)need, &hits, cfg.format_threads);
         r.st.n_hits = hits;
         for (int t = 0; t < n; ++t)
@@ -526,6 +613,7 @@ void srm_server::slot_loop(int s)
             r = slot_req[(size_t)s];
         }
         run_on_slot(s, *r);
+        if (r->st.status != SRM_OK) r->perfect.clear();   // a failed request has no records
         // an idle slot keeps its buffers for the next request, up to `retain`
         if (srm_ctx_pool_used(ctx[(size_t)s]) > base[(size_t)s] + retain) srm_job_release(job[(size_t)s]);
         {
@@ -538,7 +626,8 @@ void srm_server::slot_loop(int s)
             peak_accounted = std::max(peak_accounted, accounted(-1, 0));
             // inputs are no longer needed
             std::vector<srm_cand>().swap(r->cand);
-            std::vector<uint32_t>().swap(r->read_words);
+            r->read_words.reset();
+            r->reads.reset();
         }
         cv.notify_all();
     }
@@ -597,8 +686,6 @@ int srm_server_create(const srm_server_config *cfg, const char *genome, size_t g
         S->job.push_back(j);
     }
     S->slot_req.assign((size_t)cfg->n_slots, nullptr);
-    S->stage.assign((size_t)cfg->n_slots, nullptr);
-    S->stage_cap.assign((size_t)cfg->n_slots, 0);
     S->slot_busy.assign((size_t)cfg->n_slots, false);
     S->reserved.assign((size_t)cfg->n_slots, 0);
     for (srm_ctx *c : S->ctx) S->base.push_back(srm_ctx_pool_used(c));
@@ -632,9 +719,13 @@ long long srm_server_submit(srm_server *S, const char *reads, const uint64_t *re
         r->off[i] = acc;
         acc += read_len[i];
     }
-    r->reads.resize(acc);
-    for (size_t i = 0; i < n_reads; ++i)
-        std::memcpy(&r->reads[r->off[i]], reads + read_off[i], read_len[i]);
+    r->total = acc;
+    r->reads = S->pool->take(acc);
+    for (size_t i = 0, m; i < n_reads; i += m) {   // runs of reads that follow each other
+        size_t bytes = read_len[i];
+        for (m = 1; i + m < n_reads && read_off[i + m] == read_off[i] + bytes; ++m) bytes += read_len[i + m];
+        std::memcpy(r->reads.get() + r->off[i], reads + read_off[i], bytes);
+    }
     std::lock_guard<std::mutex> lk(S->mu);
     r->id = S->next_id++;
     r->st.t_submit = S->now();
@@ -665,18 +756,30 @@ int srm_server_wait(srm_server *S, long long id, int timeout_ms)
 long long srm_server_result(srm_server *S, long long id, char *out, size_t outcap,
                             srm_request_stats *st, int release)
 {
-    std::lock_guard<std::mutex> lk(S->mu);
-    auto it = S->all.find((uint64_t)id);
-    if (it == S->all.end() || !it->second->done) return SRM_EINVAL;
-    auto r = it->second;
+    std::shared_ptr<Request> r;
+    {
+        std::lock_guard<std::mutex> lk(S->mu);
+        auto it = S->all.find((uint64_t)id);
+        if (it == S->all.end() || !it->second->done) return SRM_EINVAL;
+        r = it->second;
+    }
+    // a finished request does not change: the copy runs beside the server's threads
     if (st) *st = r->st;
-    long long need = (long long)(r->records.size() + r->rec_len);
-    if (out && (size_t)need <= outcap) {
+    size_t need = r->records.size() + r->rec_len;
+    for (const auto &t : r->perfect) need += t.n;
+    if (out && need <= outcap) {
+        for (const auto &t : r->perfect) {
+            if (t.n) std::memcpy(out, t.mem.get(), t.n);
+            out += t.n;
+        }
         std::memcpy(out, r->records.data(), r->records.size());
         if (r->rec_len) std::memcpy(out + r->records.size(), r->rec_text.get(), r->rec_len);
+        if (release) {
+            std::lock_guard<std::mutex> lk(S->mu);
+            S->all.erase((uint64_t)id);
+        }
     }
-    if (release && out && (size_t)need <= outcap) S->all.erase(it);
-    return need;
+    return (long long)need;
 }
 
 /* HBM the alignment slots account for now (held by idle slots, reserved by busy
@@ -726,7 +829,6 @@ void srm_server_destroy(srm_server *S)
         srm_job_destroy(S->job[i]);
         srm_ctx_destroy(S->ctx[i]);
     }
-    for (char *b : S->stage) srm_host_free(b);
     srm_dfilter_destroy(S->dfilter);
     if (S->fctx) srm_ctx_destroy(S->fctx);
     srm_index_destroy(S->index);
