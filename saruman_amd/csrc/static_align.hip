@@ -38,7 +38,6 @@ std::mutex g_mu;
 unsigned char *g_scratch[MAX_DEVICES] = {};   // the array's address on each device
 
 // the host plan, rebuilt by each call (under g_mu)
-srm_cand h_cand_tile[SRM_STATIC_MAX_CAND];
 uint32_t h_perm[SRM_STATIC_MAX_CAND];
 uint32_t h_tmp[SRM_STATIC_MAX_CAND];
 uint8_t h_cls[SRM_STATIC_MAX_CAND];
@@ -46,6 +45,11 @@ uint32_t h_tiles[4 * MAX_TILES];
 uint64_t h_tile_off[MAX_TILES];
 size_t h_lcount[MAX_L + 2];
 srm::PlanSums h_sums;
+// what one copy sends: the plan's arrays as they lie in the scratch, from the descriptors
+// (candidate order, then tile order) to the tile offsets.  Five copies of a few KB were 25
+// of the 47 us of 500 candidates of 36 bp
+__attribute__((aligned(256))) unsigned char h_image[SRM_STATIC_MAX_CAND * (2 * sizeof(srm_cand) + 4) +
+                                                    MAX_TILES * 24 + 5 * 256];
 
 struct Class {
     int nw = 0, maxL = 0;
@@ -110,8 +114,8 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
     in.band_ok = in.only_band = true;
     in.merge_below = 1;
 
-    // the scratch: counters, descriptors in candidate and tile order, perm, scores,
-    // then (below) tiles, tile offsets and the band scratch
+    // the scratch: counters, descriptors in candidate and tile order, perm, then (below)
+    // tiles, tile offsets, scores and the band scratch
     size_t at = 0;
     const size_t o_queue = at;
     at = align256(at + 64 * sizeof(uint32_t));
@@ -120,8 +124,6 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
     const size_t o_cand_tile = at;
     at = align256(at + (size_t)n * sizeof(srm_cand));
     const size_t o_perm = at;
-    at = align256(at + (size_t)n * 4);
-    const size_t o_score = at;
     at = align256(at + (size_t)n * 4);
     unsigned char *base = nullptr;
     hipStream_t st = (hipStream_t)stream;
@@ -227,13 +229,14 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
             }
             i = e2;
         }
-        for (int p = 0; p < n; ++p) h_cand_tile[p] = cand[h_perm[p]];
     }
 
     const size_t o_tiles = at;
     at = align256(at + ntiles * 16);
     const size_t o_toff = at;
     at = align256(at + ntiles * 8);
+    const size_t o_score = at;
+    at = align256(at + (size_t)n * 4);
     const size_t o_band = at;
     at += words * 4;
     if (at > SRM_STATIC_SCRATCH_BYTES)
@@ -241,15 +244,19 @@ extern "C" int srm_align_static(int device, void *stream, int match, int mismatc
                                      "static scratch holds %zu; split the batch",
                          at, (size_t)SRM_STATIC_SCRATCH_BYTES);
 
+    // the arrays that the host made, in one copy
+    const size_t o_first = planned ? o_tiles : o_cand;
+    auto image = [&](size_t o) { return h_image + (o - o_first); };
     if (!planned) {
         if (const int rc = on_device()) return rc;
-        SA_TRY(hipMemcpyAsync(base + o_cand, cand, (size_t)n * sizeof(srm_cand), hipMemcpyHostToDevice, st));
-        SA_TRY(hipMemcpyAsync(base + o_cand_tile, h_cand_tile, (size_t)n * sizeof(srm_cand),
-                              hipMemcpyHostToDevice, st));
-        SA_TRY(hipMemcpyAsync(base + o_perm, h_perm, (size_t)n * 4, hipMemcpyHostToDevice, st));
+        std::memcpy(image(o_cand), cand, (size_t)n * sizeof(srm_cand));
+        auto *in_order = (srm_cand *)image(o_cand_tile);
+        for (int p = 0; p < n; ++p) in_order[p] = cand[h_perm[p]];
+        std::memcpy(image(o_perm), h_perm, (size_t)n * 4);
     }
-    SA_TRY(hipMemcpyAsync(base + o_tiles, h_tiles, ntiles * 16, hipMemcpyHostToDevice, st));
-    SA_TRY(hipMemcpyAsync(base + o_toff, h_tile_off, ntiles * 8, hipMemcpyHostToDevice, st));
+    std::memcpy(image(o_tiles), h_tiles, ntiles * 16);
+    std::memcpy(image(o_toff), h_tile_off, ntiles * 8);
+    SA_TRY(hipMemcpyAsync(base + o_first, h_image, o_toff + ntiles * 8 - o_first, hipMemcpyHostToDevice, st));
     srm::BandArgs a{};
     a.ma = match;
     a.mm = mismatch;
