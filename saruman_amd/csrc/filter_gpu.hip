@@ -1288,7 +1288,7 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
 int upload_pieces(srm_dfilter *G, Call &c, const char *reads, const uint64_t *read_off,
                   const uint16_t *read_len, const uint8_t *read_k, size_t n, bool &counted)
 {
-    Planner plan(G->ix);
+    Planner plan(G->ix, false);
     std::string err;
     // the totals: the end of the last read, and the lists of every so many reads
     const size_t bytes = read_off[n - 1] + read_len[n - 1], step = std::max<size_t>(1, n / 512);
@@ -1296,7 +1296,7 @@ int upload_pieces(srm_dfilter *G, Call &c, const char *reads, const uint64_t *re
     for (size_t i = 0; i < n; i += step, ++seen) {
         const int32_t id = plan.set_of(read_len[i], read_k[i], err);
         if (id < 0) return SRM_OK;   // the first bad read's error is the call's
-        sum += plan.lists[(size_t)id];
+        sum += (uint64_t)plan.params[(size_t)id].n;
     }
     const uint64_t room = (uint64_t)((double)sum / (double)seen * (double)n * 1.125) + 4096;
     if (room >= (uint64_t)1 << 30 || plan.params.size() > MAX_SETS) return SRM_OK;
@@ -1328,8 +1328,8 @@ int upload_pieces(srm_dfilter *G, Call &c, const char *reads, const uint64_t *re
     std::vector<DParam> dpar;
     std::vector<uint16_t> gram;
     // an eighth of the reads, so that little is left to do after the last one's arrival;
-    // a piece below 32,768 costs more calls than it hides
-    const size_t piece = std::min(PIECE, std::max<size_t>(PIECE / 4, (n + 7) / 8));
+    // a piece below 65,536 costs more calls than it hides
+    const size_t piece = std::min(PIECE, std::max<size_t>(PIECE / 2, (n + 7) / 8));
     int k = 0;
     for (size_t lo = 0; lo < n; lo += piece, ++k) {
         const size_t hi = std::min(n, lo + piece), m = hi - lo;
@@ -1432,7 +1432,7 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     }
     ReadPlan plan;
     std::string err;
-    if (int rc = plan_reads(G->ix, read_off, read_len, read_k, n_reads, plan, err))
+    if (int rc = plan_reads(G->ix, read_off, read_len, read_k, n_reads, plan, err, false))
         return srm::set_error(rc, "%s", err.c_str());
     std::vector<DParam> dpar;
     std::vector<uint16_t> gram;
