@@ -187,6 +187,10 @@ struct srm_job {
     int ma = 0, mm = 1;
     bool unit = true;
     bool one_launch = false;         // every class in one launch (set at the upload)
+    bool beside = false;             // the plain kernels on rest_st beside the band's (likewise)
+    uint64_t *back = nullptr;        // two words of page-locked memory that sizes come back to
+    hipStream_t rest_st = nullptr;
+    hipEvent_t rest_ev = nullptr;
     bool resident_genome = false;
     // device buffers
     DevBuf d_cand, d_read_words, d_win_words, d_read_bytes, d_win_bytes;
@@ -400,6 +404,45 @@ int run_launches(srm_job *j, int kernel, bool timed)
     hipStream_t st = ctx->stream;
     const bool use_band = kernel != SRM_KERNEL_PLAIN;
     if (timed) HIP_TRY(hipEventRecord(j->ev[0], st));
+    auto plain = [&](const std::vector<PlainChunk> &chunks, DevBuf &idx, DevBuf &off, bool codes,
+                     hipStream_t on) -> int {
+        for (const PlainChunk &ch : chunks) {
+            srm::PlainArgs a;
+            a.ma = j->ma;
+            a.mm = j->mm;
+            a.n = (int)ch.count;
+            a.idx = (const uint32_t *)idx.p + ch.begin;
+            a.cand = (const srm_cand *)j->d_cand.p;
+            a.read_words = (const uint32_t *)j->d_read_words.p + SRM_CODE_PAD / 16;
+            a.win_words = j->resident_genome
+                              ? ctx->genome_ptr()
+                              : (const uint32_t *)j->d_win_words.p + SRM_CODE_PAD / 16;
+            a.read_bytes = (const char *)j->d_read_bytes.p;
+            a.win_bytes = (const char *)j->d_win_bytes.p;
+            a.mat = (int16_t *)j->d_mat.p;
+            a.mat_off = (const uint64_t *)off.p + ch.begin;
+            a.res = (srm_result *)j->d_res.p;
+            a.ops = (uint32_t *)j->d_ops.p;
+            HIP_TRY(srm::launch_plain(a, codes, on));
+        }
+        return SRM_OK;
+    };
+    auto the_rest = [&](hipStream_t on) -> int {
+        const int rc = use_band ? plain(j->chunks_rest, j->d_idx_rest, j->d_off_rest, true, on)
+                                : plain(j->chunks_all, j->d_idx_all, j->d_off_all, true, on);
+        return rc ? rc : plain(j->chunks_bytes, j->d_idx_bytes, j->d_off_bytes, false, on);
+    };
+    // the candidates that the band does not take on a stream of their own, from the
+    // start: they are few and each is a serial chain as long as the band's (0.16 and
+    // 0.10 ms of a batch of 50,000 reads, 3% of them with an N, one after the other)
+    const bool beside = use_band && j->beside && !j->classes.empty();
+    int rc = SRM_OK;
+    if (beside) {
+        HIP_TRY(hipEventRecord(j->fork_ev, st));
+        HIP_TRY(hipStreamWaitEvent(j->rest_st, j->fork_ev, 0));
+        if ((rc = the_rest(j->rest_st))) return rc;
+        HIP_TRY(hipEventRecord(j->rest_ev, j->rest_st));
+    }
     if (use_band && !j->classes.empty()) {
         HIP_TRY(srm::launch_reset((uint32_t *)j->d_queue.p, (int)j->classes.size(), st));
         if (j->one_launch) {   // widest band, the longest tiles, first
@@ -446,37 +489,8 @@ int run_launches(srm_job *j, int kernel, bool timed)
             }
     }
     if (timed) HIP_TRY(hipEventRecord(j->ev[1], st));
-    auto plain = [&](const std::vector<PlainChunk> &chunks, DevBuf &idx, DevBuf &off,
-                     bool codes) -> int {
-        for (const PlainChunk &ch : chunks) {
-            srm::PlainArgs a;
-            a.ma = j->ma;
-            a.mm = j->mm;
-            a.n = (int)ch.count;
-            a.idx = (const uint32_t *)idx.p + ch.begin;
-            a.cand = (const srm_cand *)j->d_cand.p;
-            a.read_words = (const uint32_t *)j->d_read_words.p + SRM_CODE_PAD / 16;
-            a.win_words = j->resident_genome
-                              ? ctx->genome_ptr()
-                              : (const uint32_t *)j->d_win_words.p + SRM_CODE_PAD / 16;
-            a.read_bytes = (const char *)j->d_read_bytes.p;
-            a.win_bytes = (const char *)j->d_win_bytes.p;
-            a.mat = (int16_t *)j->d_mat.p;
-            a.mat_off = (const uint64_t *)off.p + ch.begin;
-            a.res = (srm_result *)j->d_res.p;
-            a.ops = (uint32_t *)j->d_ops.p;
-            HIP_TRY(srm::launch_plain(a, codes, st));
-        }
-        return SRM_OK;
-    };
-    int rc;
-    if (use_band)
-        rc = plain(j->chunks_rest, j->d_idx_rest, j->d_off_rest, true);
-    else
-        rc = plain(j->chunks_all, j->d_idx_all, j->d_off_all, true);
-    if (rc) return rc;
-    rc = plain(j->chunks_bytes, j->d_idx_bytes, j->d_off_bytes, false);
-    if (rc) return rc;
+    if (beside) HIP_TRY(hipStreamWaitEvent(st, j->rest_ev, 0));
+    else if ((rc = the_rest(st))) return rc;
     if (timed) HIP_TRY(hipEventRecord(j->ev[2], st));
     if (j->rec_stage) {
         // records of every hit into the output sized at set-up: counter reset (a
@@ -1062,6 +1076,7 @@ int srm_job_create(srm_ctx *ctx, srm_job **out)
     for (auto &e : j->ce) ok = ok && hipEventCreate(&e) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&j->fork_ev, hipEventDisableTiming) == hipSuccess;
     for (auto &e : j->join_ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    ok = ok && hipHostMalloc((void **)&j->back, 16, hipHostMallocDefault) == hipSuccess;
     if (!ok) {
         srm_job_destroy(j);
         return fail(SRM_EDEVICE, "hipEventCreate failed");
@@ -1094,6 +1109,7 @@ int srm_job_release(srm_job *j)
     HIP_TRY(hipSetDevice(c->device));
     HIP_TRY(hipStreamSynchronize(c->stream));
     for (hipStream_t q : j->side) HIP_TRY(hipStreamSynchronize(q));
+    if (j->rest_st) HIP_TRY(hipStreamSynchronize(j->rest_st));
     destroy_graph(j);
     release_job_buffers(j);
     j->plan = HostPlan();   // and the host arrays an upload keeps for the next one
@@ -1130,6 +1146,12 @@ void srm_job_destroy(srm_job *j)
             if (arr[i]) (void)hipEventDestroy(arr[i]);
     }
     if (j->fork_ev) (void)hipEventDestroy(j->fork_ev);
+    if (j->rest_st) {
+        (void)hipStreamSynchronize(j->rest_st);
+        (void)hipStreamDestroy(j->rest_st);
+    }
+    if (j->rest_ev) (void)hipEventDestroy(j->rest_ev);
+    if (j->back) (void)hipHostFree(j->back);
     delete j;
 }
 
@@ -1260,6 +1282,11 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
         hipStream_t q = nullptr;
         HIP_TRY(hipStreamCreateWithFlags(&q, hipStreamNonBlocking));
         j->side.push_back(q);
+    }
+    j->beside = concurrent && j->n_band > 0 && j->n_rest + j->n_bytes > 0;
+    if (j->beside && !j->rest_st) {
+        HIP_TRY(hipStreamCreateWithFlags(&j->rest_st, hipStreamNonBlocking));
+        HIP_TRY(hipEventCreateWithFlags(&j->rest_ev, hipEventDisableTiming));
     }
     // ---- device buffers
     if (!planned && (rc = upload(ctx, j->d_cand, cand, (size_t)n))) return rc;
@@ -1402,17 +1429,9 @@ int rec_inputs(srm_job *j, const int64_t *pos, const int32_t *read_id, const cha
     if (!pos) return fail(SRM_EINVAL, "records need the window positions");
     srm_ctx *ctx = j->ctx;
     const int n = j->n;
-    if (names) {
-        if (name_stride < 2 || name_stride > 256 || !read_id)
-            return fail(SRM_EINVAL, "a name table needs 2 <= name_stride <= 256 and read ids");
-        for (int t = 0; t < n; ++t)
-            if (read_id[t] < 0 || (size_t)read_id[t] >= n_names)
-                return fail(SRM_EINVAL, "read id %d of candidate %d is outside the name table",
-                            read_id[t], t);
-    } else if (read_id) {
-        for (int t = 0; t < n; ++t)
-            if (read_id[t] < 0) return fail(SRM_EINVAL, "negative read id at candidate %d", t);
-    }
+    if (names && (name_stride < 2 || name_stride > 256 || !read_id))
+        return fail(SRM_EINVAL, "a name table needs 2 <= name_stride <= 256 and read ids");
+    // (the ids are looked over while they are sent, below)
     const char *prefix = name_prefix ? name_prefix : "";
     const size_t plen = strlen(prefix);
     if (plen > 255) return fail(SRM_EINVAL, "name prefix longer than 255 bytes");
@@ -1433,12 +1452,41 @@ int rec_inputs(srm_job *j, const int64_t *pos, const int32_t *read_id, const cha
     HIP_TRY(srm::rec_scan(nullptr, tmp, (const uint64_t *)j->d_rec_len.p,
                           (uint64_t *)j->d_rec_off.p, n, ctx->stream));
     if ((rc = ctx->ensure(j->d_rec_tmp, std::max<size_t>(tmp, 256)))) return rc;
+    if (read_id) {
+        // an unsigned compare takes the negative ones too
+        const uint64_t bound = names ? std::min<uint64_t>(n_names, 0x80000000u) : 0x80000000u;
+        bool bad = false;
+        for (int t = 0; t < n; ++t) bad |= (uint32_t)read_id[t] >= bound;
+        if (bad) {
+            HIP_TRY(hipStreamSynchronize(ctx->stream));
+            for (int t = 0; t < n; ++t) {
+                if ((uint32_t)read_id[t] < bound) continue;
+                if (names)
+                    return fail(SRM_EINVAL, "read id %d of candidate %d is outside the name table",
+                                read_id[t], t);
+                return fail(SRM_EINVAL, "negative read id at candidate %d", t);
+            }
+        }
+    }
     j->rec_tmp = tmp;
     j->rec_names = names != nullptr;
     j->rec_ids = read_id != nullptr;
     j->rec_stride = names ? name_stride : 0;
     j->rec_prefix_len = (int)plen;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
+    return SRM_OK;
+}
+
+// the text's size and the hits, to page-locked memory (to the stack each copy waited)
+int rec_sizes(srm_job *j, uint64_t &total, uint32_t &hits)
+{
+    srm_ctx *ctx = j->ctx;
+    HIP_TRY(hipMemcpyAsync(j->back, (const uint64_t *)j->d_rec_off.p + j->n, 8, hipMemcpyDeviceToHost,
+                           ctx->stream));
+    HIP_TRY(hipMemcpyAsync(j->back + 1, j->d_rec_hits.p, 4, hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    total = j->back[0];
+    hits = (uint32_t)j->back[1];
     return SRM_OK;
 }
 }  // namespace
@@ -1459,16 +1507,13 @@ long long srm_job_records(srm_job *j, const int64_t *pos, const int32_t *read_id
     srm_ctx *ctx = j->ctx;
     const int n = j->n;
     srm::RecArgs a = rec_args(j, true);
-    HIP_TRY(hipMemsetAsync(a.hits, 0, 8, ctx->stream));
+    HIP_TRY(srm::launch_reset(a.hits, 2, ctx->stream));
     HIP_TRY(srm::launch_rec_measure(a, ctx->stream));
     size_t tmp = j->rec_tmp;
     HIP_TRY(srm::rec_scan(j->d_rec_tmp.p, tmp, a.len, (uint64_t *)j->d_rec_off.p, n, ctx->stream));
     uint64_t total = 0;
     uint32_t hits = 0;
-    HIP_TRY(hipMemcpyAsync(&total, (const uint64_t *)j->d_rec_off.p + n, 8, hipMemcpyDeviceToHost,
-                           ctx->stream));
-    HIP_TRY(hipMemcpyAsync(&hits, a.hits, 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if ((rc = rec_sizes(j, total, hits))) return rc;
     if (n_hits) *n_hits = hits;
     if (total > outcap || !out) return (long long)total;   // size query
     if ((rc = ctx->ensure(j->d_rec_out, std::max<size_t>(total, 256)))) return rc;
@@ -1506,10 +1551,7 @@ long long srm_job_records_text(srm_job *j, char *out, size_t outcap, long long *
     HIP_TRY(hipSetDevice(ctx->device));
     uint64_t total = 0;
     uint32_t hits = 0;
-    HIP_TRY(hipMemcpyAsync(&total, (const uint64_t *)j->d_rec_off.p + j->n, 8,
-                           hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipMemcpyAsync(&hits, j->d_rec_hits.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if (const int rc = rec_sizes(j, total, hits)) return rc;
     if (total > j->rec_cap) return fail(SRM_EDEVICE, "record text %llu exceeds its bound %zu",
                                         (unsigned long long)total, j->rec_cap);
     if (n_hits) *n_hits = hits;
