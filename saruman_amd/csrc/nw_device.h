@@ -75,6 +75,7 @@ struct BitsSpans {
 
 struct RecArgs {
     int n;
+    int tile_cands = 64;            // candidates per wave of the writers (launch_rec_write)
     const srm_cand *cand;
     const srm_result *res;
     const uint32_t *ops;

@@ -191,13 +191,13 @@ __global__ void __launch_bounds__(RB) rec_write(RecArgs a)
     const int wv = threadIdx.x >> 6;
     char *buf = (char *)lds[wv];
     const int nwaves = gridDim.x * (RB / 64);
-    const int ntile = (a.n + 63) / 64;
-    // a wave takes 64 consecutive candidates at a time: their metadata in one
+    const int ntile = (a.n + a.tile_cands - 1) / a.tile_cands;
+    // a wave takes tile_cands consecutive candidates at a time: their metadata in one
     // coalesced load per field (a candidate per lane), then their lines one by one
     for (int tile = __builtin_amdgcn_readfirstlane(blockIdx.x * (RB / 64) + wv); tile < ntile;
          tile += nwaves) {
-        const int tl = tile * 64 + lane;
-        const bool in = tl < a.n;
+        const int tl = tile * a.tile_cands + lane;
+        const bool in = lane < a.tile_cands && tl < a.n;
         const uint64_t len_l = in ? a.len[tl] : 0;
         if (!__ballot(len_l != 0)) continue;
         const uint4 inf_l = len_l ? a.info[tl] : make_uint4(0u, 0u, 0u, 0u);
@@ -366,7 +366,7 @@ __global__ void __launch_bounds__(RB) rec_write(RecArgs a)
 
 // ---------------------------------------------------------------------------
 // rec_write_lines: QL = 8 lines per wave at a time, TPL = 8 lanes per line.  A
-// wave takes 64 consecutive candidates (their length, offset and metadata in one
+// wave takes up to 64 consecutive candidates (their length, offset and metadata in one
 // coalesced load per field, a candidate per lane) and writes the lines
 // grouped_line() accepts, eight at a time:
 //   stage   each line's lanes load the transcript words and the read and window
@@ -486,13 +486,13 @@ __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(5))) re
     if (tid < (RB / 64) * QL) s_ops[tid / QL][tid % QL][0] = 0u;
     __syncthreads();
     const int nwaves = gridDim.x * (RB / 64);
-    const int ntile = (a.n + 63) / 64;
+    const int ntile = (a.n + a.tile_cands - 1) / a.tile_cands;
     const uint64_t e64 = 0x5555555555555555ull;
     for (int tile = __builtin_amdgcn_readfirstlane(blockIdx.x * (RB / 64) + wv); tile < ntile;
          tile += nwaves) {
         // ---- the tile's candidates, one per lane
-        const int tl = tile * 64 + lane;
-        const bool in = tl < a.n;
+        const int tl = tile * a.tile_cands + lane;
+        const bool in = lane < a.tile_cands && tl < a.n;
         const uint64_t len_l = in ? a.len[tl] : 0;
         if (!__ballot(len_l != 0)) continue;
         uint32_t cw[5] = {0u, 0u, 0u, 0u, 0u}, rw[2] = {0u, 0u};
@@ -806,22 +806,25 @@ hipError_t launch_rec_measure(const RecArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_rec_write(const RecArgs &a, hipStream_t st)
+hipError_t launch_rec_write(const RecArgs &args, hipStream_t st)
 {
+    RecArgs a = args;
     if (a.n <= 0) return hipSuccess;
-    // a wave per tile of 64 candidates for both kernels: the short lines eight at
-    // a time, then the others one at a time
-    const int tiles = (a.n + 63) / 64;
+    // a wave per tile of candidates for both kernels: the short lines eight at a time,
+    // then the others one at a time.  64 candidates a tile, which the first kernel sorts by
+    // length, while there are 4,096 tiles to fill the chip's 1,024 SIMDs; fewer below, down
+    // to one pass of eight lines, since a tile's passes follow one another: 44,000
+    // candidates, 3% of them raw, 55 + 62 us with tiles of 64, 24 + 34 with 8
+    a.tile_cands = 64;
+    while (a.tile_cands > QL && a.n / a.tile_cands < 4096) a.tile_cands /= 2;
+    const int tiles = (a.n + a.tile_cands - 1) / a.tile_cands;
     const int waves = tiles < 65536 * 4 ? tiles : 65536 * 4;
-    if (a.names)
-        hipLaunchKernelGGL(rec_write_lines<true>, dim3((waves + RB / 64 - 1) / (RB / 64)), dim3(RB), 0,
-                           st, a);
-    else
-        hipLaunchKernelGGL(rec_write_lines<false>, dim3((waves + RB / 64 - 1) / (RB / 64)), dim3(RB),
-                           0, st, a);
+    const dim3 grid((waves + RB / 64 - 1) / (RB / 64));
+    if (a.names) hipLaunchKernelGGL(rec_write_lines<true>, grid, dim3(RB), 0, st, a);
+    else hipLaunchKernelGGL(rec_write_lines<false>, grid, dim3(RB), 0, st, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(rec_write, dim3((waves + RB / 64 - 1) / (RB / 64)), dim3(RB), 0, st, a);
+    hipLaunchKernelGGL(rec_write, grid, dim3(RB), 0, st, a);
     return hipGetLastError();
 }
 
