@@ -147,6 +147,8 @@ struct Strand {
     Header *hdr;
     uint64_t flat_cap;       // entries that flat holds
     Counts *cnt, *start;     // [n_reads + 1] per read; summed over the reads before
+    uint32_t *list_sum;      // small calls: the sums of fl_count's and fl_batch_count's
+    Counts *cnt_sum;         // blocks
     uint32_t *by_rank;       // the reads with entries
     uint32_t *unsafe;        // read | leaky << 31
     uint32_t *walk;
@@ -157,6 +159,7 @@ struct Call {
     Strand s[2];
     int n;
     uint64_t n_lists;        // per strand
+    bool sums;               // block sums in place of scans (SUM_READS)
     uint64_t list_stride;    // words from a strand's list arrays to the other's
     int kmax;
     const uint8_t *blocked;
@@ -220,7 +223,84 @@ struct BlockReads {
     }
 };
 
-// the lists of reads [lo, hi)
+// list i of the block: its length with the terminator, which it writes with the first key
+__device__ __forceinline__ uint32_t count_list(const FArgs &a, const BlockReads &s, uint32_t nr, uint32_t i)
+{
+    const uint32_t t = s.read_of(i, nr);
+    const int L = s.L[t], q = s.q[t], g = gram_offset(L, q, (int)(i - s.base[t]));
+    const DQ X = a.qix[q];
+    uint64_t code;
+    uint32_t first, c;
+    if (gram_code(a.read_pk, a.read_odd, s.off[t], L, a.dr, q, g, code))
+        c = lookup_code(X, code, first);
+    else
+        c = lookup<false>(X, a.genome, a.reads + s.off[t], L, a.dr, g, nullptr, &first);
+    a.list_cnt[i] = c + 1;
+    a.list_lo[i] = first;
+    return c + 1;
+}
+
+// Sums over a block's threads, and over the blocks of a small call.  Up to SUM_READS reads
+// a kernel adds up its own blocks' parts and the next one adds the blocks before: a scan
+// kernel and its start-up between them cost 8 us and two launches, as much as the work of
+// 1,000 reads on either side (its whole call 142 -> 132 us).  Beyond, every block of
+// hundreds would read every block's sum, and the scan is the smaller part.
+constexpr size_t SUM_READS = 32768;
+constexpr size_t SUM_BLOCKS = 1024;   // blocks of either kernel, at most
+
+// the sum over the threads before this one; total: over all
+template <int N>
+__device__ __forceinline__ void block_excl(uint32_t (&v)[N], uint32_t (&total)[N])
+{
+    __shared__ uint32_t s[FB / 64][N];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    __syncthreads();   // the sums before have been read
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+        uint32_t x = v[e];
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)x, d, 64);
+            if (lane >= d) x += o;
+        }
+        if (lane == 63) s[wv][e] = x;
+        v[e] = x - v[e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+        total[e] = 0;
+#pragma unroll
+        for (int w = 0; w < FB / 64; ++w) {
+            if (w == wv) v[e] += total[e];
+            total[e] += s[w][e];
+        }
+    }
+}
+
+// of `blocks` blocks' sums of N words each: the sum over those before this block, over all
+template <int N>
+__device__ __forceinline__ void sums_before(const uint32_t *sum, uint32_t blocks, uint32_t (&before)[N],
+                                            uint32_t (&total)[N])
+{
+    uint32_t v[2 * N] = {}, t[2 * N];
+    for (uint32_t b = threadIdx.x; b < blocks; b += FB)
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            const uint32_t x = sum[(size_t)b * N + e];
+            v[N + e] += x;
+            if (b < blockIdx.x) v[e] += x;
+        }
+    block_excl<2 * N>(v, t);
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+        before[e] = t[e];
+        total[e] = t[N + e];
+    }
+}
+
+// the lists of reads [lo, hi); SUMS: with their starts in the block, and the block's sum
+template <bool SUMS>
 __global__ void __launch_bounds__(FB) fl_count(Call c_, uint32_t per, uint32_t lo, uint32_t hi)
 {
     __shared__ BlockReads s;
@@ -233,32 +313,44 @@ __global__ void __launch_bounds__(FB) fl_count(Call c_, uint32_t per, uint32_t l
         if (threadIdx.x == 0) a.list_cnt[c_.n_lists] = 0;
     }
     const uint32_t nr = s.load(a, per, lo, hi);
-    for (uint32_t i = s.base[0] + threadIdx.x; i < s.base[nr]; i += FB) {
-        const uint32_t t = s.read_of(i, nr);
-        const int L = s.L[t], q = s.q[t], g = gram_offset(L, q, (int)(i - s.base[t]));
-        const DQ X = a.qix[q];
-        uint64_t code;
-        uint32_t first, c;
-        if (gram_code(a.read_pk, a.read_odd, s.off[t], L, a.dr, q, g, code))
-            c = lookup_code(X, code, first);
-        else
-            c = lookup<false>(X, a.genome, a.reads + s.off[t], L, a.dr, g, nullptr, &first);
-        a.list_cnt[i] = c + 1;
-        a.list_lo[i] = first;
+    uint32_t carry = 0;
+    for (uint32_t i0 = s.base[0]; i0 < s.base[nr]; i0 += FB) {
+        const uint32_t i = i0 + threadIdx.x;
+        const bool in = i < s.base[nr];
+        uint32_t len[1] = {0}, all[1];
+        if (in) len[0] = count_list(a, s, nr, i);
+        if (!SUMS) continue;
+        block_excl<1>(len, all);
+        if (in) ((uint32_t *)a.list_start)[i] = carry + len[0];
+        carry += all[0];
     }
+    if (SUMS && threadIdx.x == 0) c_.s[blockIdx.y].list_sum[blockIdx.x] = carry;
 }
-
 // the lists themselves, blocks and threads as in fl_count: the positions are the
 // keys it found, or, for a q-gram holding another byte, the hash table's
+template <bool SUMS>
 __global__ void __launch_bounds__(FB) fl_fill(Call c_, uint32_t per)
 {
     __shared__ BlockReads s;
     FArgs a;
-    if (!strand_of(c_, a)) return;
+    uint32_t before[1] = {0}, total[1];
+    bool fits = true;
+    if (SUMS) {
+        const Strand &st = c_.s[blockIdx.y];
+        a = st.f;
+        a.list_org = 0;
+        sums_before<1>(st.list_sum, gridDim.x, before, total);
+        fits = total[0] <= st.flat_cap;
+        if (threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) ((uint32_t *)a.list_start)[c_.n_lists] = total[0];
+    } else if (!strand_of(c_, a)) {
+        return;
+    }
     const uint32_t nr = s.load(a, per, 0, a.n_reads);
     for (uint32_t i = s.base[0] + threadIdx.x; i < s.base[nr]; i += FB) {
-        const uint32_t c = a.list_cnt[i] - 1;
-        uint32_t *dst = a.flat + list_at(a, i);
+        const uint32_t c = a.list_cnt[i] - 1, at = list_at(a, i) + before[0];
+        if (SUMS) ((uint32_t *)a.list_start)[i] = at;
+        if (!fits) continue;
+        uint32_t *dst = a.flat + at;
         if (c) {
             const uint32_t lo = a.list_lo[i], t = s.read_of(i, nr);
             const int q = s.q[t];
@@ -509,6 +601,16 @@ __global__ void __launch_bounds__(PB) fl_pair(Call c_)
     }
 }
 
+__device__ __forceinline__ Counts counts_of(const uint32_t (&v)[4])
+{
+    Counts n;
+    n.cand = v[0];
+    n.perf = v[1];
+    n.queued = v[2];
+    n.with = v[3];
+    return n;
+}
+
 // ---- the batch pass (filter_batch.h), a thread per read: counts, and after their
 // sum the candidates and perfect hits at their places in read order.  HBM-bound
 // (12 bytes of meta per read, 5 per entry, 15 out per candidate); the host's pass
@@ -516,13 +618,14 @@ __global__ void __launch_bounds__(PB) fl_pair(Call c_)
 // With both strands in each launch and two waits in a call (one, while the output fits
 // the first copy) instead of eight, the whole call: 2M reads 96.2 -> 20.8 ms, 100,000 of
 // 36 bp 3.14 -> 0.74 ms, 1,000 0.47 -> 0.22 ms
+template <bool SUMS>
 __global__ void __launch_bounds__(FB) fl_batch_count(Call c)
 {
     FArgs a;
     if (!strand_of(c, a)) return;
     const Strand &s = c.s[blockIdx.y];
     const uint32_t r = blockIdx.x * FB + threadIdx.x;
-    if (r > a.n_reads) return;
+    if (!SUMS && r > a.n_reads) return;
     Counts n;
     if (r < a.n_reads) {
         const uint32_t m0 = a.meta[3 * (size_t)r], m2 = a.meta[3 * (size_t)r + 2];
@@ -536,7 +639,14 @@ __global__ void __launch_bounds__(FB) fl_batch_count(Call c)
             if (u < MAX_UNSAFE) s.unsafe[u] = r | (leaky ? 1u << 31 : 0u);
         }
     }
-    s.cnt[r] = n;
+    if (!SUMS) {
+        s.cnt[r] = n;
+        return;
+    }
+    uint32_t v[4] = {n.cand, n.perf, n.queued, n.with}, all[4];
+    block_excl<4>(v, all);
+    if (r <= a.n_reads) s.start[r] = counts_of(v);
+    if (threadIdx.x == 0) s.cnt_sum[blockIdx.x] = counts_of(all);
 }
 
 // the sum over a strand's reads before r
@@ -583,6 +693,7 @@ __host__ __device__ inline BlobAt blob_at(const Counts &t0, const Counts &t1)
     return b;
 }
 
+template <bool SUMS>
 __global__ void __launch_bounds__(FB) fl_batch_write(Call c)
 {
     FArgs a;
@@ -590,14 +701,30 @@ __global__ void __launch_bounds__(FB) fl_batch_write(Call c)
     const int y = blockIdx.y;
     const Strand &s = c.s[y];
     const uint32_t r = blockIdx.x * FB + threadIdx.x;
-    const BlobAt b = blob_at(counts_before(c.s[0], a.n_reads),
-                             c.n > 1 ? counts_before(c.s[1], a.n_reads) : Counts());
+    Counts total[2], at;
+    if (SUMS) {   // the other strand's sums are there too: it counted in the same launch
+        uint32_t before[4] = {}, x[4], all[4];
+        for (int z = 0; z < c.n; ++z) {
+            sums_before<4>((const uint32_t *)c.s[z].cnt_sum, gridDim.x, x, all);
+            total[z] = counts_of(all);
+            if (z == y)
+                for (int e = 0; e < 4; ++e) before[e] = x[e];
+        }
+        if (r <= a.n_reads) {
+            at = CountsSum()(s.start[r], counts_of(before));
+            s.start[r] = at;
+        }
+    } else {
+        total[0] = counts_before(c.s[0], a.n_reads);
+        if (c.n > 1) total[1] = counts_before(c.s[1], a.n_reads);
+        if (r < a.n_reads) at = counts_before(s, r);
+    }
+    const BlobAt b = blob_at(total[0], total[1]);
     const bool fits = b.bytes <= c.blob_cap;
     if (r == 0) s.hdr->blob_ok = fits;
     if (r >= a.n_reads) return;
     const uint32_t m0 = a.meta[3 * (size_t)r], m1 = a.meta[3 * (size_t)r + 1], m2 = a.meta[3 * (size_t)r + 2];
     const uint32_t ne = entries_of(m2), np = perfects_of(m2);
-    const Counts at = counts_before(s, r);
     if (ne) s.by_rank[at.with] = r;
     if (!fits) return;
     const DParam P = a.par[a.pid[r]];
@@ -836,7 +963,7 @@ struct srm_dfilter {
     size_t glen = 0;
     GBuf genome, gen_pk, gen_odd, dq;
     std::vector<GBuf> keys, pre, odd_hash, odd_pos;
-    GBuf in, read_pk, read_odd, words, blocked, list_cnt, list_lo, list_start, cub_tmp, cnt, start, by_rank,
+    GBuf in, read_pk, read_odd, words, sums, blocked, list_cnt, list_lo, list_start, cub_tmp, cnt, start, by_rank,
         unsafe, walk, out;
     GBuf flat[2], out_pos[2], out_flag[2], out_perf[2], meta[2], over[2][2];
     GBuf slot_pos, slot_flag, slot_perf;
@@ -850,7 +977,7 @@ struct srm_dfilter {
 
     ~srm_dfilter()
     {
-        for (GBuf *b : {&genome, &gen_pk, &gen_odd, &dq, &in, &read_pk, &read_odd, &words, &blocked, &list_cnt,
+        for (GBuf *b : {&genome, &gen_pk, &gen_odd, &dq, &in, &read_pk, &read_odd, &words, &sums, &blocked, &list_cnt,
                         &list_lo, &list_start, &cub_tmp, &cnt, &start, &by_rank, &unsafe, &walk, &out,
                         &slot_pos, &slot_flag, &slot_perf})
             b->release();
@@ -931,8 +1058,9 @@ uint32_t list_reads(size_t n)
 int launch_count(srm_dfilter *G, const Call &c, uint32_t lo, uint32_t hi)
 {
     const uint32_t per = list_reads(hi - lo);
-    hipLaunchKernelGGL(fl_count, dim3((hi - lo + per - 1) / per, (unsigned)c.n), dim3(FB), 0, G->st, c,
-                       per, lo, hi);
+    const dim3 grid((hi - lo + per - 1) / per, (unsigned)c.n);
+    if (c.sums) hipLaunchKernelGGL(fl_count<true>, grid, dim3(FB), 0, G->st, c, per, lo, hi);
+    else hipLaunchKernelGGL(fl_count<false>, grid, dim3(FB), 0, G->st, c, per, lo, hi);
     FL_TRY(hipGetLastError());
     return SRM_OK;
 }
@@ -948,7 +1076,7 @@ int launch_search(srm_dfilter *G, const Call &c)
     // offsets count from its first (list_org), modulo 2^32
     const bool one = c.list_stride == nl + 1;
     const int items = (int)((nl + 1) * (uint64_t)(one ? c.n : 1));
-    for (int x = 0; x < (one ? 1 : c.n); ++x) {
+    for (int x = 0; x < (c.sums ? 0 : one ? 1 : c.n); ++x) {
         size_t tmp = 0;
         const uint32_t *from = c.s[x].f.list_cnt;
         uint32_t *to = G->list_start.as<uint32_t>() + (size_t)x * c.list_stride;
@@ -956,7 +1084,8 @@ int launch_search(srm_dfilter *G, const Call &c)
         FL_RC(G->cub_tmp.ensure(tmp));
         FL_TRY(hipcub::DeviceScan::ExclusiveSum(G->cub_tmp.p, tmp, from, to, items, G->st));
     }
-    hipLaunchKernelGGL(fl_fill, grid, dim3(FB), 0, G->st, c, per);
+    if (c.sums) hipLaunchKernelGGL(fl_fill<true>, grid, dim3(FB), 0, G->st, c, per);
+    else hipLaunchKernelGGL(fl_fill<false>, grid, dim3(FB), 0, G->st, c, per);
     FL_TRY(hipGetLastError());
     // lanes per read: a wave for the reads of hundreds of entries (below); 8, about
     // the start positions of a read that maps once, for many reads; 32 for the few
@@ -976,18 +1105,25 @@ int launch_batch(srm_dfilter *G, const Call &c)
 {
     const uint32_t n = c.s[0].f.n_reads;
     const dim3 grid(n / FB + 1, (unsigned)c.n);
-    hipLaunchKernelGGL(fl_batch_count, grid, dim3(FB), 0, G->st, c);
-    FL_TRY(hipGetLastError());
-    size_t tmp = 0;
-    const int items = (int)(((uint64_t)n + 1) * (uint64_t)c.n);
-    FL_TRY(hipcub::DeviceScan::ExclusiveScan(nullptr, tmp, G->cnt.as<Counts>(), G->start.as<Counts>(),
-                                             CountsSum(), Counts(), items, G->st));
-    FL_RC(G->cub_tmp.ensure(tmp));
-    FL_TRY(hipcub::DeviceScan::ExclusiveScan(G->cub_tmp.p, tmp, G->cnt.as<Counts>(),
-                                             G->start.as<Counts>(), CountsSum(), Counts(), items,
-                                             G->st));
-    hipLaunchKernelGGL(fl_batch_write, grid, dim3(FB), 0, G->st, c);
-    FL_TRY(hipGetLastError());
+    if (c.sums) {
+        hipLaunchKernelGGL(fl_batch_count<true>, grid, dim3(FB), 0, G->st, c);
+        FL_TRY(hipGetLastError());
+        hipLaunchKernelGGL(fl_batch_write<true>, grid, dim3(FB), 0, G->st, c);
+        FL_TRY(hipGetLastError());
+    } else {
+        hipLaunchKernelGGL(fl_batch_count<false>, grid, dim3(FB), 0, G->st, c);
+        FL_TRY(hipGetLastError());
+        size_t tmp = 0;
+        const int items = (int)(((uint64_t)n + 1) * (uint64_t)c.n);
+        FL_TRY(hipcub::DeviceScan::ExclusiveScan(nullptr, tmp, G->cnt.as<Counts>(), G->start.as<Counts>(),
+                                                 CountsSum(), Counts(), items, G->st));
+        FL_RC(G->cub_tmp.ensure(tmp));
+        FL_TRY(hipcub::DeviceScan::ExclusiveScan(G->cub_tmp.p, tmp, G->cnt.as<Counts>(),
+                                                 G->start.as<Counts>(), CountsSum(), Counts(), items,
+                                                 G->st));
+        hipLaunchKernelGGL(fl_batch_write<false>, grid, dim3(FB), 0, G->st, c);
+        FL_TRY(hipGetLastError());
+    }
     hipLaunchKernelGGL(fl_batch_end, dim3(1, (unsigned)c.n), dim3(FB), 0, G->st, c);
     FL_TRY(hipGetLastError());
     return SRM_OK;
@@ -1053,6 +1189,7 @@ int ensure_lists(srm_dfilter *G, const Call &c)
     FL_RC(G->list_cnt.ensure(words * 4));
     FL_RC(G->list_lo.ensure(words * 4));
     FL_RC(G->list_start.ensure(words * 4));
+    FL_RC(G->sums.ensure(2 * SUM_BLOCKS * (4 + sizeof(Counts))));
     // candidates and perfect hits of both strands are 1-1.2 a read, 16-20 bytes each
     FL_RC(G->out.ensure(sizeof(Header) * (size_t)c.n + std::max<size_t>(STAGE_OUT, 28 * n)));
     return SRM_OK;
@@ -1067,6 +1204,8 @@ void bind_lists(const srm_dfilter *G, Call &c)
         a.list_cnt = G->list_cnt.as<uint32_t>() + (size_t)x * c.list_stride;
         a.list_lo = G->list_lo.as<uint32_t>() + (size_t)x * c.list_stride;
         a.list_start = G->list_start.as<uint32_t>() + (size_t)x * c.list_stride;
+        c.s[x].list_sum = (uint32_t *)G->sums.p + (size_t)x * SUM_BLOCKS;
+        c.s[x].cnt_sum = (Counts *)((uint32_t *)G->sums.p + 2 * SUM_BLOCKS) + (size_t)x * SUM_BLOCKS;
     }
 }
 
@@ -1480,6 +1619,7 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     c = Call{};
     c.n_lists = nl;
     c.list_stride = nl + 1;
+    c.sums = n_reads <= SUM_READS;
     for (const Params &p : plan.params) c.kmax = std::max(c.kmax, p.k);
     // both strands in each launch, while their lists fit one sum
     if (strands == 3 && nl < ((uint64_t)1 << 30) - 1) {
