@@ -77,6 +77,24 @@ __global__ void __launch_bounds__(FB) fl_pack(const uint4 *__restrict__ src, uin
     odd[i] = (uint16_t)o;
 }
 
+// A small call's inputs from page-locked host memory to dst, and the reads among them
+// (from 16-byte word `first` on) packed as by fl_pack: a copy before it takes 9 us for
+// 160 KB and starts and ends with a wait of 13
+__global__ void __launch_bounds__(FB) fl_take(const uint4 *__restrict__ src, uint4 *__restrict__ dst,
+                                              size_t first, uint32_t *__restrict__ pk,
+                                              uint16_t *__restrict__ odd, size_t n16)
+{
+    const size_t i = (size_t)blockIdx.x * FB + threadIdx.x;
+    if (i >= n16) return;
+    const uint4 v = src[i];
+    dst[i] = v;
+    if (i < first) return;
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    uint32_t o;
+    pk[i - first] = pack16(w, o);
+    odd[i - first] = (uint16_t)o;
+}
+
 constexpr size_t OVER_ROOM = (size_t)1 << 19;   // entries
 // The reads' codes as the alignment kernels take them (16 per word, the first lowest, other
 // bytes 0), `pad` codes of zero before them, every read's reverse complement after them:
@@ -142,6 +160,8 @@ struct Header {
     Flush flush[MAX_FLUSH];
 };
 
+static_assert(sizeof(Header) % 16 == 0, "the output behind it is read 16 bytes at a time");
+
 struct Strand {
     FArgs f;
     Header *hdr;
@@ -165,6 +185,8 @@ struct Call {
     const uint8_t *blocked;
     unsigned char *blob;     // the strands' candidates and perfect hits, arrays packed
     uint64_t blob_cap;
+    unsigned char *back;     // page-locked host memory for the headers and, if it fits
+    uint64_t back_cap;       // back_cap bytes, the blob
 };
 
 // a strand's arguments; false when its lists do not fit (the host makes room and
@@ -758,6 +780,26 @@ __global__ void fl_totals(Call c)
     if (threadIdx.x == 0) c.s[blockIdx.y].hdr->flat = list_at(a, c.n_lists);
 }
 
+// the strand's header and its share of the output to the host (by one block per strand),
+// as the call's last stores: a copy in their place would wait 13 us for this kernel's end
+// and take 7 more
+__device__ __forceinline__ void send_back(const Call &c, uint64_t bytes)
+{
+    __threadfence();
+    __syncthreads();
+    const uint32_t y = blockIdx.y;
+    const auto *h = (const uint32_t *)c.s[y].hdr;
+    auto *to = (uint32_t *)(c.back + y * sizeof(Header));
+    // (the atomics' words among them do not pass this CU's cache)
+    for (uint32_t i = threadIdx.x; i < sizeof(Header) / 4; i += FB)
+        to[i] = __hip_atomic_load(h + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (bytes > c.back_cap) return;
+    const auto *b = (const uint4 *)c.blob;
+    auto *out = (uint4 *)(c.back + c.n * sizeof(Header));
+    const uint64_t n16 = (bytes + 15) / 16;
+    for (uint64_t i = (uint64_t)threadIdx.x * c.n + y; i < n16; i += (uint64_t)FB * c.n) out[i] = b[i];
+}
+
 // one block per strand: the flushes (a flush ends with the first read that takes the
 // queue past chunk_value; found by a wave's 64-way search of the queued sums), and
 // the entries of the reads the host walks
@@ -766,6 +808,7 @@ __global__ void __launch_bounds__(FB) fl_batch_end(Call c)
     FArgs a;
     if (!strand_of(c, a)) {
         if (threadIdx.x == 0) c.s[blockIdx.y].hdr->flat = list_at(a, c.n_lists);
+        send_back(c, ~0ull);
         return;
     }
     const Strand &s = c.s[blockIdx.y];
@@ -832,6 +875,8 @@ __global__ void __launch_bounds__(FB) fl_batch_end(Call c)
         const uint32_t next = counts_before(s, r).with + 1;
         if ((s.unsafe[u] >> 31) && next < total.with) put(s.by_rank[next]);
     }
+    const BlobAt b = blob_at(counts_before(c.s[0], n), c.n > 1 ? counts_before(c.s[1], n) : Counts());
+    send_back(c, b.bytes <= c.blob_cap ? b.bytes : ~0ull);
 }
 
 struct GBuf {
@@ -944,10 +989,11 @@ private:
     size_t made_ = 0;
 };
 
-// inputs up to this size are put together in page-locked memory and sent in one copy
-// (a copy of a few KB takes 10-30 us of calls, whatever its size)
+// inputs up to this size are put together in page-locked memory, from which a kernel takes
+// them (a copy of a few KB takes 10-30 us of calls and waits, whatever its size)
 constexpr size_t STAGE_IN = (size_t)1 << 20;
-// and this much of the output comes back with the headers, in one copy
+// and this much of the output comes back with the headers, by the last kernel's stores:
+// 1,000 reads 132 -> 115 us with both
 constexpr size_t STAGE_OUT = (size_t)128 << 10;
 // reads of one piece of a large upload, at most, and its plan in page-locked memory
 constexpr size_t PIECE = 131072, PIECE_BYTES = (PIECE + 2) * (8 + 4 + 2);
@@ -1266,6 +1312,8 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
         }
         c.blob = G->out.as<unsigned char>() + head;
         c.blob_cap = G->out.cap - head;
+        c.back = (unsigned char *)G->stage_out;
+        c.back_cap = STAGE_OUT;
     };
     bind();
     if (!counted) FL_RC(launch_count(G, c, 0, n));
@@ -1277,8 +1325,8 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
     const auto *so = (const unsigned char *)G->stage_out;
     auto fetch = [&]() -> int {
         FL_TRY(hipEventRecord(G->ev[1], G->st));
-        FL_TRY(hipMemcpyAsync(G->stage_out, G->out.p, std::min(G->out.cap, head + STAGE_OUT),
-                              hipMemcpyDeviceToHost, G->st));
+        if (!on_device)   // (fl_batch_end sends them)
+            FL_TRY(hipMemcpyAsync(G->stage_out, G->out.p, head, hipMemcpyDeviceToHost, G->st));
         FL_TRY(hipStreamSynchronize(G->st));
         std::memcpy(h, so, head);
         return SRM_OK;
@@ -1599,15 +1647,20 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     FL_RC(G->in.ensure(all + 64));   // slack: whole 16-byte words of the reads are read
     if (all <= STAGE_IN) {
         for (const Part &p : part) std::memcpy((char *)G->stage_in + p.at, p.src, p.bytes);
-        FL_TRY(hipMemcpyAsync(G->in.p, G->stage_in, all, hipMemcpyHostToDevice, G->st));
+        FL_RC(G->pack(nullptr, rbytes, G->read_pk, G->read_odd, 0, 0));   // their room
+        const size_t n16 = (part[4].at + rbytes + 15) / 16;
+        hipLaunchKernelGGL(fl_take, dim3((unsigned)((n16 + FB - 1) / FB)), dim3(FB), 0, G->st,
+                           (const uint4 *)G->stage_in, G->in.as<uint4>(), part[4].at / 16,
+                           G->read_pk.as<uint32_t>(), G->read_odd.as<uint16_t>(), n16);
+        FL_TRY(hipGetLastError());
     } else {
         for (const Part &p : part)
             if (p.bytes)
                 FL_TRY(hipMemcpyAsync(G->in.as<char>() + p.at, p.src, p.bytes, hipMemcpyHostToDevice,
                                       G->st));
+        FL_RC(G->pack(G->in.as<char>() + part[4].at, rbytes, G->read_pk, G->read_odd));
     }
     const char *in = G->in.as<char>();
-    FL_RC(G->pack(in + part[4].at, rbytes, G->read_pk, G->read_odd));
     a.par = (const DParam *)(in + part[0].at);
     a.reads = in + part[4].at;
     a.read_pk = G->read_pk.as<uint32_t>();
