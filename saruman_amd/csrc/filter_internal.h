@@ -422,4 +422,7 @@ int dfilter_run2_words(srm_dfilter *G, const uint8_t *blocked, const char *reads
                        const uint64_t *read_off, const uint16_t *read_len, const uint8_t *read_k,
                        size_t n_reads, int chunk_value, uint32_t *words, srm_filter **out_fwd,
                        srm_filter **out_rev);
+// srm_job_download of the results without its wait: they are there after the job's next
+// call that waits (srm_job_records)
+int job_results_later(srm_job *j, srm_result *res);
 }  // namespace srm

@@ -174,10 +174,14 @@ struct HostPlan {
     std::vector<srm::PlanSums> sums;     // the device plan's (one)
     // the raw reads and windows of the candidates that take them, side by side, and
     // where each one's start
+    std::vector<srm_cand> cand_tile;     // a small upload's, in tile order
     std::vector<char> raw_read, raw_win;
     std::vector<uint32_t> raw_at;
 };
 }  // namespace
+
+// arrays of a small upload up to this size go by one launch: 5,000 candidates' plan
+constexpr size_t JOB_STAGE = (size_t)256 << 10;
 
 struct srm_job {
     srm_ctx *ctx = nullptr;
@@ -188,7 +192,8 @@ struct srm_job {
     bool unit = true;
     bool one_launch = false;         // every class in one launch (set at the upload)
     bool beside = false;             // the plain kernels on rest_st beside the band's (likewise)
-    uint64_t *back = nullptr;        // two words of page-locked memory that sizes come back to
+    char *stage = nullptr;           // JOB_STAGE bytes of page-locked memory (Staged)
+    uint64_t *back = nullptr;        // behind them two words that sizes come back to
     hipStream_t rest_st = nullptr;
     hipEvent_t rest_ev = nullptr;
     bool resident_genome = false;
@@ -527,6 +532,55 @@ __global__ void place_raw_kernel(srm_cand *__restrict__ cand, const uint32_t *__
     cand[idx[i]].read_off = at[2 * i];
     cand[idx[i]].win_off = at[2 * i + 1];
 }
+
+// a small upload's arrays, which lie in page-locked memory one after another, to their
+// buffers: a copy each takes 10 us of calls and waits, whatever its size
+struct Parts {
+    static constexpr int MAX = 8;
+    int n = 0;
+    void *dst[MAX];
+    uint32_t end[MAX];   // 16-byte words up to its end
+};
+
+__global__ void place_parts_kernel(const uint4 *__restrict__ src, Parts p)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    int x = 0;
+    while (x < p.n && i >= p.end[x]) ++x;
+    if (x < p.n) ((uint4 *)p.dst[x])[i - (x ? p.end[x - 1] : 0)] = src[i];
+}
+
+// what one launch sends from j->stage (which the job's last wait has freed)
+class Staged {
+  public:
+    explicit Staged(srm_job *job) : j(job) {}
+    static bool fits(size_t bytes, int parts) { return bytes + 16 * (size_t)parts <= JOB_STAGE && parts <= Parts::MAX; }
+    template <class T>
+    int add(DevBuf &b, const T *src, size_t count)
+    {
+        const size_t bytes = count * sizeof(T);
+        int rc = j->ctx->ensure(b, bytes + 64);   // slack as in upload(); whole words are written
+        if (rc || !bytes) return rc;
+        std::memcpy(j->stage + at, src, bytes);
+        at += (bytes + 15) & ~(size_t)15;
+        p.dst[p.n] = b.p;
+        p.end[p.n++] = (uint32_t)(at / 16);
+        return SRM_OK;
+    }
+    int send()
+    {
+        if (!p.n) return SRM_OK;
+        hipLaunchKernelGGL(place_parts_kernel, dim3((unsigned)((at / 16 + 255) / 256)), dim3(256), 0,
+                           j->ctx->stream, (const uint4 *)j->stage, p);
+        HIP_TRY(hipGetLastError());
+        return SRM_OK;
+    }
+
+  private:
+    srm_job *j;
+    size_t at = 0;
+    Parts p;
+};
 
 // The raw reads and windows that candidates take (SRM_CAND_BYTES), to d_read_bytes and
 // d_win_bytes.  Few candidates do -- those of reads with other bytes -- so their own
@@ -930,6 +984,15 @@ int ctx_device(const srm_ctx *c) { return c->device; }
 
 hipStream_t ctx_stream(const srm_ctx *c) { return c->stream; }
 
+int job_results_later(srm_job *j, srm_result *res)
+{
+    HIP_TRY(hipSetDevice(j->ctx->device));
+    if (j->n)
+        HIP_TRY(hipMemcpyAsync(res, j->d_res.p, (size_t)j->n * sizeof(srm_result), hipMemcpyDeviceToHost,
+                               j->ctx->stream));
+    return SRM_OK;
+}
+
 }  // namespace srm
 
 // ---------------------------------------------------------------------------
@@ -1076,7 +1139,8 @@ int srm_job_create(srm_ctx *ctx, srm_job **out)
     for (auto &e : j->ce) ok = ok && hipEventCreate(&e) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&j->fork_ev, hipEventDisableTiming) == hipSuccess;
     for (auto &e : j->join_ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-    ok = ok && hipHostMalloc((void **)&j->back, 16, hipHostMallocDefault) == hipSuccess;
+    ok = ok && hipHostMalloc((void **)&j->stage, JOB_STAGE + 16, hipHostMallocDefault) == hipSuccess;
+    j->back = (uint64_t *)(j->stage + JOB_STAGE);
     if (!ok) {
         srm_job_destroy(j);
         return fail(SRM_EDEVICE, "hipEventCreate failed");
@@ -1151,7 +1215,7 @@ void srm_job_destroy(srm_job *j)
         (void)hipStreamDestroy(j->rest_st);
     }
     if (j->rest_ev) (void)hipEventDestroy(j->rest_ev);
-    if (j->back) (void)hipHostFree(j->back);
+    if (j->stage) (void)hipHostFree(j->stage);
     delete j;
 }
 
@@ -1289,24 +1353,41 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
         HIP_TRY(hipEventCreateWithFlags(&j->rest_ev, hipEventDisableTiming));
     }
     // ---- device buffers
-    if (!planned && (rc = upload(ctx, j->d_cand, cand, (size_t)n))) return rc;
     if (n < PLAN_DEVICE_MIN && (rc = upload(ctx, j->d_read_words, read_words, n_read_words))) return rc;
     if (!j->resident_genome && (rc = upload(ctx, j->d_win_words, win_words, n_win_words))) return rc;
-    if (!planned) {
     const std::vector<uint32_t> &band_idx = hp.band_idx;
-    if ((rc = upload(ctx, j->d_perm, band_idx.data(), band_idx.size()))) return rc;
-    // the banded candidates in tile order (a wave reads its tile's descriptors as
-    // one contiguous run, without the indirection through perm), gathered on the
-    // device from the uploaded descriptors
-    if ((rc = ctx->ensure(j->d_cand_tile, band_idx.size() * sizeof(srm_cand) + 64))) return rc;
-    HIP_TRY(launch_gather_cand((const srm_cand *)j->d_cand.p, (const uint32_t *)j->d_perm.p,
-                               (srm_cand *)j->d_cand_tile.p, band_idx.size(), ctx->stream));
+    // the banded candidates in tile order (a wave reads its tile's descriptors as one
+    // contiguous run, without the indirection through perm), gathered on the device from
+    // the uploaded descriptors, or for a small upload here
+    const size_t in_order = planned ? 0 : band_idx.size();
+    if (!planned && Staged::fits((size_t)n * sizeof(srm_cand) + in_order * (sizeof(srm_cand) + 4) +
+                                     hp.tiles.size() * 4 + hp.tile_off.size() * 8 +
+                                     (hp.rest_idx.size() + hp.bytes_idx.size()) * 4, 7)) {
+        hp.cand_tile.resize(in_order);
+        for (size_t p = 0; p < in_order; ++p) hp.cand_tile[p] = cand[band_idx[p]];
+        Staged part(j);
+        if ((rc = part.add(j->d_cand, cand, (size_t)n))) return rc;
+        if ((rc = part.add(j->d_cand_tile, hp.cand_tile.data(), in_order))) return rc;
+        if ((rc = part.add(j->d_perm, band_idx.data(), in_order))) return rc;
+        if ((rc = part.add(j->d_tiles, hp.tiles.data(), hp.tiles.size()))) return rc;
+        if ((rc = part.add(j->d_tile_scratch, hp.tile_off.data(), hp.tile_off.size()))) return rc;
+        if ((rc = part.add(j->d_idx_rest, hp.rest_idx.data(), hp.rest_idx.size()))) return rc;
+        if ((rc = part.add(j->d_idx_bytes, hp.bytes_idx.data(), hp.bytes_idx.size()))) return rc;
+        if ((rc = part.send())) return rc;
+    } else {
+        if (!planned) {
+            if ((rc = upload(ctx, j->d_cand, cand, (size_t)n))) return rc;
+            if ((rc = upload(ctx, j->d_perm, band_idx.data(), in_order))) return rc;
+            if ((rc = ctx->ensure(j->d_cand_tile, in_order * sizeof(srm_cand) + 64))) return rc;
+            HIP_TRY(launch_gather_cand((const srm_cand *)j->d_cand.p, (const uint32_t *)j->d_perm.p,
+                                       (srm_cand *)j->d_cand_tile.p, in_order, ctx->stream));
+        }
+        if ((rc = upload(ctx, j->d_tiles, hp.tiles.data(), hp.tiles.size()))) return rc;
+        if ((rc = upload(ctx, j->d_tile_scratch, hp.tile_off.data(), hp.tile_off.size()))) return rc;
+        if ((rc = upload(ctx, j->d_idx_rest, hp.rest_idx.data(), hp.rest_idx.size()))) return rc;
+        if ((rc = upload(ctx, j->d_idx_bytes, hp.bytes_idx.data(), hp.bytes_idx.size()))) return rc;
     }
     if ((rc = ctx->ensure(j->d_tile_score, std::max<size_t>(j->n_band * 4, 64)))) return rc;
-    if ((rc = upload(ctx, j->d_tiles, hp.tiles.data(), hp.tiles.size()))) return rc;
-    if ((rc = upload(ctx, j->d_tile_scratch, hp.tile_off.data(), hp.tile_off.size()))) return rc;
-    if ((rc = upload(ctx, j->d_idx_rest, hp.rest_idx.data(), hp.rest_idx.size()))) return rc;
-    if ((rc = upload(ctx, j->d_idx_bytes, hp.bytes_idx.data(), hp.bytes_idx.size()))) return rc;
     if ((rc = ctx->ensure(j->d_queue, 64 * sizeof(uint32_t)))) return rc;
     if ((rc = ctx->ensure(j->d_scratch, std::max<size_t>(scratch_words * 4, 256)))) return rc;
     if ((rc = ctx->ensure(j->d_res, std::max<size_t>((size_t)n * sizeof(srm_result), 64)))) return rc;
@@ -1437,12 +1518,19 @@ int rec_inputs(srm_job *j, const int64_t *pos, const int32_t *read_id, const cha
     if (plen > 255) return fail(SRM_EINVAL, "name prefix longer than 255 bytes");
     HIP_TRY(hipSetDevice(ctx->device));
     int rc;
-    if ((rc = upload(ctx, j->d_rec_pos, pos, (size_t)n))) return rc;
-    if (read_id && (rc = upload(ctx, j->d_rec_id, read_id, (size_t)n))) return rc;
+    if (!names && Staged::fits((size_t)n * 12 + plen + 1, 3)) {
+        Staged part(j);
+        if ((rc = part.add(j->d_rec_pos, pos, (size_t)n))) return rc;
+        if (read_id && (rc = part.add(j->d_rec_id, read_id, (size_t)n))) return rc;
+        if ((rc = part.add(j->d_rec_names, prefix, plen + 1))) return rc;
+        if ((rc = part.send())) return rc;
+    } else {
+        if ((rc = upload(ctx, j->d_rec_pos, pos, (size_t)n))) return rc;
+        if (read_id && (rc = upload(ctx, j->d_rec_id, read_id, (size_t)n))) return rc;
+        if (!names && (rc = upload(ctx, j->d_rec_names, prefix, plen + 1))) return rc;
+    }
     if (names) {
         if ((rc = upload(ctx, j->d_rec_names, names, n_names * (size_t)name_stride))) return rc;
-    } else if ((rc = upload(ctx, j->d_rec_names, prefix, plen + 1))) {
-        return rc;
     }
     if ((rc = ctx->ensure(j->d_rec_len, ((size_t)n + 1) * 8))) return rc;
     if ((rc = ctx->ensure(j->d_rec_off, ((size_t)n + 1) * 8))) return rc;
@@ -1473,7 +1561,6 @@ int rec_inputs(srm_job *j, const int64_t *pos, const int32_t *read_id, const cha
     j->rec_ids = read_id != nullptr;
     j->rec_stride = names ? name_stride : 0;
     j->rec_prefix_len = (int)plen;
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
     return SRM_OK;
 }
 
@@ -1489,13 +1576,9 @@ int rec_sizes(srm_job *j, uint64_t &total, uint32_t &hits)
     hits = (uint32_t)j->back[1];
     return SRM_OK;
 }
-}  // namespace
-
-extern "C" {
-
-long long srm_job_records(srm_job *j, const int64_t *pos, const int32_t *read_id,
-                          const char *names, int name_stride, size_t n_names,
-                          const char *name_prefix, char *out, size_t outcap, long long *n_hits)
+long long records_now(srm_job *j, const int64_t *pos, const int32_t *read_id,
+                      const char *names, int name_stride, size_t n_names, const char *name_prefix,
+                      char *out, size_t outcap, long long *n_hits)
 {
     // this call's inputs replace those of a record stage set up before
     if (j->rec_stage) {
@@ -1524,6 +1607,19 @@ long long srm_job_records(srm_job *j, const int64_t *pos, const int32_t *read_id
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     return (long long)total;
 }
+}  // namespace
+
+extern "C" {
+
+long long srm_job_records(srm_job *j, const int64_t *pos, const int32_t *read_id,
+                          const char *names, int name_stride, size_t n_names,
+                          const char *name_prefix, char *out, size_t outcap, long long *n_hits)
+{
+    const long long got = records_now(j, pos, read_id, names, name_stride, n_names, name_prefix, out,
+                                      outcap, n_hits);
+    if (got < 0) (void)hipStreamSynchronize(j->ctx->stream);   // nothing of the caller's is still copied
+    return got;
+}
 
 int srm_job_set_records(srm_job *j, const int64_t *pos, const int32_t *read_id, const char *names,
                         int name_stride, size_t n_names, const char *name_prefix)
@@ -1532,7 +1628,9 @@ int srm_job_set_records(srm_job *j, const int64_t *pos, const int32_t *read_id, 
     j->rec_stage = false;
     j->rec_done = false;
     int rc = rec_inputs(j, pos, read_id, names, name_stride, n_names, name_prefix);
+    const hipError_t sent = hipStreamSynchronize(j->ctx->stream);   // the caller's arrays
     if (rc) return rc;
+    HIP_TRY(sent);
     // the output holds the longest text the lines can have: the name, two int32
     // coordinates (11 characters each), the strand, both rows of at most w + k
     // characters, the int16 score and 7 separators per candidate
