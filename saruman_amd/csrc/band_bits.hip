@@ -82,6 +82,16 @@ struct BitsShape {
     template <bool CK> __host__ __device__ static constexpr int win_at(int Lmax) { return CK ? ck_win_row(Lmax) : win_row(Lmax); }
 };
 
+template <int NW>
+constexpr bool rows_agree()
+{
+    for (int L = 0; L <= SRM_MAX_L; ++L)
+        if (BitsShape<NW>::rows(L) != bits_rows(NW, L)) return false;
+    return true;
+}
+static_assert(rows_agree<1>() && rows_agree<2>() && rows_agree<3>() && rows_agree<4>() &&
+              rows_agree<5>() && rows_agree<6>() && rows_agree<7>() && rows_agree<8>(), "bits_rows");
+
 // word and bit offset of diagonal i's D byte among a block's D words
 template <int NW>
 __device__ __forceinline__ void dloc(int i, int &word, int &shift)
@@ -930,18 +940,18 @@ template <bool CK>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CK ? 5 : 6)))
 void bits_all_kernel(BandArgs a, BitsSpans sp)
 {
-    uint32_t c = 0;
-    while (c + 1 < sp.n && blockIdx.x >= sp.block[c + 1]) ++c;
-    const uint32_t tile = sp.tile[c] + (blockIdx.x - sp.block[c]);
-    a.code_words = bits_code_words(sp.max_len[c]);
-    a.stage_words = bits_stage_words(sp.max_len[c]);
+    uint32_t tile;
+    int words, max_len;
+    if (!span_of(a, sp, tile, words, max_len)) return;
+    a.code_words = bits_code_words(max_len);
+    a.stage_words = bits_stage_words(max_len);
     auto both = [&](auto nw) {
         band_tile<decltype(nw)::value, CK>(a, tile);
         // both use the block's LDS, under two names: the walk's accesses stay behind
         asm volatile("" ::: "memory");
         trace_tile<decltype(nw)::value, CK>(a, tile);
     };
-    switch (sp.nw[c]) {
+    switch (words) {
     case 1: both(std::integral_constant<int, 1>{}); break;
     case 2: both(std::integral_constant<int, 2>{}); break;
     case 3: both(std::integral_constant<int, 3>{}); break;
@@ -1074,7 +1084,8 @@ hipError_t launch_bits_trace(const BandArgs &args, int nw, int maxL, hipStream_t
 // every class in one launch: a.tiles and a.tile_scratch are those of all classes
 hipError_t launch_bits_all(const BandArgs &a, const BitsSpans &sp, hipStream_t st)
 {
-    int words = 0;
+    // (without classes: what the longest staged reads take)
+    int words = sp.n ? 0 : bits_stage_words(320) > bits_code_words(250) ? bits_stage_words(320) : bits_code_words(250);
     for (uint32_t c = 0; c < sp.n; ++c) {
         const int u = bits_code_words(sp.max_len[c]), v = bits_stage_words(sp.max_len[c]);
         words = words > u ? words : u;

@@ -59,9 +59,12 @@ struct BandArgs {
 // block[c] .. block[c + 1] - 1 (a tile each, from tile[c] on) of band words nw[c] and
 // reads of up to max_len[c] codes
 constexpr int MAX_BAND_CLASSES = 16;   // 8 classes, each split at most once by read length
+// or, made on the device (n = 0), tiles in order whose w is the band and of which tiles[0]
+// run: `blocks` is what there are at most, max_len[0] the longest read there can be
 struct BitsSpans {
     uint32_t n = 0, blocks = 0;
-    uint32_t block[MAX_BAND_CLASSES], tile[MAX_BAND_CLASSES];
+    const uint32_t *tiles = nullptr;
+    uint32_t block[MAX_BAND_CLASSES], tile[MAX_BAND_CLASSES] = {};
     int nw[MAX_BAND_CLASSES], max_len[MAX_BAND_CLASSES];
     void add(int w, uint32_t tile_begin, uint32_t ntiles, int maxL)
     {
@@ -72,6 +75,27 @@ struct BitsSpans {
         blocks += ntiles;
     }
 };
+
+// the block's tile, its band's words and the read length its staging is sized for; false:
+// no tile is left
+__device__ __forceinline__ bool span_of(const BandArgs &a, const BitsSpans &sp, uint32_t &tile, int &nw,
+                                        int &max_len)
+{
+    if (sp.n == 0) {
+        tile = blockIdx.x;
+        if (tile >= sp.tiles[0]) return false;
+        const uint4 td = a.tiles[tile];
+        nw = __builtin_amdgcn_readfirstlane((int)td.w);
+        max_len = __builtin_amdgcn_readfirstlane((int)td.z);
+        return true;
+    }
+    uint32_t c = 0;
+    while (c + 1 < sp.n && blockIdx.x >= sp.block[c + 1]) ++c;
+    tile = sp.tile[c] + (blockIdx.x - sp.block[c]);
+    nw = sp.nw[c];
+    max_len = sp.max_len[c];
+    return true;
+}
 
 struct RecArgs {
     int n;
@@ -108,9 +132,17 @@ __host__ __device__ inline int band_cells(const srm_cand &c)
 // words of one tile's nibble band scratch (other costs): 8*NW diagonals x 8-column
 // blocks x 64 lanes, then the tail (columns L - 1 and L packed by diagonal,
 // equal-character bits)
-inline size_t tile_scratch_words(int nw, int maxL)
+__host__ __device__ constexpr size_t tile_scratch_words(int nw, int maxL)
 {
     return ((size_t)nw * 8 * ((maxL + 8) / 8) + 2 * (size_t)nw + 2) * 64;
+}
+
+// rows of 64 words of a tile's scratch for unit costs (stored D bits; BitsShape::rows)
+__host__ __device__ constexpr int bits_rows(int nw, int maxL)
+{
+    const int nwd = nw <= 4 ? 1 : 2, blocks = maxL >= 2 ? ((maxL - 2) >> 3) + 1 : 0;
+    return blocks * (2 * nw + 1 + 2 * nwd) + 2 * nw + 2 + ((maxL + 31) >> 4) + 1 +
+           2 * (nwd + ((maxL + 30) >> 5) + 2);
 }
 
 hipError_t launch_plain(const PlainArgs &a, bool codes, hipStream_t st);

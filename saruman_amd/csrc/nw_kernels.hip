@@ -786,15 +786,15 @@ __host__ __device__ constexpr int trace_code_words(int maxL)
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
 void nibble_all_kernel(BandArgs a, BitsSpans sp)
 {
-    uint32_t c = 0;
-    while (c + 1 < sp.n && blockIdx.x >= sp.block[c + 1]) ++c;
-    const uint32_t tile = sp.tile[c] + (blockIdx.x - sp.block[c]);
-    a.code_words = trace_code_words(sp.max_len[c]);
+    uint32_t tile;
+    int words, max_len;
+    if (!span_of(a, sp, tile, words, max_len)) return;
+    a.code_words = trace_code_words(max_len);
     auto both = [&](auto nw) {
         nibble_band_tile<decltype(nw)::value>(a, tile);
         nibble_trace_tile<decltype(nw)::value>(a, tile);
     };
-    switch (sp.nw[c]) {
+    switch (words) {
     case 1: both(std::integral_constant<int, 1>{}); break;
     case 2: both(std::integral_constant<int, 2>{}); break;
     case 3: both(std::integral_constant<int, 3>{}); break;
@@ -933,7 +933,7 @@ hipError_t launch_trace(const BandArgs &args, int nw, bool unit, int maxL, hipSt
 hipError_t launch_all(const BandArgs &a, const BitsSpans &sp, bool unit, hipStream_t st)
 {
     if (unit) return launch_bits_all(a, sp, st);
-    int words = 0;
+    int words = sp.n ? 0 : trace_code_words(sp.max_len[0]);
     for (uint32_t c = 0; c < sp.n; ++c) words = std::max(words, trace_code_words(sp.max_len[c]));
     hipLaunchKernelGGL(nibble_all_kernel, dim3(sp.blocks), dim3(64), (size_t)words * 64 * 4, st, a, sp);
     return hipGetLastError();

@@ -76,7 +76,7 @@ __host__ __device__ inline int plan_bin(const PlanIn &in, const srm_cand &c)
 {
     return (band_class(in, c) * 8 + (c.L & 7)) * 64 + 63 - (c.L >> 3);
 }
-inline int bin_len(int bin) { return 8 * (63 - (bin & 63)) + ((bin >> 6) & 7); }
+__host__ __device__ inline int bin_len(int bin) { return 8 * (63 - (bin & 63)) + ((bin >> 6) & 7); }
 
 // the tiles of the bins' counts: begin(class), tile(first place, candidates, longest
 // read) for each of its tiles, end() -- for every class that has candidates
@@ -111,17 +111,39 @@ struct PlanSums {
     uint32_t first_bad;           // the first refused candidate (~0: none)
     uint32_t n_band, n_rest, n_bytes;
     uint32_t too_long;            // banded reads of more than PLAN_MAX_L codes
-    uint32_t pad;
+    uint32_t run;                 // tiles to run, 0 when something forbids it (PlanTiles)
+    unsigned long long words;     // of the tiles' scratch (PlanTiles)
+    uint32_t n_tiles, pad;        // likewise
     uint32_t bin[PLAN_BINS];
 };
 // what the plan kernels need besides their inputs and lists
 constexpr size_t PLAN_SCRATCH = sizeof(PlanSums) + 2 * PLAN_BINS * sizeof(uint32_t);
+
+// The tiles made on the device too, for srm_align_static: in the order they run, the
+// widest band first, w the band; off: where each one's scratch starts.  They run if every
+// candidate is banded, no read is longer than PLAN_MAX_L and the call's arrays end within
+// `room` (static_end)
+struct PlanTiles {
+    bool unit;
+    uint4 *tiles;
+    uint64_t *off;
+    uint64_t o_tiles, room;
+};
+// tiles of n candidates, at most
+__host__ __device__ inline uint32_t most_tiles(uint32_t n) { return n / 64 + PLAN_CLASSES / 2 * 8; }
+__host__ __device__ inline uint64_t align256(uint64_t x) { return (x + 255) & ~(uint64_t)255; }
+// where the arrays of srm_align_static end: tiles (from o_tiles), their offsets, a score a
+// candidate, the tiles' scratch
+__host__ __device__ inline uint64_t static_end(uint64_t o_tiles, uint64_t n_tiles, uint64_t n, uint64_t words)
+{
+    return align256(align256(align256(o_tiles + n_tiles * 16) + n_tiles * 8) + n * 4) + words * 4;
+}
 
 // counts the candidates into scratch (a PlanSums at its start) and writes the banded
 // ones in tile order (perm, cand_tile) and the indexes of the others to rest and
 // bytes (null: none can come), in no order
 hipError_t launch_plan(const PlanIn &in, const srm_cand *cand, uint32_t n, void *scratch,
                        uint32_t *perm, srm_cand *cand_tile, uint32_t *rest, uint32_t *bytes,
-                       hipStream_t st);
+                       hipStream_t st, const PlanTiles *tiles = nullptr);
 
 }  // namespace srm
