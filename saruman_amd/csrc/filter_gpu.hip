@@ -493,7 +493,7 @@ __device__ __forceinline__ uint32_t pair_list(const FArgs &a, PairRead *list, ui
 // block's reads at once (without those that nothing comes of), starts that fail at
 // the read's ends are dropped before the group's compare, a start is added once, the
 // slots' entries have places of their own, and a block is one wave.  Both strands: 2M
-// reads of 50-250 bp 4.78 -> 2.82 ms, 100,000 of 36 bp 162 -> 83 us, 1,000 of
+// reads of 50-250 bp 4.78 -> 2.60 ms, 100,000 of 36 bp 162 -> 79 us, 1,000 of
 // 36-250 bp 46 -> 22 us (by a thread per read: 21 ms, 1.7 ms for the 1,000).
 template <int G, bool GLOBAL>
 __global__ void __launch_bounds__(PB) fl_pair(Call c_)

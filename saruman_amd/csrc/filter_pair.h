@@ -409,6 +409,13 @@ SRM_HD inline uint32_t chunk_end(const FArgs &a, uint32_t r)
     return list_at(a, a.list_base[next_chunk < a.n_reads ? next_chunk : a.n_reads]);
 }
 
+// |v - (gs + d)| <= lim, for positions v and gs below 2^31 and gs + 1 above -2^16, 0 <= lim
+// < 2^16: modulo 2^32 no other difference comes that near
+SRM_HD inline bool near(uint32_t v, int64_t gs, int d, int lim)
+{
+    return v - (uint32_t)gs - (uint32_t)d + (uint32_t)lim <= 2u * (uint32_t)lim;
+}
+
 // the pair passes of one start position (hash.c:606-794): list aa's element off,
 // value Pa, genome start gs + 1; lb: the read's first list.  Every match raises
 // `possible` and calls add_start_position, which acts only when possible equals
@@ -431,11 +438,16 @@ SRM_HD inline bool pair_matches(const ReadLists &ls, const DParam &P, uint32_t f
         const uint64_t at = (uint64_t)sb + off;
         const uint32_t P0 = at < flat_end ? ls.val((uint32_t)at) : 0u;
         if (P0 == 0) continue;                 // the scan never starts
-        const int64_t rstart = (int64_t)b * q + 1;
+        const int rstart = b * q + 1;
         const uint32_t lo = sb + 1;
+        if (nb - sb == 2) {
+            // a list of one element, nearly every list of a read that maps once: the scan
+            // of the rest is empty
+            if (!near(P0, gs, rstart, k) || ++hits != need) continue;
+        }
         // list b from index 1, or the next list (b + 2 <= half + 1 <= P.n: the read's)
-        const uint32_t hi = (lo < nb ? nb : ls.start(b + 2)) - 1;
-        if (!scan_run(ls, lo, hi, flat_end, gs + rstart - k, gs + rstart + k, true, P0, need, hits))
+        else if (!scan_run(ls, lo, (lo < nb ? nb : ls.start(b + 2)) - 1, flat_end, gs + rstart - k,
+                           gs + rstart + k, true, P0, need, hits))
             continue;
         if (b == half - 1 && fqm) {
             hflag = 1 + dr;
@@ -457,9 +469,13 @@ SRM_HD inline bool pair_matches(const ReadLists &ls, const DParam &P, uint32_t f
     // is negated there)
     for (int j = 0; j < half; ++j) {
         const int lim = half - 1 - j - aa < 0 ? -(half - 1 - j - aa) : half - 1 - j - aa;
-        const int64_t nin = (int64_t)(half - j - 1) * q + 1 + P.rest;
+        const int nin = (half - j - 1) * q + 1 + P.rest;
         const uint32_t lo = ls.start(half + j), hi = ls.start(half + j + 1) - 1;
-        if (!scan_run(ls, lo, hi, flat_end, gs + nin - lim, gs + nin + lim, j - aa >= 0, 0u, need,
+        if (lo == hi) continue;
+        if (hi - lo == 1 && hi <= flat_end) {   // one element: either way the same
+            const uint32_t v = ls.val(lo);
+            if (v == 0 || !near(v, gs, nin, lim) || ++hits != need) continue;
+        } else if (!scan_run(ls, lo, hi, flat_end, gs + nin - lim, gs + nin + lim, j - aa >= 0, 0u, need,
                       hits))
             continue;
         if (j == 0 && fqm) {
