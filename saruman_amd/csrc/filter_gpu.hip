@@ -331,7 +331,7 @@ __global__ void __launch_bounds__(FB) fl_count(Call c_, uint32_t per, uint32_t l
         // (the entries and perfect hits of reads that are run again follow all slots')
         if (threadIdx.x < 6)
             ((uint32_t *)c_.s[blockIdx.y].hdr)[threadIdx.x] =
-                threadIdx.x == 0 ? a.n_reads * ECAP : threadIdx.x == 1 ? a.n_reads * PCAP : 0;
+                threadIdx.x > 1 || a.packed ? 0 : threadIdx.x == 0 ? a.n_reads * ECAP : a.n_reads * PCAP;
         if (threadIdx.x == 0) a.list_cnt[c_.n_lists] = 0;
     }
     const uint32_t nr = s.load(a, per, lo, hi);
@@ -607,8 +607,8 @@ __global__ void __launch_bounds__(PB) fl_pair(Call c_)
         // own places; those of a read run again follow them all
         if (gl == 0) {
             const uint32_t ne = s.ovf ? 0 : s.n, np = s.ovf ? 0 : s.np;
-            const uint32_t be = GLOBAL ? atomicAdd(&a.counters[0], ne) : r * ECAP;
-            const uint32_t bp = GLOBAL ? atomicAdd(&a.counters[1], np) : r * PCAP;
+            const uint32_t be = GLOBAL || a.packed ? atomicAdd(&a.counters[0], ne) : r * ECAP;
+            const uint32_t bp = GLOBAL || a.packed ? atomicAdd(&a.counters[1], np) : r * PCAP;
             for (uint32_t e = 0; e < ne; ++e) {
                 a.out_pos[be + e] = s.P(e);
                 a.out_flag[be + e] = s.F(e);
@@ -1594,6 +1594,8 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     FL_TRY(hipSetDevice(G->device));
     FL_TRY(hipEventRecord(G->ev[0], G->st));
     FArgs a{};
+    // (beyond, the places of all reads leave no 32-bit offsets for the entries behind them)
+    a.packed = n_reads > ((size_t)1 << 27);
     a.qix = G->dq.as<DQ>();
     a.genome = G->genome.as<char>();
     a.glen = G->glen;
@@ -1616,8 +1618,9 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     // in pieces where the reads make two or more
     if (n_reads > PIECE / 4) {
         bool counted = false;
-        FL_RC(upload_pieces(G, c, reads, read_off, read_len, read_k, n_reads, counted));
-        if (counted) {
+        const int rc = upload_pieces(G, c, reads, read_off, read_len, read_k, n_reads, counted);
+        if (rc != SRM_OK && rc != SRM_ENOMEM) return rc;
+        if (rc == SRM_OK && counted) {
             G->last_lists = c.n_lists * (uint64_t)c.n;
             if (words) FL_RC(send_words(G, c.s[0].f, read_off[n_reads - 1] + read_len[n_reads - 1], words));
             return both(c, true);
@@ -1625,6 +1628,8 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
         FL_TRY(hipStreamSynchronize(G->copy_st));
         FL_TRY(hipStreamSynchronize(G->plan_st));
         FL_TRY(hipStreamSynchronize(G->st));
+        if (rc != SRM_OK)   // no memory for the guessed totals: the exact ones take less
+            for (GBuf *b : {&G->in, &G->list_cnt, &G->list_lo, &G->list_start}) b->release();
     }
     ReadPlan plan;
     std::string err;

@@ -58,6 +58,7 @@ struct FArgs {
     // pairing
     const uint32_t *todo;    // reads to pair; null = all reads
     uint32_t n_todo;
+    bool packed;             // entries one after another instead of at the reads' places
     int32_t *slot_pos;       // HBM slots (second and later passes)
     int8_t *slot_flag;
     int32_t *slot_perf;

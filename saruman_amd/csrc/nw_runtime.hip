@@ -1297,6 +1297,7 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
 {
     srm_ctx *ctx = j->ctx;
     HIP_TRY(hipSetDevice(ctx->device));
+    if (j->rest_st) HIP_TRY(hipStreamSynchronize(j->rest_st));   // (a run that failed did not join it)
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     destroy_graph(j);
     j->uploaded = false;
