@@ -3,12 +3,13 @@
 // Same candidates, flags, perfect hits and batch boundaries as the host filter
 // (filter.cpp); only the per-read work moves to the device:
 //   0. pack    the reads' bytes as 2-bit codes and a mask of other bytes;
-//   1. count   one thread per q-gram of a read looks it up in the device copy of
-//              the q-gram index and writes the list length + 1 and the index of
-//              the list's first key;
-//   2. scan    exclusive sum of the lengths = the offset of every 0-terminated
-//              list in one flat array, reads in order (the reference's
-//              data_array, hash.c:396-461, for all chunks at once);
+//   1. count   a lane per q-gram list looks it up in the device copy of the q-gram
+//              index and writes the list length + 1 and the index of the list's
+//              first key;
+//   2. sum     of the lengths = the offset of every 0-terminated list in one flat
+//              array, reads in order (the reference's data_array,
+//              hash.c:396-461, for all chunks at once): a scan, or for small calls
+//              the blocks' sums;
 //   3. fill    the same threads write the lists: a copy of the key run the
 //              count found, or the hash-table lookup again for a q-gram
 //              holding a byte other than ACGT;
@@ -18,14 +19,13 @@
 //              following reads' lists up to the end of the read's chunk of
 //              chunk_value reads (Q12), exactly as a walk of data_array does.
 //              The read's result-hash entries live in LDS (16 entries, 4 perfect
-//              hits per read); a read that needs more is marked and run again
-//              with slots in HBM (1024, then 65534 entries);
-//   5. compact every wave reserves space for its reads' entries with one atomic
-//              and writes them contiguously;
-//   6. batch   the sequential batch pass (Q10 leak, flush boundaries) in parallel:
+//              hits per read) and go to places of its own; a read that needs
+//              more is marked and run again with slots in HBM (1024, then
+//              65534 entries);
+//   5. batch   the sequential batch pass (Q10 leak, flush boundaries) in parallel:
 //              counts per read, their sum, candidates and perfect hits in read
-//              order in one block that the host copies; the host settles the few
-//              reads whose outcome depends on others (filter_batch.h).
+//              order in one block for the host, which settles the few reads
+//              whose outcome depends on others (filter_batch.h).
 // blockIdx.y is the strand: a call of both runs each kernel once.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
@@ -1137,11 +1137,11 @@ int launch_search(srm_dfilter *G, const Call &c)
     if (c.sums) hipLaunchKernelGGL(fl_fill<true>, grid, dim3(FB), 0, G->st, c, per);
     else hipLaunchKernelGGL(fl_fill<false>, grid, dim3(FB), 0, G->st, c, per);
     FL_TRY(hipGetLastError());
-    // lanes per read: a wave for the reads of hundreds of entries (below); 8, about
-    // the start positions of a read that maps once, for many reads; 32 for the few
-    // thousand that leave the chip idle either way, where one step covers a read's
-    // lists (1,000 reads, both strands: 0.373 ms on the device with 32, 0.414 with 8;
-    // 2M reads: 38.1 and 32.2 ms)
+    // lanes per read: a wave for the reads of hundreds of entries (run_overflow); 8, about
+    // the start positions of a read that maps once, for many reads (2M reads, both
+    // strands: 2.82 ms with 8, 3.04 with 16); 32 for the few thousand that leave the chip
+    // idle either way, where one step covers a read's lists (1,000 reads, the whole
+    // filter's kernels with a thread's chain of loads: 0.373 ms with 32, 0.414 with 8)
     auto pgrid = [&](uint32_t reads) { return dim3((n + reads - 1) / reads, (unsigned)c.n); };
     if (n < 4096)
         hipLaunchKernelGGL((fl_pair<32, false>), pgrid(pair_reads(32)), dim3(PB), 0, G->st, c);
@@ -1475,7 +1475,7 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
 //
 // Bound by the copy of the reads (57 GB/s from page-locked memory).  With the plan made
 // before it and the lookups after it, 2M reads of 143 bp took 3.5 + 6.6 + 2.9 ms; in
-// pieces 5.9 ms.
+// pieces 6.5 ms.
 int upload_pieces(srm_dfilter *G, Call &c, const char *reads, const uint64_t *read_off,
                   const uint16_t *read_len, const uint8_t *read_k, size_t n, bool &counted)
 {

@@ -38,11 +38,13 @@ def placed(reads, order, gap):
     ("ragged", 2 * PIECE + 4_097, 36, 120), ("backwards", PIECE + 999, 36, 90),
     ("shuffled", PIECE + 999, 36, 90), ("gaps", PIECE + 999, 36, 90),
     ("by_length", PIECE * 2 + 5, 36, 200), ("bad_sample", PIECE * 2 + 5, 36, 200),
-    ("others", PIECE + 7, 36, 90)])
+    ("others", PIECE + 7, 36, 90), ("repeats", PIECE + 7, 40, 60)])
 def test_pieces(name, n, lo, hi):
     print(f"[gpu] filter pieces {name}", flush=True)
     rng = np.random.default_rng(5)
-    genome = wl.synth_genome(91, [60_000], 0.5, (3, 300, 600, 10, 0.5, 0.001) if name == "others" else None)
+    # (the lists of "repeats" outgrow the room they are first given)
+    families = {"others": (3, 300, 600, 10, 0.5, 0.001), "repeats": (3, 300, 600, 60, 0.5, 0.001)}
+    genome = wl.synth_genome(91, [60_000], 0.5, families.get(name))
     reads = wl.synth_reads(92, genome, n, lo, hi, 1, p_sub=0.01, p_ins=0.001, indel_max=2, k_rate=0.05)
     if name == "others":
         seq = np.frombuffer(reads.seq, np.uint8).copy()
@@ -72,6 +74,8 @@ def test_pieces(name, n, lo, hi):
         want = {dr: wl.run_filter(idx, genome, reads, dr, 20_000) for dr in (0, 4)}
         for dr, d in zip((0, 4), df.run_both(reads, 20_000)):
             same(want[dr], d, (name, dr))
+        if name == "repeats":
+            assert df.stats()["list_entries"] > 2 * df.stats()["lists"] + 2048
         if name == "ragged":
             for dr in (4, 0):
                 same(want[dr], df.run(reads, dr, 20_000), (name, "one strand", dr))
