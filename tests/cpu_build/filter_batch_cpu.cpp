@@ -4,7 +4,7 @@
 // kernels' parts run here as plain loops.  TEST INFRASTRUCTURE ONLY.
 //
 // usage: filter_batch_cpu seed cases [plant] -> one line, exit status 1 on a difference;
-// "plant" gives the checker's pass another chunk value, which the comparison must report
+// "plant" gives the expected pass another chunk value, which the comparison must report
 #include <stdio.h>
 #include <stdlib.h>
 
