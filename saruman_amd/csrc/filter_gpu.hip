@@ -154,8 +154,10 @@ struct Header {
     uint32_t counters[3];    // entries, perfect hits, reads that outgrew their slots
     uint32_t n_unsafe, walk_words;
     uint32_t n_flush;        // MAX_FLUSH + 1: more
+    uint32_t wrapped;        // 1: more list entries than 32 bits count (list_fits)
     uint32_t flat;           // list entries (terminators included)
     uint32_t blob_ok;        // the output fitted
+    uint32_t pad[3];
     Counts total;
     Flush flush[MAX_FLUSH];
 };
@@ -165,7 +167,7 @@ static_assert(sizeof(Header) % 16 == 0, "the output behind it is read 16 bytes a
 struct Strand {
     FArgs f;
     Header *hdr;
-    uint64_t flat_cap;       // entries that flat holds
+    uint64_t flat_cap;       // entries that flat holds, MAX_FLAT at most
     Counts *cnt, *start;     // [n_reads + 1] per read; summed over the reads before
     uint32_t *list_sum;      // small calls: the sums of fl_count's and fl_batch_count's
     Counts *cnt_sum;         // blocks
@@ -190,13 +192,13 @@ struct Call {
 };
 
 // a strand's arguments; false when its lists do not fit (the host makes room and
-// runs the call again)
+// runs the call again) or are more than can be
 __device__ __forceinline__ bool strand_of(const Call &c, FArgs &a)
 {
     const Strand &s = c.s[blockIdx.y];
     a = s.f;
     a.list_org = a.list_start[0];
-    return (uint64_t)list_at(a, c.n_lists) <= s.flat_cap;
+    return !s.hdr->wrapped && (uint64_t)list_at(a, c.n_lists) <= s.flat_cap;
 }
 
 // One thread per q-gram list; a block takes the lists of `per` consecutive reads,
@@ -329,7 +331,7 @@ __global__ void __launch_bounds__(FB) fl_count(Call c_, uint32_t per, uint32_t l
     const FArgs &a = c_.s[blockIdx.y].f;
     if (blockIdx.x == 0 && hi == a.n_reads) {   // what later kernels of the call add to
         // (the entries and perfect hits of reads that are run again follow all slots')
-        if (threadIdx.x < 6)
+        if (threadIdx.x < 7)
             ((uint32_t *)c_.s[blockIdx.y].hdr)[threadIdx.x] =
                 threadIdx.x > 1 || a.packed ? 0 : threadIdx.x == 0 ? a.n_reads * ECAP : a.n_reads * PCAP;
         if (threadIdx.x == 0) a.list_cnt[c_.n_lists] = 0;
@@ -357,8 +359,8 @@ __global__ void __launch_bounds__(FB) fl_fill(Call c_, uint32_t per)
     FArgs a;
     uint32_t before[1] = {0}, total[1];
     bool fits = true;
+    const Strand &st = c_.s[blockIdx.y];
     if (SUMS) {
-        const Strand &st = c_.s[blockIdx.y];
         a = st.f;
         a.list_org = 0;
         sums_before<1>(st.list_sum, gridDim.x, before, total);
@@ -372,6 +374,10 @@ __global__ void __launch_bounds__(FB) fl_fill(Call c_, uint32_t per)
         const uint32_t c = a.list_cnt[i] - 1, at = list_at(a, i) + before[0];
         if (SUMS) ((uint32_t *)a.list_start)[i] = at;
         if (!fits) continue;
+        if (!list_fits(at, c + 1, st.flat_cap)) {
+            st.hdr->wrapped = 1;
+            continue;
+        }
         uint32_t *dst = a.flat + at;
         if (c) {
             const uint32_t lo = a.list_lo[i], t = s.read_of(i, nr);
@@ -1195,8 +1201,11 @@ int run_overflow(srm_dfilter *G, const Call &call, int x, Header &h)
         const uint32_t per = (uint32_t)std::max<size_t>(1, ((size_t)256 << 20) / ((size_t)cap * 9));
         FL_RC(G->over[x][1 - from].ensure((size_t)left * 4));
         FL_TRY(srm::launch_reset(a.counters + 2, 1, G->st));
-        for (uint32_t b = 0; b < left; b += per) {
-            const uint32_t m = std::min(per, left - b);
+        for (uint32_t b = 0, m; b < left; b += m) {
+            // (the entries' offsets are 32 bits)
+            m = (uint32_t)std::min<uint64_t>(std::min(per, left - b),
+                                             (~0u - std::max(h.counters[0], h.counters[1])) / cap);
+            if (m == 0) return srm::set_error(SRM_ENOMEM, "too many filter entries; split the call");
             FL_RC(G->slot_pos.ensure((size_t)m * cap * 4));
             FL_RC(G->slot_flag.ensure((size_t)m * cap));
             FL_RC(G->slot_perf.ensure((size_t)m * cap * 4));
@@ -1297,7 +1306,7 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
         for (int x = 0; x < c.n; ++x) {
             Strand &s = c.s[x];
             FArgs &a = s.f;
-            s.flat_cap = G->flat[x].cap / 4;
+            s.flat_cap = std::min<uint64_t>(G->flat[x].cap / 4, MAX_FLAT);
             s.cnt = G->cnt.as<Counts>() + (size_t)x * ((size_t)n + 1);
             s.start = G->start.as<Counts>() + (size_t)x * ((size_t)n + 1);
             s.by_rank = G->by_rank.as<uint32_t>() + (size_t)x * n;
@@ -1340,6 +1349,14 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
         FL_TRY(hipGetLastError());
     }
     FL_RC(fetch());
+    auto countable = [&]() -> int {
+        for (int x = 0; x < c.n; ++x)
+            if (h[x].wrapped)
+                return srm::set_error(SRM_ENOMEM, "the q-gram lists of %u reads hold more than %llu "
+                                      "positions; split the call", n, (unsigned long long)MAX_FLAT);
+        return SRM_OK;
+    };
+    FL_RC(countable());
     bool again = false;
     for (int x = 0; x < c.n; ++x)
         if ((uint64_t)h[x].flat > c.s[x].flat_cap) {
@@ -1352,6 +1369,7 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
         FL_RC(launch_search(G, c));
         if (on_device) FL_RC(launch_batch(G, c));
         FL_RC(fetch());
+        FL_RC(countable());
     }
     again = false;
     for (int x = 0; x < c.n; ++x) {

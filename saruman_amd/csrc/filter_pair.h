@@ -83,6 +83,15 @@ struct FArgs {
 // where list i starts in flat
 SRM_HD inline uint32_t list_at(const FArgs &a, uint64_t i) { return a.list_start[i] - a.list_org; }
 
+// The starts are sums modulo 2^32, and so is a strand's total, which says whether its
+// lists fit: a total past 2^32 may say so wrongly.  Until the true sum passes 2^32 every
+// start is true, so the list at which it does is one that ends past any room below 2^32:
+// a list that does not fit where the total does means that the total is not true.  A
+// strand's room is at most MAX_FLAT elements (a wave's steps past the last one must not
+// wrap either)
+constexpr uint64_t MAX_FLAT = 0xFFFFFF00ull;
+SRM_HD inline bool list_fits(uint32_t at, uint32_t len, uint64_t room) { return (uint64_t)at + len <= room; }
+
 SRM_HD inline char dcomp(char c)
 {
     switch (c) {
