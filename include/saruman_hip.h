@@ -220,6 +220,9 @@ int srm_ctx_set_pool_cap(srm_ctx *ctx, size_t pool_cap_bytes);
 /* testing hook for the failure paths: the next `count` device allocations of
  * any context fail with SRM_ENOMEM (0 clears) */
 void srm_debug_fail_allocs(int count);
+/* likewise for a device filter's buffers: `after` of their allocations succeed, the
+ * next `count` fail as on a device without memory (count 0 clears) */
+void srm_debug_fail_filter_allocs(int after, int count);
 
 /*
  * Keep a packed genome resident on the device (uploaded once).  words/n_words

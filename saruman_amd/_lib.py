@@ -41,6 +41,7 @@ _PROTOS = [
     ("srm_ctx_pool_used", C.c_size_t, [_vp]),
     ("srm_ctx_set_pool_cap", C.c_int, [_vp, C.c_size_t]),
     ("srm_debug_fail_allocs", None, [C.c_int]),
+    ("srm_debug_fail_filter_allocs", None, [C.c_int, C.c_int]),
     ("srm_ctx_set_genome", C.c_int, [_vp, _vp, C.c_size_t]),
     ("srm_job_create", C.c_int, [_vp, C.POINTER(_vp)]),
     ("srm_job_destroy", None, [_vp]),

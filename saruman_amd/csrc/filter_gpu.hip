@@ -42,6 +42,7 @@
 #include <thread>
 #include <vector>
 
+#include "alloc.h"
 #include "filter_batch.h"
 #include "filter_internal.h"
 #include "filter_pair.h"
@@ -895,12 +896,10 @@ struct GBuf {
         p = nullptr;
         cap = 0;
         size_t want = (std::max(bytes, (size_t)256) + 4095) & ~(size_t)4095;
-        hipError_t e = hipMalloc(&p, want);
-        if (e != hipSuccess) {
-            p = nullptr;
+        const hipError_t e = srm::device_alloc(&p, srm::filter_alloc_fails() ? srm::NO_DEVICE_HAS : want);
+        if (e != hipSuccess)
             return srm::set_error(SRM_ENOMEM, "hipMalloc(%zu) failed: %s", want,
                                   hipGetErrorString(e));
-        }
         cap = want;
         return SRM_OK;
     }
@@ -960,8 +959,7 @@ public:
         }
         if (make) {
             b.bytes = bytes + bytes / 4 + 4096;
-            if (hipHostMalloc(&b.p, b.bytes, hipHostMallocDefault) != hipSuccess) {
-                b.p = nullptr;
+            if (srm::host_alloc(&b.p, b.bytes) != hipSuccess) {
                 std::lock_guard<std::mutex> lk(mu_);
                 --made_;
             }
@@ -1808,9 +1806,9 @@ int srm_dfilter_create(srm_ctx *ctx, const srm_index *ix, const char *genome, si
         hipStreamCreateWithFlags(&G->plan_st, hipStreamNonBlocking) != hipSuccess ||
         hipStreamCreateWithFlags(&G->copy_st, hipStreamNonBlocking) != hipSuccess)
         return fail(srm::set_error(SRM_EDEVICE, "event creation failed"));
-    if (hipHostMalloc(&G->stage_in, STAGE_IN, hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc(&G->stage_plan, 2 * PIECE_BYTES, hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc(&G->stage_out, 2 * sizeof(Header) + STAGE_OUT, hipHostMallocDefault) != hipSuccess)
+    if (srm::host_alloc(&G->stage_in, STAGE_IN) != hipSuccess ||
+        srm::host_alloc(&G->stage_plan, 2 * PIECE_BYTES) != hipSuccess ||
+        srm::host_alloc(&G->stage_out, 2 * sizeof(Header) + STAGE_OUT) != hipSuccess)
         return fail(srm::set_error(SRM_ENOMEM, "no page-locked memory for the filter's staging"));
     int rc = G->upload(G->genome, genome, glen);
     if (!rc) rc = G->pack(G->genome.p, glen, G->gen_pk, G->gen_odd);

@@ -18,6 +18,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "alloc.h"
 #include "nw_device.h"
 #include "plan.h"
 #include "saruman_hip.h"
@@ -70,8 +71,10 @@ struct DevBuf {
     size_t cap = 0;
 };
 
-// allocations that are made to fail (srm_debug_fail_allocs), process-wide
+// allocations that are made to fail (srm_debug_fail_allocs,
+// srm_debug_fail_filter_allocs), process-wide
 std::atomic<int> g_fail_allocs{0};
+std::atomic<int> g_filter_allocs_left{0}, g_fail_filter_allocs{0};
 
 }  // namespace
 
@@ -96,8 +99,11 @@ struct srm_ctx {
     {
         if (bytes <= b.cap) return SRM_OK;
         for (int f = g_fail_allocs.load(); f > 0;)
-            if (g_fail_allocs.compare_exchange_weak(f, f - 1))
+            if (g_fail_allocs.compare_exchange_weak(f, f - 1)) {
+                void *none = nullptr;
+                (void)srm::device_alloc(&none, srm::NO_DEVICE_HAS);
                 return fail(SRM_ENOMEM, "injected allocation failure (%zu bytes)", bytes);
+            }
         // under a pool cap a buffer grows to exactly its 4 KiB-rounded need (what
         // srm_job_bytes_bound counts); otherwise by half again, for fewer regrowths
         size_t want = pool_cap ? bytes : std::max(bytes, b.cap + b.cap / 2);
@@ -114,11 +120,9 @@ struct srm_ctx {
             b.p = nullptr;
             b.cap = 0;
         }
-        hipError_t e = hipMalloc(&b.p, want);
-        if (e != hipSuccess) {
-            b.p = nullptr;
+        const hipError_t e = srm::device_alloc(&b.p, want);
+        if (e != hipSuccess)
             return fail(SRM_ENOMEM, "hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
-        }
         b.cap = want;
         pool_used += want;
         return SRM_OK;
@@ -980,6 +984,13 @@ int set_error(int code, const char *fmt, ...)
     return code;
 }
 
+bool filter_alloc_fails()
+{
+    if (g_fail_filter_allocs.load() <= 0) return false;
+    if (g_filter_allocs_left.fetch_sub(1) > 0) return false;
+    return g_fail_filter_allocs.fetch_sub(1) > 0;
+}
+
 int ctx_device(const srm_ctx *c) { return c->device; }
 
 hipStream_t ctx_stream(const srm_ctx *c) { return c->stream; }
@@ -1014,7 +1025,7 @@ int srm_device_count(void)
 void *srm_host_alloc(size_t bytes)
 {
     void *p = nullptr;
-    if (hipHostMalloc(&p, bytes ? bytes : 1, hipHostMallocDefault) != hipSuccess) {
+    if (srm::host_alloc(&p, bytes ? bytes : 1) != hipSuccess) {
         fail(SRM_ENOMEM, "hipHostMalloc(%zu) failed", bytes);
         return nullptr;
     }
@@ -1139,7 +1150,7 @@ int srm_job_create(srm_ctx *ctx, srm_job **out)
     for (auto &e : j->ce) ok = ok && hipEventCreate(&e) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&j->fork_ev, hipEventDisableTiming) == hipSuccess;
     for (auto &e : j->join_ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-    ok = ok && hipHostMalloc((void **)&j->stage, JOB_STAGE + 16, hipHostMallocDefault) == hipSuccess;
+    ok = ok && srm::host_alloc((void **)&j->stage, JOB_STAGE + 16) == hipSuccess;
     j->back = (uint64_t *)(j->stage + JOB_STAGE);
     if (!ok) {
         srm_job_destroy(j);
@@ -1191,6 +1202,13 @@ int srm_ctx_set_pool_cap(srm_ctx *c, size_t bytes)
 }
 
 void srm_debug_fail_allocs(int count) { g_fail_allocs.store(count < 0 ? 0 : count); }
+
+void srm_debug_fail_filter_allocs(int after, int count)
+{
+    g_fail_filter_allocs.store(0);
+    g_filter_allocs_left.store(after < 0 ? 0 : after);
+    g_fail_filter_allocs.store(count < 0 ? 0 : count);
+}
 
 void srm_job_destroy(srm_job *j)
 {
@@ -1687,8 +1705,8 @@ int srm_calibrate_copy(int device, size_t bytes, float *ms)
     HIP_TRY(hipSetDevice(device));
     bytes &= ~(size_t)15;
     void *a = nullptr, *b = nullptr;
-    HIP_TRY(hipMalloc(&a, bytes));
-    hipError_t e = hipMalloc(&b, bytes);
+    HIP_TRY(srm::device_alloc(&a, bytes));
+    hipError_t e = srm::device_alloc(&b, bytes);
     if (e != hipSuccess) {
         (void)hipFree(a);
         return fail(SRM_ENOMEM, "hipMalloc(%zu) failed", bytes);
@@ -1843,7 +1861,7 @@ void cuda_allocate_memory(int do_reverse)
     char **anchor = which ? &main_alloc_ptr_rev : &main_alloc_ptr_for;
     if (!*anchor) {
         (void)hipSetDevice(c->device);
-        if (hipMalloc((void **)anchor, 256) != hipSuccess) *anchor = nullptr;
+        (void)srm::device_alloc((void **)anchor, 256);
     }
 }
 
