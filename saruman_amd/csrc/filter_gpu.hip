@@ -31,6 +31,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
+#include <array>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -886,6 +887,10 @@ __global__ void __launch_bounds__(FB) fl_batch_end(Call c)
     send_back(c, b.bytes <= c.blob_cap ? b.bytes : ~0ull);
 }
 
+// GBuf::ensure's SRM_ENOMEM, as which it leaves this file: a call that needs less may
+// still do
+constexpr int NO_ROOM = -1000;
+
 struct GBuf {
     void *p = nullptr;
     size_t cap = 0;
@@ -898,8 +903,7 @@ struct GBuf {
         size_t want = (std::max(bytes, (size_t)256) + 4095) & ~(size_t)4095;
         const hipError_t e = srm::device_alloc(&p, srm::filter_alloc_fails() ? srm::NO_DEVICE_HAS : want);
         if (e != hipSuccess)
-            return srm::set_error(SRM_ENOMEM, "hipMalloc(%zu) failed: %s", want,
-                                  hipGetErrorString(e));
+            return srm::set_error(NO_ROOM, "hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
         cap = want;
         return SRM_OK;
     }
@@ -1026,16 +1030,23 @@ struct srm_dfilter {
     float last_ms = 0.f;
     size_t last_lists = 0, last_flat = 0, last_overflow = 0;
 
-    ~srm_dfilter()
+    // the buffers of a call beside its inputs
+    void release_strands()
     {
-        for (GBuf *b : {&genome, &gen_pk, &gen_odd, &dq, &in, &read_pk, &read_odd, &words, &sums, &blocked, &list_cnt,
-                        &list_lo, &list_start, &cub_tmp, &cnt, &start, &by_rank, &unsafe, &walk, &out,
-                        &slot_pos, &slot_flag, &slot_perf})
+        for (GBuf *b : {&sums, &blocked, &list_cnt, &list_lo, &list_start, &cub_tmp, &cnt, &start, &by_rank,
+                        &unsafe, &walk, &out, &slot_pos, &slot_flag, &slot_perf})
             b->release();
         for (int s = 0; s < 2; ++s)
             for (GBuf *b : {&flat[s], &out_pos[s], &out_flag[s], &out_perf[s], &meta[s], &over[s][0],
                             &over[s][1]})
                 b->release();
+        last_flat = last_overflow = 0;
+    }
+
+    ~srm_dfilter()
+    {
+        release_strands();
+        for (GBuf *b : {&genome, &gen_pk, &gen_odd, &dq, &in, &read_pk, &read_odd, &words}) b->release();
         for (auto *v : {&keys, &pre, &odd_hash, &odd_pos})
             for (auto &b : *v) b.release();
         if (stage_in) (void)hipHostFree(stage_in);
@@ -1266,10 +1277,13 @@ void bind_lists(const srm_dfilter *G, Call &c)
     }
 }
 
+// where the results of a call's strands go, in their order
+using Outs = std::array<srm_filter **, 2>;
+
 // one or both strands over the reads on the device (both while their lists fit one sum);
 // counted: their lookups are under way (upload_pieces)
 int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, const uint16_t *read_len,
-                const uint8_t *read_k, srm_filter **out)
+                const uint8_t *read_k, const Outs &out)
 {
     const uint64_t nl = c.n_lists;
     const uint32_t n = c.s[0].f.n_reads;
@@ -1408,7 +1422,7 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
         }
         FL_TRY(hipStreamSynchronize(G->st));
         auto pass = [&](int x) {
-            out[x] = batch_pass(MetaAcc{meta_h[x], pos_h[x], flag_h[x], perf_h[x]}, n, read_len, read_k,
+            *out[x] = batch_pass(MetaAcc{meta_h[x], pos_h[x], flag_h[x], perf_h[x]}, n, read_len, read_k,
                                 G->glen, blocked, (int)c.s[0].f.cv);
         };
         std::thread other;   // the two strands' passes side by side
@@ -1479,7 +1493,7 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
         R.n_perf = h[x].total.perf;
         finish(R, F->batch_end, std::vector<Flush>(h[x].flush, h[x].flush + h[x].n_flush), walked,
                read_len, read_k, G->glen, blocked);
-        out[x] = F.release();
+        *out[x] = F.release();
     }
     return SRM_OK;
 }
@@ -1619,14 +1633,7 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     a.gen_odd = G->gen_odd.as<uint32_t>();
     a.n_reads = (uint32_t)n_reads;
     a.cv = (uint32_t)chunk_value;
-    srm_filter **outs[2] = {out_fwd, out_rev};
-    auto both = [&](Call &c, bool counted) -> int {
-        srm_filter *F[2] = {nullptr, nullptr};
-        const int rc = run_strands(G, c, counted, blocked, read_len, read_k, F);
-        *outs[strands == 2 ? 1 : 0] = F[0];
-        if (strands == 3) *out_rev = F[1];
-        return rc;
-    };
+    const Outs outs = strands == 2 ? Outs{out_rev, nullptr} : Outs{out_fwd, out_rev};
     Call c{};
     c.n = strands == 3 ? 2 : 1;
     c.s[0].f = a;
@@ -1634,18 +1641,20 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     // in pieces where the reads make two or more
     if (n_reads > PIECE / 4) {
         bool counted = false;
-        const int rc = upload_pieces(G, c, reads, read_off, read_len, read_k, n_reads, counted);
-        if (rc != SRM_OK && rc != SRM_ENOMEM) return rc;
+        int rc = upload_pieces(G, c, reads, read_off, read_len, read_k, n_reads, counted);
         if (rc == SRM_OK && counted) {
             G->last_lists = c.n_lists * (uint64_t)c.n;
-            if (words) FL_RC(send_words(G, c.s[0].f, read_off[n_reads - 1] + read_len[n_reads - 1], words));
-            return both(c, true);
+            if (words) rc = send_words(G, c.s[0].f, read_off[n_reads - 1] + read_len[n_reads - 1], words);
+            if (rc == SRM_OK) rc = run_strands(G, c, true, blocked, read_len, read_k, outs);
         }
+        if (rc != NO_ROOM && (rc != SRM_OK || counted)) return rc;
         FL_TRY(hipStreamSynchronize(G->copy_st));
         FL_TRY(hipStreamSynchronize(G->plan_st));
         FL_TRY(hipStreamSynchronize(G->st));
-        if (rc != SRM_OK)   // no memory for the guessed totals: the exact ones take less
-            for (GBuf *b : {&G->in, &G->list_cnt, &G->list_lo, &G->list_start}) b->release();
+        if (rc == NO_ROOM) {   // for the guessed totals: the exact ones take less
+            G->release_strands();
+            for (GBuf *b : {&G->in, &G->read_pk, &G->read_odd, &G->words}) b->release();
+        }
     }
     ReadPlan plan;
     std::string err;
@@ -1709,14 +1718,18 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
         c.n = 2;
         c.s[0].f = c.s[1].f = a;
         c.s[1].f.dr = 4;
-        return both(c, false);
+        const int rc = run_strands(G, c, false, blocked, read_len, read_k, outs);
+        if (rc != NO_ROOM) return rc;
+        // one strand at a time holds half as much
+        FL_TRY(hipStreamSynchronize(G->st));
+        G->release_strands();
     }
     for (int x = 0; x < 2; ++x) {
         if (!(strands & (1 << x))) continue;
         c.n = 1;
         c.s[0].f = a;
         c.s[0].f.dr = x ? 4 : 0;
-        FL_RC(run_strands(G, c, false, blocked, read_len, read_k, outs[x]));
+        FL_RC(run_strands(G, c, false, blocked, read_len, read_k, {x ? out_rev : out_fwd, nullptr}));
     }
     return SRM_OK;
 }
@@ -1736,6 +1749,7 @@ int run_call(srm_dfilter *G, const uint8_t *blocked, const char *reads, const ui
     } catch (const std::bad_alloc &) {
         rc = srm::set_error(SRM_ENOMEM, "no memory on the host for %zu reads", n_reads);
     }
+    if (rc == NO_ROOM) rc = SRM_ENOMEM;
     if (rc != SRM_OK) {
         (void)hipStreamSynchronize(G->copy_st);
         (void)hipStreamSynchronize(G->plan_st);
@@ -1794,7 +1808,7 @@ int srm_dfilter_create(srm_ctx *ctx, const srm_index *ix, const char *genome, si
     G->glen = glen;
     auto fail = [&](int rc) {
         delete G;
-        return rc;
+        return rc == NO_ROOM ? SRM_ENOMEM : rc;
     };
     if (hipSetDevice(G->device) != hipSuccess ||
         hipEventCreate(&G->ev[0]) != hipSuccess || hipEventCreate(&G->ev[1]) != hipSuccess ||
