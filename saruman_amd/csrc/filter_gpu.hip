@@ -615,8 +615,8 @@ __global__ void __launch_bounds__(PB) fl_pair(Call c_)
         // own places; those of a read run again follow them all
         if (gl == 0) {
             const uint32_t ne = s.ovf ? 0 : s.n, np = s.ovf ? 0 : s.np;
-            const uint32_t be = GLOBAL || a.packed ? atomicAdd(&a.counters[0], ne) : r * ECAP;
-            const uint32_t bp = GLOBAL || a.packed ? atomicAdd(&a.counters[1], np) : r * PCAP;
+            const uint32_t be = !GLOBAL && !a.packed ? r * ECAP : ne ? atomicAdd(&a.counters[0], ne) : 0;
+            const uint32_t bp = !GLOBAL && !a.packed ? r * PCAP : np ? atomicAdd(&a.counters[1], np) : 0;
             for (uint32_t e = 0; e < ne; ++e) {
                 a.out_pos[be + e] = s.P(e);
                 a.out_flag[be + e] = s.F(e);
@@ -1280,6 +1280,17 @@ void bind_lists(const srm_dfilter *G, Call &c)
 // where the results of a call's strands go, in their order
 using Outs = std::array<srm_filter **, 2>;
 
+// The batch pass runs on the device unless separators have to come along that outweigh
+// it (a byte a base at 20 GB/s; the host's pass takes tens of nanoseconds a read), or its
+// lists of flushes and walked reads run over (run_strands): then the host's pass over the
+// downloaded entries, which come down one after another.  (From the reads' own places
+// they are 80 bytes a read and strand, empty or not: 100,000 reads over 60 Mbp in two
+// contigs 10.4 ms, 7.8 packed; 500,000 over 4 Mbp with a flush at every 100, 34.7 and 18.6)
+bool batch_on_device(const srm_dfilter *G, const uint8_t *blocked, size_t n_reads)
+{
+    return !blocked || G->glen / 512 <= n_reads;
+}
+
 // one or both strands over the reads on the device (both while their lists fit one sum);
 // counted: their lookups are under way (upload_pieces)
 int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, const uint16_t *read_len,
@@ -1287,11 +1298,7 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
 {
     const uint64_t nl = c.n_lists;
     const uint32_t n = c.s[0].f.n_reads;
-    // the batch pass runs on the device unless separators have to come along that
-    // outweigh it (a byte a base at 20 GB/s; the host's pass takes tens of nanoseconds a
-    // read and 160 bytes of slots come down for it), or its lists of flushes and walked
-    // reads run over (below): then the host's pass over the downloaded entries
-    bool on_device = !blocked || G->glen / 512 <= n;
+    bool on_device = batch_on_device(G, blocked, n);
     if (on_device && blocked) {
         FL_RC(G->upload(G->blocked, blocked, G->glen));
         c.blocked = G->blocked.as<uint8_t>();
@@ -1384,14 +1391,19 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
         FL_RC(countable());
     }
     again = false;
+    auto overflow = [&]() -> int {
+        for (int x = 0; x < c.n; ++x)
+            if (h[x].counters[2]) {
+                FL_RC(run_overflow(G, c, x, h[x]));
+                again = true;
+            }
+        return SRM_OK;
+    };
     for (int x = 0; x < c.n; ++x) {
         G->last_flat += h[x].flat;
         G->last_overflow += h[x].counters[2];
-        if (h[x].counters[2]) {
-            FL_RC(run_overflow(G, c, x, h[x]));
-            again = true;
-        }
     }
+    FL_RC(overflow());
     // the counters of the reads the batch pass lists start over
     auto batch_again = [&]() -> int {
         bind();
@@ -1410,6 +1422,14 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
     for (int x = 0; x < c.n; ++x)
         if (h[x].n_flush > MAX_FLUSH || h[x].n_unsafe > MAX_UNSAFE || h[x].walk_words > MAX_WALK)
             on_device = false;
+    if (!on_device && !c.s[0].f.packed) {
+        for (int x = 0; x < c.n; ++x) c.s[x].f.packed = true;
+        bind();
+        FL_RC(launch_count(G, c, 0, n));   // (the counters start over)
+        FL_RC(launch_search(G, c));
+        FL_RC(fetch());
+        FL_RC(overflow());
+    }
     if (!on_device) {
         std::vector<uint32_t> meta_h[2];
         std::vector<int32_t> pos_h[2], perf_h[2];
@@ -1624,8 +1644,9 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     FL_TRY(hipSetDevice(G->device));
     FL_TRY(hipEventRecord(G->ev[0], G->st));
     FArgs a{};
-    // (beyond, the places of all reads leave no 32-bit offsets for the entries behind them)
-    a.packed = n_reads > ((size_t)1 << 27);
+    // (beyond 2^27, the places of all reads leave no 32-bit offsets for the entries behind
+    // them; and the host takes the entries alone)
+    a.packed = n_reads > ((size_t)1 << 27) || !batch_on_device(G, blocked, n_reads);
     a.qix = G->dq.as<DQ>();
     a.genome = G->genome.as<char>();
     a.glen = G->glen;
