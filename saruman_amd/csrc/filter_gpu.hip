@@ -156,10 +156,8 @@ struct Header {
     uint32_t counters[3];    // entries, perfect hits, reads that outgrew their slots
     uint32_t n_unsafe, walk_words;
     uint32_t n_flush;        // MAX_FLUSH + 1: more
-    uint32_t wrapped;        // 1: more list entries than 32 bits count (list_fits)
-    uint32_t flat;           // list entries (terminators included)
+    uint32_t flat;           // list entries (terminators included; TOO_MANY)
     uint32_t blob_ok;        // the output fitted
-    uint32_t pad[3];
     Counts total;
     Flush flush[MAX_FLUSH];
 };
@@ -193,14 +191,18 @@ struct Call {
     uint64_t back_cap;       // back_cap bytes, the blob
 };
 
+// the total in place of one that 32 bits do not hold: no room has as much
+constexpr uint32_t TOO_MANY = ~0u;
+static_assert(TOO_MANY > MAX_FLAT, "");
+
 // a strand's arguments; false when its lists do not fit (the host makes room and
-// runs the call again) or are more than can be
+// runs the call again, or refuses it)
 __device__ __forceinline__ bool strand_of(const Call &c, FArgs &a)
 {
     const Strand &s = c.s[blockIdx.y];
     a = s.f;
     a.list_org = a.list_start[0];
-    return !s.hdr->wrapped && (uint64_t)list_at(a, c.n_lists) <= s.flat_cap;
+    return (uint64_t)list_at(a, c.n_lists) <= s.flat_cap;
 }
 
 // One thread per q-gram list; a block takes the lists of `per` consecutive reads,
@@ -333,10 +335,13 @@ __global__ void __launch_bounds__(FB) fl_count(Call c_, uint32_t per, uint32_t l
     const FArgs &a = c_.s[blockIdx.y].f;
     if (blockIdx.x == 0 && hi == a.n_reads) {   // what later kernels of the call add to
         // (the entries and perfect hits of reads that are run again follow all slots')
-        if (threadIdx.x < 7)
+        if (threadIdx.x < 6)
             ((uint32_t *)c_.s[blockIdx.y].hdr)[threadIdx.x] =
                 threadIdx.x > 1 || a.packed ? 0 : threadIdx.x == 0 ? a.n_reads * ECAP : a.n_reads * PCAP;
-        if (threadIdx.x == 0) a.list_cnt[c_.n_lists] = 0;
+        if (threadIdx.x == 0) {
+            a.list_cnt[c_.n_lists] = 0;
+            if (SUMS) ((uint32_t *)a.list_start)[c_.n_lists] = 0;   // (fl_fill's maximum)
+        }
     }
     const uint32_t nr = s.load(a, per, lo, hi);
     uint32_t carry = 0;
@@ -367,7 +372,8 @@ __global__ void __launch_bounds__(FB) fl_fill(Call c_, uint32_t per)
         a.list_org = 0;
         sums_before<1>(st.list_sum, gridDim.x, before, total);
         fits = total[0] <= st.flat_cap;
-        if (threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) ((uint32_t *)a.list_start)[c_.n_lists] = total[0];
+        if (threadIdx.x == 0 && blockIdx.x == gridDim.x - 1)
+            atomicMax((uint32_t *)a.list_start + c_.n_lists, total[0]);
     } else if (!strand_of(c_, a)) {
         return;
     }
@@ -377,7 +383,8 @@ __global__ void __launch_bounds__(FB) fl_fill(Call c_, uint32_t per)
         if (SUMS) ((uint32_t *)a.list_start)[i] = at;
         if (!fits) continue;
         if (!list_fits(at, c + 1, st.flat_cap)) {
-            st.hdr->wrapped = 1;
+            if (SUMS) atomicMax((uint32_t *)a.list_start + c_.n_lists, TOO_MANY);
+            else ((uint32_t *)a.list_start)[c_.n_lists] = a.list_org + TOO_MANY;
             continue;
         }
         uint32_t *dst = a.flat + at;
@@ -1370,7 +1377,7 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
     FL_RC(fetch());
     auto countable = [&]() -> int {
         for (int x = 0; x < c.n; ++x)
-            if (h[x].wrapped)
+            if (h[x].flat == TOO_MANY)
                 return srm::set_error(SRM_ENOMEM, "the q-gram lists of %u reads hold more than %llu "
                                       "positions; split the call", n, (unsigned long long)MAX_FLAT);
         return SRM_OK;
