@@ -261,7 +261,9 @@ typedef struct srm_tuning {
                                walk recomputes each 32-column segment from it */
 } srm_tuning;
 int srm_ctx_set_tuning(srm_ctx *ctx, const srm_tuning *tuning);   /* NULL = defaults */
-/* after an eager srm_job_run: grid, tiles and event time (ms) of band class nw */
+/* after an eager srm_job_run: grid, tiles and event time (ms) of band class nw.  Where the
+ * classes run in one launch (class_streams), its part of that grid, a block of one wave
+ * per tile, and the whole launch's time: the classes' run side by side in it */
 int srm_job_band_info(srm_job *job, int nw, int *blocks, int *ntiles, float *ms);
 /* resident 256-thread blocks per CU of the banded kernel for class nw */
 int srm_band_occupancy(int nw, int unit);
@@ -299,7 +301,8 @@ int srm_job_download(srm_job *job, srm_result *res, uint32_t *ops, size_t n_ops_
 /* device time (ms) of the last srm_job_run, measured with HIP events on the job's stream */
 float srm_job_last_ms(srm_job *job);
 /* device time (ms) of the last eager run by stage: kind 0 = banded, 1 = plain,
- * 2 = records (srm_job_set_records) */
+ * 2 = records (srm_job_set_records).  The plain kernels of candidates that the band does
+ * not take run beside the band's (unless class_streams is 1): the two times then overlap */
 float srm_job_kernel_ms(srm_job *job, int kind);
 /* capture srm_job_run(job, kernel) into a hipGraph and replay it; 0 = plain launches */
 int srm_job_use_graph(srm_job *job, int enable);

@@ -196,10 +196,11 @@ struct srm_job {
     bool unit = true;
     bool one_launch = false;         // every class in one launch (set at the upload)
     bool beside = false;             // the plain kernels on rest_st beside the band's (likewise)
+    bool ran_beside = false;         // and whether the last run's did
     char *stage = nullptr;           // JOB_STAGE bytes of page-locked memory (Staged)
     uint64_t *back = nullptr;        // behind them two words that sizes come back to
     hipStream_t rest_st = nullptr;
-    hipEvent_t rest_ev = nullptr;
+    hipEvent_t rest_ev = nullptr;    // their end (they start with the run)
     bool resident_genome = false;
     // device buffers
     DevBuf d_cand, d_read_words, d_win_words, d_read_bytes, d_win_bytes;
@@ -498,6 +499,7 @@ int run_launches(srm_job *j, int kernel, bool timed)
             }
     }
     if (timed) HIP_TRY(hipEventRecord(j->ev[1], st));
+    j->ran_beside = beside;
     if (beside) HIP_TRY(hipStreamWaitEvent(st, j->rest_ev, 0));
     else if ((rc = the_rest(st))) return rc;
     if (timed) HIP_TRY(hipEventRecord(j->ev[2], st));
@@ -1121,7 +1123,7 @@ int srm_job_band_info(srm_job *j, int nw, int *blocks, int *ntiles, float *ms)
     *ms = j->class_ms[nw];
     for (const auto &bc : j->classes)
         if (bc.nw == nw) {   // the two halves of a class split by read length add up
-            *blocks += bc.blocks;
+            *blocks += j->one_launch ? (int)bc.ntiles : bc.blocks;
             *ntiles += (int)bc.ntiles;
         }
     return SRM_OK;
@@ -1369,7 +1371,7 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
     j->beside = concurrent && j->n_band > 0 && j->n_rest + j->n_bytes > 0;
     if (j->beside && !j->rest_st) {
         HIP_TRY(hipStreamCreateWithFlags(&j->rest_st, hipStreamNonBlocking));
-        HIP_TRY(hipEventCreateWithFlags(&j->rest_ev, hipEventDisableTiming));
+        HIP_TRY(hipEventCreate(&j->rest_ev));
     }
     // ---- device buffers
     if (n < PLAN_DEVICE_MIN && (rc = upload(ctx, j->d_read_words, read_words, n_read_words))) return rc;
@@ -1488,7 +1490,8 @@ int srm_job_run(srm_job *j, int kernel)
     HIP_TRY(hipEventSynchronize(j->ev[3]));
     HIP_TRY(hipEventElapsedTime(&j->last_ms, j->ev[0], j->ev[3]));
     HIP_TRY(hipEventElapsedTime(&j->band_ms, j->ev[0], j->ev[1]));
-    HIP_TRY(hipEventElapsedTime(&j->plain_ms, j->ev[1], j->ev[2]));
+    HIP_TRY(hipEventElapsedTime(&j->plain_ms, j->ev[j->ran_beside ? 0 : 1],
+                                j->ran_beside ? j->rest_ev : j->ev[2]));
     HIP_TRY(hipEventElapsedTime(&j->rec_ms, j->ev[2], j->ev[3]));
     for (auto &x : j->class_ms) x = 0.f;
     if (kernel != SRM_KERNEL_PLAIN)   // the class events are recorded only with band launches
