@@ -241,20 +241,23 @@ int srm_ctx_borrow_genome(srm_ctx *dst, const srm_ctx *src);
  * blocks_per_cu[nw]: persistent 256-thread blocks per CU for band class nw
  * (8*nw band cells per lane) of the nibble kernels, 0 = as many as stay resident;
  * merge_below: band classes narrower than this run on the kernel of this class
- * (fewer launches).  The tile shape of the unit-cost kernels: tile_cands
- * candidates per wave's tile (32 or 64), block_waves waves per block (1, 2 or 4),
- * split_len: each band class splits into reads shorter than split_len and the
- * rest (two launches, each with its own LDS staging size).  walk_layout: what
- * the unit-cost forward pass leaves for the walk (1 cuts its HBM traffic; the
- * walk then does the segment's bit-parallel steps again).
+ * (fewer classes).  class_streams: the classes one after another, or side by side: in
+ * one launch for unit costs, and for others while all tiles run at once; beyond that on
+ * streams.  tile_cands: candidates per wave's tile (32 or 64).  split_len: each band
+ * class splits into reads shorter than split_len and the rest, so that a tile holds one
+ * kind (classes one after another: two launches, each with its own LDS staging size).
+ * block_waves: waves per block of the unit-cost kernels where the classes run one after
+ * another (the one launch has blocks of one wave).  walk_layout: what the unit-cost
+ * forward pass leaves for the walk (1 cuts its HBM traffic; the walk then does the
+ * segment's bit-parallel steps again).
  */
 typedef struct srm_tuning {
     int blocks_per_cu[9];   /* by band class (8 diagonals per unit); 0 = as many as fit */
     int merge_below;        /* classes below this one run with it (0/1 = none) */
-    int class_streams;      /* streams the band classes run on side by side (up to 8);
-                               0 = default (4), 1 = one after another */
+    int class_streams;      /* 1 = the band classes one after another; else (up to 8, 0 =
+                               4) side by side: in one launch, or on so many streams */
     int tile_cands;         /* candidates per tile: 0 = 64, or 32 */
-    int block_waves;        /* waves per block of the unit-cost kernels: 0 = 4, or 1, 2 */
+    int block_waves;        /* with class_streams 1, unit costs: waves per block, 0 = 4, or 1, 2 */
     int split_len;          /* 0 = no split; else the read length that splits each class */
     int walk_layout;        /* unit costs: 0 = the forward pass stores the D bits the walk
                                reads; 1 = it stores the state of every 32nd column and the

@@ -1,16 +1,18 @@
 """Autotuner for the banded kernels' launch shape on this GPU.
 
 Unit costs (match 0 / mismatch 1, every SARUMAN run): the tile shape and the
-launch order of the bit-parallel kernels, by coordinate descent over
-  class_streams   band classes side by side on 1, 2, 4 or 8 streams
-  block_waves     waves per block (1, 2, 4; one wave per tile)
+launch of the bit-parallel kernels, by coordinate descent over
+  class_streams   every band class in one launch (0), or one after another (1)
+  block_waves     waves per block of the classes one after another (4, 2, 1; the one
+                  launch has blocks of one wave)
   tile_cands      candidates per tile (64, or 32 with half the lanes idle)
   split_len       each band class split by read length at a quartile of the
-                  batch's lengths (two launches, the short reads with less LDS)
-  merge_below     narrow classes run on a wider class's kernel (fewer launches)
+                  batch's lengths
+  merge_below     narrow classes run on a wider class's kernel
   walk_layout     the forward pass stores the D bits for the walk (0), or every
                   32nd column's state from which the walk recomputes (1)
-each point timed as the median of whole band phases (HIP events).
+each point timed as the median of whole band phases (HIP events); a value takes the
+place of another if it is 5% faster (one point measured again differs by up to 4%).
 Other costs: the persistent nibble kernel with 1..max resident blocks per CU per
 band class, then merging and streams.  The result is kept only if it beats the
 default launch by 2% on a fresh measurement of both; the table -- with every
@@ -107,8 +109,8 @@ def _search_unit(ctx, job, upload, reps, log, lengths):
     """Coordinate descent over the unit-cost launch knobs; returns (best table,
     every point measured)."""
     q = [int(x) for x in np.quantile(lengths, (0.25, 0.5, 0.75))] if len(lengths) else []
-    space = [("walk_layout", [0, 1]), ("class_streams", [4, 1, 2, 8]), ("block_waves", [4, 2, 1]),
-             ("tile_cands", [64, 32]), ("split_len", [0] + sorted(set(q))),
+    space = [("walk_layout", [0, 1]), ("class_streams", [0, 1]), ("block_waves", [0, 2, 1]),
+             ("tile_cands", [0, 32]), ("split_len", [0] + sorted(set(q))),
              ("merge_below", [0, 2, 3])]
     best = defaults()
     points = []
@@ -126,11 +128,11 @@ def _search_unit(ctx, job, upload, reps, log, lengths):
         changed = False
         for knob, values in space:
             for v in values:
-                if v == best[knob] or (knob == "class_streams" and v == 4 and best[knob] == 0):
+                if v == best[knob] or (knob == "block_waves" and best["class_streams"] != 1):
                     continue
                 t = {**best, knob: v}
                 ms = measure(t)
-                if ms < best_ms:
+                if ms < 0.95 * best_ms:
                     best, best_ms, changed = t, ms, True
         if not changed:
             break
