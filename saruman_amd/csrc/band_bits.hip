@@ -904,7 +904,7 @@ __device__ __forceinline__ void trace_tile(const BandArgs &a, uint32_t tile)
 // (5: 2-7 of them spilled; 4: 1.01 instead of 0.97 ms for the step above; 6: 17-24)
 template <int NW, bool CK>
 struct TraceWaves {
-    static constexpr int value = CK ? (NW <= 4 ? 5 : 5) : (NW <= 4 ? 8 : 7);
+    static constexpr int value = CK ? 5 : NW <= 4 ? 8 : 7;
 };
 
 template <int NW, bool CK>
@@ -931,9 +931,10 @@ __host__ __device__ constexpr int bits_stage_words(int maxL) { return maxL <= 32
 // Two launches per class one after another took the sum of the classes' longest
 // chains and left the chip to the last tiles of each: 14 launches, 480 us, for the
 // 53,000 candidates of 60,000 reads of 50-250 bp.  60,000 such reads through
-// srm_align_static: 985 -> 590 us; a batch of 50,000 with its upload and records 2.35
-// -> 2.07 ms; 1.77M candidates, where the classes ran on four streams: 0.98 -> 0.95 ms
-// with their results' copy.  So it runs at every size.  Occupancy: 5 waves per SIMD
+// srm_align_static, the host's plan included: 985 -> 554 us (185 with the plan on the
+// device); a batch of 50,000 with its upload and records 2.35 -> 2.07 ms; 1.77M
+// candidates, where the classes ran on four streams: 0.98 -> 0.90-0.95 ms with their
+// results' copy.  So it runs at every size.  Occupancy: 5 waves per SIMD
 // with the checkpoint layout (4: 0.96 ms, with few registers spilled at 5 and hundreds
 // at 6), 6 with stored D bits.
 template <bool CK>

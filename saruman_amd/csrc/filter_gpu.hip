@@ -58,7 +58,7 @@ namespace {
 constexpr int FB = 256;      // threads per block
 constexpr int ECAP = 16;     // result-hash entries per read kept in LDS
 constexpr int PCAP = 4;      // perfect hits per read kept in LDS
-constexpr int PB = 64;       // threads per block of the pairing pass
+constexpr int PB = 64;       // threads per block of the pairing pass (one wave: pair_list)
 // reads per block of it with G lanes a read: half as many again as it takes at a time,
 // since about half are dropped; one each where a read may take long
 constexpr int pair_reads(int G) { return G == 8 ? PB / G * 3 / 2 : PB / G; }
@@ -459,9 +459,6 @@ struct PairRead {
 // the others, half of the reads on either strand
 __device__ __forceinline__ uint32_t pair_list(const FArgs &a, PairRead *list, uint32_t per)
 {
-    __shared__ uint32_t s_n;
-    if (PB > 64 && threadIdx.x == 0) s_n = 0;
-    if (PB > 64) __syncthreads();
     const uint32_t at = blockIdx.x * per + threadIdx.x;
     PairRead R;
     bool some = false;
@@ -485,15 +482,9 @@ __device__ __forceinline__ uint32_t pair_list(const FArgs &a, PairRead *list, ui
         }
     }
     const uint64_t m = __ballot(some);
-    const int lane = threadIdx.x & 63;
-    uint32_t n = (uint32_t)__popcll(m), first = 0;
-    if (PB > 64) {
-        if (lane == 0) first = atomicAdd(&s_n, n);
-        first = (uint32_t)__shfl((int)first, 0, 64);
-    }
-    if (some) list[first + (uint32_t)__popcll(m & ((1ull << lane) - 1))] = R;
+    if (some) list[__popcll(m & ((1ull << threadIdx.x) - 1))] = R;
     __syncthreads();
-    return PB > 64 ? s_n : n;
+    return (uint32_t)__popcll(m);
 }
 
 // run_seashore (hash.c:502-834) by G lanes per read: each lane takes a start
@@ -1666,7 +1657,7 @@ int run_device(srm_dfilter *G, const uint8_t *blocked, const char *reads,
     c.n = strands == 3 ? 2 : 1;
     c.s[0].f = a;
     c.s[0].f.dr = strands == 2 ? 4 : 0;
-    // in pieces where the reads make two or more
+    // in pieces of 65,536 reads and more; half a piece's worth is one piece
     if (n_reads > PIECE / 4) {
         bool counted = false;
         int rc = upload_pieces(G, c, reads, read_off, read_len, read_k, n_reads, counted);

@@ -34,13 +34,13 @@ struct DQ {                  // one q's index on the device
 
 struct DParam {
     int L, k, q, rest, n, half, exact;
-    uint32_t gram_off;       // into FArgs::gram
+    uint32_t gram_off;       // into FArgs::gram (no kernel reads it: gram_offset)
 };
 
 struct FArgs {
     const DQ *qix;           // [32], indexed by q
     const DParam *par;
-    const uint16_t *gram;
+    const uint16_t *gram;    // for checks on the host, as rlen: the kernels take neither
     const char *genome;
     uint64_t glen;
     const char *reads;

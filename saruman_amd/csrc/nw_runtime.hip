@@ -454,7 +454,7 @@ int run_launches(srm_job *j, int kernel, bool timed)
         HIP_TRY(hipEventRecord(j->rest_ev, j->rest_st));
     }
     if (use_band && !j->classes.empty()) {
-        HIP_TRY(srm::launch_reset((uint32_t *)j->d_queue.p, (int)j->classes.size(), st));
+        if (!j->one_launch) HIP_TRY(srm::launch_reset((uint32_t *)j->d_queue.p, (int)j->classes.size(), st));
         if (j->one_launch) {   // widest band, the longest tiles, first
             srm::BitsSpans sp;
             for (size_t c = j->classes.size(); c-- > 0;) {
@@ -1343,8 +1343,8 @@ int srm_job_upload(srm_job *j, int match, int mismatch, const srm_cand *cand, in
     j->block_waves = ctx->tuning.block_waves ? ctx->tuning.block_waves : 4;
     j->walk_ck = ctx->tuning.walk_layout;
     // band classes run side by side unless the tuning says otherwise (1 = one after
-    // another on the context's stream): in one launch, or for other costs and many tiles
-    // on 4 streams or as many as it says
+    // another on the context's stream): in one launch, or for other costs and more tiles
+    // than run at once on 4 streams or as many as it says
     const int want_streams = ctx->tuning.class_streams == 0 ? 4 : ctx->tuning.class_streams;
     const bool concurrent = want_streams > 1;
     size_t ops_end = 0, scratch_words = 0;
