@@ -42,20 +42,18 @@ OPS_PER_BAND_CELL = 6       # compare + select (substitution), 3 adds, min3
 
 # Counters of one eager step of the exact configuration profiled (workload,
 # candidates, launch tuning and the sha256 prefix of the kernel sources), from
-# rocprofv3 --pmc runs with the kernels one after another:
-#   band_bytes      HBM bytes of the band phase (bits_band_kernel and
-#                   bits_trace_kernel of every class): FETCH_SIZE x2.000 + WRITE_SIZE
-#                   x1.000, the factors a 256 MiB copy kernel reads
-#   band_valu_busy  the band phase's VALU busy fraction, weighted by kernel time
-#                   (SQ_ACTIVE_INST_VALU / CUs / GRBM_GUI_ACTIVE per kernel)
+# rocprofv3 --pmc runs:
+#   band_bytes      HBM bytes of the band phase (bits_all_kernel): FETCH_SIZE x2.000 +
+#                   WRITE_SIZE x1.000, the factors a 256 MiB copy kernel reads
+#   band_valu_busy  its VALU busy fraction (SQ_ACTIVE_INST_VALU / CUs / GRBM_GUI_ACTIVE)
 #   records_bytes   HBM bytes of the record kernels (rec_measure, rec_write_lines,
 #                   rec_write)
-# Source: profiles/bits_band_and_trace_kernels_mixed_2M_reads.md
+# Source: profiles/bits_all_kernel_mixed_2M_reads.md, profiles/record_writer_mixed_2M_reads.md
 PMC_PROFILE = [
     {"workload": "mixed", "candidates": 1774238,
-     "tuning": {"blocks_per_cu": [0, 0, 0, 0, 0, 0, 0, 0, 0], "merge_below": 2, "class_streams": 0, "tile_cands": 64, "block_waves": 1, "split_len": 0, "walk_layout": 1},
-     "kernel_sha": "05feeb9780ba", "band_bytes": 1515472944, "band_valu_busy": 0.544,
-     "records_bytes": 1501263977},
+     "tuning": {"blocks_per_cu": [0, 0, 0, 0, 0, 0, 0, 0, 0], "merge_below": 0, "class_streams": 0, "tile_cands": 0, "block_waves": 0, "split_len": 0, "walk_layout": 1},
+     "kernel_sha": "3a7f43c03a5e", "band_bytes": 1762142027, "band_valu_busy": 0.915,
+     "records_bytes": 1501308186},
 ]
 
 
@@ -551,7 +549,7 @@ def main():
         "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_INT32_TOPS,
                      "unit": "TOP/s", "frac": achieved / PEAK_INT32_TOPS,
                      "traffic": band_bytes,
-                     "kernel": "bits_band_kernel + bits_trace_kernel of every band class of one "
+                     "kernel": "bits_all_kernel, every band class's forward pass and walk of one "
                                "step (HIP events around the band phase); the dominant stage",
                      "work": "6 int32 ops per band cell of the cell-wise recurrence; the "
                              "bit-parallel kernels evaluate 32 cells per lane-op, so frac can "

@@ -468,7 +468,8 @@ void srm_filter_destroy(srm_filter *f);
  * reads, builds the position lists, pairs them on the device and returns the
  * same srm_filter (candidates, batch boundaries, perfect hits) as
  * srm_filter_run on the same arguments.  Runs on ctx's stream; not thread-safe
- * per object.
+ * per object.  A strand whose position lists hold more than 2^32 - 256 elements,
+ * terminators included, is refused with SRM_ENOMEM: split the call.
  */
 typedef struct srm_dfilter srm_dfilter;
 int srm_dfilter_create(srm_ctx *ctx, const srm_index *index, const char *genome, size_t glen,

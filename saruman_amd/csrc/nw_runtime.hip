@@ -900,12 +900,13 @@ int plan_host(srm_job *j, const srm::PlanIn &in, const srm_cand *cand, int n, si
     return SRM_OK;
 }
 
-// The same on the device (plan_gpu.hip): the descriptors go up, are checked, counted and put in tile order there, and the host makes the tiles from the
-// counts.  The host's plan of a million candidates read and wrote them five times on
-// up to 8 threads, before the first copy began: a batch of 1,000,000 reads host to host
-// 11.3 -> 7.6 ms, one of 50,000 2.1 -> 1.67 ms.  The plan's scratch is the results'
-// buffer, so the batch has to have as many as fill it (fewer: the host's plan takes
-// 0.1 ms and less).
+// The same on the device (plan_gpu.hip): the descriptors go up, are checked, counted and
+// put in tile order there, and the host makes the tiles from the counts.  The host's plan
+// of a million candidates read and wrote them five times on up to 8 threads, before the
+// first copy began: a batch of 1,000,000 reads host to host 11.3 -> 7.6 ms, one of 50,000
+// 2.1 -> 1.67 ms.  The plan's scratch is the results' buffer, so the batch has to have as
+// many as fill it.  (That is a matter of room, not where the two break even: srm_align_static,
+// with a scratch of its own, plans on the device from 4,096 candidates on.)
 constexpr int PLAN_DEVICE_MIN = 16384;
 static_assert(PLAN_DEVICE_MIN * sizeof(srm_result) >= srm::PLAN_SCRATCH, "the results' buffer holds it");
 
