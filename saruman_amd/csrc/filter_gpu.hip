@@ -1368,7 +1368,7 @@ int run_strands(srm_dfilter *G, Call c, bool counted, const uint8_t *blocked, co
     FL_RC(fetch());
     auto countable = [&]() -> int {
         for (int x = 0; x < c.n; ++x)
-            if (h[x].flat == TOO_MANY)
+            if (h[x].flat > MAX_FLAT)   // (or TOO_MANY)
                 return srm::set_error(SRM_ENOMEM, "the q-gram lists of %u reads hold more than %llu "
                                       "positions; split the call", n, (unsigned long long)MAX_FLAT);
         return SRM_OK;
